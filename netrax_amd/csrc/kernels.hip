@@ -1,14 +1,16 @@
 // HIP kernels of the network-likelihood engine (gfx950).
 //
 // Data layout in HBM (one engine):
-//   CLV arena   real [n_variants][n_sites_pad][C][S]  site-major, state innermost
+//   CLV arena   one row of S values per (variant, site, category): FP64 in
+//               state pairs (row_offset), FP32 4 states [n_sites_pad][C][4],
+//               FP32 20 states per 32-site tile (see the matrix-core kernels)
 //   scalers     int32 [n_variants][n_sites_pad]
-//   adjoints    real  [n_variants][n_sites_pad][C][S]
+//   adjoints    as the CLVs
 //   tips        uint8 (S <= 8) or uint32 (S = 20) state masks [n_tips][n_sites_pad]
 //   P, P', P''  real  [n_parts][n_edges][C][S][S]
 // Every site-parallel kernel works on tiles of TILE = 64 sites; a workgroup
 // holds TILE * C threads, thread = (site, rate category), so the C lanes of
-// a site are adjacent and a CLV row of a workgroup is one contiguous
+// a site are adjacent and a workgroup's CLV rows are one contiguous
 // TILE*C*S*sizeof(real) span.  Workgroup b of a launch over (tile, op)
 // handles tile b % n_tiles_grid of op b / n_tiles_grid; n_tiles_grid is a
 // multiple of 8, so a tile is always dispatched to the same XCD (round-robin
@@ -198,30 +200,43 @@ __host__ __device__ __forceinline__ size_t grad_index(int64_t block, int n_uses,
   return (static_cast<size_t>(block) * n_uses + g) * pw + w;
 }
 
+// FP64 rows (CLVs, adjoints, sumtables): one row of S states per (site,
+// category), stored as state pairs, each pair of the 64 rows a wave works on
+// contiguous, so a wave's 16-byte access is one span of 1 KiB:
+//   4 states   the 64 rows of a wave are 64 / C sites x C categories (lane =
+//              site C + category): [block of 64 rows][pair 2][row 64][2]
+//   20 states  a wave is one category of a 64-site tile (lane = site):
+//              [tile][category][pair 10][site 64][2]
+// A row kept whole (32 or 160 bytes) makes every access touch the lines of
+// all 64 rows and use 16 bytes of each; the vector-memory address unit was
+// the busiest unit of the 4-state reverse sweep that way (64 % on average, 89 %
+// on the fullest CUs), and a 20-state wave touched 64 lines per access.
+constexpr int PAIR_STRIDE = 128;  // doubles between a row's state pairs
+template <int S, int C>
+__device__ __forceinline__ size_t row_offset(int64_t site, int c) {
+  if constexpr (S == 4) {
+    const int64_t r = site * C + c;
+    return static_cast<size_t>((r >> 6) * (2 * PAIR_STRIDE) + (r & 63) * 2);
+  } else {
+    return static_cast<size_t>(((site >> 6) * C + c) * (S / 2 * PAIR_STRIDE) + (site & 63) * 2);
+  }
+}
+
 template <int S>
 __device__ __forceinline__ void load_clv(const double *__restrict__ p, double (&x)[S]) {
-  if constexpr (S == 4) {
-    const double2 a = reinterpret_cast<const double2 *>(p)[0];
-    const double2 b = reinterpret_cast<const double2 *>(p)[1];
-    x[0] = a.x;
-    x[1] = a.y;
-    x[2] = b.x;
-    x[3] = b.y;
-  } else {
 #pragma unroll
-    for (int i = 0; i < S; ++i) x[i] = p[i];
+  for (int i = 0; i < S / 2; ++i) {
+    const double2 v = *reinterpret_cast<const double2 *>(p + i * PAIR_STRIDE);
+    x[2 * i] = v.x;
+    x[2 * i + 1] = v.y;
   }
 }
 
 template <int S>
 __device__ __forceinline__ void store_clv(double *__restrict__ p, const double (&x)[S]) {
-  if constexpr (S == 4) {
-    reinterpret_cast<double2 *>(p)[0] = make_double2(x[0], x[1]);
-    reinterpret_cast<double2 *>(p)[1] = make_double2(x[2], x[3]);
-  } else {
 #pragma unroll
-    for (int i = 0; i < S; ++i) p[i] = x[i];
-  }
+  for (int i = 0; i < S / 2; ++i)
+    *reinterpret_cast<double2 *>(p + i * PAIR_STRIDE) = make_double2(x[2 * i], x[2 * i + 1]);
 }
 
 template <int S>
@@ -342,6 +357,7 @@ __device__ __forceinline__ void forward_ops(const DevOp *__restrict__ ops, int n
   const int c = threadIdx.x % C;
   const int64_t site = static_cast<int64_t>(tile) * TILE + threadIdx.x / C;
   const int64_t n = L.n_sites_pad;
+  const size_t slot = static_cast<size_t>(n) * (C * S), ro = row_offset<S, C>(site, c);
   {
     // load phase: raw values only (CLV rows, scaler words, tip masks), so no
     // load has to wait for the ones issued before it
@@ -357,7 +373,7 @@ __device__ __forceinline__ void forward_ops(const DevOp *__restrict__ ops, int n
           const DevOp op = ops[j];
           const int32_t kid = op.kid[k];
           if (k < op.nk && kid >= 0) {
-            load_clv<S>(clv + (static_cast<size_t>(kid) * n + site) * (C * S) + c * S, x[j][k]);
+            load_clv<S>(clv + static_cast<size_t>(kid) * slot + ro, x[j][k]);
             sk[j][k] = scl[static_cast<size_t>(kid) * n + site];
           }
         }
@@ -414,7 +430,7 @@ __device__ __forceinline__ void forward_ops(const DevOp *__restrict__ ops, int n
           for (int i = 0; i < S; ++i) v[i] *= SCALE_FACTOR;
           scj += 1;
         }
-        store_clv<S>(clv + (static_cast<size_t>(op.out) * n + site) * (C * S) + c * S, v);
+        store_clv<S>(clv + static_cast<size_t>(op.out) * slot + ro, v);
         if (c == 0) scl[static_cast<size_t>(op.out) * n + site] = scj;
       }
     }
@@ -481,14 +497,15 @@ __global__ void __launch_bounds__(TILE *C)
   const int64_t n = L.n_sites_pad;
   const size_t n_wt = static_cast<size_t>(L.n_tiles) * PW;
   const int wt = tile * PW + threadIdx.x / 64;
+  const size_t slot = static_cast<size_t>(n) * (C * S), ro = row_offset<S, C>(site, c);
   const double w = weights[site];
   // one root CLV per workgroup (grid tiles x roots): the roots' site sums
   // are independent, and a 2-D grid keeps every CU busy
   for (int rr = blockIdx.y; rr < min(n_root, static_cast<int>(blockIdx.y) + 1); ++rr) {
-    const int slot = root_slots[rr];
+    const int root = root_slots[rr];
     const int r = root_index ? root_index[rr] : rr;
     double x[S];
-    load_clv<S>(clv + (static_cast<size_t>(slot) * n + site) * (C * S) + c * S, x);
+    load_clv<S>(clv + static_cast<size_t>(root) * slot + ro, x);
     double t = 0.0;
 #pragma unroll
     for (int i = 0; i < S; ++i) t = fma(freqs[part * S + i], x[i], t);
@@ -497,7 +514,7 @@ __global__ void __launch_bounds__(TILE *C)
     if (seed && c == 0) seed[static_cast<size_t>(r) * n + site] = w != 0.0 ? w * (1.0 / C) / t : 0.0;
     double val = 0.0;
     if (c == 0 && w != 0.0)
-      val = w * (log(t) + scl[static_cast<size_t>(slot) * n + site] * LOG_SCALE_THRESHOLD);
+      val = w * (log(t) + scl[static_cast<size_t>(root) * n + site] * LOG_SCALE_THRESHOLD);
     val = wave_sum(val);
     if ((threadIdx.x & 63) == 0) partials[static_cast<size_t>(r) * n_wt + wt] = val;
   }
@@ -672,16 +689,16 @@ __device__ __forceinline__ void adjoint_inputs(const DevOp &op, int64_t site, in
                                                const double *__restrict__ seed, AdjIn<S> &in) {
   // loads only (defaults for absent inputs are applied at use), so that no
   // load waits for an earlier one
-  const size_t row = static_cast<size_t>(C * S);
+  const size_t slot = static_cast<size_t>(n) * (C * S), ro = row_offset<S, C>(site, c);
   in.kq = scl[static_cast<size_t>(op.out) * n + site];
   if (op.flags & OP_HAS_CONSUMERS)
-    load_clv<S>(adj + (static_cast<size_t>(op.out) * n + site) * row + c * S, in.a);
+    load_clv<S>(adj + static_cast<size_t>(op.out) * slot + ro, in.a);
   if (op.root >= 0) in.sd = seed[static_cast<size_t>(op.root) * n + site];
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
     const int32_t kid = op.kid[k];
     if (k < op.nk && kid >= 0) {
-      load_clv<S>(clv + (static_cast<size_t>(kid) * n + site) * row + c * S, in.x[k]);
+      load_clv<S>(clv + static_cast<size_t>(kid) * slot + ro, in.x[k]);
       in.sk[k] = scl[static_cast<size_t>(kid) * n + site];
     }
   }
@@ -721,7 +738,7 @@ __global__ void __launch_bounds__(TILE *C, S == 4 ? 3 : 1)
   const int c = threadIdx.x % C;
   const int64_t site = static_cast<int64_t>(tile) * TILE + threadIdx.x / C;
   const int64_t n = L.n_sites_pad;
-  const size_t row = static_cast<size_t>(C * S);
+  const size_t slot = static_cast<size_t>(n) * (C * S), ro = row_offset<S, C>(site, c);
   const int wave = threadIdx.x / 64;
   const double *Qc = (S == 4 ? sQ : Qd + static_cast<size_t>(part) * C * S * S) + c * (S * S);
   // 4 states: r_c Q of this lane's category in registers (every op reads it;
@@ -836,7 +853,7 @@ __global__ void __launch_bounds__(TILE *C, S == 4 ? 3 : 1)
           if ((threadIdx.x & 63) == 0) grad_partials[grad_index(tile, n_uses, op.gslot[k], PW, wave)] = g[k];
           const int32_t kid = op.kid[k];
           if (kid >= 0) {
-            double *dst = adj + (static_cast<size_t>(kid) * n + site) * row + c * S;
+            double *dst = adj + static_cast<size_t>(kid) * slot + ro;
             if (!(op.flags & (k == 0 ? OP_FIRST_KID0 : OP_FIRST_KID1))) {
               double acc[S];
               load_clv<S>(dst, acc);
@@ -865,20 +882,6 @@ __global__ void __launch_bounds__(TILE *C, S == 4 ? 3 : 1)
 using cmat = const __attribute__((address_space(4))) double *;
 __device__ __forceinline__ cmat as_cmat(const double *p) { return (cmat)p; }
 
-__device__ __forceinline__ void load_row20(const double *__restrict__ p, double (&x)[20]) {
-#pragma unroll
-  for (int i = 0; i < 10; ++i) {
-    const double2 v = reinterpret_cast<const double2 *>(p)[i];
-    x[2 * i] = v.x;
-    x[2 * i + 1] = v.y;
-  }
-}
-
-__device__ __forceinline__ void store_row20(double *__restrict__ p, const double (&x)[20]) {
-#pragma unroll
-  for (int i = 0; i < 10; ++i) reinterpret_cast<double2 *>(p)[i] = make_double2(x[2 * i], x[2 * i + 1]);
-}
-
 // Workgroup (tile, op): the op's CLV rows of one 64-site tile, C waves.
 template <int C>
 __global__ void __launch_bounds__(TILE *C)
@@ -895,7 +898,7 @@ __global__ void __launch_bounds__(TILE *C)
   const int lane = threadIdx.x & 63;
   const int64_t site = static_cast<int64_t>(tile) * TILE + lane;
   const int64_t n = L.n_sites_pad;
-  const size_t row = static_cast<size_t>(C * S);
+  const size_t slot = static_cast<size_t>(n) * (C * S), ro = row_offset<S, C>(site, c);
   // loads of both children first; the tip mask and the scaler are loaded
   // for every child (tip 0 and variant 0 stand in for the absent one): a
   // value loaded on one path only would be copied at the join, which waits
@@ -909,7 +912,7 @@ __global__ void __launch_bounds__(TILE *C)
     const int32_t kid = k < op.nk ? op.kid[k] : -1;
     tm[k] = tips[static_cast<size_t>(kid < 0 ? -kid - 1 : 0) * n + site];
     sk[k] = scl[static_cast<size_t>(kid < 0 ? 0 : kid) * n + site];
-    if (k < op.nk && kid >= 0) load_row20(clv + (static_cast<size_t>(kid) * n + site) * row + c * S, x[k]);
+    if (k < op.nk && kid >= 0) load_clv<S>(clv + static_cast<size_t>(kid) * slot + ro, x[k]);
   }
   __builtin_amdgcn_s_setprio(0);
   int sc = 0;
@@ -951,7 +954,7 @@ __global__ void __launch_bounds__(TILE *C)
     for (int i = 0; i < S; ++i) v[i] *= SCALE_FACTOR;
     sc += 1;
   }
-  store_row20(clv + (static_cast<size_t>(op.out) * n + site) * row + c * S, v);
+  store_clv<S>(clv + static_cast<size_t>(op.out) * slot + ro, v);
   if (c == 0) scl[static_cast<size_t>(op.out) * n + site] = sc;
 }
 
@@ -977,7 +980,7 @@ __global__ void __launch_bounds__(TILE *C)
   const int lane = threadIdx.x & 63;
   const int64_t site = static_cast<int64_t>(tile) * TILE + lane;
   const int64_t n = L.n_sites_pad;
-  const size_t row = static_cast<size_t>(C * S);
+  const size_t slot = static_cast<size_t>(n) * (C * S), ro = row_offset<S, C>(site, c);
   const double *Qc = Qd + (static_cast<size_t>(part) * C + c) * (S * S);
   // one op of the run (whose ops share no child) per workgroup
   ops += blockIdx.y;
@@ -990,7 +993,7 @@ __global__ void __launch_bounds__(TILE *C)
     // loaded register and waits for the loads issued before it
     double araw[S], x[2][S];
     __builtin_amdgcn_s_setprio(1);  // see the note at wait_loads
-    load_row20(adj + (static_cast<size_t>(op.out) * n + site) * row + c * S, araw);
+    load_clv<S>(adj + static_cast<size_t>(op.out) * slot + ro, araw);
     const int kq = scl[static_cast<size_t>(op.out) * n + site];
     const double sd = seed[static_cast<size_t>(op.root >= 0 ? op.root : 0) * n + site];
     uint32_t tm[2];
@@ -1000,7 +1003,7 @@ __global__ void __launch_bounds__(TILE *C)
       const int32_t kid = k < op.nk ? op.kid[k] : -1;
       tm[k] = tips[static_cast<size_t>(kid < 0 ? -kid - 1 : 0) * n + site];
       sk[k] = scl[static_cast<size_t>(kid < 0 ? 0 : kid) * n + site];
-      if (k < op.nk && kid >= 0) load_row20(clv + (static_cast<size_t>(kid) * n + site) * row + c * S, x[k]);
+      if (k < op.nk && kid >= 0) load_clv<S>(clv + static_cast<size_t>(kid) * slot + ro, x[k]);
     }
     __builtin_amdgcn_s_setprio(0);
     const bool has_adj = (op.flags & OP_HAS_CONSUMERS) != 0;
@@ -1069,14 +1072,14 @@ __global__ void __launch_bounds__(TILE *C)
       const double g = wave_sum(gk);
       if (lane == 0) grad_partials[grad_index(tile, n_uses, op.gslot[k], PW, c)] = g;
       if (kid >= 0) {
-        double *dst = adj + (static_cast<size_t>(kid) * n + site) * row + c * S;
+        double *dst = adj + static_cast<size_t>(kid) * slot + ro;
         if (!(op.flags & (k == 0 ? OP_FIRST_KID0 : OP_FIRST_KID1))) {
           double acc[S];
-          load_row20(dst, acc);
+          load_clv<S>(dst, acc);
 #pragma unroll
           for (int i = 0; i < S; ++i) back[i] += acc[i];
         }
-        store_row20(dst, back);
+        store_clv<S>(dst, back);
       }
     }
   }
@@ -1107,7 +1110,7 @@ __global__ void __launch_bounds__(TILE *C)
   const int t0 = tb + (te - tb) * slice / n_split, t1 = tb + (te - tb) * (slice + 1) / n_split;
   const int c = threadIdx.x % C;
   const int64_t n = L.n_sites_pad;
-  const size_t row = static_cast<size_t>(C * S);
+  const size_t slot = static_cast<size_t>(n) * (C * S);
   const double *Pk[2];
 #pragma unroll
   for (int k = 0; k < 2; ++k)
@@ -1120,18 +1123,19 @@ __global__ void __launch_bounds__(TILE *C)
   const double bt = op.root >= 0 ? beta[part * n_root + op.root] : 0.0;
   for (int tile = t0; tile < t1; ++tile) {
     const int64_t site = static_cast<int64_t>(tile) * TILE + threadIdx.x / C;
+    const size_t ro = row_offset<S, C>(site, c);
     const double w = weights[site];
     double a[S], x[2][S], y[2][S];
 #pragma unroll
     for (int i = 0; i < S; ++i) a[i] = 0.0;
-    if (op.flags & OP_HAS_CONSUMERS) load_clv<S>(adj + (static_cast<size_t>(op.out) * n + site) * row + c * S, a);
+    if (op.flags & OP_HAS_CONSUMERS) load_clv<S>(adj + static_cast<size_t>(op.out) * slot + ro, a);
     int ks = 0;
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       if (k >= op.nk) continue;
       const int32_t kid = op.kid[k];
       if (kid >= 0) {
-        load_clv<S>(clv + (static_cast<size_t>(kid) * n + site) * row + c * S, x[k]);
+        load_clv<S>(clv + static_cast<size_t>(kid) * slot + ro, x[k]);
         ks += scl[static_cast<size_t>(kid) * n + site];
       } else {
         tip_vec<S>(tips[static_cast<size_t>(-kid - 1) * n + site], x[k]);
@@ -1142,7 +1146,7 @@ __global__ void __launch_bounds__(TILE *C)
       // seed beta w (1/C) pi_i / Ltilde of a displayed-tree root, and the
       // frequencies' direct share beta w (1/C) x_i / Ltilde
       double xr[S];
-      load_clv<S>(clv + (static_cast<size_t>(op.out) * n + site) * row + c * S, xr);
+      load_clv<S>(clv + static_cast<size_t>(op.out) * slot + ro, xr);
       double t = 0.0;
 #pragma unroll
       for (int i = 0; i < S; ++i) t = fma(freqs[part * S + i], xr[i], t);
@@ -2592,6 +2596,15 @@ __device__ __forceinline__ void stage_path_p(double *sPp, const PathStep *__rest
 // in for absent ones, so no load sits on one path of a branch) is issued
 // before its arithmetic, which then only waits on LDS and registers.  A
 // step's own scaler is the previous step's child scaler.
+// a thread's row in a CLV slot of either form (FP32 rows are kept whole)
+template <int S, int C, typename T>
+__device__ __forceinline__ size_t clv_row(int64_t site, int c) {
+  if constexpr (std::is_same<T, double>::value)
+    return row_offset<S, C>(site, c);
+  else
+    return static_cast<size_t>(site * C + c) * S;
+}
+
 template <int S, int C, typename T>
 __device__ __forceinline__ void path_sumtable(const PathStep *__restrict__ steps, int b0, int b1,
                                               const double *sPp, int n_staged, const DevLayout &L,
@@ -2604,7 +2617,7 @@ __device__ __forceinline__ void path_sumtable(const PathStep *__restrict__ steps
   using TT = typename TipType<S>::type;
   constexpr int PB = S == 4 ? 4 : 1;
   const int64_t n = L.n_sites_pad;
-  const size_t row = static_cast<size_t>(C * S);
+  const size_t slot = static_cast<size_t>(n) * (C * S), ro = clv_row<S, C, T>(site, c);
   auto slot_of = [](int32_t x) { return x >= 0 ? x : 0; };
   auto tip_of = [](int32_t x) { return (x < 0 && x != NO_CHILD) ? -x - 1 : 0; };
   auto prow = [&](int j, int which, int edge) -> const double * {
@@ -2613,9 +2626,9 @@ __device__ __forceinline__ void path_sumtable(const PathStep *__restrict__ steps
   };
   const int32_t root = steps[b0].out, low = steps[b1 - 1].child;
   double xr[S], xc[S];
-  load_any<S>(clv + (static_cast<size_t>(root) * n + site) * row + c * S, xr);
+  load_any<S>(clv + static_cast<size_t>(root) * slot + ro, xr);
   int kq = scl[static_cast<size_t>(root) * n + site];
-  load_any<S>(clv + (static_cast<size_t>(slot_of(low)) * n + site) * row + c * S, xc);
+  load_any<S>(clv + static_cast<size_t>(slot_of(low)) * slot + ro, xc);
   const TT tmc = tips[static_cast<size_t>(tip_of(low)) * n + site];
   double a[S];
   {
@@ -2637,7 +2650,7 @@ __device__ __forceinline__ void path_sumtable(const PathStep *__restrict__ steps
         kc[u] = scl[static_cast<size_t>(slot_of(ps.child)) * n + site];
         ks[u] = scl[static_cast<size_t>(slot_of(ps.sib)) * n + site];
         tm[u] = tips[static_cast<size_t>(tip_of(ps.sib)) * n + site];
-        load_any<S>(clv + (static_cast<size_t>(slot_of(ps.sib)) * n + site) * row + c * S, xs[u]);
+        load_any<S>(clv + static_cast<size_t>(slot_of(ps.sib)) * slot + ro, xs[u]);
       }
     }
 #pragma unroll
@@ -2692,7 +2705,6 @@ __global__ void __launch_bounds__(TILE *C)
   const int part = tile_part[tile];
   const int c = threadIdx.x % C;
   const int64_t site = static_cast<int64_t>(tile) * TILE + threadIdx.x / C;
-  const size_t row = static_cast<size_t>(C * S);
   // one displayed tree's path per workgroup (grid tiles x paths): the path
   // walks are independent, and one per workgroup fills the GPU
   const int j = blockIdx.y;
@@ -2703,9 +2715,7 @@ __global__ void __launch_bounds__(TILE *C)
   double stv[S];
   path_sumtable<S, C, T>(steps, b0, b1, sPp, n_staged, L, part, site, c, clv, scl, scale_unit, tips, P, V, Vinv,
                          freqs, stv);
-  double *out = st + (static_cast<size_t>(j) * L.n_sites_pad + site) * row + c * S;
-#pragma unroll
-  for (int kk = 0; kk < S; ++kk) out[kk] = stv[kk];
+  store_clv<S>(st + static_cast<size_t>(j) * L.n_sites_pad * (C * S) + row_offset<S, C>(site, c), stv);
 }
 
 // Per displayed tree j and wave: sums over sites of w log rho(b),
@@ -2773,7 +2783,7 @@ __global__ void __launch_bounds__(TILE *C)
   const int c = threadIdx.x % C;
   const int64_t site = static_cast<int64_t>(tile) * TILE + threadIdx.x / C;
   const int64_t n = L.n_sites_pad;
-  const size_t row = static_cast<size_t>(C * S);
+  const size_t slot = static_cast<size_t>(n) * (C * S), ro = row_offset<S, C>(site, c);
   const size_t n_wt = static_cast<size_t>(L.n_tiles) * PW;
   const int wt = tile * PW + threadIdx.x / 64;
   const double w = weights[site];
@@ -2781,10 +2791,8 @@ __global__ void __launch_bounds__(TILE *C)
   stage_exps<S, C>(ev, rates, part, brlen, c, ex, lr);
   // one path per workgroup (grid tiles x paths)
   for (int j = blockIdx.y; j < min(n_paths, static_cast<int>(blockIdx.y) + 1); ++j) {
-    const double *in = st + (static_cast<size_t>(j) * n + site) * row + c * S;
     double stv[S], v[3];
-#pragma unroll
-    for (int k = 0; k < S; ++k) stv[k] = in[k];
+    load_clv<S>(st + static_cast<size_t>(j) * slot + ro, stv);
     sumtable_partials<S, C>(stv, ex, lr, w, c, v);
     if ((threadIdx.x & 63) == 0)
 #pragma unroll
@@ -2816,7 +2824,7 @@ __global__ void __launch_bounds__(TILE *C)
   const int c = threadIdx.x % C;
   const int64_t site = static_cast<int64_t>(tile) * TILE + threadIdx.x / C;
   const int64_t n = L.n_sites_pad;
-  const size_t row = static_cast<size_t>(C * S);
+  const size_t slot = static_cast<size_t>(n) * (C * S), ro = row_offset<S, C>(site, c);
   const size_t n_wt = static_cast<size_t>(L.n_tiles) * PW;
   const int wt = tile * PW + threadIdx.x / 64;
   const double w = weights[site];
@@ -2824,10 +2832,8 @@ __global__ void __launch_bounds__(TILE *C)
   stage_exps<S, C>(ev, rates, part, brlen, c, ex, lr);
   // one path per workgroup (grid tiles x the largest path count)
   for (int j = blockIdx.y; j < min(n_paths, static_cast<int>(blockIdx.y) + 1); ++j) {
-    const double *in = st + (static_cast<size_t>(j) * n + site) * row + c * S;
     double stv[S], v[3];
-#pragma unroll
-    for (int k = 0; k < S; ++k) stv[k] = in[k];
+    load_clv<S>(st + static_cast<size_t>(j) * slot + ro, stv);
     sumtable_partials<S, C>(stv, ex, lr, w, c, v);
     if ((threadIdx.x & 63) == 0)
 #pragma unroll
