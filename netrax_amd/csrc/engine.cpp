@@ -264,11 +264,46 @@ static void plan_budget(Engine &e) {
       }
     bp.seg_root_begin.push_back(static_cast<int>(bp.root_phys.size()));
   }
+  if (e.walks()) {
+    // a segment is a launch: a slot hands on only what it made itself
+    std::vector<DevOp> adj = ops;
+    for (int j = 0; j < bp.n_seg; ++j) {
+      const int b = bp.seg_chunk[j], n = bp.seg_chunk[j + 1] - b, r = bp.rec_begin[b];
+      assign_forward_slots(ops.data() + b, n, e.fwd_slots);
+      assign_forward_slots(rec.data() + r, bp.rec_begin[b + n] - r, e.fwd_slots);
+      assign_reverse_slots(adj.data() + b, n, e.adj_slots);
+    }
+    upload(e.d_ops_b_adj, adj, e.stream);
+  }
   upload(e.d_ops_b, ops, e.stream);
   upload(e.d_ops_rec, rec, e.stream);
   upload(e.d_root_phys, bp.root_phys, e.stream);
   upload(e.d_root_index, bp.root_index, e.stream);
   resize_rows(e, bp.n_phys);
+}
+
+// Granules and LDS slots per wave of the 4-state FP64 walks.  Four granules
+// share an op's fixed work best (41,345 patterns x 4 categories, gradient:
+// 0.66 ms, 0.92 with two, 1.00 with one); fewer once they would leave SIMDs
+// without a wave (8,719 patterns: 0.303 / 0.285 / 0.286 ms, 611 patterns, lnL:
+// 53.4 / 50.8 / 50.4 us).  As many slots as let the launch's waves, at most
+// three per SIMD, be resident together.
+static void choose_walk_shape(Engine &e) {
+  constexpr int CUS = 256, LDS_PER_CU = 160 * 1024, SIMDS = 4 * CUS;
+  const int64_t granules = e.L.n_sites_pad * e.C / 16;
+  const int least = e.C == 8 ? 2 : 1;
+  e.walk_nq = e.C == 8 ? 2 : 4;
+  while (e.walk_nq > least && granules / e.walk_nq < SIMDS) e.walk_nq /= 2;
+  e.rpw = TILE * e.C / (16 * e.walk_nq);
+  const int64_t waves = granules / e.walk_nq;
+  const int per_cu = static_cast<int>(std::min<int64_t>(12, (waves + CUS - 1) / CUS));
+  auto slots = [&](auto lds) {
+    int n = 2;
+    while (n < WALK_SLOTS && lds(e.walk_nq, n + 1) <= static_cast<size_t>(LDS_PER_CU / per_cu)) ++n;
+    return n;
+  };
+  e.fwd_slots = slots(forward_walk_lds);
+  e.adj_slots = slots(adjoint_walk_lds);
 }
 
 // Builds the level schedule, the batched order, root CLV set and gradient
@@ -321,11 +356,18 @@ static void build_schedule(Engine &e) {
     return op;
   };
 
-  // plain form: level chunks (one per pruning level), ops in slot order;
-  // the 4-state passes walk them in one launch, 20 states launch per level
+  // plain form: level chunks (one per pruning level), ops in slot order, one
+  // launch each; the 4-state walks take a depth-first order instead, each op
+  // a chunk
   e.ops_all.clear();
   e.chunks.clear();
-  for (int l = 1; l <= max_level; ++l) {
+  if (e.walks())
+    for (int s : depth_first_order(e.dag, e.root_slots)) {
+      const int i = static_cast<int>(e.ops_all.size());
+      e.ops_all.push_back(make_op(s));
+      e.chunks.push_back(LevelChunk{e.dag.var[s].level, i, i + 1});
+    }
+  for (int l = 1; l <= max_level && !e.walks(); ++l) {
     const auto &lv = e.level_ops[l];
     if (lv.empty()) continue;
     LevelChunk ch{};
@@ -402,10 +444,14 @@ static void build_schedule(Engine &e) {
     dc[k].use = e.class_use[k];
   }
   upload(e.d_ops, e.ops_all, e.stream);
-  {
-    std::vector<LevelChunk> walk(e.chunks.rbegin(), e.chunks.rend());
-    upload(e.d_adj_walk, walk, e.stream);
-    upload(e.d_fwd_walk, e.chunks, e.stream);
+  if (e.walks()) {
+    choose_walk_shape(e);
+    const int n_ops = static_cast<int>(e.ops_all.size());
+    e.ops_fwd = e.ops_adj = e.ops_all;
+    assign_forward_slots(e.ops_fwd.data(), n_ops, e.fwd_slots);
+    assign_reverse_slots(e.ops_adj.data(), n_ops, e.adj_slots);
+    upload(e.d_ops_fwd, e.ops_fwd, e.stream);
+    upload(e.d_ops_adj, e.ops_adj, e.stream);
   }
   upload(e.d_ops_dfs, e.ops_dfs, e.stream);
   upload(e.d_group_begin, e.group_begin, e.stream);
@@ -415,10 +461,13 @@ static void build_schedule(Engine &e) {
   upload(e.d_class_dlogprob, e.class_dlogprob, e.stream);
   std::vector<int32_t> rs(e.root_slots.begin(), e.root_slots.end());
   upload(e.d_root_slots, rs, e.stream);
-  // gradient partials per site block: plain form 64-site tiles of C waves;
-  // FP32 form its reverse-sweep workgroups (tune_tile sites of tune_lanes
+  // gradient partials per site block: plain form a wave of the walks (4
+  // states) or 64-site tiles of C waves; FP32 form its reverse-sweep workgroups (tune_tile sites of tune_lanes
   // lanes per row, or 32 sites for 20-state data)
-  if (e.opt.precision != NRX_FP32) {
+  if (e.walks()) {
+    e.gpw = 1;
+    e.gbpt = e.rpw;
+  } else if (e.opt.precision != NRX_FP32) {
     e.gpw = TILE * e.C / 64;
     e.gbpt = 1;
   } else if (e.S == AA_STATES) {
@@ -428,8 +477,8 @@ static void build_schedule(Engine &e) {
     e.gpw = e.tune_tile * e.C * e.tune_lanes / 64;
     e.gbpt = TILE / e.tune_tile;
   }
-  if (e.gpw * e.gbpt < e.pw) throw std::logic_error("gradient partial layout does not cover the tile");
-  const size_t n_wt = static_cast<size_t>(e.L.n_tiles) * e.pw;
+  if (e.gpw * e.gbpt < e.rpw) throw std::logic_error("gradient partial layout does not cover the tile");
+  const size_t n_wt = static_cast<size_t>(e.L.n_tiles) * e.rpw;
   const size_t n_gwt = static_cast<size_t>(e.L.n_tiles) * e.gpw * e.gbpt;
   e.d_root_partials.alloc(sizeof(double) * std::max<size_t>(1, rs.size()) * n_wt);
   e.d_beta.alloc(sizeof(double) * std::max<size_t>(1, rs.size()) * e.P);
@@ -664,14 +713,13 @@ static void forward(Engine &e, bool incremental) {
       all = false;
       break;
     }
-  // 4 states: one launch walking the levels (a workgroup per tile); 20
+  // 4 states: one launch (a wave walks its sites through the ops); 20
   // states: one launch per level (one op per workgroup, so a level fills
   // the GPU)
-  const bool walk = e.S != AA_STATES;
   if (all) {
-    if (walk) {
+    if (e.walks()) {
       record_kernel_begin(e, 0);
-      launch_forward_walk(e, e.d_ops.as<DevOp>(), e.d_fwd_walk.as<LevelChunk>(), static_cast<int>(e.chunks.size()));
+      launch_forward_walk(e, e.d_ops_fwd.as<DevOp>(), static_cast<int>(e.ops_all.size()));
       record_kernel_end(e, 0);
     } else {
       for (const LevelChunk &ch : e.chunks) {
@@ -693,11 +741,11 @@ static void forward(Engine &e, bool incremental) {
       if (d.op_end > d.op_begin) lv.push_back(d);
     }
     if (!dirty.empty()) {
+      if (e.walks()) assign_forward_slots(dirty.data(), static_cast<int>(dirty.size()), e.fwd_slots);
       stage_upload(e, e.d_ops_dirty, dirty);
-      if (walk) {
-        stage_upload(e, e.d_dirty_walk, lv);
+      if (e.walks()) {
         record_kernel_begin(e, 0);
-        launch_forward_walk(e, e.d_ops_dirty.as<DevOp>(), e.d_dirty_walk.as<LevelChunk>(), static_cast<int>(lv.size()));
+        launch_forward_walk(e, e.d_ops_dirty.as<DevOp>(), static_cast<int>(dirty.size()));
         record_kernel_end(e, 0);
       } else {
         for (const LevelChunk &d : lv) {
@@ -746,10 +794,8 @@ static void fetch_results(Engine &e) {
 // Reverse sweep of level chunks c_hi down to c_lo (plain form).  20
 // states: one launch per run of ops without a common child, one op per
 // workgroup, so that a level fills the GPU.  4 states: one launch for all
-// of them, a workgroup per tile walking the levels and their ops in order
-// (the order the first-delivery flags were set in); per-level launches
-// cost a fixed time each against little work per op.
-static void adjoint_chunks(Engine &e, int c_hi, int c_lo, const DevOp *ops) {
+// of them.
+static void adjoint_chunks(Engine &e, int c_hi, int c_lo, const DevOp *ops, bool keep = false) {
   if (e.S == AA_STATES) {
     for (int c = c_hi; c >= c_lo; --c)
       for (int r = e.adj_run_begin[c]; r < e.adj_run_begin[c + 1]; ++r) {
@@ -759,7 +805,7 @@ static void adjoint_chunks(Engine &e, int c_hi, int c_lo, const DevOp *ops) {
       }
   } else if (c_hi >= c_lo) {
     record_kernel_begin(e, 1);
-    launch_adjoint_levels(e, ops, c_hi, c_lo);
+    launch_adjoint_walk(e, ops + e.chunks[c_lo].op_begin, e.chunks[c_hi].op_end - e.chunks[c_lo].op_begin, keep);
     record_kernel_end(e, 1);
   }
 }
@@ -770,6 +816,12 @@ static void budget_forward(Engine &e, bool gradient) {
   const auto &bp = e.bp;
   const DevOp *ops = e.d_ops_b.as<DevOp>();
   for (int j = 0; j < bp.n_seg; ++j) {
+    if (e.walks()) {
+      record_kernel_begin(e, 0);
+      launch_forward_walk(e, ops + bp.seg_chunk[j], bp.seg_chunk[j + 1] - bp.seg_chunk[j]);
+      record_kernel_end(e, 0);
+      continue;
+    }
     for (int c = bp.seg_chunk[j]; c < bp.seg_chunk[j + 1]; ++c) {
       const LevelChunk &ch = e.chunks[c];
       record_kernel_begin(e, 0);
@@ -783,9 +835,14 @@ static void budget_forward(Engine &e, bool gradient) {
 
 static void budget_adjoint(Engine &e) {
   const auto &bp = e.bp;
-  const DevOp *ops = e.d_ops_b.as<DevOp>(), *rec = e.d_ops_rec.as<DevOp>();
+  const DevOp *ops = (e.walks() ? e.d_ops_b_adj : e.d_ops_b).as<DevOp>(), *rec = e.d_ops_rec.as<DevOp>();
   for (int j = bp.n_seg - 1; j >= 0; --j) {
-    if (j < bp.n_seg - 1)  // the last segment's pool still holds its CLVs
+    const int c0 = bp.seg_chunk[j], c1 = bp.seg_chunk[j + 1];
+    if (e.walks() && j < bp.n_seg - 1 && bp.rec_begin[c1] > bp.rec_begin[c0]) {
+      record_kernel_begin(e, 0);
+      launch_forward_walk(e, rec + bp.rec_begin[c0], bp.rec_begin[c1] - bp.rec_begin[c0]);
+      record_kernel_end(e, 0);
+    } else if (!e.walks() && j < bp.n_seg - 1)  // the last segment's pool still holds its CLVs
       for (int c = bp.seg_chunk[j]; c < bp.seg_chunk[j + 1]; ++c) {
         const int n = bp.rec_begin[c + 1] - bp.rec_begin[c];
         if (n == 0) continue;
@@ -845,7 +902,10 @@ static int stage_invalid_ops(Engine &e, const NetDesc *&desc) {
 // `fetch` false: the results stay on the device (for a caller that reads
 // them there, such as the device Newton sweep) and no host wait is made;
 // the host copy is then stale, so the cache is marked invalid.
-static int evaluate(Engine &e, int variant, bool incremental, bool update_pm, bool gradient, bool fetch = true) {
+// `keep_adjoints`: the reverse sweep of the 4-state FP64 form leaves every
+// CLV's adjoint in HBM (the model gradient reads them).
+static int evaluate(Engine &e, int variant, bool incremental, bool update_pm, bool gradient, bool fetch = true,
+                    bool keep_adjoints = false) {
   check_ready(e);
   if (variant != NRX_AVERAGE_DISPLAYED_TREES && variant != NRX_BEST_DISPLAYED_TREE)
     throw std::invalid_argument("unknown likelihood variant");
@@ -917,7 +977,7 @@ static int evaluate(Engine &e, int variant, bool incremental, bool update_pm, bo
   } else if (e.bp.n_seg > 1) {
     // memory budget: segments forward, then the reverse sweep recomputing
     budget_forward(e, gradient);
-    launch_mixture(e, variant, e.pw);
+    launch_mixture(e, variant, e.rpw);
     if (gradient) {
       budget_adjoint(e);
       launch_grad_reduce(e);
@@ -925,11 +985,12 @@ static int evaluate(Engine &e, int variant, bool incremental, bool update_pm, bo
     std::fill(e.clv_dirty.begin(), e.clv_dirty.end(), 0);
   } else {
     forward(e, incremental);
-    launch_root_partials(e, gradient);
-    launch_mixture(e, variant, e.pw);
+    if (!e.walks()) launch_root_partials(e, gradient);
+    launch_mixture(e, variant, e.rpw);
     if (gradient) {
       e.d_adj.alloc(sizeof(double) * e.clv_elems_per_slot * e.dag.var.size());
-      adjoint_chunks(e, static_cast<int>(e.chunks.size()) - 1, 0, e.d_ops.as<DevOp>());
+      adjoint_chunks(e, static_cast<int>(e.chunks.size()) - 1, 0, (e.walks() ? e.d_ops_adj : e.d_ops).as<DevOp>(),
+                     keep_adjoints);
       launch_grad_reduce(e);
     }
   }
@@ -1455,6 +1516,7 @@ int nrx_create(const nrx_network_desc *net, const nrx_partition_desc *parts, int
     // site-sum partials per 64-site tile: one per wave (the 20-state FP32
     // form runs two 32-site workgroups of C waves per tile)
     e->pw = aa32 ? 2 * e->C : TILE * e->C / 64;
+    e->rpw = e->pw;
     e->parts.resize(n_parts);
     int64_t off = 0;
     int tile = 0;
@@ -1925,7 +1987,8 @@ int nrx_model_gradient(nrx_engine *eng, int32_t variant, double *total, double *
     if (e.opt.precision != NRX_FP64 || e.S != 4)
       return fail(NRX_ERR_UNSUPPORTED, "model gradients are provided for the FP64 form with 4-state data");
     require_resident(e);
-    const int rc = evaluate(e, variant, true, true, true);  // CLVs, adjoints, mixture weights
+    // CLVs, adjoints, mixture weights
+    const int rc = evaluate(e, variant, true, true, true, /*fetch=*/true, /*keep_adjoints=*/true);
     if (rc != NRX_OK) return rc;
     *total = e.cached_total;
     const int S = e.S, C = e.C, P = e.P, nr = S * (S - 1) / 2;
@@ -2258,11 +2321,15 @@ int nrx_get_stats(nrx_engine *eng, nrx_stats *out) {
     const double scl = 4.0 * sites;            // one scaler row
     const double tip_b = (e.S == 4 ? 1.0 : 4.0) * sites;
     double fwd_ops = 0.0;
-    for (const DevOp &op : e.ops_all) {
-      for (int k = 0; k < op.nk; ++k) fwd_ops += op.kid[k] >= 0 ? row + scl : tip_b;
+    for (const DevOp &op : e.walks() ? e.ops_fwd : e.ops_all) {
+      for (int k = 0; k < op.nk; ++k) {
+        if (e.walks() && (op.flags & (k == 0 ? OP_PASS_KID0 : OP_PASS_KID1))) continue;  // handed over in LDS
+        fwd_ops += op.kid[k] >= 0 ? row + scl : tip_b;
+      }
       fwd_ops += row + scl;  // parent CLV and scaler written
     }
-    const double root = e.root_slots.size() * (row + scl + 8.0 * sites);
+    // the walks form the root sums in place and write the seed factors
+    const double root = e.root_slots.size() * ((e.walks() ? 0.0 : row + scl) + 8.0 * sites);
     const double pm = static_cast<double>(e.P) * e.E * e.C * e.S * e.S * b;
     // push-form adjoint, over the op list and flags of the engine's form:
     // per op read its scaler, its adjoint (when accumulated) and its children
@@ -2274,13 +2341,14 @@ int nrx_get_stats(nrx_engine *eng, nrx_stats *out) {
     // 20-state FP32.
     const bool fp32 = e.opt.precision == NRX_FP32;
     const double aexp = fp32 ? (e.S == AA_STATES ? scl * e.C : scl) : 0.0;
-    const bool pass = fp32 && e.S == 4;
+    const bool pass = e.S == 4;
+    const std::vector<DevOp> &adj_ops = fp32 ? e.ops_dfs : e.walks() ? e.ops_adj : e.ops_all;
     out->n_lds_handoffs = 0;
     if (pass)
-      for (const DevOp &op : e.ops_dfs)
+      for (const DevOp &op : adj_ops)
         out->n_lds_handoffs += ((op.flags & OP_PASS_KID0) != 0) + ((op.flags & OP_PASS_KID1) != 0);
     double adj = 0.0;
-    for (const DevOp &op : fp32 ? e.ops_dfs : e.ops_all) {
+    for (const DevOp &op : adj_ops) {
       adj += scl;
       if ((op.flags & OP_HAS_CONSUMERS) && !(pass && (op.flags & OP_A_PASS))) adj += row + aexp;
       if (op.root >= 0) adj += fp32 ? row : 8.0 * sites;
@@ -2289,7 +2357,7 @@ int nrx_get_stats(nrx_engine *eng, nrx_stats *out) {
           adj += tip_b;
           continue;
         }
-        adj += row + scl;  // child CLV and scaler
+        adj += e.walks() ? row : row + scl;  // child CLV and scaler (the walks read only their own CLV's)
         if (pass && (op.flags & (k == 0 ? OP_PASS_KID0 : OP_PASS_KID1))) continue;
         adj += row + aexp;  // delivered adjoint
         if (!(op.flags & (k == 0 ? OP_FIRST_KID0 : OP_FIRST_KID1))) adj += row + aexp;

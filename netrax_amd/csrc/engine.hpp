@@ -102,20 +102,24 @@ constexpr int32_t OP_ACC_EARLY1 = 32;
 constexpr int32_t OP_PASS_KID0 = 64;
 constexpr int32_t OP_PASS_KID1 = 128;
 constexpr int32_t OP_A_PASS = 256;
+// FP64 form, 4 states: the op's own adjoint lies in HBM and the op before it
+// in the sweep delivered to it last, so it is read after that delivery
+// instead of one op ahead
+constexpr int32_t OP_A_LATE = 512;
+// FP64 form, 4 states: child k's adjoint lies in HBM and holds deliveries
+constexpr int32_t OP_ACC0 = 1024;
+constexpr int32_t OP_ACC1 = 2048;
+constexpr int WALK_SLOTS = 8;  // FP64 form: LDS slots of a wave, at most (3 bits per use)
 constexpr int PASS_SLOTS = 5;  // at most; fewer where LDS would cost residency
 constexpr int PASS_SHIFT = 12;  // slot of use u (0, 1: children, 2: own) in bits 12 + 3u
 constexpr int32_t PASS_BITS = 0x1FF << PASS_SHIFT;
 inline __host__ __device__ int pass_slot(int32_t flags, int u) { return (flags >> (PASS_SHIFT + 3 * u)) & 7; }
 
-// A launch of the plain form: the ops [op_begin, op_end) of one pruning
-// level.  The forward runs one workgroup per (tile, PLAIN_G consecutive
-// ops); the adjoint one workgroup per tile walking all ops in order.
+// Plain form: the ops [op_begin, op_end), one pruning level of 20-state data
+// (a launch), or one op of the 4-state walk (where a memory budget may cut it).
 struct LevelChunk {
   int level, op_begin, op_end;
 };
-constexpr int PLAIN_G = 4;  // forward ops per workgroup
-// adjoint: ops of a level whose P matrices are staged in LDS (48 KiB)
-constexpr int plain_staged_ops(int C) { return 49152 / (2 * C * 16 * 8); }
 
 // One step of a root-to-branch path: the op (its output slot), the child
 // the path continues into and the other child (NO_CHILD for a one-child
@@ -242,10 +246,14 @@ int adjoint_pass_slots(int C, int G, int TS, int H, int E, int64_t n_work);
 
 // Kernel launchers (kernels.hip)
 void launch_pmatrices(Engine &e);
+// 20 states: one level
 void launch_forward_level(Engine &e, const DevOp *ops, int n_ops, const LevelChunk &ch);
-// 4 states: the levels of `walk` (device array of op ranges into `ops`,
-// lowest level first) in one launch
-void launch_forward_walk(Engine &e, const DevOp *ops, const LevelChunk *walk, int n_walk);
+// 4 states: ops in an order with children first, with their LDS slots
+// assigned (assign_forward_slots); root site sums and seed factors included
+void launch_forward_walk(Engine &e, const DevOp *ops, int n_ops);
+// dynamic LDS of the walks' one-wave workgroups (nq granules per wave)
+size_t forward_walk_lds(int nq, int n_slots);
+size_t adjoint_walk_lds(int nq, int n_slots);
 void launch_root_partials(Engine &e, bool seeds);
 // root partials of n roots: physical rows `rows`, root indices `index`
 void launch_root_partials(Engine &e, bool seeds, const int32_t *rows, const int32_t *index, int n);
@@ -253,8 +261,9 @@ void launch_mixture(Engine &e, int variant, int partials_per_tile);
 // 20 states: one run of ops, taken from `ops` (same positions as in the
 // op list)
 void launch_adjoint_level(Engine &e, const LevelChunk &ch, const DevOp *ops);
-// 4 states: level chunks c_hi down to c_lo in one launch
-void launch_adjoint_levels(Engine &e, const DevOp *ops, int c_hi, int c_lo);
+// 4 states: the ops backwards (slots from assign_reverse_slots); keep: every
+// adjoint is also stored in HBM
+void launch_adjoint_walk(Engine &e, const DevOp *ops, int n_ops, bool keep);
 void launch_grad_reduce(Engine &e);
 // nets: a descriptor other than the engine's own (its invalid ops only)
 void launch_forward_persistent(Engine &e, const NetDesc *nets = nullptr);

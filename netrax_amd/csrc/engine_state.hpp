@@ -72,8 +72,10 @@ struct Engine : nrx_engine {
   std::vector<std::vector<int>> level_ops;  // variant slots per level (needed only)
   std::vector<int> root_slots;              // distinct displayed-tree-root CLVs
   std::vector<int> class_root_index;        // [nc]
-  // plain form: ops in level order, cut into launches with bounded LDS tables
-  std::vector<DevOp> ops_all;
+  // plain form: ops in level order (20 states; FP32 engines likewise), or in
+  // the depth-first order of the 4-state walks, with their LDS slots in the
+  // two lists the walks read
+  std::vector<DevOp> ops_all, ops_fwd, ops_adj;
   std::vector<LevelChunk> chunks;
   // plain form reverse sweep: runs of ops without a common child, per chunk
   std::vector<LevelChunk> adj_runs;
@@ -83,7 +85,10 @@ struct Engine : nrx_engine {
   std::vector<int32_t> group_begin;  // [n_groups + 1] into ops_dfs
   std::vector<int32_t> edge_use_begin, edge_use_list;  // gradient rows per edge
   int n_uses = 0;
-  int pw = 1;  // site-sum partials per tile (one per wave)
+  int pw = 1;   // site-sum partials per tile (one per wave)
+  int rpw = 1;  // root site-sum partials per tile
+  // FP64 form, 4 states: granules per wave of the walks and LDS slots per wave
+  int walk_nq = 4, fwd_slots = 2, adj_slots = 2;
   // gradient partials [site block][row][wave]: waves per block, blocks per tile
   int gpw = 1, gbpt = 1;
   // FP32 form shape (nrx_autotune / nrx_set_tuning): ops per group of the
@@ -123,7 +128,7 @@ struct Engine : nrx_engine {
     std::vector<int32_t> root_index;    // ... and their root indices
     std::vector<int> seg_root_begin;    // [n_seg + 1] ranges of the two above
   } bp;
-  DevBuf d_ops_b, d_ops_rec, d_root_phys, d_root_index;
+  DevBuf d_ops_b, d_ops_b_adj, d_ops_rec, d_root_phys, d_root_index;
   hipGraphExec_t nr_graph = nullptr;
   int nr_graph_key[4] = {-1, -1, -1, -1};  // variant, mode, max_iters, paths
   const void *nr_graph_bufs[3] = {nullptr, nullptr, nullptr};
@@ -150,9 +155,7 @@ struct Engine : nrx_engine {
   DevBuf d_clv, d_scl, d_adj, d_adj_exp, d_Qf;
   DevBuf d_Pa;  // 20-state FP32 form: matrix-core operand tables
   DevBuf d_ops, d_ops_dirty, d_Qd;
-  DevBuf d_adj_walk;  // the level chunks top level first (the reverse sweep's walk)
-  DevBuf d_fwd_walk;  // the level chunks lowest level first (the forward pass's walk)
-  DevBuf d_dirty_walk;  // op ranges of d_ops_dirty per level (incremental forward)
+  DevBuf d_ops_fwd, d_ops_adj;  // 4 states: the walks' op lists
   // FP32 form, incremental evaluation: the invalid ops, their groups and
   // their descriptor
   DevBuf d_ops_inc, d_group_begin_inc, d_netdesc_inc;
@@ -179,6 +182,8 @@ struct Engine : nrx_engine {
   std::vector<hipEvent_t> ev_k[2];
   int n_k[2] = {0, 0};
   nrx_timing last_timing{};
+
+  bool walks() const { return S == 4 && opt.precision == NRX_FP64; }
 
   ~Engine();
 };

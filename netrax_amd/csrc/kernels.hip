@@ -1,20 +1,18 @@
 // HIP kernels of the network-likelihood engine (gfx950).
 //
 // Data layout in HBM (one engine):
-//   CLV arena   one row of S values per (variant, site, category): FP64 in
-//               state pairs (row_offset), FP32 4 states [n_sites_pad][C][4],
+//   CLV arena   one row of S values per (variant, site, category): FP64 in the
+//               order of row_offset, FP32 4 states [n_sites_pad][C][4],
 //               FP32 20 states per 32-site tile (see the matrix-core kernels)
 //   scalers     int32 [n_variants][n_sites_pad]
 //   adjoints    as the CLVs
 //   tips        uint8 (S <= 8) or uint32 (S = 20) state masks [n_tips][n_sites_pad]
 //   P, P', P''  real  [n_parts][n_edges][C][S][S]
-// Every site-parallel kernel works on tiles of TILE = 64 sites; a workgroup
-// holds TILE * C threads, thread = (site, rate category), so the C lanes of
-// a site are adjacent and a workgroup's CLV rows are one contiguous
-// TILE*C*S*sizeof(real) span.  Workgroup b of a launch over (tile, op)
-// handles tile b % n_tiles_grid of op b / n_tiles_grid; n_tiles_grid is a
-// multiple of 8, so a tile is always dispatched to the same XCD (round-robin
-// over workgroup ids) and its children's CLVs stay in that XCD's L2.
+// The FP64 kernels of 20 states and the path kernels work on tiles of TILE =
+// 64 sites with TILE * C threads; the 20-state launches cover (tile, op) with
+// the tile count rounded up to a multiple of 8, so a tile always goes to the
+// same XCD (round-robin over workgroup ids) and its children's CLVs stay in
+// that XCD's L2.
 #include <cfloat>
 #include <cmath>
 #include <map>
@@ -200,20 +198,22 @@ __host__ __device__ __forceinline__ size_t grad_index(int64_t block, int n_uses,
   return (static_cast<size_t>(block) * n_uses + g) * pw + w;
 }
 
-// FP64 rows (CLVs, adjoints, sumtables): one row of S states per (site,
-// category), stored as state pairs, each pair of the 64 rows a wave works on
-// contiguous, so a wave's 16-byte access is one span of 1 KiB:
-//   4 states   the 64 rows of a wave are 64 / C sites x C categories (lane =
-//              site C + category): [block of 64 rows][pair 2][row 64][2]
-//   20 states  a wave is one category of a 64-site tile (lane = site):
-//              [tile][category][pair 10][site 64][2]
-// A row kept whole (32 or 160 bytes) makes every access touch the lines of
-// all 64 rows and use 16 bytes of each; the vector-memory address unit was
-// the busiest unit of the 4-state reverse sweep that way (64 % on average, 89 %
-// on the fullest CUs), and a 20-state wave touched 64 lines per access.
+// FP64 rows: S states of one (site, category).
+//   20 states  state pairs, each pair of a wave's 64 sites contiguous (a wave
+//              is one category of a 64-site tile, lane = site):
+//              [tile][category][pair 10][site 64][2], so a wave's 16-byte
+//              access is one span of 1 KiB
+//   4 states   granules of 64 doubles in the lane order of the matrix
+//              instruction (see k_forward_walk): [state 4][block 4][site 4],
+//              a block being one category of 4 sites.  A granule holds all
+//              categories of 16 / C sites (8 categories: half the categories
+//              of 4 sites, two granules in turn).
+// A row kept whole (32 or 160 bytes) would make every access of a wave touch
+// the lines of all its 64 rows and use 16 bytes of each.
 constexpr int PAIR_STRIDE = 128;  // doubles between a row's state pairs
+constexpr int STATE_STRIDE = 16;  // doubles between a 4-state row's entries
 template <int S, int C>
-__device__ __forceinline__ size_t row_offset(int64_t site, int c) {
+__device__ __forceinline__ size_t pair_offset(int64_t site, int c) {
   if constexpr (S == 4) {
     const int64_t r = site * C + c;
     return static_cast<size_t>((r >> 6) * (2 * PAIR_STRIDE) + (r & 63) * 2);
@@ -221,9 +221,21 @@ __device__ __forceinline__ size_t row_offset(int64_t site, int c) {
     return static_cast<size_t>(((site >> 6) * C + c) * (S / 2 * PAIR_STRIDE) + (site & 63) * 2);
   }
 }
+template <int S, int C>
+__device__ __forceinline__ size_t row_offset(int64_t site, int c) {
+  if constexpr (S != 4) {
+    return pair_offset<S, C>(site, c);
+  } else if constexpr (C == 8) {
+    return static_cast<size_t>(((site >> 2) * 2 + (c >> 2)) * 64 + (c & 3) * 4 + (site & 3));
+  } else {
+    constexpr int SB = 4 / C;  // 4-site groups of a granule
+    const int64_t g = site >> 2;
+    return static_cast<size_t>(g / SB * 64 + (c * SB + g % SB) * 4 + (site & 3));
+  }
+}
 
 template <int S>
-__device__ __forceinline__ void load_clv(const double *__restrict__ p, double (&x)[S]) {
+__device__ __forceinline__ void load_pairs(const double *__restrict__ p, double (&x)[S]) {
 #pragma unroll
   for (int i = 0; i < S / 2; ++i) {
     const double2 v = *reinterpret_cast<const double2 *>(p + i * PAIR_STRIDE);
@@ -233,10 +245,26 @@ __device__ __forceinline__ void load_clv(const double *__restrict__ p, double (&
 }
 
 template <int S>
-__device__ __forceinline__ void store_clv(double *__restrict__ p, const double (&x)[S]) {
+__device__ __forceinline__ void store_pairs(double *__restrict__ p, const double (&x)[S]) {
 #pragma unroll
   for (int i = 0; i < S / 2; ++i)
     *reinterpret_cast<double2 *>(p + i * PAIR_STRIDE) = make_double2(x[2 * i], x[2 * i + 1]);
+}
+
+template <int S>
+__device__ __forceinline__ void load_clv(const double *__restrict__ p, double (&x)[S]) {
+  if constexpr (S == 4) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = p[i * STATE_STRIDE];
+  } else {
+    load_pairs<S>(p, x);
+  }
+}
+
+template <int S>
+__device__ __forceinline__ void store_clv(double *__restrict__ p, const double (&x)[S]) {
+  static_assert(S != 4, "4-state rows are written by k_forward_walk and k_adjoint_level");
+  store_pairs<S>(p, x);
 }
 
 template <int S>
@@ -308,173 +336,6 @@ __global__ void k_pmatrices(DevLayout L, const double *__restrict__ V,
   d2P[idx] = a2;
   if (Pf) Pf[idx] = static_cast<float>(a0);
   if (dPf) dPf[idx] = static_cast<float>(a1);
-}
-
-// ------------------------------------------------------- forward (FP64)
-// Plain form: a workgroup per tile walks the levels in one launch
-// (k_forward_walk), or, under a memory budget, one launch per level on a
-// 2-D grid of (tile, group of ops of the level).  In the latter blockIdx.x
-// is the tile and gridDim.x a multiple of 8,
-// so every workgroup of a tile lands on the same XCD (workgroup ids are
-// dealt round-robin to the 8 XCDs) and finds the children it reads, written
-// by the same tile in earlier levels, in that XCD's L2.  For 4-state data
-// the P matrices of the group's ops are staged in LDS first: row 2j + k
-// holds op j's child-k edge.
-template <int S, int C>
-__device__ __forceinline__ void stage_ops_p(double *sP, const double *__restrict__ P,
-                                            const DevOp *__restrict__ ops, int n_staged, int part,
-                                            const DevLayout &L) {
-  if constexpr (S == 4) {
-    constexpr int ROW = C * S * S;
-    for (int i = threadIdx.x; i < n_staged * 2 * ROW; i += blockDim.x) {
-      const int slot = i / ROW, r = i % ROW;
-      const int j = slot >> 1, k = slot & 1;
-      if (k < ops[j].nk)
-        sP[i] = P[(static_cast<size_t>(part) * L.n_edges + ops[j].edge[k]) * ROW + r];
-    }
-    __syncthreads();
-  }
-}
-
-// P row block of op j's child k for category c: staged in LDS, or read from
-// memory (20 states, or ops of an adjoint group beyond the staged ones)
-template <int S, int C>
-__device__ __forceinline__ const double *op_p(const double *sP, int n_staged,
-                                              const double *__restrict__ P, int part,
-                                              const DevLayout &L, int j, int k, int edge, int c) {
-  if constexpr (S == 4)
-    if (j < n_staged) return sP + ((j * 2 + k) * C + c) * (S * S);
-  return P + ((static_cast<size_t>(part) * L.n_edges + edge) * C + c) * (S * S);
-}
-
-// ops[0, nb) of one pruning level for one tile: all children of the ops are
-// loaded before any is combined; their P matrices are staged in sP.
-template <int S, int C, int G>
-__device__ __forceinline__ void forward_ops(const DevOp *__restrict__ ops, int nb, const DevLayout &L, int part,
-                                            int tile, double *__restrict__ clv, int32_t *__restrict__ scl,
-                                            const typename TipType<S>::type *__restrict__ tips,
-                                            const double *__restrict__ P, double *sP) {
-  const int c = threadIdx.x % C;
-  const int64_t site = static_cast<int64_t>(tile) * TILE + threadIdx.x / C;
-  const int64_t n = L.n_sites_pad;
-  const size_t slot = static_cast<size_t>(n) * (C * S), ro = row_offset<S, C>(site, c);
-  {
-    // load phase: raw values only (CLV rows, scaler words, tip masks), so no
-    // load has to wait for the ones issued before it
-    __builtin_amdgcn_s_setprio(1);
-    double x[G][2][S];
-    int sk[G][2];
-    uint32_t tm[G][2];
-#pragma unroll
-    for (int j = 0; j < G; ++j) {
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        if (j < nb) {
-          const DevOp op = ops[j];
-          const int32_t kid = op.kid[k];
-          if (k < op.nk && kid >= 0) {
-            load_clv<S>(clv + static_cast<size_t>(kid) * slot + ro, x[j][k]);
-            sk[j][k] = scl[static_cast<size_t>(kid) * n + site];
-          }
-        }
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < G; ++j) {
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        if (j < nb) {
-          const DevOp op = ops[j];
-          const int32_t kid = op.kid[k];
-          if (k < op.nk && kid < 0) tm[j][k] = tips[static_cast<size_t>(-kid - 1) * n + site];
-        }
-      }
-    }
-    // the P matrices after the children's loads: one round trip for both
-    __builtin_amdgcn_s_setprio(0);
-    stage_ops_p<S, C>(sP, P, ops, nb, part, L);  // ends with a barrier (4 states)
-    wait_loads();
-#pragma unroll
-    for (int j = 0; j < G; ++j) {
-      if (j < nb) {
-        const DevOp op = ops[j];
-        int sc_j = 0;
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          if (k < op.nk) {
-            if (op.kid[k] < 0)
-              tip_vec<S>(tm[j][k], x[j][k]);
-            else
-              sc_j += sk[j][k];
-          }
-        }
-        double v[S];
-#pragma unroll
-        for (int i = 0; i < S; ++i) v[i] = 1.0;
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          if (k < op.nk) {
-            double y[S];
-            matvec<S>(op_p<S, C>(sP, nb, P, part, L, j, k, op.edge[k], c), x[j][k], y);
-#pragma unroll
-            for (int i = 0; i < S; ++i) v[i] *= y[i];
-          }
-        }
-        double m = v[0];
-#pragma unroll
-        for (int i = 1; i < S; ++i) m = fmax(m, v[i]);
-        m = cat_max<C>(m);
-        int scj = sc_j;
-        if (m < SCALE_THRESHOLD) {
-#pragma unroll
-          for (int i = 0; i < S; ++i) v[i] *= SCALE_FACTOR;
-          scj += 1;
-        }
-        store_clv<S>(clv + static_cast<size_t>(op.out) * slot + ro, v);
-        if (c == 0) scl[static_cast<size_t>(op.out) * n + site] = scj;
-      }
-    }
-  }
-}
-
-// Workgroup (tile, g) computes ops [gG, gG + G) of the launch for one tile.
-template <int S, int C, int G>
-__global__ void __launch_bounds__(TILE *C)
-    k_forward_level(const DevOp *__restrict__ ops, int n_ops, DevLayout L,
-                    double *__restrict__ clv, int32_t *__restrict__ scl,
-                    const typename TipType<S>::type *__restrict__ tips,
-                    const double *__restrict__ P, const int32_t *__restrict__ tile_part) {
-  __shared__ double sP[S == 4 ? G * 2 * C * S * S : 1];
-  const int tile = blockIdx.x;
-  if (tile >= L.n_tiles) return;  // grid padded to a multiple of 8 tiles
-  const int g0 = blockIdx.y * G;
-  forward_ops<S, C, G>(ops + g0, min(G, n_ops - g0), L, tile_part[tile], tile, clv, scl, tips, P, sP);
-}
-
-// The whole forward pass (or its invalid CLVs) in one launch: a workgroup
-// per tile walks the levels of `walk` (op ranges of `ops`, lowest level
-// first) and each level's ops G at a time.  A CLV and its scaler are read
-// back only by the lanes of the wave that stored them (a site's C lanes
-// share a wave), so no level boundary needs a launch.
-template <int S, int C, int G>
-__global__ void __launch_bounds__(TILE *C, 3)
-    k_forward_walk(const DevOp *__restrict__ ops, const LevelChunk *__restrict__ walk, int n_walk, DevLayout L,
-                   double *__restrict__ clv, int32_t *__restrict__ scl,
-                   const typename TipType<S>::type *__restrict__ tips,
-                   const double *__restrict__ P, const int32_t *__restrict__ tile_part) {
-  __shared__ double sP[S == 4 ? G * 2 * C * S * S : 1];
-  const int tile = blockIdx.x;
-  if (tile >= L.n_tiles) return;  // grid padded to a multiple of 8 tiles
-  const int part = tile_part[tile];
-  bool staged = false;
-  for (int w = 0; w < n_walk; ++w) {
-    const LevelChunk lv = walk[w];
-    for (int g0 = lv.op_begin; g0 < lv.op_end; g0 += G) {
-      if (S == 4 && staged) __syncthreads();  // every lane is done with the previous group's staged P
-      staged = true;
-      forward_ops<S, C, G>(ops + g0, min(G, lv.op_end - g0), L, part, tile, clv, scl, tips, P, sP);
-    }
-  }
 }
 
 // ---------------------------------------------------- root site sums (FP64)
@@ -653,218 +514,474 @@ __global__ void __launch_bounds__(256)
   mixture_body(L, n_root, nc, R, variant, classes, class_dlogprob, root_sums, beta, res, rl);
 }
 
-// ------------------------------------------------------- adjoint (FP64)
+// ------------------------------------------------ 4 states, FP64 plain form
+// The pruning walks on the matrix cores.  v_mfma_f64_4x4x4 multiplies four
+// independent 4 x 4 blocks: A lane (l & 3, block, l >> 4) = A[row][k], B lane
+// = B[k = l >> 4][col = l & 3], D lane = D[row = l >> 4][col = l & 3], block =
+// (l >> 2) & 3.  With blocks = rate categories (and 4-site groups when there
+// are fewer than 4 categories), rows = states and columns = sites, D has B's
+// layout: a product of a CLV is itself a CLV operand, and the stored rows are
+// these registers (see row_offset), one coalesced 512-byte access per 16
+// rows.  P is one register per lane (a 512-byte load of all categories of an
+// edge) instead of 16 LDS reads per lane, and r_c Q stays in one.
+//
+// One wave walks its sites through the whole op list, in depth-first order,
+// and hands a CLV (forward) or an adjoint (reverse) to its consumer through
+// an LDS slot of the wave; a row travels through HBM only where no slot was
+// free (schedule.cpp).  Every CLV is still stored once: the reverse sweep,
+// later incremental passes and the branch derivatives read it.  The loads of
+// an op are issued one op ahead.
+//
+// NQ granules (64 (state, site, category) entries each) per wave: 4 share
+// each matrix load, sum and scalar step among 16 sites at 4 categories; 2 or
+// 1 spread few sites over more waves.
+template <int C, int NQ>
+struct Quad {
+  static constexpr int SPW = 16 * NQ / C;    // sites of a wave
+  static constexpr int NA = C == 8 ? 2 : 1;  // matrix registers per edge (halves of 8 categories)
+  static constexpr int SB = C >= 4 ? 1 : 4 / C;  // 4-site groups of a granule
+  static constexpr int NW = SPW / 4;         // 4-site tip words of a wave
+  static __device__ __forceinline__ int cat(int lane, int h) { return ((lane >> 2) & 3) / SB + 4 * h; }
+  static __device__ __forceinline__ constexpr int half(int q) { return C == 8 ? q & 1 : 0; }
+  // first 4-site group of granule q, and a lane's site within the wave
+  static __device__ __forceinline__ constexpr int group(int q) { return C == 8 ? q >> 1 : q * SB; }
+  static __device__ __forceinline__ int site(int lane, int q) {
+    return 4 * (group(q) + ((lane >> 2) & 3) % SB) + (lane & 3);
+  }
+};
+
+__device__ __forceinline__ double mfma4(double a, double b, double c) {
+  return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
+}
+
+// Granule q of a tip's 0/1 vectors; lane w of `words` holds the masks of the
+// wave's 4-site group w.
+template <int C, int NQ>
+__device__ __forceinline__ double tip_entry(uint32_t words, int q, int lane, int shift) {
+  using W = Quad<C, NQ>;
+  uint32_t w;
+  if constexpr (W::SB == 1)
+    w = __builtin_amdgcn_readlane(words, W::group(q));
+  else
+    w = __shfl(words, W::group(q) + ((lane >> 2) & 3) % W::SB);
+  return __hiloint2double(-static_cast<int>((w >> shift) & 1u) & 0x3FF00000, 0);  // 1.0 or 0.0
+}
+
+// Sites of the wave (bit s = site s) all of whose entries' bits are set in
+// the granules' lane masks.
+template <int C, int NQ>
+__device__ __forceinline__ uint64_t whole_sites(const uint64_t (&m)[NQ]) {
+  using W = Quad<C, NQ>;
+  uint64_t sites = 0;
+#pragma unroll
+  for (int q = 0; q < NQ; q += W::NA) {
+    uint64_t t = m[q];
+    if constexpr (C == 8) t &= m[q + 1];
+    t &= t >> 32;
+    t &= t >> 16;  // over the states
+    if constexpr (C >= 4) {
+      t &= t >> 8;
+      t &= t >> 4;
+      t &= 0xF;
+    } else if constexpr (C == 2) {
+      t &= t >> 8;
+      t &= 0xFF;
+    } else {
+      t &= 0xFFFF;
+    }
+    sites |= t << (4 * W::group(q));
+  }
+  return sites;
+}
+
+// Sums over the 64 lanes of two values at once: lane 31 ends with a's total,
+// lane 63 with b's (the halves of the wave trade one value each, then five
+// DPP steps serve both).
+__device__ __forceinline__ double pair_wave_sum(double a, double b) {
+  const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+  double v = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+  v += dpp<0x111>(v);
+  v += dpp<0x112>(v);
+  v += dpp<0x114>(v);
+  v += dpp<0x118>(v);
+  v += dpp<0x142>(v);
+  return v;
+}
+
+// A use of every register of x here: the wait for the loads into them goes
+// here, ahead of the next op's loads, whose count a condition may change.
+template <typename T, int N>
+__device__ __forceinline__ void arrive(T (&x)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(x[i]));
+}
+
+template <int C, int NQ>
+struct FwdIn4 {
+  double A[2 * Quad<C, NQ>::NA];  // P of both children
+  double x[2 * NQ];               // children read from HBM
+  uint32_t raw[2];                // their scaler words, or a tip child's mask words
+};
+
+// Scaler words: 2 x (rescalings below and at this CLV) + (rescaled here).
+//
+// Bound: HBM (a CLV written per op; 50 taxa, 41,345 patterns: 0.92 GB in 0.223
+// ms, 4.1 TB/s; a thread per row with P in LDS and CLVs through HBM took
+// 0.311 + 0.023 ms for the root sums), or a wave's chain of ops for few sites.
+template <int S, int C, int NQ>
+__global__ void __launch_bounds__(64, 3)
+    k_forward_walk(const DevOp *__restrict__ ops_, int n_ops, int n_slots, DevLayout L, double *__restrict__ clv_,
+                   int32_t *__restrict__ scl_, const uint8_t *__restrict__ tips_, const double *__restrict__ P_,
+                   const double *__restrict__ freqs, const double *__restrict__ weights,
+                   const int32_t *__restrict__ tile_part, double *__restrict__ root_partials,
+                   double *__restrict__ seed) {
+  static_assert(S == 4, "20 states take k_forward_level_aa");
+  using W = Quad<C, NQ>;
+  constexpr int NA = W::NA, SPW = W::SPW;
+  const CAS DevOp *ops = to_constant(ops_);
+  const int lane = threadIdx.x, state = lane >> 4;
+  const int64_t n = L.n_sites_pad, row = n * (C * 4);
+  const int64_t site0 = static_cast<int64_t>(blockIdx.x) * SPW;
+  const int part = to_constant(tile_part)[site0 / TILE];
+  double *slots = dyn_lds<double>();  // [slot][granule][lane], then the slots' scaler words
+  uint32_t *slot_scl = reinterpret_cast<uint32_t *>(slots + n_slots * (NQ * 64));
+  GAS double *clv = to_global(clv_) + static_cast<int64_t>(blockIdx.x) * (NQ * 64);
+  GAS int32_t *scl = to_global(scl_) + site0;
+  const GAS uint8_t *tips = to_global(tips_) + site0;
+  const GAS double *P = to_global(P_) + static_cast<int64_t>(part) * L.n_edges * (C * 16);
+  const uint32_t off = lane * 8, soff = (lane % SPW) * 4, woff = (lane % W::NW) * 4;
+  const int tip_shift = 8 * (lane & 3) + state;
+  uint32_t aoff[NA];
+#pragma unroll
+  for (int h = 0; h < NA; ++h) aoff[h] = (W::cat(lane, h) * 16 + (lane & 3) * 4 + state) * 8;
+  const double w = weights[site0 + lane % SPW];
+  const double pi_c = freqs[part * 4 + state] * (1.0 / C);
+
+  auto load = [&](const DevOp &op, FwdIn4<C, NQ> &in) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int h = 0; h < NA; ++h) in.A[k * NA + h] = *at(P + op.edge[k] * (C * 16), aoff[h]);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      if (k >= op.nk) continue;
+      const int64_t kid = op.kid[k];
+      if (kid < 0) {
+        in.raw[k] = *at(reinterpret_cast<const GAS uint32_t *>(tips + (-kid - 1) * n), woff);
+      } else if (!(op.flags & (k == 0 ? OP_PASS_KID0 : OP_PASS_KID1))) {
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) in.x[k * NQ + q] = *at(clv + kid * row, off + q * 512);
+        in.raw[k] = static_cast<uint32_t>(*at(scl + kid * n, soff));
+      }
+    }
+  };
+  // y = P x of child k
+  auto child = [&](const DevOp &op, const FwdIn4<C, NQ> &in, int k, double (&y)[NQ], uint32_t &count) {
+    double x[NQ];
+    if (op.kid[k] < 0) {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) x[q] = tip_entry<C, NQ>(in.raw[k], q, lane, tip_shift);
+    } else if (op.flags & (k == 0 ? OP_PASS_KID0 : OP_PASS_KID1)) {
+      const int slot = pass_slot(op.flags, k);
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) x[q] = slots[slot * (NQ * 64) + q * 64 + lane];
+      count += slot_scl[slot * 64 + lane] >> 1;
+    } else {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) x[q] = in.x[k * NQ + q];
+      count += in.raw[k] >> 1;
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) y[q] = mfma4(in.A[k * NA + W::half(q)], x[q], 0.0);
+  };
+  auto step = [&](int t, FwdIn4<C, NQ> &in, FwdIn4<C, NQ> &next) {
+    const DevOp op = ops[t];
+    arrive(in.A);
+    arrive(in.x);
+    arrive(in.raw);
+    __builtin_amdgcn_sched_barrier(0);
+    {
+      const DevOp ahead = ops[min(t + 1, n_ops - 1)];
+      load(ahead, next);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    double v[NQ];
+    uint32_t count = 0;
+    child(op, in, 0, v, count);
+    if (op.nk == 2) {
+      double y[NQ];
+      child(op, in, 1, y, count);
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) v[q] *= y[q];
+    }
+    // a site is rescaled when all its entries are below the threshold; most
+    // ops have no entry there at all
+    uint32_t word = count << 1;
+    uint64_t small[NQ], any = 0;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      small[q] = __builtin_amdgcn_ballot_w64(v[q] < SCALE_THRESHOLD);
+      any |= small[q];
+    }
+    if (any) {
+      const uint64_t sites = whole_sites<C, NQ>(small);
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+        if ((sites >> W::site(lane, q)) & 1) v[q] *= SCALE_FACTOR;
+      if ((sites >> (lane % SPW)) & 1) word += 3;
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) *at(clv + op.out * row, off + q * 512) = v[q];
+    *at(scl + op.out * n, soff) = static_cast<int32_t>(word);  // lanes of a site store the same word
+    if (op.flags & OP_A_PASS) {
+      const int slot = pass_slot(op.flags, 2);
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) slots[slot * (NQ * 64) + q * 64 + lane] = v[q];
+      slot_scl[slot * 64 + lane] = word;
+    }
+    if (op.root >= 0) {
+      // site likelihoods Ltilde = (1/C) sum_c pi . x: the sum over the states
+      // as a product with rows pi / C (every row of D holds it), then over
+      // the categories; lane l takes site l % SPW
+      double t_site = 0.0;
+#pragma unroll
+      for (int q = 0; q < NQ; q += NA) {
+        double t = mfma4(pi_c, v[q], 0.0);
+        if constexpr (C == 8) t += mfma4(pi_c, v[q + 1], 0.0);
+        if constexpr (C >= 4) t += dpp<0x124>(t);  // row_ror:4
+        if constexpr (C >= 2) t += dpp<0x128>(t);  // row_ror:8
+        if ((lane % SPW) / (4 * W::SB) == q / NA) t_site = t;
+      }
+      const double wk = lane < SPW ? w : 0.0;
+      const double val = wk != 0.0 ? wk * (log(t_site) + static_cast<double>(word >> 1) * LOG_SCALE_THRESHOLD) : 0.0;
+      const double sum = wave_sum(val);
+      if (lane == 0) root_partials[static_cast<int64_t>(op.root) * gridDim.x + blockIdx.x] = sum;
+      // the adjoint's seed factor at this root and site, w / (C Ltilde)
+      seed[op.root * n + site0 + lane % SPW] = w != 0.0 ? w * (1.0 / C) / t_site : 0.0;
+    }
+  };
+  FwdIn4<C, NQ> a, b;
+  load(ops[0], a);
+  for (int t = 0; t < n_ops; t += 2) {
+    step(t, a, b);
+    if (t + 1 < n_ops) step(t + 1, b, a);
+  }
+}
+
 // Reverse pruning in push form.  For op q with children k (edge e_k, CLV
-// x_k, y_k = P_k x_k) and rescale factor F = 2^(256 (k_q - sum k_k)):
+// x_k, y_k = P_k x_k) and rescale factor F = 2^256 where q was rescaled:
 //   z_k      = Abar_q * F * prod_{j != k} y_j
 //   Abar_k  += P_k^T z_k            (delivered to child k)
 //   dJ/dt_k += z_k . (P'_k x_k),    P'_k x_k = r_c Q y_k
 // where J = sum_p sum_t beta_{p,t} lnL_{p,t} and Abar is the derivative of
 // J w.r.t. the *scaled* CLV values; a root CLV adds the seed
-// beta * w_s * (1/C) pi_i / Ltilde_s.  Ops are walked in reverse
-// topological order; every consumer of a CLV delivers before the CLV's
-// own op runs, the first one writes and later ones accumulate.  The same
-// thread owns (site, category) in every op, so accumulation needs neither
-// atomics nor barriers and is deterministic.
-// One workgroup per tile walks the levels of `walk` (level chunks, top
-// level first) and each level's ops in order; since every (site, category)
-// has one owning thread in every op, a level's deliveries are read back by
-// the thread that stored them, and a single launch can cover any number of
-// levels.  The P matrices of each level's first max_staged ops are staged
-// in LDS when the walk enters the level.
-template <int S>
-struct AdjIn {
-  double a[S];
-  double x[2][S];  // inner children; tips are expanded from tm at use
-  double sd;       // seed factor w / (C Ltilde) of a displayed-tree root's site
-  int kq, sk[2];   // sk: a child's scaler, or a tip child's code (one register for both)
+// beta * w_s * (1/C) pi_i / Ltilde_s.  The ops are walked backwards: every
+// consumer of a CLV delivers before the CLV's own op runs, the first one
+// writes and later ones accumulate (in the matrix instruction's C operand).
+// The same lane owns an entry in every op: no atomics, no barriers,
+// deterministic.
+template <int C, int NQ>
+struct AdjIn4 {
+  double A[2 * Quad<C, NQ>::NA], AT[2 * Quad<C, NQ>::NA];  // P and P^T of both children
+  double x[2 * NQ];    // inner children
+  double a[NQ];        // own adjoint, where no slot holds it
+  double sd[1];        // seed factor of a displayed-tree root (lane l: site l % SPW)
+  uint32_t raw[2];     // tip children's mask words
+  uint32_t word[1];    // own scaler word
 };
 
-template <int S, int C>
-__device__ __forceinline__ void adjoint_inputs(const DevOp &op, int64_t site, int64_t n, int c,
-                                               const double *__restrict__ clv,
-                                               const int32_t *__restrict__ scl,
-                                               const double *__restrict__ adj,
-                                               const typename TipType<S>::type *__restrict__ tips,
-                                               const double *__restrict__ seed, AdjIn<S> &in) {
-  // loads only (defaults for absent inputs are applied at use), so that no
-  // load waits for an earlier one
-  const size_t slot = static_cast<size_t>(n) * (C * S), ro = row_offset<S, C>(site, c);
-  in.kq = scl[static_cast<size_t>(op.out) * n + site];
-  if (op.flags & OP_HAS_CONSUMERS)
-    load_clv<S>(adj + static_cast<size_t>(op.out) * slot + ro, in.a);
-  if (op.root >= 0) in.sd = seed[static_cast<size_t>(op.root) * n + site];
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const int32_t kid = op.kid[k];
-    if (k < op.nk && kid >= 0) {
-      load_clv<S>(clv + static_cast<size_t>(kid) * slot + ro, in.x[k]);
-      in.sk[k] = scl[static_cast<size_t>(kid) * n + site];
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const int32_t kid = op.kid[k];
-    if (k < op.nk && kid < 0) in.sk[k] = static_cast<int>(tips[static_cast<size_t>(-kid - 1) * n + site]);
-  }
-}
+constexpr int GRAD_RING = 128;  // gradient sums of a wave on their way to HBM, 64 at a time
 
-// At least 3 waves per SIMD (the register count the kernel needs anyway):
-// a launch has one wave per 64 (site, category) pairs, about 2.5 per SIMD
-// at 41k patterns, so every wave is resident from the start.
-template <int S, int C>
-__global__ void __launch_bounds__(TILE *C, S == 4 ? 3 : 1)
-    k_adjoint_level(const DevOp *__restrict__ ops, const LevelChunk *__restrict__ walk, int n_walk,
-                    int max_staged, DevLayout L,
-                    const double *__restrict__ clv, const int32_t *__restrict__ scl,
-                    double *__restrict__ adj, const typename TipType<S>::type *__restrict__ tips,
-                    const double *__restrict__ P, const double *__restrict__ Qd,
+// Bound: HBM (every inner child's CLV once per use; 50 taxa, 41,345 patterns:
+// 1.6 GB in 0.363 ms, 4.5 TB/s; with P in LDS and every adjoint through HBM
+// 2.99 GB in 0.648 ms).
+template <int C, int NQ>
+__global__ void __launch_bounds__(64, 3)
+    k_adjoint_level(const DevOp *__restrict__ ops_, int n_ops, int n_slots, int keep, DevLayout L,
+                    const double *__restrict__ clv_, const int32_t *__restrict__ scl_, double *__restrict__ adj_,
+                    const uint8_t *__restrict__ tips_, const double *__restrict__ P_, const double *__restrict__ Qd,
                     const double *__restrict__ freqs, const double *__restrict__ seed,
-                    const int32_t *__restrict__ tile_part, const double *__restrict__ beta,
-                    int n_root, int n_uses, double *__restrict__ grad_partials) {
-  // LDS: r_c Q of every category (4 states), then the staged P matrices
-  double *sQ = dyn_lds<double>();
-  double *sP = sQ + (S == 4 ? C * S * S : 0);
-  constexpr int PW = TILE * C / 64;
-  const int tile = blockIdx.x;
-  if (tile >= L.n_tiles) return;  // grid padded to a multiple of 8 tiles
-
-  const int part = tile_part[tile];
-  if constexpr (S == 4) {
-    for (int i = threadIdx.x; i < C * S * S; i += blockDim.x)
-      sQ[i] = Qd[static_cast<size_t>(part) * C * S * S + i];
-    __syncthreads();
+                    const int32_t *__restrict__ tile_part, const double *__restrict__ beta, int n_root, int n_uses,
+                    double *__restrict__ grad_partials) {
+  using W = Quad<C, NQ>;
+  constexpr int NA = W::NA, SPW = W::SPW;
+  const CAS DevOp *ops = to_constant(ops_);
+  const int lane = threadIdx.x, state = lane >> 4;
+  const int64_t n = L.n_sites_pad, row = n * (C * 4);
+  const int64_t site0 = static_cast<int64_t>(blockIdx.x) * SPW;
+  const int part = to_constant(tile_part)[site0 / TILE];
+  double *ring = dyn_lds<double>();
+  double *slots = ring + GRAD_RING;  // [slot][granule][lane]
+  const GAS double *clv = to_global(clv_) + static_cast<int64_t>(blockIdx.x) * (NQ * 64);
+  GAS double *adj = to_global(adj_) + static_cast<int64_t>(blockIdx.x) * (NQ * 64);
+  const GAS int32_t *scl = to_global(scl_) + site0;
+  const GAS uint8_t *tips = to_global(tips_) + site0;
+  const GAS double *P = to_global(P_) + static_cast<int64_t>(part) * L.n_edges * (C * 16);
+  GAS double *grad = to_global(grad_partials) + static_cast<int64_t>(blockIdx.x) * n_uses;
+  const uint32_t off = lane * 8, soff = (lane % SPW) * 4, woff = (lane % W::NW) * 4;
+  const int tip_shift = 8 * (lane & 3) + state;
+  uint32_t aoff[NA], toff[NA];
+  double Q[NA];
+#pragma unroll
+  for (int h = 0; h < NA; ++h) {
+    aoff[h] = (W::cat(lane, h) * 16 + (lane & 3) * 4 + state) * 8;
+    toff[h] = (W::cat(lane, h) * 16 + state * 4 + (lane & 3)) * 8;
+    Q[h] = Qd[part * (C * 16) + aoff[h] / 8];
   }
-  const int c = threadIdx.x % C;
-  const int64_t site = static_cast<int64_t>(tile) * TILE + threadIdx.x / C;
-  const int64_t n = L.n_sites_pad;
-  const size_t slot = static_cast<size_t>(n) * (C * S), ro = row_offset<S, C>(site, c);
-  const int wave = threadIdx.x / 64;
-  const double *Qc = (S == 4 ? sQ : Qd + static_cast<size_t>(part) * C * S * S) + c * (S * S);
-  // 4 states: r_c Q of this lane's category in registers (every op reads it;
-  // from LDS it would cost as many LDS bytes as a P matrix per child)
-  double Qr[S == 4 ? 16 : 1];
-  if constexpr (S == 4)
+  const double pi = freqs[part * 4 + state];
+
+  auto load = [&](const DevOp &op, AdjIn4<C, NQ> &in) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) Qr[i] = Qc[i];
-  for (int w = 0; w < n_walk; ++w) {
-    const LevelChunk lv = walk[w];
-    const DevOp *__restrict__ lops = ops + lv.op_begin;
-    const int n_ops = lv.op_end - lv.op_begin;
-    const int n_staged = min(n_ops, max_staged);
-    if (S == 4 && w > 0) __syncthreads();  // every lane is done with the previous level's staged P
-    stage_ops_p<S, C>(sP, P, lops, n_staged, part, L);  // ends with a barrier (4 states)
-    for (int j = 0; j < n_ops; ++j) {
-      const DevOp op = lops[j];
-      AdjIn<S> cur;
-      __builtin_amdgcn_s_setprio(1);  // see the note at wait_loads
-      adjoint_inputs<S, C>(op, site, n, c, clv, scl, adj, tips, seed, cur);
-      __builtin_amdgcn_s_setprio(0);
-      double a[S];
-      const bool has_adj = (op.flags & OP_HAS_CONSUMERS) != 0;
+    for (int k = 0; k < 2; ++k)
 #pragma unroll
-      for (int i = 0; i < S; ++i) a[i] = has_adj ? cur.a[i] : 0.0;
-      int ks = 0;
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        if (k < op.nk) {
-          if (op.kid[k] < 0)
-            tip_vec<S>(static_cast<uint32_t>(cur.sk[k]), cur.x[k]);
-          else
-            ks += cur.sk[k];
-        }
+      for (int h = 0; h < NA; ++h) {
+        in.A[k * NA + h] = *at(P + op.edge[k] * (C * 16), aoff[h]);
+        in.AT[k * NA + h] = *at(P + op.edge[k] * (C * 16), toff[h]);
       }
-      if (op.root >= 0) {
-        // seed beta * w * (1/C) pi_i / Ltilde at a displayed-tree root
-        const double f = beta[part * n_root + op.root] * cur.sd;
+    in.word[0] = static_cast<uint32_t>(*at(scl + op.out * n, soff));
 #pragma unroll
-        for (int i = 0; i < S; ++i) a[i] = fma(f, freqs[part * S + i], a[i]);
-      }
-      double y[2][S];
-      const double F = (cur.kq - ks) > 0 ? SCALE_FACTOR : 1.0;
-      // arithmetic of both children first, memory traffic after
-      double back[2][S], g[2];
-      if constexpr (S == 4) {
-        // y_k = P_k x_k, z_0 = a F y_1 (or a F), z_1 = a F y_0, back_k = P_k^T
-        // z_k: P_0 is read once (row i gives y_0[i], z_0[i] and row i's share
-        // of back_0), P_1 twice -- three matrix reads per op instead of four
-        const double *P0 = op_p<S, C>(sP, n_staged, P, part, L, j, 0, op.edge[0], c);
-        // (selects, not op.edge[op.nk - 1]: a runtime index would put op on the stack)
-        const double *P1 = op.nk == 2 ? op_p<S, C>(sP, n_staged, P, part, L, j, 1, op.edge[1], c) : P0;
-        double z[2][S];
-        if (op.nk == 2) matvec<S>(P1, cur.x[1], y[1]);
-#pragma unroll
-        for (int i = 0; i < S; ++i) {
-          const double2 r01 = reinterpret_cast<const double2 *>(P0 + i * S)[0];
-          const double2 r23 = reinterpret_cast<const double2 *>(P0 + i * S)[1];
-          y[0][i] = fma(r23.y, cur.x[0][3], fma(r23.x, cur.x[0][2], fma(r01.y, cur.x[0][1], r01.x * cur.x[0][0])));
-          z[0][i] = a[i] * F * (op.nk == 2 ? y[1][i] : 1.0);
-          if (i == 0) {
-            back[0][0] = r01.x * z[0][0];
-            back[0][1] = r01.y * z[0][0];
-            back[0][2] = r23.x * z[0][0];
-            back[0][3] = r23.y * z[0][0];
-          } else {
-            back[0][0] = fma(r01.x, z[0][i], back[0][0]);
-            back[0][1] = fma(r01.y, z[0][i], back[0][1]);
-            back[0][2] = fma(r23.x, z[0][i], back[0][2]);
-            back[0][3] = fma(r23.y, z[0][i], back[0][3]);
-          }
-        }
-        if (op.nk == 2) {
-#pragma unroll
-          for (int i = 0; i < S; ++i) z[1][i] = a[i] * F * y[0][i];
-          if (op.kid[1] >= 0) matvec_t<S>(P1, z[1], back[1]);
-        }
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          if (k < op.nk) {
-            double dx[S];
-            matvec<S>(Qr, y[k], dx);
-            double gk = 0.0;
-#pragma unroll
-            for (int i = 0; i < S; ++i) gk = fma(z[k][i], dx[i], gk);
-            g[k] = wave_sum(gk);
-          }
-        }
+    for (int k = 0; k < 2; ++k) {
+      if (k >= op.nk) continue;
+      const int64_t kid = op.kid[k];
+      if (kid < 0) {
+        in.raw[k] = *at(reinterpret_cast<const GAS uint32_t *>(tips + (-kid - 1) * n), woff);
       } else {
 #pragma unroll
-        for (int k = 0; k < 2; ++k)
-          if (k < op.nk) matvec<S>(op_p<S, C>(sP, n_staged, P, part, L, j, k, op.edge[k], c), cur.x[k], y[k]);
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          if (k < op.nk) {
-            double z[S], dx[S];
-#pragma unroll
-            for (int i = 0; i < S; ++i) z[i] = a[i] * F * (op.nk == 2 ? y[1 - k][i] : 1.0);
-            matvec<S>(Qc, y[k], dx);
-            double gk = 0.0;
-#pragma unroll
-            for (int i = 0; i < S; ++i) gk = fma(z[i], dx[i], gk);
-            g[k] = wave_sum(gk);
-            if (op.kid[k] >= 0)
-              matvec_t<S>(op_p<S, C>(sP, n_staged, P, part, L, j, k, op.edge[k], c), z, back[k]);
-          }
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        if (k < op.nk) {
-          if ((threadIdx.x & 63) == 0) grad_partials[grad_index(tile, n_uses, op.gslot[k], PW, wave)] = g[k];
-          const int32_t kid = op.kid[k];
-          if (kid >= 0) {
-            double *dst = adj + static_cast<size_t>(kid) * slot + ro;
-            if (!(op.flags & (k == 0 ? OP_FIRST_KID0 : OP_FIRST_KID1))) {
-              double acc[S];
-              load_clv<S>(dst, acc);
-#pragma unroll
-              for (int i = 0; i < S; ++i) back[k][i] += acc[i];
-            }
-            store_clv<S>(dst, back[k]);
-          }
-        }
+        for (int q = 0; q < NQ; ++q) in.x[k * NQ + q] = *at(clv + kid * row, off + q * 512);
       }
     }
+    if ((op.flags & (OP_HAS_CONSUMERS | OP_A_PASS | OP_A_LATE)) == OP_HAS_CONSUMERS)
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) in.a[q] = *at(adj + op.out * row, off + q * 512);
+    if (op.root >= 0) in.sd[0] = seed[op.root * n + site0 + lane % SPW];
+  };
+  // back-propagated vectors to child k's adjoint
+  auto deliver = [&](const DevOp &op, const AdjIn4<C, NQ> &in, int k, const double (&z)[NQ], double (&b)[NQ]) {
+    const bool first = (op.flags & (k == 0 ? OP_FIRST_KID0 : OP_FIRST_KID1)) != 0;
+    const bool pass = (op.flags & (k == 0 ? OP_PASS_KID0 : OP_PASS_KID1)) != 0;
+    double *slot = slots + pass_slot(op.flags, k) * (NQ * 64) + lane;
+    GAS double *dst = adj + static_cast<int64_t>(op.kid[k]) * row;
+    if (pass && !first) {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) b[q] = slot[q * 64];
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) b[q] = mfma4(in.AT[k * NA + W::half(q)], z[q], b[q]);
+    if (pass) {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) slot[q * 64] = b[q];
+    } else {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) *at(dst, off + q * 512) = b[q];
+    }
+  };
+  auto product = [&](const DevOp &op, const AdjIn4<C, NQ> &in, int k, double (&y)[NQ]) {
+    double x[NQ];
+    if (op.kid[k] < 0) {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) x[q] = tip_entry<C, NQ>(in.raw[k], q, lane, tip_shift);
+    } else {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) x[q] = in.x[k * NQ + q];
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) y[q] = mfma4(in.A[k * NA + W::half(q)], x[q], 0.0);
+  };
+  const int last = ops[n_ops - 1].gslot[0];  // the sweep's first gradient row
+  int flushed = last;
+  auto step = [&](int t, AdjIn4<C, NQ> &in, AdjIn4<C, NQ> &next) {
+    const DevOp op = ops[t];
+    arrive(in.A);
+    arrive(in.AT);
+    arrive(in.x);
+    arrive(in.a);
+    arrive(in.sd);
+    arrive(in.raw);
+    arrive(in.word);
+    __builtin_amdgcn_sched_barrier(0);
+    // what the children's adjoints hold already, where no slot does (the
+    // deliveries before this op's are stores of this wave, so in order)
+    double acc[2][NQ];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) acc[k][q] = 0.0;
+      if (op.flags & (k == 0 ? OP_ACC0 : OP_ACC1))
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) acc[k][q] = *at(adj + op.kid[k] * row, off + q * 512);
+    }
+    {
+      const DevOp ahead = ops[max(t - 1, 0)];
+      load(ahead, next);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    double a[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) a[q] = 0.0;
+    if (op.flags & OP_A_PASS) {
+      const double *slot = slots + pass_slot(op.flags, 2) * (NQ * 64) + lane;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) a[q] = slot[q * 64];
+    } else if (op.flags & OP_A_LATE) {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) a[q] = *at(adj + op.out * row, off + q * 512);
+      wait_loads();
+    } else if (op.flags & OP_HAS_CONSUMERS) {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) a[q] = in.a[q];
+    }
+    if (op.root >= 0) {
+      // seed beta * w * (1/C) pi_i / Ltilde at a displayed-tree root
+      const double f = beta[part * n_root + op.root] * in.sd[0];
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) a[q] = fma(__shfl(f, W::site(lane, q)), pi, a[q]);
+    }
+    if (keep)  // the model gradient reads every adjoint
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) *at(adj + op.out * row, off + q * 512) = a[q];
+    const uint64_t scaled = __builtin_amdgcn_ballot_w64(lane < SPW && (in.word[0] & 1u));
+    if (scaled)
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+        if ((scaled >> W::site(lane, q)) & 1) a[q] *= SCALE_FACTOR;
+    double y[2][NQ], z[NQ], g[2] = {0.0, 0.0};
+    auto use = [&](int k) {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) g[k] = fma(z[q], mfma4(Q[W::half(q)], y[k][q], 0.0), g[k]);
+      if (op.kid[k] >= 0) deliver(op, in, k, z, acc[k]);
+    };
+    product(op, in, 0, y[0]);
+    if (op.nk == 2) {
+      product(op, in, 1, y[1]);
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) z[q] = a[q] * y[1][q];
+      use(0);
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) z[q] = a[q] * y[0][q];
+      use(1);
+    } else {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) z[q] = a[q];
+      use(0);
+    }
+    // rows are numbered in the order of the sweep: row r waits in ring[r %
+    // GRAD_RING], and 64 at a time leave as one store
+    const double total = pair_wave_sum(g[0], g[1]);
+    const int k = lane >> 5;
+    if ((lane & 31) == 31 && k < op.nk) ring[(op.gslot[0] + k) % GRAD_RING] = total;
+    const int done = op.gslot[0] + op.nk;
+    if (done - flushed >= 64) {
+      grad[flushed + lane] = ring[(flushed + lane) % GRAD_RING];
+      flushed += 64;
+    }
+    if (t == 0 && lane < done - flushed) grad[flushed + lane] = ring[(flushed + lane) % GRAD_RING];
+  };
+  AdjIn4<C, NQ> u, v;
+  load(ops[n_ops - 1], u);
+  for (int t = n_ops - 1; t >= 0; t -= 2) {
+    step(t, u, v);
+    if (t > 0) step(t - 1, v, u);
   }
 }
 
@@ -1087,9 +1204,8 @@ __global__ void __launch_bounds__(TILE *C)
 
 // ---------------------------------------------- model gradient (FP64)
 // dlnL / dP_{e,c} for every (op, child) use: G = sum over sites of z (x)^T
-// with z the adjoint of y = P x (recomputed from the op's stored adjoint,
-// its children and the displayed-tree seed, exactly as k_adjoint_level
-// forms it) and x the child's CLV; and, at displayed-tree roots, the direct
+// with z the adjoint of y = P x (recomputed from the op's stored adjoint
+// and its children, as k_adjoint_level forms it) and x the child's CLV; and, at displayed-tree roots, the direct
 // dependence of lnL on the frequencies, sum_s beta w (1/C) x_i / Ltilde.
 // Grid (op, chunk): a chunk is a 1/n_split slice of one partition's tiles,
 // so every partial belongs to one partition; a workgroup walks its tiles
@@ -1128,23 +1244,20 @@ __global__ void __launch_bounds__(TILE *C)
     double a[S], x[2][S], y[2][S];
 #pragma unroll
     for (int i = 0; i < S; ++i) a[i] = 0.0;
-    if (op.flags & OP_HAS_CONSUMERS) load_clv<S>(adj + static_cast<size_t>(op.out) * slot + ro, a);
-    int ks = 0;
+    load_clv<S>(adj + static_cast<size_t>(op.out) * slot + ro, a);
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       if (k >= op.nk) continue;
       const int32_t kid = op.kid[k];
       if (kid >= 0) {
         load_clv<S>(clv + static_cast<size_t>(kid) * slot + ro, x[k]);
-        ks += scl[static_cast<size_t>(kid) * n + site];
       } else {
         tip_vec<S>(tips[static_cast<size_t>(-kid - 1) * n + site], x[k]);
       }
       matvec<S>(Pk[k], x[k], y[k]);
     }
     if (op.root >= 0) {
-      // seed beta w (1/C) pi_i / Ltilde of a displayed-tree root, and the
-      // frequencies' direct share beta w (1/C) x_i / Ltilde
+      // the frequencies' direct share beta w (1/C) x_i / Ltilde
       double xr[S];
       load_clv<S>(clv + static_cast<size_t>(op.out) * slot + ro, xr);
       double t = 0.0;
@@ -1153,12 +1266,9 @@ __global__ void __launch_bounds__(TILE *C)
       t = cat_sum<C>(t) * (1.0 / C);
       const double f = w != 0.0 ? bt * w * (1.0 / C) / t : 0.0;
 #pragma unroll
-      for (int i = 0; i < S; ++i) {
-        a[i] = fma(f, freqs[part * S + i], a[i]);
-        rr[i] = fma(f, xr[i], rr[i]);
-      }
+      for (int i = 0; i < S; ++i) rr[i] = fma(f, xr[i], rr[i]);
     }
-    const double F = (scl[static_cast<size_t>(op.out) * n + site] - ks) > 0 ? SCALE_FACTOR : 1.0;
+    const double F = (scl[static_cast<size_t>(op.out) * n + site] & 1) ? SCALE_FACTOR : 1.0;
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       if (k >= op.nk) continue;
@@ -2596,6 +2706,11 @@ __device__ __forceinline__ void stage_path_p(double *sPp, const PathStep *__rest
 // in for absent ones, so no load sits on one path of a branch) is issued
 // before its arithmetic, which then only waits on LDS and registers.  A
 // step's own scaler is the previous step's child scaler.
+// rescalings a scaler word counts (FP64 4-state words: see k_forward_walk)
+template <int S, typename T>
+__device__ __forceinline__ int scl_count(int32_t word) {
+  return S == 4 && std::is_same<T, double>::value ? word >> 1 : word;
+}
 // a thread's row in a CLV slot of either form (FP32 rows are kept whole)
 template <int S, int C, typename T>
 __device__ __forceinline__ size_t clv_row(int64_t site, int c) {
@@ -2627,7 +2742,7 @@ __device__ __forceinline__ void path_sumtable(const PathStep *__restrict__ steps
   const int32_t root = steps[b0].out, low = steps[b1 - 1].child;
   double xr[S], xc[S];
   load_any<S>(clv + static_cast<size_t>(root) * slot + ro, xr);
-  int kq = scl[static_cast<size_t>(root) * n + site];
+  int kq = scl_count<S, T>(scl[static_cast<size_t>(root) * n + site]);
   load_any<S>(clv + static_cast<size_t>(slot_of(low)) * slot + ro, xc);
   const TT tmc = tips[static_cast<size_t>(tip_of(low)) * n + site];
   double a[S];
@@ -2664,13 +2779,13 @@ __device__ __forceinline__ void path_sumtable(const PathStep *__restrict__ steps
           if (ps.sib < 0)
             tip_vec<S>(tm[u], xs[u]);
           else
-            ksu = ks[u];
+            ksu = scl_count<S, T>(ks[u]);
           matvec<S>(prow(j, 1, ps.edge_sib), xs[u], y);
         } else {
 #pragma unroll
           for (int i = 0; i < S; ++i) y[i] = 1.0;
         }
-        const int kcu = ps.child >= 0 ? kc[u] : 0;
+        const int kcu = ps.child >= 0 ? scl_count<S, T>(kc[u]) : 0;
         const double F = ldexp(1.0, scale_unit * (kq - kcu - ksu));
         double z[S];
 #pragma unroll
@@ -2715,7 +2830,7 @@ __global__ void __launch_bounds__(TILE *C)
   double stv[S];
   path_sumtable<S, C, T>(steps, b0, b1, sPp, n_staged, L, part, site, c, clv, scl, scale_unit, tips, P, V, Vinv,
                          freqs, stv);
-  store_clv<S>(st + static_cast<size_t>(j) * L.n_sites_pad * (C * S) + row_offset<S, C>(site, c), stv);
+  store_pairs<S>(st + static_cast<size_t>(j) * L.n_sites_pad * (C * S) + pair_offset<S, C>(site, c), stv);
 }
 
 // Per displayed tree j and wave: sums over sites of w log rho(b),
@@ -2783,7 +2898,7 @@ __global__ void __launch_bounds__(TILE *C)
   const int c = threadIdx.x % C;
   const int64_t site = static_cast<int64_t>(tile) * TILE + threadIdx.x / C;
   const int64_t n = L.n_sites_pad;
-  const size_t slot = static_cast<size_t>(n) * (C * S), ro = row_offset<S, C>(site, c);
+  const size_t slot = static_cast<size_t>(n) * (C * S), ro = pair_offset<S, C>(site, c);
   const size_t n_wt = static_cast<size_t>(L.n_tiles) * PW;
   const int wt = tile * PW + threadIdx.x / 64;
   const double w = weights[site];
@@ -2792,7 +2907,7 @@ __global__ void __launch_bounds__(TILE *C)
   // one path per workgroup (grid tiles x paths)
   for (int j = blockIdx.y; j < min(n_paths, static_cast<int>(blockIdx.y) + 1); ++j) {
     double stv[S], v[3];
-    load_clv<S>(st + static_cast<size_t>(j) * slot + ro, stv);
+    load_pairs<S>(st + static_cast<size_t>(j) * slot + ro, stv);
     sumtable_partials<S, C>(stv, ex, lr, w, c, v);
     if ((threadIdx.x & 63) == 0)
 #pragma unroll
@@ -2824,7 +2939,7 @@ __global__ void __launch_bounds__(TILE *C)
   const int c = threadIdx.x % C;
   const int64_t site = static_cast<int64_t>(tile) * TILE + threadIdx.x / C;
   const int64_t n = L.n_sites_pad;
-  const size_t slot = static_cast<size_t>(n) * (C * S), ro = row_offset<S, C>(site, c);
+  const size_t slot = static_cast<size_t>(n) * (C * S), ro = pair_offset<S, C>(site, c);
   const size_t n_wt = static_cast<size_t>(L.n_tiles) * PW;
   const int wt = tile * PW + threadIdx.x / 64;
   const double w = weights[site];
@@ -2833,7 +2948,7 @@ __global__ void __launch_bounds__(TILE *C)
   // one path per workgroup (grid tiles x the largest path count)
   for (int j = blockIdx.y; j < min(n_paths, static_cast<int>(blockIdx.y) + 1); ++j) {
     double stv[S], v[3];
-    load_clv<S>(st + static_cast<size_t>(j) * slot + ro, stv);
+    load_pairs<S>(st + static_cast<size_t>(j) * slot + ro, stv);
     sumtable_partials<S, C>(stv, ex, lr, w, c, v);
     if ((threadIdx.x & 63) == 0)
 #pragma unroll
@@ -3294,37 +3409,45 @@ void launch_forward_level(Engine &e, const DevOp *ops, int n_ops, const LevelChu
     NRX_HIP(hipGetLastError());
     return;
   }
-  dispatch_sc(e.S, e.C, [&](auto s, auto c) {
-    constexpr int S = decltype(s)::value, C = decltype(c)::value;
-    constexpr int G = S == 4 ? PLAIN_G : 1;
-    using TT = typename TipType<S>::type;
-    hipLaunchKernelGGL((k_forward_level<S, C, G>), dim3(e.L.n_tiles_grid, (n_ops + G - 1) / G),
-                       dim3(TILE * C), 0, e.stream, ops, n_ops, e.L, e.d_clv.as<double>(),
-                       e.d_scl.as<int32_t>(), e.d_tips.as<TT>(), e.d_P.as<double>(),
-                       e.d_tile_part.as<int32_t>());
-  });
-  NRX_HIP(hipGetLastError());
+  throw std::logic_error("launch_forward_level: 4-state passes go through launch_forward_walk");
 }
 
-void launch_forward_walk(Engine &e, const DevOp *ops, const LevelChunk *walk, int n_walk) {
-  if (e.S == AA_STATES) throw std::logic_error("launch_forward_walk: 20-state levels go through launch_forward_level");
-  if (n_walk == 0) return;
-  dispatch_sc(e.S, e.C, [&](auto s, auto c) {
-    constexpr int S = decltype(s)::value, C = decltype(c)::value;
-    constexpr int G = S == 4 ? PLAIN_G : 1;
-    using TT = typename TipType<S>::type;
-    if constexpr (S != AA_STATES)
-      hipLaunchKernelGGL((k_forward_walk<S, C, G>), dim3(e.L.n_tiles_grid), dim3(TILE * C), 0, e.stream, ops, walk,
-                         n_walk, e.L, e.d_clv.as<double>(), e.d_scl.as<int32_t>(), e.d_tips.as<TT>(),
-                         e.d_P.as<double>(), e.d_tile_part.as<int32_t>());
+// Shapes of the 4-state FP64 walks: C categories, NQ granules per wave (8
+// categories take granules in pairs, and 4 of them would spill registers).
+template <typename F>
+static void dispatch_walk(int C, int NQ, F &&f) {
+  dispatch_c(C, [&](auto c) {
+    constexpr int CC = decltype(c)::value;
+    if constexpr (CC != 8)
+      if (NQ == 4) return f(c, std::integral_constant<int, 4>{});
+    if (NQ == 2) return f(c, std::integral_constant<int, 2>{});
+    if constexpr (CC != 8)
+      if (NQ == 1) return f(c, std::integral_constant<int, 1>{});
+    throw std::logic_error("unsupported walk shape");
+  });
+}
+
+size_t forward_walk_lds(int nq, int n_slots) { return static_cast<size_t>(n_slots) * (nq * 512 + 256); }
+size_t adjoint_walk_lds(int nq, int n_slots) { return sizeof(double) * GRAD_RING + static_cast<size_t>(n_slots) * nq * 512; }
+
+void launch_forward_walk(Engine &e, const DevOp *ops, int n_ops) {
+  if (n_ops == 0) return;
+  const unsigned waves = static_cast<unsigned>(e.L.n_tiles) * e.rpw;
+  dispatch_walk(e.C, e.walk_nq, [&](auto c, auto nq) {
+    constexpr int C = decltype(c)::value, NQ = decltype(nq)::value;
+    hipLaunchKernelGGL((k_forward_walk<4, C, NQ>), dim3(waves), dim3(64), forward_walk_lds(NQ, e.fwd_slots), e.stream,
+                       ops, n_ops, e.fwd_slots, e.L, e.d_clv.as<double>(), e.d_scl.as<int32_t>(),
+                       e.d_tips.as<uint8_t>(), e.d_P.as<double>(), e.d_freqs.as<double>(), e.d_weights.as<double>(),
+                       e.d_tile_part.as<int32_t>(), e.d_root_partials.as<double>(), e.d_site_seed.as<double>());
   });
   NRX_HIP(hipGetLastError());
 }
 
 void launch_root_partials(Engine &e, bool seeds, const int32_t *rows, const int32_t *index, int n) {
   if (n == 0) return;
-  dispatch_sc(e.S, e.C, [&](auto s, auto c) {
-    constexpr int S = decltype(s)::value, C = decltype(c)::value;
+  if (e.S != AA_STATES) throw std::logic_error("launch_root_partials: the 4-state forward walk forms the root sums");
+  dispatch_c(e.C, [&](auto c) {
+    constexpr int S = AA_STATES, C = decltype(c)::value;
     hipLaunchKernelGGL((k_root_partials<S, C>), dim3(e.L.n_tiles, n), dim3(TILE * C), 0, e.stream, rows, n, e.L,
                        e.d_clv.as<double>(), e.d_scl.as<int32_t>(), e.d_freqs.as<double>(),
                        e.d_weights.as<double>(), e.d_tile_part.as<int32_t>(), e.d_root_partials.as<double>(),
@@ -3367,31 +3490,20 @@ void launch_adjoint_level(Engine &e, const LevelChunk &ch, const DevOp *ops) {
     NRX_HIP(hipGetLastError());
     return;
   }
-  throw std::logic_error("launch_adjoint_level: 4-state sweeps go through launch_adjoint_levels");
+  throw std::logic_error("launch_adjoint_level: 4-state sweeps go through launch_adjoint_walk");
 }
 
-void launch_adjoint_levels(Engine &e, const DevOp *ops, int c_hi, int c_lo) {
-  const int nch = static_cast<int>(e.chunks.size());
-  if (e.S == AA_STATES || c_lo < 0 || c_hi >= nch || c_lo > c_hi)
-    throw std::logic_error("launch_adjoint_levels: 4-state level chunks expected");
-  int widest = 0;
-  for (int c = c_lo; c <= c_hi; ++c) widest = std::max(widest, e.chunks[c].op_end - e.chunks[c].op_begin);
-  if (widest == 0) return;
-  // the walk list holds the chunks top level first: chunk c at nch - 1 - c
-  const LevelChunk *walk = e.d_adj_walk.as<LevelChunk>() + (nch - 1 - c_hi);
-  const int n_walk = c_hi - c_lo + 1;
-  dispatch_sc(e.S, e.C, [&](auto s, auto c) {
-    constexpr int S = decltype(s)::value, C = decltype(c)::value;
-    using TT = typename TipType<S>::type;
-    const int max_staged = S == 4 ? std::min(widest, plain_staged_ops(C)) : 0;
-    const size_t lds = S == 4 ? sizeof(double) * (max_staged * 2 + 1) * C * S * S : 0;
-    if constexpr (S != AA_STATES)  // 20 states take k_adjoint_level_aa (refused above)
-      hipLaunchKernelGGL((k_adjoint_level<S, C>), dim3(e.L.n_tiles_grid), dim3(TILE * C), lds, e.stream,
-                         ops, walk, n_walk, max_staged, e.L, e.d_clv.as<double>(),
-                         e.d_scl.as<int32_t>(), e.d_adj.as<double>(), e.d_tips.as<TT>(),
-                         e.d_P.as<double>(), e.d_Qd.as<double>(), e.d_freqs.as<double>(),
-                         e.d_site_seed.as<double>(), e.d_tile_part.as<int32_t>(), e.d_beta.as<double>(),
-                         static_cast<int>(e.root_slots.size()), e.n_uses, e.d_grad_partials.as<double>());
+void launch_adjoint_walk(Engine &e, const DevOp *ops, int n_ops, bool keep) {
+  if (n_ops == 0) return;
+  const unsigned waves = static_cast<unsigned>(e.L.n_tiles) * e.rpw;
+  dispatch_walk(e.C, e.walk_nq, [&](auto c, auto nq) {
+    constexpr int C = decltype(c)::value, NQ = decltype(nq)::value;
+    hipLaunchKernelGGL((k_adjoint_level<C, NQ>), dim3(waves), dim3(64), adjoint_walk_lds(NQ, e.adj_slots), e.stream,
+                       ops, n_ops, e.adj_slots, keep ? 1 : 0, e.L, e.d_clv.as<double>(), e.d_scl.as<int32_t>(),
+                       e.d_adj.as<double>(), e.d_tips.as<uint8_t>(), e.d_P.as<double>(), e.d_Qd.as<double>(),
+                       e.d_freqs.as<double>(), e.d_site_seed.as<double>(), e.d_tile_part.as<int32_t>(),
+                       e.d_beta.as<double>(), static_cast<int>(e.root_slots.size()), e.n_uses,
+                       e.d_grad_partials.as<double>());
   });
   NRX_HIP(hipGetLastError());
 }

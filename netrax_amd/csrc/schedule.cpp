@@ -2,6 +2,7 @@
 #include "schedule.hpp"
 
 #include <algorithm>
+#include <array>
 #include <stdexcept>
 #include <utility>
 
@@ -59,6 +60,142 @@ void split_level_runs(std::vector<DevOp> &ops, const std::vector<LevelChunk> &ch
     }
     std::copy(ordered.begin(), ordered.end(), ops.begin() + ch.op_begin);
     run_begin.push_back(static_cast<int>(runs.size()));
+  }
+}
+
+std::vector<int> depth_first_order(const Dag &dag, const std::vector<int> &root_slots) {
+  const int nv = static_cast<int>(dag.var.size());
+  // rows held at once below a variant, counted as for a tree
+  std::vector<int> held(nv, 1);
+  for (int v = 0; v < nv; ++v) {  // children have smaller slot ids
+    int a = 0, b = 0;
+    for (int k = 0; k < dag.var[v].nkids; ++k) {
+      const int32_t kid = dag.var[v].kid[k];
+      (k == 0 ? a : b) = kid >= 0 ? held[kid] : 0;
+    }
+    held[v] = std::max(1, a == b ? a + 1 : std::max(a, b));
+  }
+  std::vector<int> order;
+  std::vector<char> seen(nv, 0);
+  std::vector<std::pair<int, int>> stack;
+  for (int rs : root_slots) {
+    if (seen[rs]) continue;
+    seen[rs] = 1;
+    stack.push_back({rs, 0});
+    while (!stack.empty()) {
+      const int v = stack.back().first, i = stack.back().second++;
+      const Variant &var = dag.var[v];
+      if (i >= var.nkids) {
+        order.push_back(v);
+        stack.pop_back();
+        continue;
+      }
+      const bool second_first = var.nkids == 2 && var.kid[0] >= 0 && var.kid[1] >= 0 && held[var.kid[1]] > held[var.kid[0]];
+      const int32_t kid = var.kid[second_first ? 1 - i : i];
+      if (kid >= 0 && !seen[kid]) {
+        seen[kid] = 1;
+        stack.push_back({kid, 0});
+      }
+    }
+  }
+  return order;
+}
+
+// The row with the furthest next read gives up its slot (it was stored in
+// HBM anyway), which keeps the most reads in LDS.
+void assign_forward_slots(DevOp *ops, int n, int n_slots) {
+  constexpr int NEVER = INT32_MAX;
+  int rows = 0;
+  for (int i = 0; i < n; ++i) {
+    rows = std::max(rows, ops[i].out + 1);
+    for (int k = 0; k < ops[i].nk; ++k) rows = std::max(rows, ops[i].kid[k] + 1);
+  }
+  std::vector<int> next(rows, NEVER), first_read(n), made(rows, -1);
+  std::vector<std::array<int, 2>> later(n);  // next read of child k after op i
+  for (int i = n - 1; i >= 0; --i) {
+    first_read[i] = next[ops[i].out];
+    for (int k = 0; k < ops[i].nk; ++k)
+      if (ops[i].kid[k] >= 0) later[i][k] = next[ops[i].kid[k]];
+    for (int k = 0; k < ops[i].nk; ++k)
+      if (ops[i].kid[k] >= 0) next[ops[i].kid[k]] = i;
+  }
+  std::vector<int> row_in(n_slots, -1), read_at(n_slots, NEVER);
+  for (int i = 0; i < n; ++i) {
+    DevOp &op = ops[i];
+    op.flags &= ~(OP_PASS_KID0 | OP_PASS_KID1 | OP_A_PASS | PASS_BITS);
+    for (int k = 0; k < op.nk; ++k) {
+      if (op.kid[k] < 0) continue;
+      const auto it = std::find(row_in.begin(), row_in.end(), op.kid[k]);
+      if (it != row_in.end()) {
+        const int q = static_cast<int>(it - row_in.begin());
+        op.flags |= (k == 0 ? OP_PASS_KID0 : OP_PASS_KID1) | (q << (PASS_SHIFT + 3 * k));
+        read_at[q] = later[i][k];
+      } else if (made[op.kid[k]] == i - 1 && i > 0) {
+        // the kernel loads an op's inputs before the op before it stores
+        throw std::logic_error("forward walk: a child is read from HBM right after it was made");
+      }
+    }
+    for (int q = 0; q < n_slots; ++q)
+      if (read_at[q] == NEVER) row_in[q] = -1;
+    made[op.out] = i;
+    if (first_read[i] == NEVER) continue;
+    int q = static_cast<int>(std::find(row_in.begin(), row_in.end(), -1) - row_in.begin());
+    if (q == n_slots) {
+      q = static_cast<int>(std::max_element(read_at.begin(), read_at.end()) - read_at.begin());
+      if (read_at[q] <= first_read[i]) continue;
+    }
+    row_in[q] = op.out;
+    read_at[q] = first_read[i];
+    op.flags |= OP_A_PASS | (q << (PASS_SHIFT + 6));
+  }
+}
+
+// A row keeps its slot from its first delivery to its own op, or lives in
+// HBM throughout; rows are taken by earliest release (interval scheduling).
+// A slot's old row is read before the op that releases it delivers, so the
+// slot can take a new row at that op.
+void assign_reverse_slots(DevOp *ops, int n, int n_slots) {
+  constexpr int32_t ALL =
+      OP_PASS_KID0 | OP_PASS_KID1 | OP_A_PASS | PASS_BITS | OP_A_LATE | OP_ACC0 | OP_ACC1;
+  int rows = 0;
+  for (int i = 0; i < n; ++i) {
+    rows = std::max(rows, ops[i].out + 1);
+    for (int k = 0; k < ops[i].nk; ++k) rows = std::max(rows, ops[i].kid[k] + 1);
+  }
+  // positions in the sweep: t = n - 1 - op
+  std::vector<int> start(rows, -1), slot_of(rows, -1), last(rows, -2);
+  std::vector<int> busy_until(n_slots, -1);
+  for (int t = 0; t < n; ++t) {
+    DevOp &op = ops[n - 1 - t];
+    op.flags &= ~ALL;
+    for (int k = 0; k < op.nk; ++k)
+      if (op.kid[k] >= 0 && (op.flags & (k == 0 ? OP_FIRST_KID0 : OP_FIRST_KID1))) start[op.kid[k]] = t;
+  }
+  for (int t = 0; t < n; ++t) {  // by release: the position of the row's own op
+    const int32_t row = ops[n - 1 - t].out;
+    if (start[row] < 0 || start[row] >= t) continue;  // no delivery, or one of an earlier launch
+    int best = -1;
+    for (int q = 0; q < n_slots; ++q)
+      if (busy_until[q] <= start[row] && (best < 0 || busy_until[q] > busy_until[best])) best = q;
+    if (best < 0) continue;
+    busy_until[best] = t;
+    slot_of[row] = best;
+  }
+  for (int t = 0; t < n; ++t) {
+    DevOp &op = ops[n - 1 - t];
+    if (slot_of[op.out] >= 0)
+      op.flags |= OP_A_PASS | (slot_of[op.out] << (PASS_SHIFT + 6));
+    else if (last[op.out] == t - 1)
+      op.flags |= OP_A_LATE;
+    for (int k = 0; k < op.nk; ++k) {
+      const int32_t kid = op.kid[k];
+      if (kid < 0) continue;
+      if (slot_of[kid] >= 0)
+        op.flags |= (k == 0 ? OP_PASS_KID0 : OP_PASS_KID1) | (slot_of[kid] << (PASS_SHIFT + 3 * k));
+      else if (!(op.flags & (k == 0 ? OP_FIRST_KID0 : OP_FIRST_KID1)))
+        op.flags |= k == 0 ? OP_ACC0 : OP_ACC1;
+      last[kid] = t;
+    }
   }
 }
 
