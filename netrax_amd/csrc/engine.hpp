@@ -109,6 +109,9 @@ constexpr int32_t OP_A_LATE = 512;
 // FP64 form, 4 states: child k's adjoint lies in HBM and holds deliveries
 constexpr int32_t OP_ACC0 = 1024;
 constexpr int32_t OP_ACC1 = 2048;
+// FP64 form, 4 states, forward: child k's CLV is read from HBM
+constexpr int32_t OP_LOAD0 = 1 << 21;
+constexpr int32_t OP_LOAD1 = 1 << 22;
 constexpr int WALK_SLOTS = 8;  // FP64 form: LDS slots of a wave, at most (3 bits per use)
 constexpr int PASS_SLOTS = 5;  // at most; fewer where LDS would cost residency
 constexpr int PASS_SHIFT = 12;  // slot of use u (0, 1: children, 2: own) in bits 12 + 3u

@@ -617,11 +617,52 @@ __device__ __forceinline__ void arrive(T (&x)[N]) {
   for (int i = 0; i < N; ++i) asm volatile("" : "+v"(x[i]));
 }
 
+// Brings a walk's P matrices (one 128-byte line each) and op list into the
+// XCD's L2: the kernels before it left them in other XCDs, and every op of
+// the walk would otherwise wait for its matrices' first read from memory.
+// Each wave touches one 64-line piece; workgroups b, b + 8, ... share an XCD.
+__device__ __forceinline__ uint32_t warm_l2(const GAS double *P, int n_mats, const DevOp *ops, int n_ops, int lane) {
+  const int op_lines = (n_ops * static_cast<int>(sizeof(DevOp)) + 127) / 128;
+  const int pieces = (n_mats + op_lines + 63) / 64;
+  const int line = (static_cast<int>(blockIdx.x >> 3) % pieces) * 64 + lane;
+  uint32_t v = 0;
+  if (line < n_mats)
+    v = *reinterpret_cast<const GAS uint32_t *>(P + line * 16);
+  else if (line < n_mats + op_lines)
+    v = *(reinterpret_cast<const GAS uint32_t *>(to_global(ops)) + (line - n_mats) * 32);
+  return v;
+}
+
+// One op's descriptor in scalar registers, fetched whole: read field by
+// field where it is used, every field would be a scalar load with a wait.
+typedef int32_t i32x8 __attribute__((ext_vector_type(8), aligned(8)));
+typedef int32_t i32x2 __attribute__((ext_vector_type(2), aligned(8)));
+struct OpRegs {
+  i32x8 a;
+  i32x2 b;
+  __device__ __forceinline__ uint32_t out() const { return a[0]; }
+  __device__ __forceinline__ int nk() const { return a[1]; }
+  __device__ __forceinline__ int32_t kid(int k) const { return a[2 + k]; }
+  __device__ __forceinline__ uint32_t edge(int k) const { return a[4 + k]; }
+  __device__ __forceinline__ int root() const { return a[6]; }
+  __device__ __forceinline__ int flags() const { return a[7]; }
+  __device__ __forceinline__ bool has(int f0, int f1, int k) const { return (a[7] & (k == 0 ? f0 : f1)) != 0; }
+  __device__ __forceinline__ int gslot() const { return b[0]; }
+};
+static_assert(sizeof(DevOp) == 40, "OpRegs restates DevOp");
+__device__ __forceinline__ OpRegs fetch_op(const CAS DevOp *ops, int t) {
+  OpRegs r;
+  r.a = *reinterpret_cast<const CAS i32x8 *>(ops + t);
+  r.b = *reinterpret_cast<const CAS i32x2 *>(reinterpret_cast<const CAS int32_t *>(ops + t) + 8);
+  return r;
+}
+__device__ __forceinline__ void arrive(OpRegs &r) { asm volatile("" : "+s"(r.a), "+s"(r.b)); }
+
 template <int C, int NQ>
 struct FwdIn4 {
   double A[2 * Quad<C, NQ>::NA];  // P of both children
   double x[2 * NQ];               // children read from HBM
-  uint32_t raw[2];                // their scaler words, or a tip child's mask words
+  uint32_t raw[2];                // the children's scaler words, or tip mask words
 };
 
 // Scaler words: 2 x (rescalings below and at this CLV) + (rescaled here).
@@ -641,7 +682,7 @@ __global__ void __launch_bounds__(64, 3)
   constexpr int NA = W::NA, SPW = W::SPW;
   const CAS DevOp *ops = to_constant(ops_);
   const int lane = threadIdx.x, state = lane >> 4;
-  const int64_t n = L.n_sites_pad, row = n * (C * 4);
+  const uint64_t n = L.n_sites_pad, row = n * (C * 4);
   const int64_t site0 = static_cast<int64_t>(blockIdx.x) * SPW;
   const int part = to_constant(tile_part)[site0 / TILE];
   double *slots = dyn_lds<double>();  // [slot][granule][lane], then the slots' scaler words
@@ -658,58 +699,59 @@ __global__ void __launch_bounds__(64, 3)
   const double w = weights[site0 + lane % SPW];
   const double pi_c = freqs[part * 4 + state] * (1.0 / C);
 
-  auto load = [&](const DevOp &op, FwdIn4<C, NQ> &in) {
+  auto load = [&](const OpRegs &op, FwdIn4<C, NQ> &in) {
 #pragma unroll
     for (int k = 0; k < 2; ++k)
 #pragma unroll
-      for (int h = 0; h < NA; ++h) in.A[k * NA + h] = *at(P + op.edge[k] * (C * 16), aoff[h]);
+      for (int h = 0; h < NA; ++h) in.A[k * NA + h] = *at(P + op.edge(k) * (C * 16), aoff[h]);
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-      if (k >= op.nk) continue;
-      const int64_t kid = op.kid[k];
-      if (kid < 0) {
-        in.raw[k] = *at(reinterpret_cast<const GAS uint32_t *>(tips + (-kid - 1) * n), woff);
-      } else if (!(op.flags & (k == 0 ? OP_PASS_KID0 : OP_PASS_KID1))) {
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) in.x[k * NQ + q] = *at(clv + kid * row, off + q * 512);
-        in.raw[k] = static_cast<uint32_t>(*at(scl + kid * n, soff));
-      }
+      // a tip's mask words, or the row's scaler words (a one-child op's
+      // second child stands for its first)
+      const int32_t kid = k < op.nk() ? op.kid(k) : op.kid(0);
+      const GAS char *tip = reinterpret_cast<const GAS char *>(tips) + static_cast<uint32_t>(~kid) * n;
+      const GAS char *word = reinterpret_cast<const GAS char *>(scl) + static_cast<uint32_t>(kid) * (n * 4);
+      in.raw[k] = *at(reinterpret_cast<const GAS uint32_t *>(kid < 0 ? tip : word), kid < 0 ? woff : soff);
     }
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      if (op.has(OP_LOAD0, OP_LOAD1, k))
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+          in.x[k * NQ + q] = *at(clv + static_cast<uint32_t>(op.kid(k)) * row, off + q * 512);
   };
   // y = P x of child k
-  auto child = [&](const DevOp &op, const FwdIn4<C, NQ> &in, int k, double (&y)[NQ], uint32_t &count) {
-    double x[NQ];
-    if (op.kid[k] < 0) {
+  auto child = [&](const OpRegs &op, FwdIn4<C, NQ> &in, int k, double (&y)[NQ], uint32_t &count) {
+    uint32_t below = in.raw[k] >> 1;
+    if (op.kid(k) < 0) {
 #pragma unroll
-      for (int q = 0; q < NQ; ++q) x[q] = tip_entry<C, NQ>(in.raw[k], q, lane, tip_shift);
-    } else if (op.flags & (k == 0 ? OP_PASS_KID0 : OP_PASS_KID1)) {
-      const int slot = pass_slot(op.flags, k);
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) x[q] = slots[slot * (NQ * 64) + q * 64 + lane];
-      count += slot_scl[slot * 64 + lane] >> 1;
-    } else {
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) x[q] = in.x[k * NQ + q];
-      count += in.raw[k] >> 1;
+      for (int q = 0; q < NQ; ++q) in.x[k * NQ + q] = tip_entry<C, NQ>(in.raw[k], q, lane, tip_shift);
+      below = 0;
     }
+    if (op.has(OP_PASS_KID0, OP_PASS_KID1, k)) {
+      const int slot = pass_slot(op.flags(), k);
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) y[q] = mfma4(in.A[k * NA + W::half(q)], x[q], 0.0);
+      for (int q = 0; q < NQ; ++q) in.x[k * NQ + q] = slots[slot * (NQ * 64) + q * 64 + lane];
+      below = slot_scl[slot * 64 + lane] >> 1;
+    }
+    count += below;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) y[q] = mfma4(in.A[k * NA + W::half(q)], in.x[k * NQ + q], 0.0);
   };
-  auto step = [&](int t, FwdIn4<C, NQ> &in, FwdIn4<C, NQ> &next) {
-    const DevOp op = ops[t];
+  // op t with its inputs `in`; loads those of op t + 1 and fetches op t + 2
+  auto step = [&](int t, const OpRegs &op, OpRegs &ahead, OpRegs &after, FwdIn4<C, NQ> &in, FwdIn4<C, NQ> &next) {
     arrive(in.A);
     arrive(in.x);
     arrive(in.raw);
+    arrive(ahead);
     __builtin_amdgcn_sched_barrier(0);
-    {
-      const DevOp ahead = ops[min(t + 1, n_ops - 1)];
-      load(ahead, next);
-    }
+    load(ahead, next);
+    after = fetch_op(ops, min(t + 2, n_ops - 1));
     __builtin_amdgcn_sched_barrier(0);
     double v[NQ];
     uint32_t count = 0;
     child(op, in, 0, v, count);
-    if (op.nk == 2) {
+    if (op.nk() == 2) {
       double y[NQ];
       child(op, in, 1, y, count);
 #pragma unroll
@@ -732,15 +774,15 @@ __global__ void __launch_bounds__(64, 3)
       if ((sites >> (lane % SPW)) & 1) word += 3;
     }
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) *at(clv + op.out * row, off + q * 512) = v[q];
-    *at(scl + op.out * n, soff) = static_cast<int32_t>(word);  // lanes of a site store the same word
-    if (op.flags & OP_A_PASS) {
-      const int slot = pass_slot(op.flags, 2);
+    for (int q = 0; q < NQ; ++q) *at(clv + op.out() * row, off + q * 512) = v[q];
+    *at(scl + op.out() * n, soff) = static_cast<int32_t>(word);  // lanes of a site store the same word
+    if (op.flags() & OP_A_PASS) {
+      const int slot = pass_slot(op.flags(), 2);
 #pragma unroll
       for (int q = 0; q < NQ; ++q) slots[slot * (NQ * 64) + q * 64 + lane] = v[q];
       slot_scl[slot * 64 + lane] = word;
     }
-    if (op.root >= 0) {
+    if (op.root() >= 0) {
       // site likelihoods Ltilde = (1/C) sum_c pi . x: the sum over the states
       // as a product with rows pi / C (every row of D holds it), then over
       // the categories; lane l takes site l % SPW
@@ -756,16 +798,30 @@ __global__ void __launch_bounds__(64, 3)
       const double wk = lane < SPW ? w : 0.0;
       const double val = wk != 0.0 ? wk * (log(t_site) + static_cast<double>(word >> 1) * LOG_SCALE_THRESHOLD) : 0.0;
       const double sum = wave_sum(val);
-      if (lane == 0) root_partials[static_cast<int64_t>(op.root) * gridDim.x + blockIdx.x] = sum;
+      if (lane == 0) root_partials[static_cast<int64_t>(op.root()) * gridDim.x + blockIdx.x] = sum;
       // the adjoint's seed factor at this root and site, w / (C Ltilde)
-      seed[op.root * n + site0 + lane % SPW] = w != 0.0 ? w * (1.0 / C) / t_site : 0.0;
+      seed[op.root() * n + site0 + lane % SPW] = w != 0.0 ? w * (1.0 / C) / t_site : 0.0;
     }
   };
-  FwdIn4<C, NQ> a, b;
-  load(ops[0], a);
+  OpRegs op0 = fetch_op(ops, 0), op1 = fetch_op(ops, min(1, n_ops - 1));
+  uint32_t warm[1] = {warm_l2(P, L.n_edges * C, ops_, n_ops, lane)};
+  FwdIn4<C, NQ> a;
+  load(op0, a);
+  arrive(warm);
+  // complete before the loop, so that the waits inside it count only what the
+  // step before issued (its stores need not have ended)
+  arrive(a.A);
+  arrive(a.x);
+  arrive(a.raw);
   for (int t = 0; t < n_ops; t += 2) {
-    step(t, a, b);
-    if (t + 1 < n_ops) step(t + 1, b, a);
+    FwdIn4<C, NQ> b, c;  // what an op does not load stays undefined: nothing is carried over
+    OpRegs op2, op3;
+    step(t, op0, op1, op2, a, b);
+    if (t + 1 >= n_ops) break;
+    step(t + 1, op1, op2, op3, b, c);
+    a = c;
+    op0 = op2;
+    op1 = op3;
   }
 }
 
@@ -808,7 +864,7 @@ __global__ void __launch_bounds__(64, 3)
   constexpr int NA = W::NA, SPW = W::SPW;
   const CAS DevOp *ops = to_constant(ops_);
   const int lane = threadIdx.x, state = lane >> 4;
-  const int64_t n = L.n_sites_pad, row = n * (C * 4);
+  const uint64_t n = L.n_sites_pad, row = n * (C * 4);
   const int64_t site0 = static_cast<int64_t>(blockIdx.x) * SPW;
   const int part = to_constant(tile_part)[site0 / TILE];
   double *ring = dyn_lds<double>();
@@ -831,37 +887,35 @@ __global__ void __launch_bounds__(64, 3)
   }
   const double pi = freqs[part * 4 + state];
 
-  auto load = [&](const DevOp &op, AdjIn4<C, NQ> &in) {
+  auto load = [&](const OpRegs &op, AdjIn4<C, NQ> &in) {
 #pragma unroll
     for (int k = 0; k < 2; ++k)
 #pragma unroll
       for (int h = 0; h < NA; ++h) {
-        in.A[k * NA + h] = *at(P + op.edge[k] * (C * 16), aoff[h]);
-        in.AT[k * NA + h] = *at(P + op.edge[k] * (C * 16), toff[h]);
+        in.A[k * NA + h] = *at(P + op.edge(k) * (C * 16), aoff[h]);
+        in.AT[k * NA + h] = *at(P + op.edge(k) * (C * 16), toff[h]);
       }
-    in.word[0] = static_cast<uint32_t>(*at(scl + op.out * n, soff));
+    in.word[0] = static_cast<uint32_t>(*at(scl + op.out() * n, soff));
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-      if (k >= op.nk) continue;
-      const int64_t kid = op.kid[k];
-      if (kid < 0) {
-        in.raw[k] = *at(reinterpret_cast<const GAS uint32_t *>(tips + (-kid - 1) * n), woff);
-      } else {
+      // (a one-child op's second child stands for its first)
+      const int32_t kid = k < op.nk() ? op.kid(k) : op.kid(0);
+      if (kid < 0)
+        in.raw[k] = *at(reinterpret_cast<const GAS uint32_t *>(tips + static_cast<uint32_t>(~kid) * n), woff);
+      else if (k < op.nk())
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) in.x[k * NQ + q] = *at(clv + kid * row, off + q * 512);
-      }
+        for (int q = 0; q < NQ; ++q) in.x[k * NQ + q] = *at(clv + static_cast<uint32_t>(kid) * row, off + q * 512);
     }
-    if ((op.flags & (OP_HAS_CONSUMERS | OP_A_PASS | OP_A_LATE)) == OP_HAS_CONSUMERS)
+    if ((op.flags() & (OP_HAS_CONSUMERS | OP_A_PASS | OP_A_LATE)) == OP_HAS_CONSUMERS)
 #pragma unroll
-      for (int q = 0; q < NQ; ++q) in.a[q] = *at(adj + op.out * row, off + q * 512);
-    if (op.root >= 0) in.sd[0] = seed[op.root * n + site0 + lane % SPW];
+      for (int q = 0; q < NQ; ++q) in.a[q] = *at(adj + op.out() * row, off + q * 512);
+    if (op.root() >= 0) in.sd[0] = seed[op.root() * n + site0 + lane % SPW];
   };
   // back-propagated vectors to child k's adjoint
-  auto deliver = [&](const DevOp &op, const AdjIn4<C, NQ> &in, int k, const double (&z)[NQ], double (&b)[NQ]) {
-    const bool first = (op.flags & (k == 0 ? OP_FIRST_KID0 : OP_FIRST_KID1)) != 0;
-    const bool pass = (op.flags & (k == 0 ? OP_PASS_KID0 : OP_PASS_KID1)) != 0;
-    double *slot = slots + pass_slot(op.flags, k) * (NQ * 64) + lane;
-    GAS double *dst = adj + static_cast<int64_t>(op.kid[k]) * row;
+  auto deliver = [&](const OpRegs &op, const AdjIn4<C, NQ> &in, int k, const double (&z)[NQ], double (&b)[NQ]) {
+    const bool first = op.has(OP_FIRST_KID0, OP_FIRST_KID1, k), pass = op.has(OP_PASS_KID0, OP_PASS_KID1, k);
+    double *slot = slots + pass_slot(op.flags(), k) * (NQ * 64) + lane;
+    GAS double *dst = adj + static_cast<uint32_t>(op.kid(k)) * row;
     if (pass && !first) {
 #pragma unroll
       for (int q = 0; q < NQ; ++q) b[q] = slot[q * 64];
@@ -876,22 +930,16 @@ __global__ void __launch_bounds__(64, 3)
       for (int q = 0; q < NQ; ++q) *at(dst, off + q * 512) = b[q];
     }
   };
-  auto product = [&](const DevOp &op, const AdjIn4<C, NQ> &in, int k, double (&y)[NQ]) {
-    double x[NQ];
-    if (op.kid[k] < 0) {
+  auto product = [&](const OpRegs &op, AdjIn4<C, NQ> &in, int k, double (&y)[NQ]) {
+    if (op.kid(k) < 0)
 #pragma unroll
-      for (int q = 0; q < NQ; ++q) x[q] = tip_entry<C, NQ>(in.raw[k], q, lane, tip_shift);
-    } else {
+      for (int q = 0; q < NQ; ++q) in.x[k * NQ + q] = tip_entry<C, NQ>(in.raw[k], q, lane, tip_shift);
 #pragma unroll
-      for (int q = 0; q < NQ; ++q) x[q] = in.x[k * NQ + q];
-    }
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) y[q] = mfma4(in.A[k * NA + W::half(q)], x[q], 0.0);
+    for (int q = 0; q < NQ; ++q) y[q] = mfma4(in.A[k * NA + W::half(q)], in.x[k * NQ + q], 0.0);
   };
-  const int last = ops[n_ops - 1].gslot[0];  // the sweep's first gradient row
-  int flushed = last;
-  auto step = [&](int t, AdjIn4<C, NQ> &in, AdjIn4<C, NQ> &next) {
-    const DevOp op = ops[t];
+  int flushed = ops[n_ops - 1].gslot[0];  // the sweep's first gradient row
+  // op t with its inputs `in`; loads those of op t - 1 and fetches op t - 2
+  auto step = [&](int t, const OpRegs &op, OpRegs &ahead, OpRegs &after, AdjIn4<C, NQ> &in, AdjIn4<C, NQ> &next) {
     arrive(in.A);
     arrive(in.AT);
     arrive(in.x);
@@ -899,6 +947,7 @@ __global__ void __launch_bounds__(64, 3)
     arrive(in.sd);
     arrive(in.raw);
     arrive(in.word);
+    arrive(ahead);
     __builtin_amdgcn_sched_barrier(0);
     // what the children's adjoints hold already, where no slot does (the
     // deliveries before this op's are stores of this wave, so in order)
@@ -907,39 +956,37 @@ __global__ void __launch_bounds__(64, 3)
     for (int k = 0; k < 2; ++k) {
 #pragma unroll
       for (int q = 0; q < NQ; ++q) acc[k][q] = 0.0;
-      if (op.flags & (k == 0 ? OP_ACC0 : OP_ACC1))
+      if (op.has(OP_ACC0, OP_ACC1, k))
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) acc[k][q] = *at(adj + op.kid[k] * row, off + q * 512);
+        for (int q = 0; q < NQ; ++q) acc[k][q] = *at(adj + static_cast<uint32_t>(op.kid(k)) * row, off + q * 512);
     }
-    {
-      const DevOp ahead = ops[max(t - 1, 0)];
-      load(ahead, next);
-    }
+    load(ahead, next);
+    after = fetch_op(ops, max(t - 2, 0));
     __builtin_amdgcn_sched_barrier(0);
     double a[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) a[q] = 0.0;
-    if (op.flags & OP_A_PASS) {
-      const double *slot = slots + pass_slot(op.flags, 2) * (NQ * 64) + lane;
+    if (op.flags() & OP_A_PASS) {
+      const double *slot = slots + pass_slot(op.flags(), 2) * (NQ * 64) + lane;
 #pragma unroll
       for (int q = 0; q < NQ; ++q) a[q] = slot[q * 64];
-    } else if (op.flags & OP_A_LATE) {
+    } else if (op.flags() & OP_A_LATE) {
 #pragma unroll
-      for (int q = 0; q < NQ; ++q) a[q] = *at(adj + op.out * row, off + q * 512);
+      for (int q = 0; q < NQ; ++q) a[q] = *at(adj + op.out() * row, off + q * 512);
       wait_loads();
-    } else if (op.flags & OP_HAS_CONSUMERS) {
+    } else if (op.flags() & OP_HAS_CONSUMERS) {
 #pragma unroll
       for (int q = 0; q < NQ; ++q) a[q] = in.a[q];
     }
-    if (op.root >= 0) {
+    if (op.root() >= 0) {
       // seed beta * w * (1/C) pi_i / Ltilde at a displayed-tree root
-      const double f = beta[part * n_root + op.root] * in.sd[0];
+      const double f = beta[part * n_root + op.root()] * in.sd[0];
 #pragma unroll
       for (int q = 0; q < NQ; ++q) a[q] = fma(__shfl(f, W::site(lane, q)), pi, a[q]);
     }
     if (keep)  // the model gradient reads every adjoint
 #pragma unroll
-      for (int q = 0; q < NQ; ++q) *at(adj + op.out * row, off + q * 512) = a[q];
+      for (int q = 0; q < NQ; ++q) *at(adj + op.out() * row, off + q * 512) = a[q];
     const uint64_t scaled = __builtin_amdgcn_ballot_w64(lane < SPW && (in.word[0] & 1u));
     if (scaled)
 #pragma unroll
@@ -949,10 +996,10 @@ __global__ void __launch_bounds__(64, 3)
     auto use = [&](int k) {
 #pragma unroll
       for (int q = 0; q < NQ; ++q) g[k] = fma(z[q], mfma4(Q[W::half(q)], y[k][q], 0.0), g[k]);
-      if (op.kid[k] >= 0) deliver(op, in, k, z, acc[k]);
+      if (op.kid(k) >= 0) deliver(op, in, k, z, acc[k]);
     };
     product(op, in, 0, y[0]);
-    if (op.nk == 2) {
+    if (op.nk() == 2) {
       product(op, in, 1, y[1]);
 #pragma unroll
       for (int q = 0; q < NQ; ++q) z[q] = a[q] * y[1][q];
@@ -969,19 +1016,28 @@ __global__ void __launch_bounds__(64, 3)
     // GRAD_RING], and 64 at a time leave as one store
     const double total = pair_wave_sum(g[0], g[1]);
     const int k = lane >> 5;
-    if ((lane & 31) == 31 && k < op.nk) ring[(op.gslot[0] + k) % GRAD_RING] = total;
-    const int done = op.gslot[0] + op.nk;
+    if ((lane & 31) == 31 && k < op.nk()) ring[(op.gslot() + k) % GRAD_RING] = total;
+    const int done = op.gslot() + op.nk();
     if (done - flushed >= 64) {
       grad[flushed + lane] = ring[(flushed + lane) % GRAD_RING];
       flushed += 64;
     }
     if (t == 0 && lane < done - flushed) grad[flushed + lane] = ring[(flushed + lane) % GRAD_RING];
   };
-  AdjIn4<C, NQ> u, v;
-  load(ops[n_ops - 1], u);
+  OpRegs op0 = fetch_op(ops, n_ops - 1), op1 = fetch_op(ops, max(n_ops - 2, 0));
+  uint32_t warm[1] = {warm_l2(P, L.n_edges * C, ops_, n_ops, lane)};
+  AdjIn4<C, NQ> u;
+  load(op0, u);
+  arrive(warm);
   for (int t = n_ops - 1; t >= 0; t -= 2) {
-    step(t, u, v);
-    if (t > 0) step(t - 1, v, u);
+    AdjIn4<C, NQ> v, w;  // what an op does not load stays undefined: nothing is carried over
+    OpRegs op2, op3;
+    step(t, op0, op1, op2, u, v);
+    if (t == 0) break;
+    step(t - 1, op1, op2, op3, v, w);
+    u = w;
+    op0 = op2;
+    op1 = op3;
   }
 }
 

@@ -122,7 +122,7 @@ void assign_forward_slots(DevOp *ops, int n, int n_slots) {
   std::vector<int> row_in(n_slots, -1), read_at(n_slots, NEVER);
   for (int i = 0; i < n; ++i) {
     DevOp &op = ops[i];
-    op.flags &= ~(OP_PASS_KID0 | OP_PASS_KID1 | OP_A_PASS | PASS_BITS);
+    op.flags &= ~(OP_PASS_KID0 | OP_PASS_KID1 | OP_A_PASS | PASS_BITS | OP_LOAD0 | OP_LOAD1);
     for (int k = 0; k < op.nk; ++k) {
       if (op.kid[k] < 0) continue;
       const auto it = std::find(row_in.begin(), row_in.end(), op.kid[k]);
@@ -130,9 +130,11 @@ void assign_forward_slots(DevOp *ops, int n, int n_slots) {
         const int q = static_cast<int>(it - row_in.begin());
         op.flags |= (k == 0 ? OP_PASS_KID0 : OP_PASS_KID1) | (q << (PASS_SHIFT + 3 * k));
         read_at[q] = later[i][k];
-      } else if (made[op.kid[k]] == i - 1 && i > 0) {
+      } else {
         // the kernel loads an op's inputs before the op before it stores
-        throw std::logic_error("forward walk: a child is read from HBM right after it was made");
+        if (made[op.kid[k]] == i - 1 && i > 0)
+          throw std::logic_error("forward walk: a child is read from HBM right after it was made");
+        op.flags |= k == 0 ? OP_LOAD0 : OP_LOAD1;
       }
     }
     for (int q = 0; q < n_slots; ++q)

@@ -31,7 +31,7 @@ std::vector<int> depth_first_order(const Dag &dag, const std::vector<int> &root_
 // LDS slots of the forward walk over ops[0, n) (OP_PASS_KID*: the child is
 // read from the slot its op left it in; OP_A_PASS: the op leaves its CLV in
 // a slot), of which the wave has n_slots (2 to WALK_SLOTS).  Rows are the
-// numbers in the ops; a child no slot holds is read from HBM.
+// numbers in the ops; a child no slot holds is read from HBM (OP_LOAD*).
 void assign_forward_slots(DevOp *ops, int n, int n_slots);
 
 // LDS slots and load flags (OP_PASS_*, OP_A_PASS, OP_A_LATE, OP_ACC*)
