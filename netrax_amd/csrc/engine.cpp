@@ -282,6 +282,19 @@ static void plan_budget(Engine &e) {
   resize_rows(e, bp.n_phys);
 }
 
+constexpr int CUS = 256, LDS_PER_CU = 160 * 1024, LDS_PER_GROUP = 64 * 1024;
+
+// LDS slots per wave of a walk of `waves` waves.
+template <typename Lds>
+static int walk_slots(int64_t waves, Lds &&lds) {
+  const int per_cu = static_cast<int>(std::min<int64_t>(12, (waves + CUS - 1) / CUS));
+  // (LDS is given out in pieces of 1280 bytes)
+  const size_t most = std::min<size_t>(LDS_PER_CU / per_cu / 1280 * 1280, LDS_PER_GROUP);
+  int n = 2;
+  while (n < WALK_SLOTS && lds(n + 1) <= most) ++n;
+  return n;
+}
+
 // Granules and LDS slots per wave of the 4-state FP64 walks.  Four granules
 // share an op's fixed work best (41,345 patterns x 4 categories, gradient:
 // 0.66 ms, 0.92 with two, 1.00 with one); fewer once they would leave SIMDs
@@ -289,21 +302,40 @@ static void plan_budget(Engine &e) {
 // 53.4 / 50.8 / 50.4 us).  As many slots as let the launch's waves, at most
 // three per SIMD, be resident together.
 static void choose_walk_shape(Engine &e) {
-  constexpr int CUS = 256, LDS_PER_CU = 160 * 1024, SIMDS = 4 * CUS;
   const int64_t granules = e.L.n_sites_pad * e.C / 16;
   const int least = e.C == 8 ? 2 : 1;
   e.walk_nq = e.C == 8 ? 2 : 4;
-  while (e.walk_nq > least && granules / e.walk_nq < SIMDS) e.walk_nq /= 2;
+  while (e.walk_nq > least && granules / e.walk_nq < 4 * CUS) e.walk_nq /= 2;
   e.rpw = TILE * e.C / (16 * e.walk_nq);
-  const int64_t waves = granules / e.walk_nq;
-  const int per_cu = static_cast<int>(std::min<int64_t>(12, (waves + CUS - 1) / CUS));
-  auto slots = [&](auto lds) {
-    int n = 2;
-    while (n < WALK_SLOTS && lds(e.walk_nq, n + 1) <= static_cast<size_t>(LDS_PER_CU / per_cu)) ++n;
-    return n;
-  };
-  e.fwd_slots = slots(forward_walk_lds);
-  e.adj_slots = slots(adjoint_walk_lds);
+  e.fwd_slots = walk_slots(granules / e.walk_nq, [&](int n) { return forward_walk_lds(e.walk_nq, n); });
+  e.adj_slots = walk_slots(granules / e.walk_nq, [&](int n) { return adjoint_walk_lds(e.walk_nq, n); });
+}
+
+// 64-row blocks per wave of the FP32 walks, `blocks` of them in a launch: two
+// share an op's fixed work once a launch fills the GPU either way (batch of 32
+// networks, 387,000 patterns, gradients: 2.41 ms against 2.86; 41,345 patterns:
+// 0.44 against 0.41, 1,294 waves leaving most SIMDs one).  Group widths 2 and
+// 3 of a tuned shape name two and one.
+static int walk_blocks_of(int tune_group, int64_t blocks) {
+  if (tune_group == 2 || tune_group == 3) return tune_group == 2 ? 2 : 1;
+  return blocks / 2 >= 8 * CUS ? 2 : 1;
+}
+
+// LDS slots of the FP32 walks for a launch of `blocks` 64-row blocks.
+static void choose_slots32(Engine &e, int64_t blocks) {
+  e.rpw = e.C / e.walk_blocks;
+  e.fwd_slots = walk_slots(blocks / e.walk_blocks, [&](int n) { return forward_lds32(e.C, e.walk_blocks, n); });
+  e.adj_slots = walk_slots(blocks / e.walk_blocks, [&](int n) { return adjoint_lds32(e.C, e.walk_blocks, n); });
+}
+
+// The walks' two op lists with their slots.
+static void assign_walk_slots(Engine &e) {
+  const int n = static_cast<int>(e.ops_all.size());
+  e.ops_fwd = e.ops_adj = e.ops_all;
+  assign_forward_slots(e.ops_fwd.data(), n, e.fwd_slots);
+  assign_reverse_slots(e.ops_adj.data(), n, e.adj_slots);
+  upload(e.d_ops_fwd, e.ops_fwd, e.stream);
+  upload(e.d_ops_adj, e.ops_adj, e.stream);
 }
 
 // Builds the level schedule, the batched order, root CLV set and gradient
@@ -387,18 +419,15 @@ static void build_schedule(Engine &e) {
     set_adjoint_flags(e.ops_all, order, nv);
   }
 
-  // batched form (FP32): groups of up to tune_group independent ops in
-  // depth-first priority, then the LDS pass slots of the 4-state sweep
-  {
+  // 20 states FP32: groups of up to tune_group independent ops in
+  // depth-first priority
+  e.ops_dfs.clear();
+  e.group_begin.assign(1, 0);
+  if (!e.walks()) {
     std::vector<DevOp> proto(nv);
     for (int v = 0; v < nv; ++v)
       if (e.needed[v]) proto[v] = make_op(v);
     build_batched_order(e.dag, e.root_slots, proto, e.tune_group, e.ops_dfs, e.group_begin);
-    e.pass_slots = 0;
-    if (e.S == 4 && e.opt.precision == NRX_FP32)
-      e.pass_slots = adjoint_pass_slots(e.C, e.tune_group, e.tune_tile, e.tune_lanes, e.E,
-                                        e.L.n_sites_pad / e.tune_tile);
-    set_pass_slots(e.ops_dfs, e.group_begin, nv, e.pass_slots);
   }
 
   // gradient rows, one per (op, child), numbered in the order this engine's
@@ -406,8 +435,9 @@ static void build_schedule(Engine &e) {
   // backwards), so that a workgroup's consecutive ops write consecutive rows
   {
     std::vector<int> walk;  // indices into the form's op list
-    std::vector<DevOp> &ops = e.opt.precision == NRX_FP32 ? e.ops_dfs : e.ops_all;
-    if (e.opt.precision == NRX_FP32) {
+    const bool grouped = e.opt.precision == NRX_FP32 && !e.walks();
+    std::vector<DevOp> &ops = grouped ? e.ops_dfs : e.ops_all;
+    if (grouped) {
       for (int g = static_cast<int>(e.group_begin.size()) - 2; g >= 0; --g)
         for (int i = e.group_begin[g]; i < e.group_begin[g + 1]; ++i) walk.push_back(i);
     } else {
@@ -445,13 +475,15 @@ static void build_schedule(Engine &e) {
   }
   upload(e.d_ops, e.ops_all, e.stream);
   if (e.walks()) {
-    choose_walk_shape(e);
-    const int n_ops = static_cast<int>(e.ops_all.size());
-    e.ops_fwd = e.ops_adj = e.ops_all;
-    assign_forward_slots(e.ops_fwd.data(), n_ops, e.fwd_slots);
-    assign_reverse_slots(e.ops_adj.data(), n_ops, e.adj_slots);
-    upload(e.d_ops_fwd, e.ops_fwd, e.stream);
-    upload(e.d_ops_adj, e.ops_adj, e.stream);
+    if (e.opt.precision == NRX_FP64) {
+      choose_walk_shape(e);
+    } else {
+      const int64_t blocks = e.L.n_sites_pad * e.C / 64;
+      // (a single 64-site tile of 1 category is one block)
+      e.walk_blocks = e.C == 1 ? 1 : walk_blocks_of(e.tune_group, blocks);
+      choose_slots32(e, blocks);
+    }
+    assign_walk_slots(e);
   }
   upload(e.d_ops_dfs, e.ops_dfs, e.stream);
   upload(e.d_group_begin, e.group_begin, e.stream);
@@ -461,21 +493,17 @@ static void build_schedule(Engine &e) {
   upload(e.d_class_dlogprob, e.class_dlogprob, e.stream);
   std::vector<int32_t> rs(e.root_slots.begin(), e.root_slots.end());
   upload(e.d_root_slots, rs, e.stream);
-  // gradient partials per site block: plain form a wave of the walks (4
-  // states) or 64-site tiles of C waves; FP32 form its reverse-sweep workgroups (tune_tile sites of tune_lanes
-  // lanes per row, or 32 sites for 20-state data)
+  // gradient partials per site block: a wave of the walks (4 states), 64-site
+  // tiles of C waves (20 states FP64) or 32-site workgroups (FP32)
   if (e.walks()) {
     e.gpw = 1;
     e.gbpt = e.rpw;
   } else if (e.opt.precision != NRX_FP32) {
     e.gpw = TILE * e.C / 64;
     e.gbpt = 1;
-  } else if (e.S == AA_STATES) {
+  } else {
     e.gpw = e.C;
     e.gbpt = TILE / AA_TILE;
-  } else {
-    e.gpw = e.tune_tile * e.C * e.tune_lanes / 64;
-    e.gbpt = TILE / e.tune_tile;
   }
   if (e.gpw * e.gbpt < e.rpw) throw std::logic_error("gradient partial layout does not cover the tile");
   const size_t n_wt = static_cast<size_t>(e.L.n_tiles) * e.rpw;
@@ -502,7 +530,13 @@ NetDesc make_netdesc(const Engine &e) {
   d.n_groups = static_cast<int32_t>(e.group_begin.size()) - 1;
   d.n_root = static_cast<int32_t>(e.root_slots.size());
   d.n_uses = e.n_uses;
-  d.n_pass = e.pass_slots;
+  d.ops_fwd = e.d_ops_fwd.as<DevOp>();
+  d.ops_adj = e.d_ops_adj.as<DevOp>();
+  d.n_fwd = d.n_adj = static_cast<int32_t>(e.ops_all.size());
+  d.fwd_slots = e.fwd_slots;
+  d.adj_slots = e.adj_slots;
+  d.seed = e.d_site_seed.as<double>();
+  d.PfT = e.d_PfT.as<float>();
   d.clv = e.d_clv.as<float>();
   d.scl = e.d_scl.as<int32_t>();
   d.adj = e.d_adj.as<float>();
@@ -520,9 +554,10 @@ NetDesc make_netdesc(const Engine &e) {
   // every buffer the persistent kernels read must exist before its address
   // is handed to the device
   const bool aa = e.S == AA_STATES;
-  const void *need[] = {d.ops, d.group_begin, d.clv, d.scl, d.adj, d.adj_exp, d.tips,
-                        aa ? static_cast<const void *>(d.Pa) : d.Pf, d.Qf,
-                        d.tile_part, d.freqs, d.weights, d.beta, d.root_partials, d.grad_partials};
+  const void *need[] = {aa ? d.ops : d.ops_fwd, aa ? static_cast<const void *>(d.group_begin) : d.ops_adj,
+                        d.clv, d.scl, d.adj, d.adj_exp, d.tips, aa ? static_cast<const void *>(d.Pa) : d.Pf,
+                        aa ? static_cast<const void *>(d.Pa) : d.PfT, d.Qf, d.tile_part, d.freqs, d.weights, d.beta,
+                        d.root_partials, d.grad_partials, d.seed};
   for (const void *p : need)
     if (!p) throw std::logic_error("device descriptor built before its buffers were allocated");
   return d;
@@ -532,8 +567,8 @@ static void upload_netdesc(Engine &e) {
   if (e.opt.precision != NRX_FP32) return;
   std::vector<NetDesc> nd{make_netdesc(e)};
   upload(e.d_netdesc, nd, e.stream);
-  // work items: tiles of tune_tile sites, or of 32 sites for 20-state data
-  const int n_work = static_cast<int>(e.L.n_sites_pad / (e.S == AA_STATES ? AA_TILE : e.tune_tile));
+  // work items: the walks' waves, or tiles of 32 sites for 20-state data
+  const int n_work = e.L.n_tiles * (e.S == AA_STATES ? TILE / AA_TILE : e.rpw);
   std::vector<WorkItem> work(n_work);
   for (int t = 0; t < n_work; ++t) work[t] = WorkItem{0, t};
   upload(e.d_work, work, e.stream);
@@ -741,7 +776,8 @@ static void forward(Engine &e, bool incremental) {
       if (d.op_end > d.op_begin) lv.push_back(d);
     }
     if (!dirty.empty()) {
-      if (e.walks()) assign_forward_slots(dirty.data(), static_cast<int>(dirty.size()), e.fwd_slots);
+      if (e.walks())
+        assign_forward_slots(dirty.data(), static_cast<int>(dirty.size()), e.fwd_slots);
       stage_upload(e, e.d_ops_dirty, dirty);
       if (e.walks()) {
         record_kernel_begin(e, 0);
@@ -854,7 +890,26 @@ static void budget_adjoint(Engine &e) {
   }
 }
 
-// FP32 form, incremental evaluation: the ops whose CLVs are invalid, in the
+// FP32 form, 4 states, incremental evaluation: the ops whose CLVs are invalid
+// in walk order, with slots of their own.  Returns as stage_invalid_ops.
+static int stage_invalid_walk(Engine &e, const NetDesc *&desc) {
+  std::vector<DevOp> ops;
+  for (const DevOp &op : e.ops_all)
+    if (e.clv_dirty[op.out]) ops.push_back(op);
+  if (ops.size() == e.ops_all.size()) return -1;
+  const int n = static_cast<int>(ops.size());
+  if (n == 0) return 0;
+  assign_forward_slots(ops.data(), n, e.fwd_slots);
+  stage_upload(e, e.d_ops_inc, ops);
+  NetDesc d = make_netdesc(e);
+  d.ops_fwd = e.d_ops_inc.as<DevOp>();
+  d.n_fwd = n;
+  stage_upload(e, e.d_netdesc_inc, std::vector<NetDesc>{d});
+  desc = e.d_netdesc_inc.as<NetDesc>();
+  return n;
+}
+
+// FP32 form, 20 states, incremental evaluation: the ops whose CLVs are invalid, in the
 // forward order and groups of the full list (a subset of a group of
 // independent ops is independent), as a device descriptor of their own.
 // A group is flagged independent of the one before it when it reads none of
@@ -930,7 +985,7 @@ static int evaluate(Engine &e, int variant, bool incremental, bool update_pm, bo
     const bool aa32 = e.S == AA_STATES;
     const NetDesc *inc = nullptr;
     int n_inc_groups = -1;
-    if (incremental) n_inc_groups = stage_invalid_ops(e, inc);
+    if (incremental) n_inc_groups = e.walks() ? stage_invalid_walk(e, inc) : stage_invalid_ops(e, inc);
     const bool partial = n_inc_groups >= 0;
     auto enqueue = [&e, aa32, variant, gradient, pm_in_graph, inc, n_inc_groups](bool timed) {
       if (pm_in_graph) enqueue_pmatrices(e);
@@ -943,7 +998,7 @@ static int evaluate(Engine &e, int variant, bool incremental, bool update_pm, bo
         launch_forward_persistent(e, inc);
       }
       if (timed) record_kernel_end(e, 0);
-      launch_mixture(e, variant, e.pw);
+      launch_mixture(e, variant, e.rpw);
       if (gradient) {
         if (timed) record_kernel_begin(e, 1);
         if (aa32)
@@ -1195,9 +1250,10 @@ struct Batch {
   std::vector<int64_t> offsets;
   int n_work = 0, C = 0, max_pm = 0, max_root_rows = 0, max_use_rows = 0, max_edges = 0,
       max_res = 0;
-  size_t lds_fwd = 0, lds_adj = 0;
+  int fwd_slots = 0, adj_slots = 0;  // the most any engine has
   bool use_graph = false;
   int G = 4, TS = TILE, H = 1;  // shape of the persistent kernels, shared by all engines
+  int blocks = 1;               // 64-row blocks per wave, likewise
   hipGraphExec_t graph_exec[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};  // [variant][gradient]
   ~Batch() {
     if (stream) (void)hipStreamSynchronize(stream);
@@ -1221,6 +1277,7 @@ static SmallDesc make_smalldesc(const Engine &e) {
   d.dP = e.d_dP.as<double>();
   d.d2P = e.d_d2P.as<double>();
   d.Pf = e.d_Pf.as<float>();
+  d.PfT = e.d_PfT.as<float>();
   d.n_root = static_cast<int32_t>(e.root_slots.size());
   d.nc = static_cast<int32_t>(e.dag.classes.size());
   d.R = e.R;
@@ -1244,10 +1301,10 @@ static SmallDesc make_smalldesc(const Engine &e) {
   d.rl_dbrlen = e.rl.dbrlen;
   d.rl_part_dbrlen = e.rl.part_dbrlen;
   d.rl_dprob = e.rl.dprob;
-  d.pw = e.pw;
+  d.pw = e.rpw;
   d.gpw = e.gpw;
   d.gbpt = e.gbpt;
-  const void *need[] = {d.V, d.Vinv, d.ev, d.rates, d.brlen, d.P, d.dP, d.d2P, d.Pf,
+  const void *need[] = {d.V, d.Vinv, d.ev, d.rates, d.brlen, d.P, d.dP, d.d2P, d.Pf, d.PfT,
                         d.part_tile_begin, d.classes, d.class_dlogprob, d.root_partials,
                         d.root_sums, d.grad_partials, d.use_sums, d.beta, d.edge_use_begin,
                         d.edge_use_list, d.res};
@@ -1266,44 +1323,56 @@ static void build_batch(Batch &b) {
   std::vector<std::pair<int, int>> order;  // (cost, engine)
   b.offsets.assign(n + 1, 0);
   b.max_pm = b.max_root_rows = b.max_use_rows = b.max_edges = b.max_res = 0;
-  b.lds_fwd = b.lds_adj = 0;
+  b.fwd_slots = b.adj_slots = 0;
   b.versions.resize(n);
   b.G = b.engines[0]->tune_group;
   b.TS = b.engines[0]->tune_tile;
   b.H = b.engines[0]->tune_lanes;
-  // One batch launch holds far more workgroups than one engine's, so each
-  // engine keeps only as many LDS pass slots as leave the launch's
-  // workgroups per CU unchanged (a slot given up moves its deliveries back
-  // to HBM); its own graphs then re-capture.
-  int64_t total_work = 0;
-  for (const Engine *e : b.engines) total_work += e->L.n_sites_pad / b.TS;
+  for (const Engine *e : b.engines)
+    if (e->tune_group != b.G || e->tune_tile != b.TS || e->tune_lanes != b.H)
+      throw std::invalid_argument("batch engines must share the FP32 kernel shape (nrx_set_tuning)");
+  // One batch launch holds far more waves than one engine's: its engines take
+  // the wave shape of the whole (never back to one block, so that batches
+  // with an engine in common settle), and each keeps only as many LDS slots
+  // as let the launch's waves be resident (a row without a slot goes through
+  // HBM); their own graphs then re-capture.
+  int64_t blocks = 0;
+  for (const Engine *e : b.engines) blocks += e->L.n_sites_pad * e->C / 64;
+  b.blocks = b.C == 1 ? 1 : walk_blocks_of(b.G, blocks);
+  for (const Engine *e : b.engines) b.blocks = std::max(b.blocks, e->walk_blocks);
   for (Engine *e : b.engines) {
-    if (e->S != 4 || e->tune_group != b.G || e->tune_tile != b.TS || e->tune_lanes != b.H) continue;
-    const int k = adjoint_pass_slots(e->C, b.G, b.TS, b.H, e->E, total_work);
-    if (k >= e->pass_slots) continue;
-    e->pass_slots = k;
-    set_pass_slots(e->ops_dfs, e->group_begin, static_cast<int>(e->dag.var.size()), k);
-    upload(e->d_ops_dfs, e->ops_dfs, e->stream);
+    const bool reshaped = e->walk_blocks != b.blocks;
+    const int fwd = reshaped ? WALK_SLOTS : e->fwd_slots, adj = reshaped ? WALK_SLOTS : e->adj_slots;
+    e->walk_blocks = b.blocks;
+    choose_slots32(*e, blocks);
+    e->fwd_slots = std::min(fwd, e->fwd_slots);
+    e->adj_slots = std::min(adj, e->adj_slots);
+    if (reshaped) {  // the root sums and gradient rows are per wave
+      e->gbpt = e->rpw;
+      std::fill(e->clv_dirty.begin(), e->clv_dirty.end(), 1);
+      e->cache_valid = false;
+    } else if (e->fwd_slots == fwd && e->adj_slots == adj) {
+      continue;
+    }
+    assign_walk_slots(*e);
     upload_netdesc(*e);
     NRX_HIP(hipStreamSynchronize(e->stream));
     e->schedule_version++;
   }
   for (int i = 0; i < n; ++i) {
     const Engine &e = *b.engines[i];
-    if (e.tune_group != b.G || e.tune_tile != b.TS || e.tune_lanes != b.H)
-      throw std::invalid_argument("batch engines must share the FP32 kernel shape (nrx_set_tuning)");
     nets[i] = make_netdesc(e);
     small[i] = make_smalldesc(e);
     b.versions[i] = e.schedule_version;
-    order.push_back({static_cast<int>(e.ops_dfs.size()), i});
+    order.push_back({static_cast<int>(e.ops_all.size()), i});
     b.offsets[i + 1] = b.offsets[i] + e.rl.size;
     b.max_pm = std::max(b.max_pm, e.P * e.E * e.C * e.S * e.S);
     b.max_root_rows = std::max(b.max_root_rows, static_cast<int>(e.root_slots.size()) * e.P);
     b.max_use_rows = std::max(b.max_use_rows, e.n_uses * e.P);
     b.max_edges = std::max(b.max_edges, e.E);
     b.max_res = std::max(b.max_res, e.rl.size);
-    b.lds_fwd = std::max(b.lds_fwd, sizeof(float) * e.E * e.C * 16);
-    b.lds_adj = std::max(b.lds_adj, adjoint_persistent_lds(e.E, e.C, b.TS, e.pass_slots));
+    b.fwd_slots = std::max(b.fwd_slots, e.fwd_slots);
+    b.adj_slots = std::max(b.adj_slots, e.adj_slots);
   }
   std::stable_sort(order.begin(), order.end(),
                    [](const std::pair<int, int> &x, const std::pair<int, int> &y) {
@@ -1311,7 +1380,7 @@ static void build_batch(Batch &b) {
                    });
   std::vector<WorkItem> work;
   for (const auto &o : order)
-    for (int t = 0; t < b.engines[o.second]->L.n_sites_pad / b.TS; ++t) work.push_back({o.second, t});
+    for (int t = 0; t < b.engines[o.second]->L.n_tiles * b.engines[o.second]->rpw; ++t) work.push_back({o.second, t});
   b.n_work = static_cast<int>(work.size());
   upload(b.d_nets, nets, b.stream);
   upload(b.d_small, small, b.stream);
@@ -1391,13 +1460,13 @@ int nrx_batch_evaluate(nrx_batch *batch, int32_t variant, double *lnl, double *d
     auto enqueue = [&]() {
       const SmallDesc *sd = b.d_small.as<SmallDesc>();
       launch_pmatrices_multi(b.stream, sd, n, b.max_pm);
-      launch_forward_persistent_multi(b.stream, b.C, b.G, b.TS, b.d_nets.as<NetDesc>(),
-                                      b.d_work.as<WorkItem>(), b.n_work, b.lds_fwd);
+      launch_forward_persistent_multi(b.stream, b.C, b.blocks, b.d_nets.as<NetDesc>(),
+                                      b.d_work.as<WorkItem>(), b.n_work, b.fwd_slots);
       launch_root_reduce_multi(b.stream, sd, n, b.max_root_rows);
       launch_mixture_multi(b.stream, sd, n, variant);
       if (grad) {
-        launch_adjoint_persistent_multi(b.stream, b.C, b.G, b.TS, b.H, b.d_nets.as<NetDesc>(),
-                                        b.d_work.as<WorkItem>(), b.n_work, b.lds_adj);
+        launch_adjoint_persistent_multi(b.stream, b.C, b.blocks, b.d_nets.as<NetDesc>(),
+                                        b.d_work.as<WorkItem>(), b.n_work, b.adj_slots);
         launch_grad_reduce_multi(b.stream, sd, n, b.max_use_rows, b.max_edges);
       }
       launch_gather_results(b.stream, sd, n, b.d_offsets.as<int64_t>(), b.d_out.as<double>(),
@@ -1614,6 +1683,7 @@ int nrx_create(const nrx_network_desc *net, const nrx_partition_desc *parts, int
     e->d_scl.alloc(sizeof(int32_t) * static_cast<size_t>(n) * std::max<size_t>(nv, 1));
     if (e->opt.precision == NRX_FP32) {
       e->d_Pf.alloc(sizeof(float) * pm);
+      if (!aa32) e->d_PfT.alloc(sizeof(float) * pm);
       e->d_adj.alloc(sizeof(float) * e->clv_elems_per_slot * std::max<size_t>(nv, 1));
       // adjoint exponents: per site (4 states) or per (site, category) (20 states)
       const size_t per_slot = aa32 ? static_cast<size_t>(n) * e->C : static_cast<size_t>(n);
@@ -2342,7 +2412,7 @@ int nrx_get_stats(nrx_engine *eng, nrx_stats *out) {
     const bool fp32 = e.opt.precision == NRX_FP32;
     const double aexp = fp32 ? (e.S == AA_STATES ? scl * e.C : scl) : 0.0;
     const bool pass = e.S == 4;
-    const std::vector<DevOp> &adj_ops = fp32 ? e.ops_dfs : e.walks() ? e.ops_adj : e.ops_all;
+    const std::vector<DevOp> &adj_ops = e.walks() ? e.ops_adj : fp32 ? e.ops_dfs : e.ops_all;
     out->n_lds_handoffs = 0;
     if (pass)
       for (const DevOp &op : adj_ops)
@@ -2351,7 +2421,7 @@ int nrx_get_stats(nrx_engine *eng, nrx_stats *out) {
     for (const DevOp &op : adj_ops) {
       adj += scl;
       if ((op.flags & OP_HAS_CONSUMERS) && !(pass && (op.flags & OP_A_PASS))) adj += row + aexp;
-      if (op.root >= 0) adj += fp32 ? row : 8.0 * sites;
+      if (op.root >= 0) adj += fp32 && !e.walks() ? row : 8.0 * sites;
       for (int k = 0; k < op.nk; ++k) {
         if (op.kid[k] < 0) {
           adj += tip_b;
@@ -2475,10 +2545,10 @@ int nrx_batch_optimize(nrx_batch *batch, int32_t variant, int32_t mode, const in
 
 namespace nrx {
 
-// Shapes of the FP32 form's persistent kernels: 4-state data takes G ops
-// per group, TS sites per workgroup (TS C threads, a multiple of 64) and H
-// lanes per (site, category) row in the reverse sweep; 20-state data has 32
-// sites per workgroup and tunes G only.
+// Shapes of the FP32 form's kernels.  20-state data has 32 sites per
+// workgroup and tunes the group width g.  For 4-state data g chooses the row
+// blocks of a wave (walk_blocks_of); ts and h are part of a shape's name and
+// choose nothing.
 struct Shape {
   int g, ts, h;
   bool operator==(const Shape &o) const { return g == o.g && ts == o.ts && h == o.h; }
@@ -2552,6 +2622,15 @@ int nrx_autotune(nrx_engine *eng, int32_t variant, int32_t reps, nrx_tuning *bes
     int rc = NRX_OK;
     try {
       for (size_t i = 0; i < cands.size() && rc == NRX_OK; ++i) {
+        if (e.walks()) {  // shapes that run the same kernels are timed once
+          const int64_t blocks = e.L.n_sites_pad * e.C / 64;
+          size_t j = 0;
+          while (walk_blocks_of(cands[j].g, blocks) != walk_blocks_of(cands[i].g, blocks)) ++j;
+          if (j < i) {
+            ms[i] = ms[j];
+            continue;
+          }
+        }
         apply_shape(e, cands[i]);
         rc = evaluate(e, variant, false, true, true);  // warm-up (and graph capture)
         for (int r = 0; r < reps && rc == NRX_OK; ++r) {

@@ -80,7 +80,10 @@ struct DevOp {
   int32_t root;      // index of the root-CLV site sum this op feeds, or -1
   int32_t flags;     // OP_HAS_CONSUMERS | OP_FIRST_KID0 | OP_FIRST_KID1
   int32_t gslot[2];  // gradient-partial row of (this op, child k)
+  int32_t slots;     // 4-state walks: LDS slots of the uses 0, 1 (children) and 2 (own row), see walk_slot
+  int32_t pad;
 };
+inline __host__ __device__ int walk_slot(const DevOp &op, int u) { return (op.slots >> (8 * u)) & 255; }
 constexpr int32_t OP_HAS_CONSUMERS = 1;  // adjoint of `out` was accumulated by consumers
 constexpr int32_t OP_FIRST_KID0 = 2;     // first consumer of kid[0] in adjoint order
 constexpr int32_t OP_FIRST_KID1 = 4;
@@ -102,17 +105,17 @@ constexpr int32_t OP_ACC_EARLY1 = 32;
 constexpr int32_t OP_PASS_KID0 = 64;
 constexpr int32_t OP_PASS_KID1 = 128;
 constexpr int32_t OP_A_PASS = 256;
-// FP64 form, 4 states: the op's own adjoint lies in HBM and the op before it
+// 4-state walks (OP_PASS_* and OP_A_PASS name slots of DevOp::slots): the op's own adjoint lies in HBM and the op before it
 // in the sweep delivered to it last, so it is read after that delivery
 // instead of one op ahead
 constexpr int32_t OP_A_LATE = 512;
-// FP64 form, 4 states: child k's adjoint lies in HBM and holds deliveries
+// 4-state walks: child k's adjoint lies in HBM and holds deliveries
 constexpr int32_t OP_ACC0 = 1024;
 constexpr int32_t OP_ACC1 = 2048;
-// FP64 form, 4 states, forward: child k's CLV is read from HBM
+// 4-state walks, forward: child k's CLV is read from HBM
 constexpr int32_t OP_LOAD0 = 1 << 21;
 constexpr int32_t OP_LOAD1 = 1 << 22;
-constexpr int WALK_SLOTS = 8;  // FP64 form: LDS slots of a wave, at most (3 bits per use)
+constexpr int WALK_SLOTS = 32;  // LDS slots of a wave, at most
 constexpr int PASS_SLOTS = 5;  // at most; fewer where LDS would cost residency
 constexpr int PASS_SHIFT = 12;  // slot of use u (0, 1: children, 2: own) in bits 12 + 3u
 constexpr int32_t PASS_BITS = 0x1FF << PASS_SHIFT;
@@ -185,7 +188,11 @@ struct NetDesc {
   int32_t n_groups;
   int32_t n_root;
   int32_t n_uses;  // gradient rows
-  int32_t n_pass;  // LDS pass slots of the 4-state reverse sweep (layout of its dynamic LDS)
+  // 4-state walks: op lists (forward and reverse) and LDS slots per wave
+  const DevOp *ops_fwd, *ops_adj;
+  int32_t n_fwd, n_adj, fwd_slots, adj_slots;
+  double *seed;      // root seed factors [root][site]
+  const float *PfT;  // transposes of Pf's matrices
   float *clv;
   int32_t *scl;
   float *adj;
@@ -213,7 +220,7 @@ struct SmallDesc {
   // P matrices
   const double *V, *Vinv, *ev, *rates, *brlen;
   double *P, *dP, *d2P;
-  float *Pf;
+  float *Pf, *PfT;
   // reductions and mixture
   int32_t n_root, nc, R, n_uses;
   const int32_t *part_tile_begin;
@@ -237,15 +244,25 @@ void launch_mixture_multi(hipStream_t s, const SmallDesc *d, int n, int variant)
 void launch_grad_reduce_multi(hipStream_t s, const SmallDesc *d, int n, int max_rows, int max_edges);
 void launch_gather_results(hipStream_t s, const SmallDesc *d, int n, const int64_t *offsets,
                            double *out, int max_size);
-// G = ops per group, TS = sites per workgroup (the autotuned shape)
-void launch_forward_persistent_multi(hipStream_t stream, int C, int G, int TS, const NetDesc *nets,
-                                     const WorkItem *work, int n_work, size_t lds);
-// H = lanes per (site, category) row of the 4-state reverse sweep (1 or 2)
-void launch_adjoint_persistent_multi(hipStream_t stream, int C, int G, int TS, int H, const NetDesc *nets,
-                                     const WorkItem *work, int n_work, size_t lds);
-// dynamic LDS of the FP32 4-state adjoint (P/Q tables and pass slots)
-size_t adjoint_persistent_lds(int E, int C, int TS, int n_pass);
-int adjoint_pass_slots(int C, int G, int TS, int H, int E, int64_t n_work);
+// blocks: 64-row blocks per wave (1 or 2)
+void launch_forward_persistent_multi(hipStream_t stream, int C, int blocks, const NetDesc *nets, const WorkItem *work,
+                                     int n_work, int max_slots);
+void launch_adjoint_persistent_multi(hipStream_t stream, int C, int blocks, const NetDesc *nets, const WorkItem *work,
+                                     int n_work, int max_slots);
+
+// Dynamic LDS of the 4-state walks: the reverse walk's ring of gradient sums
+// on their way to HBM, and n_slots rows with their scaler words or exponents.
+constexpr int GRAD_RING = 128;
+constexpr size_t forward_walk_lds(int nq, int n_slots) { return static_cast<size_t>(n_slots) * (nq * 512 + 256); }
+constexpr size_t adjoint_walk_lds(int nq, int n_slots) {
+  return sizeof(double) * GRAD_RING + static_cast<size_t>(n_slots) * nq * 512;
+}
+constexpr size_t forward_lds32(int C, int blocks, int n_slots) {
+  return static_cast<size_t>(n_slots) * blocks * (1024 + 256 / C);
+}
+constexpr size_t adjoint_lds32(int C, int blocks, int n_slots) {
+  return sizeof(float) * GRAD_RING + forward_lds32(C, blocks, n_slots);
+}
 
 // Kernel launchers (kernels.hip)
 void launch_pmatrices(Engine &e);
@@ -254,9 +271,6 @@ void launch_forward_level(Engine &e, const DevOp *ops, int n_ops, const LevelChu
 // 4 states: ops in an order with children first, with their LDS slots
 // assigned (assign_forward_slots); root site sums and seed factors included
 void launch_forward_walk(Engine &e, const DevOp *ops, int n_ops);
-// dynamic LDS of the walks' one-wave workgroups (nq granules per wave)
-size_t forward_walk_lds(int nq, int n_slots);
-size_t adjoint_walk_lds(int nq, int n_slots);
 void launch_root_partials(Engine &e, bool seeds);
 // root partials of n roots: physical rows `rows`, root indices `index`
 void launch_root_partials(Engine &e, bool seeds, const int32_t *rows, const int32_t *index, int n);

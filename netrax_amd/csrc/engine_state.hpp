@@ -72,32 +72,32 @@ struct Engine : nrx_engine {
   std::vector<std::vector<int>> level_ops;  // variant slots per level (needed only)
   std::vector<int> root_slots;              // distinct displayed-tree-root CLVs
   std::vector<int> class_root_index;        // [nc]
-  // plain form: ops in level order (20 states; FP32 engines likewise), or in
-  // the depth-first order of the 4-state walks, with their LDS slots in the
-  // two lists the walks read
+  // ops in level order (20 states), or in the depth-first order of the
+  // 4-state walks, with their LDS slots in the two lists the walks read
   std::vector<DevOp> ops_all, ops_fwd, ops_adj;
   std::vector<LevelChunk> chunks;
   // plain form reverse sweep: runs of ops without a common child, per chunk
   std::vector<LevelChunk> adj_runs;
   std::vector<int> adj_run_begin;
-  // batched form: groups of independent ops in a depth-first-biased order
+  // FP32 form, 20 states: groups of independent ops in a depth-first-biased order
   std::vector<DevOp> ops_dfs;
   std::vector<int32_t> group_begin;  // [n_groups + 1] into ops_dfs
   std::vector<int32_t> edge_use_begin, edge_use_list;  // gradient rows per edge
   int n_uses = 0;
   int pw = 1;   // site-sum partials per tile (one per wave)
   int rpw = 1;  // root site-sum partials per tile
-  // FP64 form, 4 states: granules per wave of the walks and LDS slots per wave
-  int walk_nq = 4, fwd_slots = 2, adj_slots = 2;
+  // 4-state walks: LDS slots per wave, and granules per wave (FP64)
+  int walk_nq = 4, fwd_slots = 4, adj_slots = 4;
+  int walk_blocks = 1;  // 64-row blocks per wave (FP32)
   // gradient partials [site block][row][wave]: waves per block, blocks per tile
   int gpw = 1, gbpt = 1;
   // FP32 form shape (nrx_autotune / nrx_set_tuning): ops per group of the
-  // persistent kernels and sites per workgroup (4-state data; 32 for 20)
+  // 20-state kernels; for 4 states see walk_blocks_of.  The other two are
+  // part of a shape's name only.
   int tune_group = 4;
   int tune_tile = TILE;
-  int tune_lanes = 1;  // lanes per (site, category) row of the 4-state reverse sweep
+  int tune_lanes = 1;
   int schedule_version = 0;  // bumped by every schedule rebuild
-  int pass_slots = 0;        // LDS pass slots the FP32 4-state reverse sweep uses
 
   // branch derivatives: sumtables of one branch for every displayed tree
   // containing it (valid while nothing but that branch's length changes)
@@ -151,13 +151,13 @@ struct Engine : nrx_engine {
   hipStream_t stream = nullptr;
   DevBuf d_tips, d_weights, d_tile_part, d_part_tile_begin;
   DevBuf d_V, d_Vinv, d_eval, d_rates, d_freqs, d_brlen;
-  DevBuf d_P, d_dP, d_d2P, d_Pf, d_dPf;
+  DevBuf d_P, d_dP, d_d2P, d_Pf, d_PfT;
   DevBuf d_clv, d_scl, d_adj, d_adj_exp, d_Qf;
   DevBuf d_Pa;  // 20-state FP32 form: matrix-core operand tables
   DevBuf d_ops, d_ops_dirty, d_Qd;
   DevBuf d_ops_fwd, d_ops_adj;  // 4 states: the walks' op lists
-  // FP32 form, incremental evaluation: the invalid ops, their groups and
-  // their descriptor
+  // FP32 form, incremental evaluation: the invalid ops, their groups (20
+  // states) and their descriptor
   DevBuf d_ops_inc, d_group_begin_inc, d_netdesc_inc;
   DevBuf d_ops_dfs, d_group_begin, d_edge_use_begin, d_edge_use_list;
   DevBuf d_netdesc, d_work;  // FP32 form: this engine's NetDesc and (0, tile) work table
@@ -183,7 +183,7 @@ struct Engine : nrx_engine {
   int n_k[2] = {0, 0};
   nrx_timing last_timing{};
 
-  bool walks() const { return S == 4 && opt.precision == NRX_FP64; }
+  bool walks() const { return S == 4; }
 
   ~Engine();
 };

@@ -308,7 +308,7 @@ __global__ void k_pmatrices(DevLayout L, const double *__restrict__ V,
                             const double *__restrict__ rates, const double *__restrict__ brlen,
                             double *__restrict__ P, double *__restrict__ dP,
                             double *__restrict__ d2P, float *__restrict__ Pf,
-                            float *__restrict__ dPf) {
+                            float *__restrict__ PfT) {
   const int S = L.S, C = L.C;
   const int64_t total = static_cast<int64_t>(L.n_parts) * L.n_edges * C * S * S;
   const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -335,7 +335,7 @@ __global__ void k_pmatrices(DevLayout L, const double *__restrict__ V,
   dP[idx] = a1;
   d2P[idx] = a2;
   if (Pf) Pf[idx] = static_cast<float>(a0);
-  if (dPf) dPf[idx] = static_cast<float>(a1);
+  if (PfT) PfT[idx - (i * S + j) + (j * S + i)] = static_cast<float>(a0);
 }
 
 // ---------------------------------------------------- root site sums (FP64)
@@ -635,11 +635,11 @@ __device__ __forceinline__ uint32_t warm_l2(const GAS double *P, int n_mats, con
 
 // One op's descriptor in scalar registers, fetched whole: read field by
 // field where it is used, every field would be a scalar load with a wait.
-typedef int32_t i32x8 __attribute__((ext_vector_type(8), aligned(8)));
-typedef int32_t i32x2 __attribute__((ext_vector_type(2), aligned(8)));
+typedef int32_t i32x8 __attribute__((ext_vector_type(8), aligned(16)));
+typedef int32_t i32x4 __attribute__((ext_vector_type(4), aligned(16)));
 struct OpRegs {
   i32x8 a;
-  i32x2 b;
+  i32x4 b;
   __device__ __forceinline__ uint32_t out() const { return a[0]; }
   __device__ __forceinline__ int nk() const { return a[1]; }
   __device__ __forceinline__ int32_t kid(int k) const { return a[2 + k]; }
@@ -648,15 +648,24 @@ struct OpRegs {
   __device__ __forceinline__ int flags() const { return a[7]; }
   __device__ __forceinline__ bool has(int f0, int f1, int k) const { return (a[7] & (k == 0 ? f0 : f1)) != 0; }
   __device__ __forceinline__ int gslot() const { return b[0]; }
+  __device__ __forceinline__ int slot(int u) const { return (b[2] >> (8 * u)) & 255; }
 };
-static_assert(sizeof(DevOp) == 40, "OpRegs restates DevOp");
+static_assert(sizeof(DevOp) == 48, "OpRegs restates DevOp");
 __device__ __forceinline__ OpRegs fetch_op(const CAS DevOp *ops, int t) {
   OpRegs r;
   r.a = *reinterpret_cast<const CAS i32x8 *>(ops + t);
-  r.b = *reinterpret_cast<const CAS i32x2 *>(reinterpret_cast<const CAS int32_t *>(ops + t) + 8);
+  r.b = *reinterpret_cast<const CAS i32x4 *>(reinterpret_cast<const CAS int32_t *>(ops + t) + 8);
   return r;
 }
 __device__ __forceinline__ void arrive(OpRegs &r) { asm volatile("" : "+s"(r.a), "+s"(r.b)); }
+
+// A lane's byte offset, hidden from the optimiser: it would otherwise keep
+// base + offset of every buffer as a register pair across the op loop and add
+// each row to that, instead of addressing with a scalar base plus the offset.
+__device__ __forceinline__ uint32_t opaque(uint32_t x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
 
 template <int C, int NQ>
 struct FwdIn4 {
@@ -700,10 +709,11 @@ __global__ void __launch_bounds__(64, 3)
   const double pi_c = freqs[part * 4 + state] * (1.0 / C);
 
   auto load = [&](const OpRegs &op, FwdIn4<C, NQ> &in) {
+    const uint32_t o = opaque(off);
 #pragma unroll
     for (int k = 0; k < 2; ++k)
 #pragma unroll
-      for (int h = 0; h < NA; ++h) in.A[k * NA + h] = *at(P + op.edge(k) * (C * 16), aoff[h]);
+      for (int h = 0; h < NA; ++h) in.A[k * NA + h] = *at(P + op.edge(k) * (C * 16), opaque(aoff[h]));
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       // a tip's mask words, or the row's scaler words (a one-child op's
@@ -718,7 +728,7 @@ __global__ void __launch_bounds__(64, 3)
       if (op.has(OP_LOAD0, OP_LOAD1, k))
 #pragma unroll
         for (int q = 0; q < NQ; ++q)
-          in.x[k * NQ + q] = *at(clv + static_cast<uint32_t>(op.kid(k)) * row, off + q * 512);
+          in.x[k * NQ + q] = *at(clv + static_cast<uint32_t>(op.kid(k)) * row, o + q * 512);
   };
   // y = P x of child k
   auto child = [&](const OpRegs &op, FwdIn4<C, NQ> &in, int k, double (&y)[NQ], uint32_t &count) {
@@ -729,7 +739,7 @@ __global__ void __launch_bounds__(64, 3)
       below = 0;
     }
     if (op.has(OP_PASS_KID0, OP_PASS_KID1, k)) {
-      const int slot = pass_slot(op.flags(), k);
+      const int slot = op.slot(k);
 #pragma unroll
       for (int q = 0; q < NQ; ++q) in.x[k * NQ + q] = slots[slot * (NQ * 64) + q * 64 + lane];
       below = slot_scl[slot * 64 + lane] >> 1;
@@ -748,6 +758,7 @@ __global__ void __launch_bounds__(64, 3)
     load(ahead, next);
     after = fetch_op(ops, min(t + 2, n_ops - 1));
     __builtin_amdgcn_sched_barrier(0);
+    const uint32_t o = opaque(off);
     double v[NQ];
     uint32_t count = 0;
     child(op, in, 0, v, count);
@@ -774,10 +785,10 @@ __global__ void __launch_bounds__(64, 3)
       if ((sites >> (lane % SPW)) & 1) word += 3;
     }
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) *at(clv + op.out() * row, off + q * 512) = v[q];
-    *at(scl + op.out() * n, soff) = static_cast<int32_t>(word);  // lanes of a site store the same word
+    for (int q = 0; q < NQ; ++q) *at(clv + op.out() * row, o + q * 512) = v[q];
+    *at(scl + op.out() * n, opaque(soff)) = static_cast<int32_t>(word);  // lanes of a site store the same word
     if (op.flags() & OP_A_PASS) {
-      const int slot = pass_slot(op.flags(), 2);
+      const int slot = op.slot(2);
 #pragma unroll
       for (int q = 0; q < NQ; ++q) slots[slot * (NQ * 64) + q * 64 + lane] = v[q];
       slot_scl[slot * 64 + lane] = word;
@@ -847,8 +858,6 @@ struct AdjIn4 {
   uint32_t word[1];    // own scaler word
 };
 
-constexpr int GRAD_RING = 128;  // gradient sums of a wave on their way to HBM, 64 at a time
-
 // Bound: HBM (every inner child's CLV once per use; 50 taxa, 41,345 patterns:
 // 1.6 GB in 0.363 ms, 4.5 TB/s; with P in LDS and every adjoint through HBM
 // 2.99 GB in 0.648 ms).
@@ -888,33 +897,34 @@ __global__ void __launch_bounds__(64, 3)
   const double pi = freqs[part * 4 + state];
 
   auto load = [&](const OpRegs &op, AdjIn4<C, NQ> &in) {
+    const uint32_t o = opaque(off);
 #pragma unroll
     for (int k = 0; k < 2; ++k)
 #pragma unroll
       for (int h = 0; h < NA; ++h) {
-        in.A[k * NA + h] = *at(P + op.edge(k) * (C * 16), aoff[h]);
-        in.AT[k * NA + h] = *at(P + op.edge(k) * (C * 16), toff[h]);
+        in.A[k * NA + h] = *at(P + op.edge(k) * (C * 16), opaque(aoff[h]));
+        in.AT[k * NA + h] = *at(P + op.edge(k) * (C * 16), opaque(toff[h]));
       }
-    in.word[0] = static_cast<uint32_t>(*at(scl + op.out() * n, soff));
+    in.word[0] = static_cast<uint32_t>(*at(scl + op.out() * n, opaque(soff)));
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       // (a one-child op's second child stands for its first)
       const int32_t kid = k < op.nk() ? op.kid(k) : op.kid(0);
       if (kid < 0)
-        in.raw[k] = *at(reinterpret_cast<const GAS uint32_t *>(tips + static_cast<uint32_t>(~kid) * n), woff);
+        in.raw[k] = *at(reinterpret_cast<const GAS uint32_t *>(tips + static_cast<uint32_t>(~kid) * n), opaque(woff));
       else if (k < op.nk())
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) in.x[k * NQ + q] = *at(clv + static_cast<uint32_t>(kid) * row, off + q * 512);
+        for (int q = 0; q < NQ; ++q) in.x[k * NQ + q] = *at(clv + static_cast<uint32_t>(kid) * row, o + q * 512);
     }
     if ((op.flags() & (OP_HAS_CONSUMERS | OP_A_PASS | OP_A_LATE)) == OP_HAS_CONSUMERS)
 #pragma unroll
-      for (int q = 0; q < NQ; ++q) in.a[q] = *at(adj + op.out() * row, off + q * 512);
+      for (int q = 0; q < NQ; ++q) in.a[q] = *at(adj + op.out() * row, o + q * 512);
     if (op.root() >= 0) in.sd[0] = seed[op.root() * n + site0 + lane % SPW];
   };
   // back-propagated vectors to child k's adjoint
   auto deliver = [&](const OpRegs &op, const AdjIn4<C, NQ> &in, int k, const double (&z)[NQ], double (&b)[NQ]) {
     const bool first = op.has(OP_FIRST_KID0, OP_FIRST_KID1, k), pass = op.has(OP_PASS_KID0, OP_PASS_KID1, k);
-    double *slot = slots + pass_slot(op.flags(), k) * (NQ * 64) + lane;
+    double *slot = slots + op.slot(k) * (NQ * 64) + lane;
     GAS double *dst = adj + static_cast<uint32_t>(op.kid(k)) * row;
     if (pass && !first) {
 #pragma unroll
@@ -922,12 +932,13 @@ __global__ void __launch_bounds__(64, 3)
     }
 #pragma unroll
     for (int q = 0; q < NQ; ++q) b[q] = mfma4(in.AT[k * NA + W::half(q)], z[q], b[q]);
+    const uint32_t o = opaque(off);
     if (pass) {
 #pragma unroll
       for (int q = 0; q < NQ; ++q) slot[q * 64] = b[q];
     } else {
 #pragma unroll
-      for (int q = 0; q < NQ; ++q) *at(dst, off + q * 512) = b[q];
+      for (int q = 0; q < NQ; ++q) *at(dst, o + q * 512) = b[q];
     }
   };
   auto product = [&](const OpRegs &op, AdjIn4<C, NQ> &in, int k, double (&y)[NQ]) {
@@ -958,25 +969,23 @@ __global__ void __launch_bounds__(64, 3)
       for (int q = 0; q < NQ; ++q) acc[k][q] = 0.0;
       if (op.has(OP_ACC0, OP_ACC1, k))
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) acc[k][q] = *at(adj + static_cast<uint32_t>(op.kid(k)) * row, off + q * 512);
+        for (int q = 0; q < NQ; ++q) acc[k][q] = *at(adj + static_cast<uint32_t>(op.kid(k)) * row, opaque(off) + q * 512);
     }
     load(ahead, next);
     after = fetch_op(ops, max(t - 2, 0));
     __builtin_amdgcn_sched_barrier(0);
-    double a[NQ];
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) a[q] = 0.0;
+    double (&a)[NQ] = in.a;
     if (op.flags() & OP_A_PASS) {
-      const double *slot = slots + pass_slot(op.flags(), 2) * (NQ * 64) + lane;
+      const double *slot = slots + op.slot(2) * (NQ * 64) + lane;
 #pragma unroll
       for (int q = 0; q < NQ; ++q) a[q] = slot[q * 64];
     } else if (op.flags() & OP_A_LATE) {
 #pragma unroll
       for (int q = 0; q < NQ; ++q) a[q] = *at(adj + op.out() * row, off + q * 512);
       wait_loads();
-    } else if (op.flags() & OP_HAS_CONSUMERS) {
+    } else if (!(op.flags() & OP_HAS_CONSUMERS)) {
 #pragma unroll
-      for (int q = 0; q < NQ; ++q) a[q] = in.a[q];
+      for (int q = 0; q < NQ; ++q) a[q] = 0.0;
     }
     if (op.root() >= 0) {
       // seed beta * w * (1/C) pi_i / Ltilde at a displayed-tree root
@@ -1425,292 +1434,116 @@ __global__ void k_grad_total(DevLayout L, const int32_t *__restrict__ edge_use_b
   res[rl.dbrlen + e] = tot;
 }
 
-// ==================================================== FP32 batched form
-// One workgroup per 64-site tile walks the whole op list (children before
-// parents, depth-first post-order so a child is consumed soon after it is
-// written).  Thread (site, category) owns its CLV row in every op, so every
-// value a thread reads was written by the same thread: no barrier is needed
-// after the P tables are staged in LDS.  CLVs are FP32, renormalised at
-// every op by an exact power of two so the site maximum lies in [0.5, 1);
-// the per-site exponent k (true = stored * 2^-k) is carried as an int32.
-// Site sums, the mixture and the gradient reduction across waves are FP64;
-// inside a wave the gradient's per-(site, category) shares (each of order
-// weight / branch length) are summed in FP32 per row of 16 lanes.
+// ==================================================== FP32 form, 4 states
+// The walks of the FP64 form (k_forward_walk, k_adjoint_level) in FP32.  A
+// product of 64 rows with their 4 x 4 matrices is four v_mfma_f32_4x4x1 (16
+// blocks): step k takes A lane (l & 3, block l >> 2) = P[l & 3][k] and B lane
+// l = x[k] of the lane's own row, and register i of D is entry i of that row,
+// so a lane owns a (site, category) row in every op and its four entries stay
+// in four registers.  A lane's part of P is one row of it (16 bytes), of P^T
+// (back-propagation) one column, stored apart.
+//
+// CLVs are renormalised at every op by an exact power of two so the site
+// maximum lies in [0.5, 1); the per-site exponent k (true = stored * 2^-k) is
+// carried as an int32.  Site sums, the mixture and the gradient reduction
+// across waves are FP64; inside a wave the gradient's per-(site, category)
+// shares (each of order weight / branch length) are summed in FP32.
 constexpr double LN2 = 0.69314718055994530941723212145818;
 constexpr int EXP_EMPTY = -(1 << 28);  // exponent of an all-zero adjoint
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 template <int CTRL>
 __device__ __forceinline__ int dpp_i(int v) {
   return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, false);
 }
 
-// Maximum over the C category lanes of a site, comparing the float bit
+// A wave's rows: NR blocks of 64 rows, a block being 64 / C sites.  Lane l
+// holds site j = l & 3 of a 4-site group and one category; the categories of
+// a site are 4 or 8 lanes apart in a row of 16 lanes (8 categories: in two
+// rows of 16), where DPP rotations reach them.
+template <int C, int NR>
+struct Rows {
+  static constexpr int SPB = 64 / C;    // sites of a block
+  static constexpr int SPW = SPB * NR;  // sites of a wave
+  static __device__ __forceinline__ int cat(int lane) {
+    return C == 2 ? (lane >> 3) & 1 : (lane >> 2) & (C - 1);
+  }
+  static __device__ __forceinline__ int site(int lane) {  // within the block
+    const int b = lane >> 2;
+    const int group = C == 8 ? b >> 3 : C == 4 ? b >> 2 : C == 2 ? (b & 1) | ((b >> 2) << 1) : b;
+    return 4 * group + (lane & 3);
+  }
+  static __device__ __forceinline__ int lane_of(int site, int c) {
+    const int g = site >> 2;
+    const int b = C == 8 ? g * 8 + c : C == 4 ? g * 4 + c : C == 2 ? (g & 1) | (c << 1) | ((g >> 1) << 2) : g;
+    return 4 * b + (site & 3);
+  }
+};
+
+// Maximum over the category lanes of a site, comparing the float bit
 // patterns as signed integers: the float order for values >= 0, and every
 // positive value beats every negative one, which is all a site maximum
 // needs.  (fmaxf would add a NaN canonicalisation around every cross-lane
 // move; the integer max takes the DPP move as an operand modifier.)
 template <int C>
-__device__ __forceinline__ float cat_maxf(float m) {
+__device__ __forceinline__ float site_max(float m) {
   int u = __float_as_int(m);
-  if constexpr (C > 1) u = max(u, dpp_i<DPP_XOR1>(u));
-  if constexpr (C > 2) u = max(u, dpp_i<DPP_XOR2>(u));
-  if constexpr (C > 4) u = max(u, __shfl_xor(u, 4));
+  if constexpr (C >= 4) u = max(u, dpp_i<0x124>(u));  // row_ror:4
+  if constexpr (C >= 2) u = max(u, dpp_i<0x128>(u));  // row_ror:8
+  if constexpr (C == 8) {
+    const auto s = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    u = max(static_cast<int>(s[0]), static_cast<int>(s[1]));
+  }
   return __int_as_float(u);
 }
+template <int C>
+__device__ __forceinline__ double site_total(double t) {
+  if constexpr (C >= 4) t += dpp<0x124>(t);
+  if constexpr (C >= 2) t += dpp<0x128>(t);
+  if constexpr (C == 8) t += __shfl_xor(t, 16);
+  return t;
+}
+template <int C>
+__device__ __forceinline__ float site_absmax(const f32x4 &x) {
+  return site_max<C>(fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))));
+}
 
-// Sum over the 64 lanes of a wave of FP32 values, in FP32 and a fixed order,
-// returned in FP64: four row_shr steps inside each row of 16 lanes (lane 15
-// of a row ends with the row's sum S_r), then row_bcast:15 (0x142: each row
-// adds lane 15 of the row before it, so lane 31 = S0 + S1 and lane 63 =
-// S2 + S3) and row_bcast:31 (0x143: rows 2 and 3 add lane 31), after which
-// lane 63 holds the total; one lane read instead of four.
-__device__ __forceinline__ double wave_sum_f32(float v) {
+__device__ __forceinline__ f32x4 product4(const f32x4 &M, const f32x4 &x) {
+  f32x4 y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) y = __builtin_amdgcn_mfma_f32_4x4x1f32(M[k], x[k], y, 0, 0, 0);
+  return y;
+}
+__device__ __forceinline__ f32x4 tip_row(uint32_t mask) {
+  f32x4 x;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) x[i] = __int_as_float(-static_cast<int>((mask >> i) & 1u) & 0x3F800000);  // 1.0f or 0.0f
+  return x;
+}
+__device__ __forceinline__ f32x4 scale4(const f32x4 &x, int e) {
+  f32x4 y;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) y[i] = ldexpf(x[i], e);
+  return y;
+}
+
+// Sums over the 64 lanes of two FP32 values at once, in a fixed order: lane
+// 31 ends with a's total, lane 63 with b's (see pair_wave_sum).
+__device__ __forceinline__ float pair_wave_sum_f32(float a, float b) {
+  const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  float v = __uint_as_float(s[0]) + __uint_as_float(s[1]);
   v += dpp<0x111>(v);
   v += dpp<0x112>(v);
   v += dpp<0x114>(v);
   v += dpp<0x118>(v);
   v += dpp<0x142>(v);
-  v += dpp<0x143>(v);
-  return static_cast<double>(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63)));
-}
-
-__device__ __forceinline__ void tip_vec4(uint32_t mask, float (&x)[4]) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) x[i] = ((mask >> i) & 1u) ? 1.0f : 0.0f;
-}
-
-__device__ __forceinline__ void load4(const float *__restrict__ p, float (&x)[4]) {
-  const float4 v = *reinterpret_cast<const float4 *>(p);
-  x[0] = v.x;
-  x[1] = v.y;
-  x[2] = v.z;
-  x[3] = v.w;
-}
-
-__device__ __forceinline__ void store4(float *__restrict__ p, const float (&x)[4]) {
-  *reinterpret_cast<float4 *>(p) = make_float4(x[0], x[1], x[2], x[3]);
-}
-
-#ifdef __HIP_DEVICE_COMPILE__
-__device__ __forceinline__ void load4(const GAS float *__restrict__ p, float (&x)[4]) {
-  const float4 v = *reinterpret_cast<const GAS float4 *>(p);
-  x[0] = v.x;
-  x[1] = v.y;
-  x[2] = v.z;
-  x[3] = v.w;
-}
-
-__device__ __forceinline__ void store4(GAS float *__restrict__ p, const float (&x)[4]) {
-  *reinterpret_cast<GAS float4 *>(p) = make_float4(x[0], x[1], x[2], x[3]);
-}
-#endif
-
-__device__ __forceinline__ void mv4(const float *__restrict__ M, const float (&x)[4], float (&y)[4]) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    y[i] = fmaf(M[4 * i + 3], x[3], fmaf(M[4 * i + 2], x[2], fmaf(M[4 * i + 1], x[1], M[4 * i] * x[0])));
-}
-
-__device__ __forceinline__ void mv4t(const float *__restrict__ M, const float (&x)[4], float (&y)[4]) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-    y[j] = fmaf(M[12 + j], x[3], fmaf(M[8 + j], x[2], fmaf(M[4 + j], x[1], M[j] * x[0])));
-}
-
-// Raw inputs of one group of the 4-state FP32 forward: child rows, child
-// scaler words and tip masks (expanded when used).
-template <int G>
-struct FwdIn {
-  float x[G][2][4];
-  int sk[G][2];
-  uint32_t tm[G][2];
-};
-
-// Issues every load of group [g0, g0 + nb): inner children in one pass, tip
-// masks in another (no join of a load path with a non-load path between two
-// loads), nothing waits.
-template <int C, int G>
-__device__ __forceinline__ void fwd_load(const CAS DevOp *__restrict__ ops, int g0, int nb,
-                                         const GAS float *__restrict__ clv,
-                                         const GAS int32_t *__restrict__ scl,
-                                         const GAS uint8_t *__restrict__ tips, int64_t n,
-                                         int64_t site, int c, FwdIn<G> &in) {
-#pragma unroll
-  for (int j = 0; j < G; ++j) {
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      if (j < nb) {
-        const DevOp op = ops[g0 + j];
-        const int32_t kid = op.kid[kk];
-        if (kk < op.nk && kid >= 0) {
-          load4(clv + (static_cast<size_t>(kid) * n + site) * (C * 4) + c * 4, in.x[j][kk]);
-          in.sk[j][kk] = scl[static_cast<size_t>(kid) * n + site];
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < G; ++j) {
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      if (j < nb) {
-        const DevOp op = ops[g0 + j];
-        const int32_t kid = op.kid[kk];
-        if (kk < op.nk && kid < 0) in.tm[j][kk] = tips[static_cast<size_t>(-kid - 1) * n + site];
-      }
-    }
-  }
-}
-
-// TS sites per workgroup (TS C threads, a multiple of 64, TS <= 64 so a
-// workgroup never straddles partitions) and G ops per group are the
-// autotuned shape parameters.
-// The bodies of the persistent kernels take every buffer as a __restrict__
-// parameter: restrict only reaches the optimiser through parameters, and it
-// lets the compiler keep op-table loads scalar and move CLV loads past
-// stores to other buffers.
-template <int C, int G, int TS>
-__device__ __forceinline__ void forward_persistent_body(
-    const CAS DevOp *__restrict__ ops, const CAS int32_t *__restrict__ group_begin, int n_groups,
-    const DevLayout L, GAS float *__restrict__ clv, GAS int32_t *__restrict__ scl,
-    const GAS uint8_t *__restrict__ tips, const GAS float *__restrict__ Pf,
-    const GAS int32_t *__restrict__ tile_part, const GAS double *__restrict__ freqs,
-    const GAS double *__restrict__ weights, GAS double *__restrict__ root_partials, int tile) {
-  float *sP = dyn_lds<float>();  // P of this tile's partition: [edge][cat][4][4]
-  constexpr int PW = TILE * C / 64;  // site-sum partials (waves) per 64-site tile
-  const int64_t site0 = static_cast<int64_t>(tile) * TS;
-  const int part = tile_part[site0 / TILE];
-  const int np = L.n_edges * C * 16;
-  const GAS float *gP = Pf + static_cast<size_t>(part) * np;
-  for (int i = threadIdx.x; i < np; i += blockDim.x) sP[i] = gP[i];
-  __syncthreads();
-  const int c = threadIdx.x % C;
-  const int64_t site = site0 + threadIdx.x / C;
-  const int64_t n = L.n_sites_pad;
-  const size_t n_wt = static_cast<size_t>(L.n_tiles) * PW;
-  const size_t wt = static_cast<size_t>(site0 * C / 64) + threadIdx.x / 64;  // global wave
-  const double w = weights[site];
-  double pi[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) pi[i] = freqs[part * 4 + i];
-  // The inputs of a group are loaded as raw values (rows, scaler words, tip
-  // masks) in one phase with no wait inside it.  When the next group does
-  // not consume this one (OP_GROUP_INDEP on its first op), its loads are
-  // issued before this group's arithmetic and stores, so the two groups'
-  // memory round trips overlap.
-  FwdIn<G> cur, nxt;
-  fwd_load<C, G>(ops, group_begin[0], group_begin[1] - group_begin[0], clv, scl, tips, n, site, c, cur);
-  wait_loads();
-  for (int gi = 0; gi < n_groups; ++gi) {
-    const int g0 = group_begin[gi];
-    const int nb = group_begin[gi + 1] - g0;
-    const bool has_next = gi + 1 < n_groups;
-    int n0 = 0, nn = 0;
-    bool early = false;
-    if (has_next) {
-      n0 = group_begin[gi + 1];
-      nn = group_begin[gi + 2] - n0;
-      early = (ops[n0].flags & OP_GROUP_INDEP) != 0;
-    }
-    if (early) {
-      __builtin_amdgcn_s_setprio(1);  // see the note at wait_loads
-      fwd_load<C, G>(ops, n0, nn, clv, scl, tips, n, site, c, nxt);
-      __builtin_amdgcn_s_setprio(0);
-    }
-    float v[G][4];
-    int kk_[G];
-    double rv[G];
-#pragma unroll
-    for (int j = 0; j < G; ++j) {
-      if (j < nb) {
-        const DevOp op = ops[g0 + j];
-        int ks = 0;
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-          if (kk < op.nk) {
-            if (op.kid[kk] < 0)
-              tip_vec4(cur.tm[j][kk], cur.x[j][kk]);
-            else
-              ks += cur.sk[j][kk];
-          }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[j][i] = 1.f;
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-          if (kk < op.nk) {
-            float y[4];
-            mv4(sP + (op.edge[kk] * C + c) * 16, cur.x[j][kk], y);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) v[j][i] *= y[i];
-          }
-        }
-        const float m = cat_maxf<C>(fmaxf(fmaxf(v[j][0], v[j][1]), fmaxf(v[j][2], v[j][3])));
-        int e = 0;
-        if (m > 0.f) (void)frexpf(m, &e);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[j][i] = ldexpf(v[j][i], -e);
-        kk_[j] = ks - e;
-        rv[j] = 0.0;
-        if (op.root >= 0) {
-          double t = 0.0;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) t = fma(pi[i], static_cast<double>(v[j][i]), t);
-          t = cat_sum<C>(t) * (1.0 / C);
-          const double val = (c == 0 && w != 0.0) ? w * (log(t) - kk_[j] * LN2) : 0.0;
-          rv[j] = wave_sum(val);
-        }
-      }
-    }
-    if (early) wait_loads();  // the next group's inputs, before this group's stores
-#pragma unroll
-    for (int j = 0; j < G; ++j) {
-      if (j < nb) {
-        const DevOp op = ops[g0 + j];
-        store4(clv + (static_cast<size_t>(op.out) * n + site) * (C * 4) + c * 4, v[j]);
-        if (c == 0) scl[static_cast<size_t>(op.out) * n + site] = kk_[j];
-        if (op.root >= 0 && (threadIdx.x & 63) == 0)
-          root_partials[static_cast<size_t>(op.root) * n_wt + wt] = rv[j];
-      }
-    }
-    if (has_next) {
-      if (!early) {
-        __builtin_amdgcn_s_setprio(1);
-        fwd_load<C, G>(ops, n0, nn, clv, scl, tips, n, site, c, nxt);
-        __builtin_amdgcn_s_setprio(0);
-        wait_loads();
-      }
-      cur = nxt;
-    }
-  }
-}
-
-template <int C, int G, int TS>
-__global__ void __launch_bounds__(TS *C)
-    k_forward_persistent(const NetDesc *__restrict__ nets, const WorkItem *__restrict__ work) {
-  const WorkItem wi = work[blockIdx.x];
-  const NetDesc &nd = nets[wi.net];
-  forward_persistent_body<C, G, TS>(to_constant(nd.ops), to_constant(nd.group_begin), nd.n_groups, nd.L,
-                                    to_global(nd.clv), to_global(nd.scl), to_global(nd.tips),
-                                    to_global(nd.Pf), to_global(nd.tile_part), to_global(nd.freqs),
-                                    to_global(nd.weights), to_global(nd.root_partials), wi.tile);
-}
-
-// Push-form reverse sweep (as k_adjoint_level) over the groups of the
-// forward order, backwards.  The adjoint of every CLV is stored as FP32
-// mantissas with a per-site exponent g: dJ/d(stored CLV) = stored * 2^g,
-// renormalised at every write; contributions are aligned to the larger
-// exponent before they are added, so no intermediate can overflow.
-// Site maximum of |x| over the C category lanes of a site.
-template <int C>
-__device__ __forceinline__ float site_absmax(const float (&x)[4]) {
-  return cat_maxf<C>(fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))));
+  return v;
 }
 
 // x 2^ex + y 2^ey with both aligned to the larger exponent, which is
 // returned.  Branch-free (one side shifts by zero): the comparison differs
 // between the sites of a wave.
-__device__ __forceinline__ int align_add(float (&x)[4], int ex, const float (&y)[4], int ey) {
+__device__ __forceinline__ int align_add(f32x4 &x, int ex, const f32x4 &y, int ey) {
   const int e = max(ex, ey);
   // power-of-two scales: the products are exact, as ldexp would be
   const float sx = ldexpf(1.0f, ex - e), sy = ldexpf(1.0f, ey - e);
@@ -1719,574 +1552,457 @@ __device__ __forceinline__ int align_add(float (&x)[4], int ex, const float (&y)
   return e;
 }
 
-// Scales x so that its site maximum m of |x| lands in [0.5, 1) and returns
-// the new exponent; EXP_EMPTY for an all-zero site (frexp of 0 gives 0, so
-// the scaling is then the identity).
-__device__ __forceinline__ int renorm(float (&x)[4], int ex, float m) {
-  int e = 0;
-  (void)frexpf(m, &e);
+__device__ __forceinline__ void arrive(f32x4 &x) { asm volatile("" : "+v"(x)); }
+template <int N>
+__device__ __forceinline__ void arrive(f32x4 (&x)[N]) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) x[i] = ldexpf(x[i], -e);
-  return m > 0.f ? ex + e : EXP_EMPTY;
+  for (int i = 0; i < N; ++i) arrive(x[i]);
 }
 
-// Adds delivered vector b (adjoint exponent eb) to the accumulated value
-// (acc, ea) unless this is the child's first delivery, renormalises and
-// stores.  An all-zero delivery takes exponent EXP_EMPTY so that it cannot
-// scale the accumulated value away.
-template <int C>
-__device__ __forceinline__ void finish_delivery(GAS float *__restrict__ dst_m, GAS int32_t *__restrict__ dst_e,
-                                                bool first, bool lane0, float (&b)[4], int eb,
-                                                const float (&acc)[4], int ea) {
-  float mb = site_absmax<C>(b);
-  if (!first) {  // uniform: a flag of the op
-    eb = align_add(b, mb > 0.f ? eb : EXP_EMPTY, acc, ea);
-    mb = site_absmax<C>(b);
-  }
-  eb = renorm(b, eb, mb);
-  store4(dst_m, b);
-  if (lane0) *dst_e = eb;
-}
-
-// A delivery to a child whose adjoint lives in an LDS pass slot (see
-// OP_PASS_KID0): the same arithmetic as finish_delivery, on the thread's
-// slot instead of HBM.  slot_e is the site's exponent, shared by the C
-// lanes of the site (each writes the same value).
-template <int C>
-__device__ __forceinline__ void pass_delivery(float *__restrict__ slot_m, int *__restrict__ slot_e, bool first,
-                                              float (&b)[4], int eb) {
-  float mb = site_absmax<C>(b);
-  if (!first) {  // uniform: a flag of the op
-    const float4 v = *reinterpret_cast<const float4 *>(slot_m);
-    const float acc[4] = {v.x, v.y, v.z, v.w};
-    eb = align_add(b, mb > 0.f ? eb : EXP_EMPTY, acc, *slot_e);
-    mb = site_absmax<C>(b);
-  }
-  eb = renorm(b, eb, mb);
-  *reinterpret_cast<float4 *>(slot_m) = make_float4(b[0], b[1], b[2], b[3]);
-  *slot_e = eb;
-}
-
-template <int C, int G, int TS>
-__device__ __forceinline__ void adjoint_persistent_body(
-    const CAS DevOp *__restrict__ ops, const CAS int32_t *__restrict__ group_begin, int n_groups,
-    const DevLayout L, const GAS float *__restrict__ clv, const GAS int32_t *__restrict__ scl,
-    GAS float *__restrict__ adj, GAS int32_t *__restrict__ adj_exp,
-    const GAS uint8_t *__restrict__ tips, const GAS float *__restrict__ Pf,
-    const GAS float *__restrict__ Qf, const GAS int32_t *__restrict__ tile_part,
-    const GAS double *__restrict__ freqs, const GAS double *__restrict__ weights,
-    const GAS double *__restrict__ beta, int n_root, int n_uses, int n_pass,
-    GAS double *__restrict__ grad_partials, int tile) {
-  float *sP = dyn_lds<float>();  // [edge][cat][16] then Q: [cat][16], then the pass slots
-  constexpr int PWB = TS * C / 64;  // waves of this site block
-  constexpr int NT = TS * C;
-  const int64_t site0 = static_cast<int64_t>(tile) * TS;
-  const int part = tile_part[site0 / TILE];
-  const int np = L.n_edges * C * 16;
-  const GAS float *gP = Pf + static_cast<size_t>(part) * np;
-  for (int i = threadIdx.x; i < np; i += blockDim.x) sP[i] = gP[i];
-  for (int i = threadIdx.x; i < C * 16; i += blockDim.x) sP[np + i] = Qf[part * C * 16 + i];
-  __syncthreads();
-  const int c = threadIdx.x % C;
-  // r_c Q of this lane's category, kept in registers (every op reads it)
-  float Qr[16];
+// The loop of a walk over ops[0, n) (backwards: ops[n - 1] first): the inputs
+// of an op are loaded one op ahead, its descriptor one op before that (loading
+// two ops ahead measured the same).  `early` issues what the op must read
+// after the stores of the op before it.
+template <typename In, typename Load, typename Early, typename Step>
+__device__ __forceinline__ void walk_ops(const CAS DevOp *ops, int n, bool backwards, Load load, Early early, Step step) {
+  auto at_step = [&](int i) { return backwards ? max(n - 1 - i, 0) : min(i, n - 1); };
+  OpRegs op[2] = {fetch_op(ops, at_step(0)), fetch_op(ops, at_step(1))};
+  In in[2];
+  load(op[0], in[0]);
+  // complete before the loop, so that the waits inside it count only what the
+  // step before issued (its stores need not have ended)
+  in[0].arrive_all();
+  for (int t = 0;; t += 2) {
 #pragma unroll
-  for (int i = 0; i < 16; ++i) Qr[i] = sP[np + c * 16 + i];
-  // pass slots: mantissas [slot][thread][4], site exponents [slot][site]
-  float *pass_m = sP + ((np + C * 16 + 3) & ~3);
-  int *pass_e = reinterpret_cast<int *>(pass_m + n_pass * NT * 4);
-  const int site_in_tile = threadIdx.x / C;
-  const int64_t site = site0 + threadIdx.x / C;
-  const int64_t n = L.n_sites_pad;
-  const int wave = threadIdx.x / 64;
-  const bool lane0 = c == 0;
-  const double w = weights[site];
+    for (int u = 0; u < 2; ++u) {
+      if (t + u >= n) return;
+      in[u].arrive_all();
+      arrive(op[1 - u]);
+      __builtin_amdgcn_sched_barrier(0);
+      const OpRegs now = op[u];
+      auto held = early(now);
+      In next;  // what an op does not load stays undefined: nothing is carried over
+      load(op[1 - u], next);
+      op[u] = fetch_op(ops, at_step(t + u + 2));
+      __builtin_amdgcn_sched_barrier(0);
+      step(now, in[u], held);
+      in[1 - u] = next;
+    }
+  }
+}
+
+// Scaler words: exponent k of the CLV << 9 | exponent of this op's
+// renormalisation in 9 bits (-149 .. 1); k stays far below 2^22 for the
+// networks the form takes.
+__device__ __forceinline__ int word_k(int32_t word) { return word >> 9; }
+__device__ __forceinline__ int word_step(int32_t word) { return (word << 23) >> 23; }
+
+template <int C, int NR>
+struct FwdIn32 {
+  f32x4 A[2], x[2 * NR];
+  uint32_t raw[2 * NR];  // the children's scaler words, or tip masks
+  __device__ __forceinline__ void arrive_all() {
+    arrive(A);
+    arrive(x);
+    arrive(raw);
+  }
+};
+
+struct Nothing {};
+
+template <int C, int NR>
+__device__ __forceinline__ void forward_walk32(const NetDesc &nd, float *lds, int64_t site0) {
+  using W = Rows<C, NR>;
+  const int lane = threadIdx.x & 63;
+  const uint64_t n = nd.L.n_sites_pad, row = n * (C * 16);  // bytes of a CLV row
+  const int part = to_constant(nd.tile_part)[site0 / TILE];
+  const int n_slots = nd.fwd_slots;
+  f32x4 *slots = reinterpret_cast<f32x4 *>(lds);  // [slot][block][lane], then the scaler words [slot][block][site]
+  int32_t *slot_scl = reinterpret_cast<int32_t *>(slots + n_slots * (NR * 64));
+  const int sl = W::site(lane);
+  GAS char *clv = reinterpret_cast<GAS char *>(to_global(nd.clv)) + site0 * (C * 16);
+  GAS char *scl = reinterpret_cast<GAS char *>(to_global(nd.scl)) + site0 * 4;
+  const GAS char *tips = reinterpret_cast<const GAS char *>(to_global(nd.tips)) + site0;
+  const GAS char *P =
+      reinterpret_cast<const GAS char *>(to_global(nd.Pf)) + static_cast<int64_t>(part) * nd.L.n_edges * (C * 64);
+  const uint32_t off = lane * 16, soff = sl * 4, aoff = W::cat(lane) * 64 + (lane & 3) * 16;
+  double w[NR], pi[4];
+#pragma unroll
+  for (int r = 0; r < NR; ++r) w[r] = to_global(nd.weights)[site0 + r * W::SPB + sl];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) pi[i] = to_global(nd.freqs)[part * 4 + i];
+  GAS double *root_partials = to_global(nd.root_partials) + site0 / W::SPW;
+  GAS double *seed = to_global(nd.seed) + site0 + sl;
+  const int64_t n_waves = static_cast<int64_t>(n) / W::SPW;
+
+  auto load = [&](const OpRegs &op, FwdIn32<C, NR> &in) {
+    const uint32_t o = opaque(off), so = opaque(soff), tip_o = opaque(sl), ao = opaque(aoff);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) in.A[k] = *reinterpret_cast<const GAS f32x4 *>(P + op.edge(k) * (C * 64) + ao);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      if (op.has(OP_LOAD0, OP_LOAD1, k)) {
+        const GAS char *src = clv + static_cast<uint32_t>(op.kid(k)) * row;
+        const GAS char *word = scl + static_cast<uint32_t>(op.kid(k)) * (n * 4);
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          in.x[k * NR + r] = *reinterpret_cast<const GAS f32x4 *>(src + o + r * 1024);
+          in.raw[k * NR + r] = *reinterpret_cast<const GAS uint32_t *>(word + so + r * (W::SPB * 4));
+        }
+      }
+      if (k < op.nk() && op.kid(k) < 0) {
+        const GAS char *tip = tips + static_cast<uint32_t>(~op.kid(k)) * n;
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+          in.raw[k * NR + r] = *reinterpret_cast<const GAS uint8_t *>(tip + tip_o + r * W::SPB);
+      }
+    }
+  };
+  auto child = [&](const OpRegs &op, FwdIn32<C, NR> &in, int k, f32x4 (&y)[NR], int (&ks)[NR]) {
+    if (op.kid(k) < 0) {
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        in.x[k * NR + r] = tip_row(in.raw[k * NR + r]);
+        in.raw[k * NR + r] = 0;
+      }
+    }
+    if (op.has(OP_PASS_KID0, OP_PASS_KID1, k)) {
+      const int slot = op.slot(k);
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        in.x[k * NR + r] = slots[(slot * NR + r) * 64 + lane];
+        in.raw[k * NR + r] = slot_scl[(slot * NR + r) * W::SPB + sl];
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      y[r] = product4(in.A[k], in.x[k * NR + r]);
+      ks[r] += word_k(static_cast<int32_t>(in.raw[k * NR + r]));
+    }
+  };
+  auto step = [&](const OpRegs &op, FwdIn32<C, NR> &in, Nothing) {
+    f32x4 v[NR];
+    int word[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) word[r] = 0;
+    child(op, in, 0, v, word);
+    if (op.nk() == 2) {
+      f32x4 y[NR];
+      child(op, in, 1, y, word);
+#pragma unroll
+      for (int r = 0; r < NR; ++r) v[r] *= y[r];
+    }
+    GAS char *dst = clv + op.out() * row, *dst_scl = scl + op.out() * (n * 4);
+    const uint32_t o = opaque(off), so = opaque(soff);
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      const float m = site_max<C>(fmaxf(fmaxf(v[r][0], v[r][1]), fmaxf(v[r][2], v[r][3])));
+      const int e = m > 0.f ? __builtin_amdgcn_frexp_expf(m) : 0;
+      v[r] = scale4(v[r], -e);
+      word[r] = ((word[r] - e) << 9) | (e & 511);
+      *reinterpret_cast<GAS f32x4 *>(dst + o + r * 1024) = v[r];
+      // (the lanes of a site store the same word)
+      *reinterpret_cast<GAS int32_t *>(dst_scl + so + r * (W::SPB * 4)) = word[r];
+    }
+    if (op.flags() & OP_A_PASS) {
+      const int slot = op.slot(2);
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        slots[(slot * NR + r) * 64 + lane] = v[r];
+        slot_scl[(slot * NR + r) * W::SPB + sl] = word[r];
+      }
+    }
+    if (op.root() >= 0) {
+      double val = 0.0;
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        double t = 0.0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) t = fma(pi[i], static_cast<double>(v[r][i]), t);
+        t = site_total<C>(t) * (1.0 / C);
+        if (W::cat(lane) == 0 && w[r] != 0.0) val += w[r] * (log(t) - word_k(word[r]) * LN2);
+        // the adjoint's seed factor at this root and site, w / (C Ltilde)
+        seed[op.root() * static_cast<int64_t>(n) + r * W::SPB] = w[r] != 0.0 ? w[r] / (C * t) : 0.0;
+      }
+      val = wave_sum(val);
+      if (lane == 0) root_partials[op.root() * n_waves] = val;
+    }
+  };
+  walk_ops<FwdIn32<C, NR>>(to_constant(nd.ops_fwd), nd.n_fwd, false, load,
+                              [](const OpRegs &) { return Nothing{}; }, step);
+}
+
+// Reverse sweep in push form (as k_adjoint_level).  The adjoint of every CLV
+// is FP32 mantissas with a per-site exponent g: dJ/d(stored CLV) = stored *
+// 2^g, renormalised at its op; contributions are aligned to the
+// larger exponent before they are added, so no intermediate can overflow.
+template <int C, int NR>
+struct AdjIn32 {
+  f32x4 A[2], AT[2], x[2 * NR], a[NR];
+  double sd[NR];
+  int32_t ea[NR], word[NR];
+  uint32_t raw[2 * NR];  // tip masks
+  __device__ __forceinline__ void arrive_all() {
+    arrive(A);
+    arrive(AT);
+    arrive(x);
+    arrive(a);
+    arrive(sd);
+    arrive(ea);
+    arrive(word);
+    arrive(raw);
+  }
+};
+// What the children's adjoints hold already, where no slot does.
+template <int NR>
+struct Held32 {
+  f32x4 m[2 * NR];
+  int32_t e[2 * NR];
+};
+
+template <int C, int NR>
+__device__ __forceinline__ void adjoint_walk32(const NetDesc &nd, float *lds, int64_t site0) {
+  using W = Rows<C, NR>;
+  const int lane = threadIdx.x & 63;
+  const uint64_t n = nd.L.n_sites_pad, row = n * (C * 16);
+  const int part = to_constant(nd.tile_part)[site0 / TILE];
+  const int n_slots = nd.adj_slots;
+  float *ring = lds;
+  f32x4 *slots = reinterpret_cast<f32x4 *>(ring + GRAD_RING);  // [slot][block][lane], then exponents [slot][block][site]
+  int32_t *slot_e = reinterpret_cast<int32_t *>(slots + n_slots * (NR * 64));
+  const int sl = W::site(lane);
+  const GAS char *clv = reinterpret_cast<const GAS char *>(to_global(nd.clv)) + site0 * (C * 16);
+  GAS char *adj = reinterpret_cast<GAS char *>(to_global(nd.adj)) + site0 * (C * 16);
+  GAS char *adj_exp = reinterpret_cast<GAS char *>(to_global(nd.adj_exp)) + site0 * 4;
+  const GAS char *scl = reinterpret_cast<const GAS char *>(to_global(nd.scl)) + site0 * 4;
+  const GAS char *tips = reinterpret_cast<const GAS char *>(to_global(nd.tips)) + site0;
+  const int64_t p0 = static_cast<int64_t>(part) * nd.L.n_edges * (C * 64);
+  const GAS char *P = reinterpret_cast<const GAS char *>(to_global(nd.Pf)) + p0;
+  const GAS char *PT = reinterpret_cast<const GAS char *>(to_global(nd.PfT)) + p0;
+  const uint32_t off = lane * 16, soff = sl * 4, aoff = W::cat(lane) * 64 + (lane & 3) * 16;
+  const f32x4 Q = *reinterpret_cast<const GAS f32x4 *>(reinterpret_cast<const GAS char *>(to_global(nd.Qf)) +
+                                                       part * (C * 64) + aoff);
   double pi[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) pi[i] = freqs[part * 4 + i];
-  const int64_t row_elems = n * C * 4;  // floats of one CLV / adjoint slot
-  const uint32_t off_row = static_cast<uint32_t>((site * C + c) * 4) * 4u;  // bytes into such a slot
-  const uint32_t off_site = static_cast<uint32_t>(site) * 4u;  // bytes into a scaler / exponent slot
-  for (int gi = n_groups - 1; gi >= 0; --gi) {
-    const int g0 = group_begin[gi];
-    const int nb = group_begin[gi + 1] - g0;
-    // load the adjoints and children of the whole group first, as raw
-    // values: nothing in this phase waits for an earlier load
-    __builtin_amdgcn_s_setprio(1);
-    float aq[G][4], x[G][2][4], xq[G][4], acc[G][2][4];
-    // sk: a child's scaler, or a tip child's code (one register for both)
-    int gq[G], kq[G], sk[G][2], eacc[G][2];
+  for (int i = 0; i < 4; ++i) pi[i] = to_global(nd.freqs)[part * 4 + i];
+  const GAS double *seed = to_global(nd.seed) + site0 + sl;
+  const GAS double *beta = to_global(nd.beta) + part * nd.n_root;
+  GAS double *grad = to_global(nd.grad_partials) + site0 / W::SPW * nd.n_uses;
+  const CAS DevOp *ops = to_constant(nd.ops_adj);
+  const int n_ops = nd.n_adj;
+
+  auto load = [&](const OpRegs &op, AdjIn32<C, NR> &in) {
+    const uint32_t o = opaque(off), so = opaque(soff), tip_o = opaque(sl), ao = opaque(aoff);
 #pragma unroll
-    for (int j = 0; j < G; ++j) {
-      if (j < nb) {
-        const DevOp op = ops[g0 + j];
-        kq[j] = *at(scl + op.out * n, off_site);
-        if (op.flags & OP_HAS_CONSUMERS) {
-          if (op.flags & OP_A_PASS) {
-            const int slot = pass_slot(op.flags, 2);
-            const float4 v = reinterpret_cast<const float4 *>(pass_m)[slot * NT + threadIdx.x];
-            aq[j][0] = v.x;
-            aq[j][1] = v.y;
-            aq[j][2] = v.z;
-            aq[j][3] = v.w;
-            gq[j] = pass_e[slot * TS + site_in_tile];
-          } else {
-            load4(at(adj + op.out * row_elems, off_row), aq[j]);
-            gq[j] = *at(adj_exp + op.out * n, off_site);
-          }
-        }
-        if (op.root >= 0) load4(at(clv + op.out * row_elems, off_row), xq[j]);
-      }
+    for (int k = 0; k < 2; ++k) {
+      in.A[k] = *reinterpret_cast<const GAS f32x4 *>(P + op.edge(k) * (C * 64) + ao);
+      in.AT[k] = *reinterpret_cast<const GAS f32x4 *>(PT + op.edge(k) * (C * 64) + ao);
     }
 #pragma unroll
-    for (int j = 0; j < G; ++j) {
+    for (int r = 0; r < NR; ++r)
+      in.word[r] = *reinterpret_cast<const GAS int32_t *>(scl + op.out() * (n * 4) + so + r * (W::SPB * 4));
 #pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
-        if (j < nb) {
-          const DevOp op = ops[g0 + j];
-          const int32_t kid = op.kid[kk];
-          if (kk < op.nk && kid >= 0) {
-            load4(at(clv + kid * row_elems, off_row), x[j][kk]);
-            sk[j][kk] = *at(scl + kid * n, off_site);
-            if (op.flags & (kk == 0 ? OP_ACC_EARLY0 : OP_ACC_EARLY1)) {
-              // the child's accumulated adjoint, last written two or more groups ago
-              load4(at(adj + kid * row_elems, off_row), acc[j][kk]);
-              eacc[j][kk] = *at(adj_exp + kid * n, off_site);
-            }
-          }
-        }
+    for (int k = 0; k < 2; ++k) {
+      // (a one-child op's second child stands for its first)
+      const int32_t kid = k < op.nk() ? op.kid(k) : op.kid(0);
+      if (kid < 0) {
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+          in.raw[k * NR + r] =
+              *reinterpret_cast<const GAS uint8_t *>(tips + static_cast<uint32_t>(~kid) * n + tip_o + r * W::SPB);
+      } else if (k < op.nk()) {
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+          in.x[k * NR + r] = *reinterpret_cast<const GAS f32x4 *>(clv + static_cast<uint32_t>(kid) * row + o + r * 1024);
       }
     }
+    if ((op.flags() & (OP_HAS_CONSUMERS | OP_A_PASS | OP_A_LATE)) == OP_HAS_CONSUMERS)
 #pragma unroll
-    for (int j = 0; j < G; ++j) {
+      for (int r = 0; r < NR; ++r) {
+        in.a[r] = *reinterpret_cast<const GAS f32x4 *>(adj + op.out() * row + o + r * 1024);
+        in.ea[r] = *reinterpret_cast<const GAS int32_t *>(adj_exp + op.out() * (n * 4) + so + r * (W::SPB * 4));
+      }
+    if (op.root() >= 0)
 #pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
-        if (j < nb) {
-          const DevOp op = ops[g0 + j];
-          const int32_t kid = op.kid[kk];
-          if (kk < op.nk && kid < 0) sk[j][kk] = *at(tips + (-kid - 1) * n, static_cast<uint32_t>(site));
+      for (int r = 0; r < NR; ++r) in.sd[r] = seed[op.root() * static_cast<int64_t>(n) + r * W::SPB];
+  };
+  auto early = [&](const OpRegs &op) {
+    Held32<NR> held;
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      if (op.has(OP_ACC0, OP_ACC1, k))
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          const uint64_t kid = static_cast<uint32_t>(op.kid(k));
+          const uint32_t o = opaque(off), so = opaque(soff);
+          held.m[k * NR + r] = *reinterpret_cast<const GAS f32x4 *>(adj + kid * row + o + r * 1024);
+          held.e[k * NR + r] = *reinterpret_cast<const GAS int32_t *>(adj_exp + kid * (n * 4) + so + r * (W::SPB * 4));
         }
+    return held;
+  };
+  // Delivers the vectors b (exponents ez) to child k's adjoint, adding what is
+  // there already unless this is the first delivery.  The sum is left as it
+  // is: mantissas between an op's factor (far above FP32's smallest) and the
+  // number of deliveries; the child's op renormalises it.
+  auto deliver = [&](const OpRegs &op, int k, f32x4 (&b)[NR], const int (&ez)[NR], Held32<NR> &held) {
+    const bool pass = op.has(OP_PASS_KID0, OP_PASS_KID1, k);
+    f32x4 *slot = slots + op.slot(k) * (NR * 64) + lane;
+    int32_t *se = slot_e + op.slot(k) * (NR * W::SPB) + sl;
+    int eb[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) eb[r] = ez[r];
+    if (!op.has(OP_FIRST_KID0, OP_FIRST_KID1, k)) {
+      if (pass)
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          held.m[k * NR + r] = slot[r * 64];
+          held.e[k * NR + r] = se[r * W::SPB];
+        }
+#pragma unroll
+      for (int r = 0; r < NR; ++r) eb[r] = align_add(b[r], eb[r], held.m[k * NR + r], held.e[k * NR + r]);
+    }
+    if (pass) {
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        slot[r * 64] = b[r];
+        se[r * W::SPB] = eb[r];  // (the lanes of a site store the same exponent)
+      }
+    } else {
+      const uint64_t kid = static_cast<uint32_t>(op.kid(k));
+      const uint32_t o = opaque(off), so = opaque(soff);
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        *reinterpret_cast<GAS f32x4 *>(adj + kid * row + o + r * 1024) = b[r];
+        *reinterpret_cast<GAS int32_t *>(adj_exp + kid * (n * 4) + so + r * (W::SPB * 4)) = eb[r];
       }
     }
-    __builtin_amdgcn_s_setprio(0);
-    wait_loads();
-    int ks[G];
+  };
+  int flushed = ops[n_ops - 1].gslot[0];  // the sweep's first gradient row
+  const int rows_end = nd.n_uses;
+  auto step = [&](const OpRegs &op, AdjIn32<C, NR> &in, Held32<NR> &held) {
+    f32x4 (&a)[NR] = in.a;
+    int32_t (&ez)[NR] = in.ea;
+    if (op.flags() & OP_A_PASS) {
 #pragma unroll
-    for (int j = 0; j < G; ++j) {
-      if (j < nb) {
-        const DevOp op = ops[g0 + j];
-        ks[j] = 0;
+      for (int r = 0; r < NR; ++r) {
+        a[r] = slots[(op.slot(2) * NR + r) * 64 + lane];
+        ez[r] = slot_e[(op.slot(2) * NR + r) * W::SPB + sl];
+      }
+    } else if (op.flags() & OP_A_LATE) {
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-          if (kk < op.nk) {
-            if (op.kid[kk] < 0)
-              tip_vec4(static_cast<uint32_t>(sk[j][kk]), x[j][kk]);
-            else
-              ks[j] += sk[j][kk];
-          }
-        }
-        const bool has_adj = (op.flags & OP_HAS_CONSUMERS) != 0;
-        float a[4];
+      for (int r = 0; r < NR; ++r) {
+        a[r] = *reinterpret_cast<const GAS f32x4 *>(adj + op.out() * row + off + r * 1024);
+        ez[r] = *reinterpret_cast<const GAS int32_t *>(adj_exp + op.out() * (n * 4) + soff + r * (W::SPB * 4));
+      }
+      wait_loads();
+    } else if (!(op.flags() & OP_HAS_CONSUMERS)) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) a[i] = has_adj ? aq[j][i] : 0.f;
-        int ea = has_adj ? gq[j] : EXP_EMPTY;
-        if (op.root >= 0) {
-          double t = 0.0;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) t = fma(pi[i], static_cast<double>(xq[j][i]), t);
-          t = cat_sum<C>(t) * (1.0 / C);
-          const double b = beta[part * n_root + op.root] * w;
-          int ef = EXP_EMPTY;
-          float sd[4] = {0.f, 0.f, 0.f, 0.f};
-          if (b != 0.0) {
-            const double mf = frexp(b / (C * t), &ef);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) sd[i] = static_cast<float>(mf * pi[i]);
-          }
-          ea = align_add(a, ea, sd, ef);
-        }
-        // y_k = P_k x_k, z_0 = a y_1 (or a), z_1 = a y_0 and back_k = P_k^T z_k
-        // read P_0 once (row i gives y_0[i], then z_0[i] and row i's share of
-        // back_0) and P_1 twice: three matrix reads from LDS per op, not four
-        float y[2][4], z[2][4], back[2][4];
-        const float *P0 = sP + (op.edge[0] * C + c) * 16;
-        // (a select, not op.edge[op.nk - 1]: a runtime index would put op on the stack)
-        const float *P1 = sP + ((op.nk == 2 ? op.edge[1] : op.edge[0]) * C + c) * 16;
-        if (op.nk == 2) mv4(P1, x[j][1], y[1]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float4 r = reinterpret_cast<const float4 *>(P0)[i];
-          y[0][i] = fmaf(r.w, x[j][0][3], fmaf(r.z, x[j][0][2], fmaf(r.y, x[j][0][1], r.x * x[j][0][0])));
-          z[0][i] = op.nk == 2 ? a[i] * y[1][i] : a[i];
-          if (i == 0) {
-            back[0][0] = r.x * z[0][0];
-            back[0][1] = r.y * z[0][0];
-            back[0][2] = r.z * z[0][0];
-            back[0][3] = r.w * z[0][0];
-          } else {
-            back[0][0] = fmaf(r.x, z[0][i], back[0][0]);
-            back[0][1] = fmaf(r.y, z[0][i], back[0][1]);
-            back[0][2] = fmaf(r.z, z[0][i], back[0][2]);
-            back[0][3] = fmaf(r.w, z[0][i], back[0][3]);
-          }
-        }
-        if (op.nk == 2) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) z[1][i] = a[i] * y[0][i];
-          mv4t(P1, z[1], back[1]);
-        }
-        const int ez = ea + kq[j] - ks[j];
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-          if (kk < op.nk) {
-            float qx[4];
-            mv4(Qr, y[kk], qx);
-            const float gd =
-                fmaf(z[kk][3], qx[3], fmaf(z[kk][2], qx[2], fmaf(z[kk][1], qx[1], z[kk][0] * qx[0])));
-            // the site's share of dlnL/dt is O(weight / t): FP32 holds it
-            const double gv = wave_sum_f32(ldexpf(gd, ez));
-            if ((threadIdx.x & 63) == 0) grad_partials[grad_index(tile, n_uses, op.gslot[kk], PWB, wave)] = gv;
-            const int32_t kid = op.kid[kk];
-            if (kid >= 0 && (op.flags & (kk == 0 ? OP_PASS_KID0 : OP_PASS_KID1))) {
-              const int slot = pass_slot(op.flags, kk);
-              pass_delivery<C>(pass_m + 4 * (slot * NT + threadIdx.x), pass_e + slot * TS + site_in_tile,
-                               (op.flags & (kk == 0 ? OP_FIRST_KID0 : OP_FIRST_KID1)) != 0, back[kk], ez);
-            } else if (kid >= 0) {
-              GAS float *dst_m = at(adj + kid * row_elems, off_row);
-              GAS int32_t *dst_e = at(adj_exp + kid * n, off_site);
-              const bool first = (op.flags & (kk == 0 ? OP_FIRST_KID0 : OP_FIRST_KID1)) != 0;
-              if (first || (op.flags & (kk == 0 ? OP_ACC_EARLY0 : OP_ACC_EARLY1))) {
-                finish_delivery<C>(dst_m, dst_e, first, lane0, back[kk], ez, acc[j][kk], eacc[j][kk]);
-              } else {
-                // the schedule keeps two deliveries to one child out of a
-                // group, so this read-back of the adjoint written by an
-                // earlier op of this group is never taken; kept for any schedule
-                float acc_now[4];
-                load4(dst_m, acc_now);
-                finish_delivery<C>(dst_m, dst_e, false, lane0, back[kk], ez, acc_now, *dst_e);
-              }
-            }
-          }
-        }
+      for (int r = 0; r < NR; ++r) {
+        a[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+        ez[r] = EXP_EMPTY;
       }
     }
-  }
+    if (op.root() >= 0) {
+      // seed beta * w * (1/C) pi_i / Ltilde at a displayed-tree root
+      const double bt = beta[op.root()];
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        int ef = EXP_EMPTY;
+        f32x4 sd = {0.f, 0.f, 0.f, 0.f};
+        const double f = bt * in.sd[r];
+        if (f != 0.0) {
+          const double mf = frexp(f, &ef);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) sd[i] = static_cast<float>(mf * pi[i]);
+        }
+        ez[r] = align_add(a[r], ez[r], sd, ef);
+      }
+    }
+    // the site maximum of |a| to [0.5, 1), an all-zero adjoint to exponent
+    // EXP_EMPTY (so that what it delivers cannot scale another delivery away),
+    // and the exponent of z: the CLV's exponent less its children's is the
+    // op's step
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      const float m = site_absmax<C>(a[r]);
+      const int e = __builtin_amdgcn_frexp_expf(m);  // 0 of 0
+      a[r] = scale4(a[r], -e);
+      ez[r] = m > 0.f ? ez[r] + e - word_step(in.word[r]) : EXP_EMPTY;
+    }
+    f32x4 y[2][NR];
+    float g[2] = {0.f, 0.f};
+    auto product = [&](int k) {
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        if (op.kid(k) < 0) in.x[k * NR + r] = tip_row(in.raw[k * NR + r]);
+        y[k][r] = product4(in.A[k], in.x[k * NR + r]);
+      }
+    };
+    auto use = [&](int k, f32x4 (&z)[NR]) {
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        const f32x4 d = product4(Q, y[k][r]);
+        const float gd = fmaf(z[r][3], d[3], fmaf(z[r][2], d[2], fmaf(z[r][1], d[1], z[r][0] * d[0])));
+        // the site's share of dlnL/dt is O(weight / t): FP32 holds it
+        g[k] += ldexpf(gd, ez[r]);
+      }
+      if (op.kid(k) >= 0) {
+#pragma unroll
+        for (int r = 0; r < NR; ++r) z[r] = product4(in.AT[k], z[r]);
+        deliver(op, k, z, ez, held);
+      }
+    };
+    product(0);
+    f32x4 z[NR];
+    if (op.nk() == 2) {
+      product(1);
+#pragma unroll
+      for (int r = 0; r < NR; ++r) z[r] = a[r] * y[1][r];
+      use(0, z);
+#pragma unroll
+      for (int r = 0; r < NR; ++r) z[r] = a[r] * y[0][r];
+      use(1, z);
+    } else {
+#pragma unroll
+      for (int r = 0; r < NR; ++r) z[r] = a[r];
+      use(0, z);
+    }
+    // (rows leave as in k_adjoint_level)
+    const float total = pair_wave_sum_f32(g[0], g[1]);
+    const int k = lane >> 5;
+    if ((lane & 31) == 31 && k < op.nk()) ring[(op.gslot() + k) % GRAD_RING] = total;
+    const int done = op.gslot() + op.nk();
+    if (done - flushed >= 64) {
+      grad[flushed + lane] = ring[(flushed + lane) % GRAD_RING];
+      flushed += 64;
+    }
+    if (done == rows_end && lane < done - flushed) grad[flushed + lane] = ring[(flushed + lane) % GRAD_RING];
+  };
+  walk_ops<AdjIn32<C, NR>>(ops, n_ops, true, load, early, step);
 }
 
-template <int C, int G, int TS>
-__global__ void __launch_bounds__(TS *C, 3)
+// WG threads per workgroup: one wave, which the device places wherever a SIMD
+// has room (41,345 patterns, gradient: 0.41 ms, 0.54 with four waves per
+// workgroup).  G = 2: two row blocks per wave, G = 3: one (see walk_blocks).
+template <int G>
+constexpr int row_blocks = G == 2 ? 2 : 1;
+
+template <int C, int G, int WG>
+__global__ void __launch_bounds__(WG, 3)
+    k_forward_persistent(const NetDesc *__restrict__ nets, const WorkItem *__restrict__ work) {
+  static_assert(WG == 64, "a workgroup is one wave");
+  const WorkItem wi = to_constant(work)[blockIdx.x];
+  forward_walk32<C, row_blocks<G>>(nets[wi.net], dyn_lds<float>(),
+                                   static_cast<int64_t>(wi.tile) * Rows<C, row_blocks<G>>::SPW);
+}
+
+template <int C, int G, int WG>
+__global__ void __launch_bounds__(WG, 3)
     k_adjoint_persistent(const NetDesc *__restrict__ nets, const WorkItem *__restrict__ work) {
-  const WorkItem wi = work[blockIdx.x];
-  const NetDesc &nd = nets[wi.net];
-  adjoint_persistent_body<C, G, TS>(to_constant(nd.ops), to_constant(nd.group_begin), nd.n_groups, nd.L,
-                                    to_global(nd.clv), to_global(nd.scl), to_global(nd.adj),
-                                    to_global(nd.adj_exp), to_global(nd.tips), to_global(nd.Pf),
-                                    to_global(nd.Qf), to_global(nd.tile_part), to_global(nd.freqs),
-                                    to_global(nd.weights), to_global(nd.beta), nd.n_root, nd.n_uses,
-                                    nd.n_pass, to_global(nd.grad_partials), wi.tile);
-}
-
-// ------------------------------------------- reverse sweep, two lanes per row
-// The same sweep (ops, groups, flags, LDS pass slots, arithmetic) with each
-// (site, category) row of 4 states held by two adjacent lanes: lane h = 0
-// holds states 0, 1 and lane h = 1 states 2, 3 (threadIdx.x = (site C +
-// category) 2 + h).  A tile then has twice the waves, each carrying half the
-// registers per op, so more groups' loads are in flight per SIMD.  Products
-// with a 4 x 4 matrix need the partner's two values (one DPP move each):
-//   y = P x      my rows of P times (mine, partner's) x
-//   back = P^T z partial sums over my two rows for all four columns; the
-//                partner's partials for my columns arrive by DPP
-//   Q y          as P x, on the exchanged y
-// The P and Q tables in LDS are stored per lane half: block h of a (edge,
-// category) holds rows 2h, 2h+1 with the columns reordered (2h, 2h+1, then
-// the partner's two), so every lane reads its operands in one fixed order.
-__device__ __forceinline__ float pair_swap(float v) { return dpp<DPP_XOR1>(v); }
-
-// maximum / sum over the 2C lanes of a site (halves at lane bit 0,
-// categories at bits 1 ..)
-template <int C>
-__device__ __forceinline__ float site_max2(float m) {  // integer max, as cat_maxf
-  int u = __float_as_int(m);
-  u = max(u, dpp_i<DPP_XOR1>(u));
-  if constexpr (C > 1) u = max(u, dpp_i<DPP_XOR2>(u));
-  if constexpr (C > 2) u = max(u, __shfl_xor(u, 4));
-  if constexpr (C > 4) u = max(u, __shfl_xor(u, 8));
-  return __int_as_float(u);
-}
-template <int C>
-__device__ __forceinline__ double site_sum2(double m) {
-  m += dpp<DPP_XOR1>(m);
-  if constexpr (C > 1) m += dpp<DPP_XOR2>(m);
-  if constexpr (C > 2) m += __shfl_xor(m, 4);
-  if constexpr (C > 4) m += __shfl_xor(m, 8);
-  return m;
-}
-
-// source index in a row-major 4 x 4 matrix of entry r (0..15) of lane half
-// h's block: rows 2h + r / 4 % 2, columns (2h, 2h+1, partner's two)
-__device__ __forceinline__ int half_block_src(int r) {
-  const int h = r >> 3, k = (r >> 2) & 1, q = r & 3;
-  const int row = 2 * h + k;
-  const int col = q < 2 ? 2 * h + q : 2 * (1 - h) + (q - 2);
-  return row * 4 + col;
-}
-
-// y (my two rows) = M (x, partner's x); M = the lane's 8-entry block
-__device__ __forceinline__ void mv2(const float *__restrict__ M, float x0, float x1, float o0, float o1,
-                                    float &y0, float &y1) {
-  y0 = fmaf(M[3], o1, fmaf(M[2], o0, fmaf(M[1], x1, M[0] * x0)));
-  y1 = fmaf(M[7], o1, fmaf(M[6], o0, fmaf(M[5], x1, M[4] * x0)));
-}
-
-// (P^T z) for my two states from my block and my two z values
-__device__ __forceinline__ void mv2t(const float *__restrict__ M, float z0, float z1, float &b0, float &b1) {
-  const float p0 = fmaf(M[4], z1, M[0] * z0);  // columns 2h, 2h+1: my states
-  const float p1 = fmaf(M[5], z1, M[1] * z0);
-  const float q0 = fmaf(M[6], z1, M[2] * z0);  // the partner's states
-  const float q1 = fmaf(M[7], z1, M[3] * z0);
-  b0 = p0 + pair_swap(q0);
-  b1 = p1 + pair_swap(q1);
-}
-
-// x 2^ex + y 2^ey (two values), aligned to the larger exponent
-__device__ __forceinline__ int align_add2(float &x0, float &x1, int ex, float y0, float y1, int ey) {
-  const int e = max(ex, ey);
-  const float sx = ldexpf(1.0f, ex - e), sy = ldexpf(1.0f, ey - e);
-  x0 = fmaf(x0, sx, y0 * sy);
-  x1 = fmaf(x1, sx, y1 * sy);
-  return e;
-}
-
-__device__ __forceinline__ int renorm2(float &x0, float &x1, int ex, float m) {
-  int e = 0;
-  (void)frexpf(m, &e);
-  x0 = ldexpf(x0, -e);
-  x1 = ldexpf(x1, -e);
-  return m > 0.f ? ex + e : EXP_EMPTY;
-}
-
-__device__ __forceinline__ void load2(const GAS float *__restrict__ p, float &a, float &b) {
-  const float2 v = *reinterpret_cast<const GAS float2 *>(p);
-  a = v.x;
-  b = v.y;
-}
-__device__ __forceinline__ void store2(GAS float *__restrict__ p, float a, float b) {
-  *reinterpret_cast<GAS float2 *>(p) = make_float2(a, b);
-}
-
-// delivered (b, eb) plus the accumulated (acc, ea) unless first, then
-// renormalised (as finish_delivery)
-template <int C>
-__device__ __forceinline__ void finish_delivery2(float &b0, float &b1, int &eb, bool first, float a0, float a1,
-                                                 int ea) {
-  float mb = site_max2<C>(fmaxf(fabsf(b0), fabsf(b1)));
-  if (!first) {
-    eb = align_add2(b0, b1, mb > 0.f ? eb : EXP_EMPTY, a0, a1, ea);
-    mb = site_max2<C>(fmaxf(fabsf(b0), fabsf(b1)));
-  }
-  eb = renorm2(b0, b1, eb, mb);
-}
-
-template <int C, int G, int TS>
-__device__ __forceinline__ void adjoint_split_body(
-    const CAS DevOp *__restrict__ ops, const CAS int32_t *__restrict__ group_begin, int n_groups,
-    const DevLayout L, const GAS float *__restrict__ clv, const GAS int32_t *__restrict__ scl,
-    GAS float *__restrict__ adj, GAS int32_t *__restrict__ adj_exp,
-    const GAS uint8_t *__restrict__ tips, const GAS float *__restrict__ Pf,
-    const GAS float *__restrict__ Qf, const GAS int32_t *__restrict__ tile_part,
-    const GAS double *__restrict__ freqs, const GAS double *__restrict__ weights,
-    const GAS double *__restrict__ beta, int n_root, int n_uses, int n_pass,
-    GAS double *__restrict__ grad_partials, int tile) {
-  float *sP = dyn_lds<float>();  // [edge][cat][half][8] then Q [cat][half][8], then pass slots
-  constexpr int NT = TS * C * 2;
-  constexpr int PWB = NT / 64;  // waves of this site block
-  const int64_t site0 = static_cast<int64_t>(tile) * TS;
-  const int part = tile_part[site0 / TILE];
-  const int np = L.n_edges * C * 16;
-  const GAS float *gP = Pf + static_cast<size_t>(part) * np;
-  for (int i = threadIdx.x; i < np; i += NT) sP[i] = gP[(i & ~15) + half_block_src(i & 15)];
-  for (int i = threadIdx.x; i < C * 16; i += NT) sP[np + i] = Qf[part * C * 16 + (i & ~15) + half_block_src(i & 15)];
-  __syncthreads();
-  const int h = threadIdx.x & 1;
-  const int c = (threadIdx.x >> 1) % C;
-  float Qr[8];  // this lane's half block of r_c Q, kept in registers
-#pragma unroll
-  for (int i = 0; i < 8; ++i) Qr[i] = sP[np + c * 16 + h * 8 + i];
-  // pass slots: mantissas [slot][thread][2], site exponents [slot][site]
-  float *pass_m = sP + ((np + C * 16 + 3) & ~3);
-  int *pass_e = reinterpret_cast<int *>(pass_m + n_pass * NT * 2);
-  const int site_in_tile = threadIdx.x / (2 * C);
-  const int64_t site = site0 + site_in_tile;
-  const int64_t n = L.n_sites_pad;
-  const int wave = threadIdx.x / 64;
-  const bool lead = (threadIdx.x & (2 * C - 1)) == 0;  // writes the site's exponent
-  const double w = weights[site];
-  const double pi0 = freqs[part * 4 + 2 * h], pi1 = freqs[part * 4 + 2 * h + 1];
-  const size_t row = C * 4;
-  const int off = c * 4 + 2 * h;  // my two states within a site's row
-  for (int gi = n_groups - 1; gi >= 0; --gi) {
-    const int g0 = group_begin[gi];
-    const int nb = group_begin[gi + 1] - g0;
-    float aq[G][2], x[G][2][2], xq[G][2], acc[G][2][2];
-    int gq[G], kq[G], sk[G][2], eacc[G][2];
-    uint32_t tm[G][2];
-#pragma unroll
-    for (int j = 0; j < G; ++j) {
-      if (j < nb) {
-        const DevOp op = ops[g0 + j];
-        kq[j] = scl[static_cast<size_t>(op.out) * n + site];
-        if (op.flags & OP_HAS_CONSUMERS) {
-          if (op.flags & OP_A_PASS) {
-            const int slot = pass_slot(op.flags, 2);
-            const float2 v = reinterpret_cast<const float2 *>(pass_m)[slot * NT + threadIdx.x];
-            aq[j][0] = v.x;
-            aq[j][1] = v.y;
-            gq[j] = pass_e[slot * TS + site_in_tile];
-          } else {
-            load2(adj + (static_cast<size_t>(op.out) * n + site) * row + off, aq[j][0], aq[j][1]);
-            gq[j] = adj_exp[static_cast<size_t>(op.out) * n + site];
-          }
-        }
-        if (op.root >= 0) load2(clv + (static_cast<size_t>(op.out) * n + site) * row + off, xq[j][0], xq[j][1]);
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < G; ++j) {
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
-        if (j < nb) {
-          const DevOp op = ops[g0 + j];
-          const int32_t kid = op.kid[kk];
-          if (kk < op.nk && kid >= 0) {
-            load2(clv + (static_cast<size_t>(kid) * n + site) * row + off, x[j][kk][0], x[j][kk][1]);
-            sk[j][kk] = scl[static_cast<size_t>(kid) * n + site];
-            if (op.flags & (kk == 0 ? OP_ACC_EARLY0 : OP_ACC_EARLY1)) {
-              load2(adj + (static_cast<size_t>(kid) * n + site) * row + off, acc[j][kk][0], acc[j][kk][1]);
-              eacc[j][kk] = adj_exp[static_cast<size_t>(kid) * n + site];
-            }
-          }
-        }
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < G; ++j) {
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
-        if (j < nb) {
-          const DevOp op = ops[g0 + j];
-          const int32_t kid = op.kid[kk];
-          if (kk < op.nk && kid < 0) tm[j][kk] = tips[static_cast<size_t>(-kid - 1) * n + site];
-        }
-      }
-    }
-    wait_loads();
-#pragma unroll
-    for (int j = 0; j < G; ++j) {
-      if (j < nb) {
-        const DevOp op = ops[g0 + j];
-        int ks = 0;
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-          if (kk < op.nk) {
-            if (op.kid[kk] < 0) {
-              const uint32_t m = tm[j][kk] >> (2 * h);
-              x[j][kk][0] = (m & 1u) ? 1.f : 0.f;
-              x[j][kk][1] = (m & 2u) ? 1.f : 0.f;
-            } else {
-              ks += sk[j][kk];
-            }
-          }
-        }
-        const bool has_adj = (op.flags & OP_HAS_CONSUMERS) != 0;
-        float a0 = has_adj ? aq[j][0] : 0.f, a1 = has_adj ? aq[j][1] : 0.f;
-        int ea = has_adj ? gq[j] : EXP_EMPTY;
-        if (op.root >= 0) {
-          double t = site_sum2<C>(fma(pi0, static_cast<double>(xq[j][0]), pi1 * static_cast<double>(xq[j][1])));
-          t *= 1.0 / C;
-          const double b = beta[part * n_root + op.root] * w;
-          int ef = EXP_EMPTY;
-          float sd0 = 0.f, sd1 = 0.f;
-          if (b != 0.0) {
-            const double mf = frexp(b / (C * t), &ef);
-            sd0 = static_cast<float>(mf * pi0);
-            sd1 = static_cast<float>(mf * pi1);
-          }
-          ea = align_add2(a0, a1, ea, sd0, sd1, ef);
-        }
-        float y[2][2];
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk)
-          if (kk < op.nk)
-            mv2(sP + (op.edge[kk] * C + c) * 16 + h * 8, x[j][kk][0], x[j][kk][1], pair_swap(x[j][kk][0]),
-                pair_swap(x[j][kk][1]), y[kk][0], y[kk][1]);
-        const int ez = ea + kq[j] - ks;
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-          if (kk < op.nk) {
-            const float z0 = op.nk == 2 ? a0 * y[1 - kk][0] : a0;
-            const float z1 = op.nk == 2 ? a1 * y[1 - kk][1] : a1;
-            float q0, q1, b0, b1;
-            mv2(Qr, y[kk][0], y[kk][1], pair_swap(y[kk][0]), pair_swap(y[kk][1]), q0, q1);
-            mv2t(sP + (op.edge[kk] * C + c) * 16 + h * 8, z0, z1, b0, b1);
-            const float gd = fmaf(z1, q1, z0 * q0);
-            const double gv = wave_sum_f32(ldexpf(gd, ez));
-            if ((threadIdx.x & 63) == 0) grad_partials[grad_index(tile, n_uses, op.gslot[kk], PWB, wave)] = gv;
-            const int32_t kid = op.kid[kk];
-            if (kid < 0) continue;
-            const bool first = (op.flags & (kk == 0 ? OP_FIRST_KID0 : OP_FIRST_KID1)) != 0;
-            int eb = ez;
-            if (op.flags & (kk == 0 ? OP_PASS_KID0 : OP_PASS_KID1)) {
-              const int slot = pass_slot(op.flags, kk);
-              float2 *sm = reinterpret_cast<float2 *>(pass_m) + slot * NT + threadIdx.x;
-              int *se = pass_e + slot * TS + site_in_tile;
-              float p0 = 0.f, p1 = 0.f;
-              int pe = EXP_EMPTY;
-              if (!first) {
-                const float2 v = *sm;
-                p0 = v.x;
-                p1 = v.y;
-                pe = *se;
-              }
-              finish_delivery2<C>(b0, b1, eb, first, p0, p1, pe);
-              *sm = make_float2(b0, b1);
-              *se = eb;  // every lane of the site writes the same value
-            } else {
-              GAS float *dst_m = adj + (static_cast<size_t>(kid) * n + site) * row + off;
-              GAS int32_t *dst_e = adj_exp + static_cast<size_t>(kid) * n + site;
-              float p0 = 0.f, p1 = 0.f;
-              int pe = EXP_EMPTY;
-              if (!first) {
-                if (op.flags & (kk == 0 ? OP_ACC_EARLY0 : OP_ACC_EARLY1)) {
-                  p0 = acc[j][kk][0];
-                  p1 = acc[j][kk][1];
-                  pe = eacc[j][kk];
-                } else {
-                  // an earlier op of this group or the previous group wrote it: read it now
-                  load2(dst_m, p0, p1);
-                  pe = *dst_e;
-                }
-              }
-              finish_delivery2<C>(b0, b1, eb, first, p0, p1, pe);
-              store2(dst_m, b0, b1);
-              if (lead) *dst_e = eb;
-            }
-          }
-        }
-      }
-    }
-  }
-}
-
-template <int C, int G, int TS>
-__global__ void __launch_bounds__(TS *C * 2)
-    k_adjoint_split(const NetDesc *__restrict__ nets, const WorkItem *__restrict__ work) {
-  const WorkItem wi = work[blockIdx.x];
-  const NetDesc &nd = nets[wi.net];
-  adjoint_split_body<C, G, TS>(to_constant(nd.ops), to_constant(nd.group_begin), nd.n_groups, nd.L,
-                               to_global(nd.clv), to_global(nd.scl), to_global(nd.adj), to_global(nd.adj_exp),
-                               to_global(nd.tips), to_global(nd.Pf), to_global(nd.Qf), to_global(nd.tile_part),
-                               to_global(nd.freqs), to_global(nd.weights), to_global(nd.beta), nd.n_root,
-                               nd.n_uses, nd.n_pass, to_global(nd.grad_partials), wi.tile);
+  static_assert(WG == 64, "a workgroup is one wave");
+  const WorkItem wi = to_constant(work)[blockIdx.x];
+  adjoint_walk32<C, row_blocks<G>>(nets[wi.net], dyn_lds<float>(),
+                                   static_cast<int64_t>(wi.tile) * Rows<C, row_blocks<G>>::SPW);
 }
 
 // ============================================= FP32 form, 20 states (MFMA)
@@ -2762,18 +2478,23 @@ __device__ __forceinline__ void stage_path_p(double *sPp, const PathStep *__rest
 // in for absent ones, so no load sits on one path of a branch) is issued
 // before its arithmetic, which then only waits on LDS and registers.  A
 // step's own scaler is the previous step's child scaler.
-// rescalings a scaler word counts (FP64 4-state words: see k_forward_walk)
+// rescalings (FP64) or exponent (FP32) that a CLV's scaler word counts
 template <int S, typename T>
 __device__ __forceinline__ int scl_count(int32_t word) {
-  return S == 4 && std::is_same<T, double>::value ? word >> 1 : word;
+  if constexpr (S != 4) return word;
+  return std::is_same<T, double>::value ? word >> 1 : word_k(word);
 }
 // a thread's row in a CLV slot of either form (FP32 rows are kept whole)
 template <int S, int C, typename T>
 __device__ __forceinline__ size_t clv_row(int64_t site, int c) {
-  if constexpr (std::is_same<T, double>::value)
+  if constexpr (std::is_same<T, double>::value) {
     return row_offset<S, C>(site, c);
-  else
+  } else if constexpr (S == 4) {
+    constexpr int SPB = Rows<C, 1>::SPB;
+    return static_cast<size_t>(site / SPB * 64 + Rows<C, 1>::lane_of(static_cast<int>(site % SPB), c)) * 4;
+  } else {
     return static_cast<size_t>(site * C + c) * S;
+  }
 }
 
 template <int S, int C, typename T>
@@ -3314,6 +3035,7 @@ __global__ void k_pmatrices_multi(const SmallDesc *__restrict__ descs) {
   d.dP[idx] = a1;
   d.d2P[idx] = a2;
   d.Pf[idx] = static_cast<float>(a0);
+  d.PfT[idx - (i * S + j) + (j * S + i)] = static_cast<float>(a0);
 }
 
 __device__ void reduce_segments_body(const double *__restrict__ in, size_t row_stride, int pw,
@@ -3438,7 +3160,7 @@ void launch_pmatrices(Engine &e) {
   hipLaunchKernelGGL(k_pmatrices, dim3(nb), dim3(256), 0, e.stream, e.L, e.d_V.as<double>(),
                      e.d_Vinv.as<double>(), e.d_eval.as<double>(), e.d_rates.as<double>(),
                      e.d_brlen.as<double>(), e.d_P.as<double>(), e.d_dP.as<double>(),
-                     e.d_d2P.as<double>(), e.d_Pf.as<float>(), e.d_dPf.as<float>());
+                     e.d_d2P.as<double>(), e.d_Pf.as<float>(), e.d_PfT.as<float>());
   NRX_HIP(hipGetLastError());
 }
 
@@ -3483,8 +3205,6 @@ static void dispatch_walk(int C, int NQ, F &&f) {
   });
 }
 
-size_t forward_walk_lds(int nq, int n_slots) { return static_cast<size_t>(n_slots) * (nq * 512 + 256); }
-size_t adjoint_walk_lds(int nq, int n_slots) { return sizeof(double) * GRAD_RING + static_cast<size_t>(n_slots) * nq * 512; }
 
 void launch_forward_walk(Engine &e, const DevOp *ops, int n_ops) {
   if (n_ops == 0) return;
@@ -3576,103 +3296,41 @@ void launch_grad_reduce(Engine &e) {
 
 
 
-// Shapes of the 4-state persistent kernels: group width G in {2, 3, 4, 8}
-// and TS in {16, 32, 64} sites per workgroup with TS C a multiple of 64.
+// Shapes of the 4-state FP32 walks: C categories, one or two row blocks.
 template <typename F>
-void dispatch_shape(int C, int G, int TS, F &&f) {
-  auto with_ts = [&](auto c, auto g) {
-    constexpr int CC = decltype(c)::value;
-    if (TS == 64) return f(c, g, std::integral_constant<int, 64>{});
-    if constexpr (32 * CC % 64 == 0)
-      if (TS == 32) return f(c, g, std::integral_constant<int, 32>{});
-    if constexpr (16 * CC % 64 == 0)
-      if (TS == 16) return f(c, g, std::integral_constant<int, 16>{});
-    throw std::invalid_argument("unsupported sites per workgroup for this number of categories");
-  };
+static void dispatch_walk32(int C, int blocks, F &&f) {
   dispatch_c(C, [&](auto c) {
-    switch (G) {
-      case 2: with_ts(c, std::integral_constant<int, 2>{}); break;
-      case 3: with_ts(c, std::integral_constant<int, 3>{}); break;
-      case 4: with_ts(c, std::integral_constant<int, 4>{}); break;
-      case 8: with_ts(c, std::integral_constant<int, 8>{}); break;
-      default: throw std::invalid_argument("unsupported group width");
-    }
+    if (blocks == 2)
+      f(c, std::integral_constant<int, 2>{});
+    else
+      f(c, std::integral_constant<int, 3>{});
   });
 }
 
 void launch_forward_persistent(Engine &e, const NetDesc *nets) {
-  launch_forward_persistent_multi(e.stream, e.C, e.tune_group, e.tune_tile,
-                                  nets ? nets : e.d_netdesc.as<NetDesc>(), e.d_work.as<WorkItem>(),
-                                  static_cast<int>(e.L.n_sites_pad / e.tune_tile),
-                                  sizeof(float) * e.E * e.C * 16);
+  launch_forward_persistent_multi(e.stream, e.C, e.walk_blocks, nets ? nets : e.d_netdesc.as<NetDesc>(),
+                                  e.d_work.as<WorkItem>(), e.L.n_tiles * e.rpw, e.fwd_slots);
 }
 
 void launch_adjoint_persistent(Engine &e) {
-  launch_adjoint_persistent_multi(e.stream, e.C, e.tune_group, e.tune_tile, e.tune_lanes,
-                                  e.d_netdesc.as<NetDesc>(), e.d_work.as<WorkItem>(),
-                                  static_cast<int>(e.L.n_sites_pad / e.tune_tile),
-                                  adjoint_persistent_lds(e.E, e.C, e.tune_tile, e.pass_slots));
+  launch_adjoint_persistent_multi(e.stream, e.C, e.walk_blocks, e.d_netdesc.as<NetDesc>(), e.d_work.as<WorkItem>(),
+                                  e.L.n_tiles * e.rpw, e.adj_slots);
 }
 
-size_t adjoint_persistent_lds(int E, int C, int TS, int n_pass) {
-  // P and Q tables, padded to 16 bytes, then n_pass slots of 16 bytes per
-  // thread and 4 per site
-  const size_t tables = (static_cast<size_t>(E) * C * 16 + C * 16 + 3) & ~size_t(3);
-  return sizeof(float) * tables + static_cast<size_t>(n_pass) * TS * (C * 4 * sizeof(float) + sizeof(int));
-}
-
-// Pass slots for a reverse-sweep launch of n_work workgroups on the current
-// device: the most slots (at most PASS_SLOTS) whose LDS still lets as many
-// workgroups per CU be resident as the launch can use (its registers and
-// tables allow, and its size fills); 0 when the tables alone do not fit.
-int adjoint_pass_slots(int C, int G, int TS, int H, int E, int64_t n_work) {
-  int dev = 0, n_cu = 0;
-  NRX_HIP(hipGetDevice(&dev));
-  NRX_HIP(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
-  int best = 0;
-  dispatch_shape(C, G, TS, [&](auto c, auto g, auto ts) {
-    constexpr int CC = decltype(c)::value, GG = decltype(g)::value, T = decltype(ts)::value;
-    const void *kern = H == 2 ? reinterpret_cast<const void *>(&k_adjoint_split<CC, GG, T>)
-                              : reinterpret_cast<const void *>(&k_adjoint_persistent<CC, GG, T>);
-    auto resident = [&](int k) {
-      int nb = 0;
-      NRX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, T * CC * H,
-                                                           adjoint_persistent_lds(E, C, TS, k)));
-      return nb;
-    };
-    const int r0 = resident(0);
-    if (r0 == 0) return;
-    const int64_t want = std::min<int64_t>(r0, (n_work + n_cu - 1) / std::max(1, n_cu));
-    for (int k = PASS_SLOTS; k > 0; --k)
-      if (resident(k) >= want) {
-        best = k;
-        return;
-      }
-  });
-  return best;
-}
-
-void launch_forward_persistent_multi(hipStream_t stream, int C, int G, int TS, const NetDesc *nets,
-                                     const WorkItem *work, int n_work, size_t lds) {
-  dispatch_shape(C, G, TS, [&](auto c, auto g, auto ts) {
-    constexpr int CC = decltype(c)::value, GG = decltype(g)::value, T = decltype(ts)::value;
-    hipLaunchKernelGGL((k_forward_persistent<CC, GG, T>), dim3(n_work), dim3(T * CC), lds, stream,
-                       nets, work);
+void launch_forward_persistent_multi(hipStream_t stream, int C, int blocks, const NetDesc *nets, const WorkItem *work,
+                                     int n_work, int max_slots) {
+  dispatch_walk32(C, blocks, [&](auto c, auto g) {
+    hipLaunchKernelGGL((k_forward_persistent<decltype(c)::value, decltype(g)::value, 64>), dim3(n_work), dim3(64),
+                       forward_lds32(C, blocks, max_slots), stream, nets, work);
   });
   NRX_HIP(hipGetLastError());
 }
 
-void launch_adjoint_persistent_multi(hipStream_t stream, int C, int G, int TS, int H, const NetDesc *nets,
-                                     const WorkItem *work, int n_work, size_t lds) {
-  if (H != 1 && H != 2) throw std::invalid_argument("lanes per row must be 1 or 2");
-  dispatch_shape(C, G, TS, [&](auto c, auto g, auto ts) {
-    constexpr int CC = decltype(c)::value, GG = decltype(g)::value, T = decltype(ts)::value;
-    if (H == 2)
-      hipLaunchKernelGGL((k_adjoint_split<CC, GG, T>), dim3(n_work), dim3(T * CC * 2), lds, stream, nets,
-                         work);
-    else
-      hipLaunchKernelGGL((k_adjoint_persistent<CC, GG, T>), dim3(n_work), dim3(T * CC), lds, stream,
-                         nets, work);
+void launch_adjoint_persistent_multi(hipStream_t stream, int C, int blocks, const NetDesc *nets, const WorkItem *work,
+                                     int n_work, int max_slots) {
+  dispatch_walk32(C, blocks, [&](auto c, auto g) {
+    hipLaunchKernelGGL((k_adjoint_persistent<decltype(c)::value, decltype(g)::value, 64>), dim3(n_work), dim3(64),
+                       adjoint_lds32(C, blocks, max_slots), stream, nets, work);
   });
   NRX_HIP(hipGetLastError());
 }

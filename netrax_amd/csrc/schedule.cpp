@@ -122,18 +122,20 @@ void assign_forward_slots(DevOp *ops, int n, int n_slots) {
   std::vector<int> row_in(n_slots, -1), read_at(n_slots, NEVER);
   for (int i = 0; i < n; ++i) {
     DevOp &op = ops[i];
-    op.flags &= ~(OP_PASS_KID0 | OP_PASS_KID1 | OP_A_PASS | PASS_BITS | OP_LOAD0 | OP_LOAD1);
+    op.flags &= ~(OP_PASS_KID0 | OP_PASS_KID1 | OP_A_PASS | OP_LOAD0 | OP_LOAD1);
+    op.slots = 0;
     for (int k = 0; k < op.nk; ++k) {
       if (op.kid[k] < 0) continue;
       const auto it = std::find(row_in.begin(), row_in.end(), op.kid[k]);
       if (it != row_in.end()) {
         const int q = static_cast<int>(it - row_in.begin());
-        op.flags |= (k == 0 ? OP_PASS_KID0 : OP_PASS_KID1) | (q << (PASS_SHIFT + 3 * k));
+        op.flags |= k == 0 ? OP_PASS_KID0 : OP_PASS_KID1;
+        op.slots |= q << (8 * k);
         read_at[q] = later[i][k];
       } else {
-        // the kernel loads an op's inputs before the op before it stores
-        if (made[op.kid[k]] == i - 1 && i > 0)
-          throw std::logic_error("forward walk: a child is read from HBM right after it was made");
+        // the kernel loads an op's inputs one op early
+        if (i > 0 && made[op.kid[k]] == i - 1)
+          throw std::logic_error("forward walk: a child is read from HBM before it is stored");
         op.flags |= k == 0 ? OP_LOAD0 : OP_LOAD1;
       }
     }
@@ -148,7 +150,8 @@ void assign_forward_slots(DevOp *ops, int n, int n_slots) {
     }
     row_in[q] = op.out;
     read_at[q] = first_read[i];
-    op.flags |= OP_A_PASS | (q << (PASS_SHIFT + 6));
+    op.flags |= OP_A_PASS;
+    op.slots |= q << 16;
   }
 }
 
@@ -157,8 +160,7 @@ void assign_forward_slots(DevOp *ops, int n, int n_slots) {
 // A slot's old row is read before the op that releases it delivers, so the
 // slot can take a new row at that op.
 void assign_reverse_slots(DevOp *ops, int n, int n_slots) {
-  constexpr int32_t ALL =
-      OP_PASS_KID0 | OP_PASS_KID1 | OP_A_PASS | PASS_BITS | OP_A_LATE | OP_ACC0 | OP_ACC1;
+  constexpr int32_t ALL = OP_PASS_KID0 | OP_PASS_KID1 | OP_A_PASS | OP_A_LATE | OP_ACC0 | OP_ACC1;
   int rows = 0;
   for (int i = 0; i < n; ++i) {
     rows = std::max(rows, ops[i].out + 1);
@@ -170,6 +172,7 @@ void assign_reverse_slots(DevOp *ops, int n, int n_slots) {
   for (int t = 0; t < n; ++t) {
     DevOp &op = ops[n - 1 - t];
     op.flags &= ~ALL;
+    op.slots = 0;
     for (int k = 0; k < op.nk; ++k)
       if (op.kid[k] >= 0 && (op.flags & (k == 0 ? OP_FIRST_KID0 : OP_FIRST_KID1))) start[op.kid[k]] = t;
   }
@@ -185,17 +188,21 @@ void assign_reverse_slots(DevOp *ops, int n, int n_slots) {
   }
   for (int t = 0; t < n; ++t) {
     DevOp &op = ops[n - 1 - t];
-    if (slot_of[op.out] >= 0)
-      op.flags |= OP_A_PASS | (slot_of[op.out] << (PASS_SHIFT + 6));
-    else if (last[op.out] == t - 1)
+    if (slot_of[op.out] >= 0) {
+      op.flags |= OP_A_PASS;
+      op.slots |= slot_of[op.out] << 16;
+    } else if (last[op.out] >= 0 && last[op.out] == t - 1) {
       op.flags |= OP_A_LATE;
+    }
     for (int k = 0; k < op.nk; ++k) {
       const int32_t kid = op.kid[k];
       if (kid < 0) continue;
-      if (slot_of[kid] >= 0)
-        op.flags |= (k == 0 ? OP_PASS_KID0 : OP_PASS_KID1) | (slot_of[kid] << (PASS_SHIFT + 3 * k));
-      else if (!(op.flags & (k == 0 ? OP_FIRST_KID0 : OP_FIRST_KID1)))
+      if (slot_of[kid] >= 0) {
+        op.flags |= k == 0 ? OP_PASS_KID0 : OP_PASS_KID1;
+        op.slots |= slot_of[kid] << (8 * k);
+      } else if (!(op.flags & (k == 0 ? OP_FIRST_KID0 : OP_FIRST_KID1))) {
         op.flags |= k == 0 ? OP_ACC0 : OP_ACC1;
+      }
       last[kid] = t;
     }
   }

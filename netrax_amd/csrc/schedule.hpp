@@ -23,7 +23,7 @@ void set_adjoint_flags(std::vector<DevOp> &ops, const std::vector<int> &adj_orde
 void split_level_runs(std::vector<DevOp> &ops, const std::vector<LevelChunk> &chunks, std::vector<LevelChunk> &runs,
                       std::vector<int> &run_begin);
 
-// 4-state FP64 walks: every variant the roots need, children first, each
+// 4-state walks: every variant the roots need, children first, each
 // root's subtrees depth first and the child that needs more rows at once
 // before the other, so that few rows are held at a time.
 std::vector<int> depth_first_order(const Dag &dag, const std::vector<int> &root_slots);
@@ -31,12 +31,15 @@ std::vector<int> depth_first_order(const Dag &dag, const std::vector<int> &root_
 // LDS slots of the forward walk over ops[0, n) (OP_PASS_KID*: the child is
 // read from the slot its op left it in; OP_A_PASS: the op leaves its CLV in
 // a slot), of which the wave has n_slots (2 to WALK_SLOTS).  Rows are the
-// numbers in the ops; a child no slot holds is read from HBM (OP_LOAD*).
+// numbers in the ops; a child no slot holds is read from HBM (OP_LOAD*), one
+// op early.
 void assign_forward_slots(DevOp *ops, int n, int n_slots);
 
 // LDS slots and load flags (OP_PASS_*, OP_A_PASS, OP_A_LATE, OP_ACC*)
 // of the reverse walk over ops[n - 1] .. ops[0]; the adjoint flags
 // (set_adjoint_flags) hold for the whole sweep, of which the ops may be a part.
+// An op's own adjoint, where HBM holds it, is read one op early unless
+// OP_A_LATE.
 void assign_reverse_slots(DevOp *ops, int n, int n_slots);
 
 // OP_ACC_EARLY* for the FP32 reverse sweep (groups backwards).

@@ -1,4 +1,4 @@
-// Host-side check of the 4-state FP64 walks' schedule (netrax_amd/csrc/
+// Host-side check of the 4-state walks' schedule (netrax_amd/csrc/
 // schedule.cpp): the depth-first op order and the LDS slots of both walks,
 // replayed for one network, whole and cut into launches.
 //
@@ -64,14 +64,15 @@ static void check(const Dag &dag, const std::vector<int> &order, int n_slots, in
         if (made[kid] < 0) fail("child after its parent");
         if (op.flags & (k == 0 ? OP_PASS_KID0 : OP_PASS_KID1)) {
           ++slot_reads;
-          if (pass_slot(op.flags, k) >= n_slots || held[pass_slot(op.flags, k)] != kid) fail("slot holds another CLV");
-        } else if (i > cut[j] && made[kid] == i - 1) {
-          fail("CLV loaded before it is stored");
+          if (walk_slot(op, k) >= n_slots || held[walk_slot(op, k)] != kid) fail("slot holds another CLV");
+        } else {
+          if (made[kid] >= cut[j] && made[kid] == i - 1) fail("CLV loaded before it is stored");
+          if (!(op.flags & (k == 0 ? OP_LOAD0 : OP_LOAD1))) fail("CLV not loaded");
         }
       }
       if (made[op.out] >= 0) fail("variant twice");
       made[op.out] = i;
-      if (op.flags & OP_A_PASS) held[pass_slot(op.flags, 2)] = op.out;
+      if (op.flags & OP_A_PASS) held[walk_slot(op, 2)] = op.out;
     }
   }
   // reverse: deliveries made to a row, where they lie, and when the last was made
@@ -83,10 +84,10 @@ static void check(const Dag &dag, const std::vector<int> &order, int n_slots, in
       if (((op.flags & OP_HAS_CONSUMERS) != 0) != (uses[op.out] > 0)) fail("OP_HAS_CONSUMERS");
       if (got[op.out] != uses[op.out]) fail("adjoint read before its deliveries");
       if (op.flags & OP_A_PASS) {
-        const int q = pass_slot(op.flags, 2);
+        const int q = walk_slot(op, 2);
         if (q >= n_slots || held[q] != op.out) fail("adjoint not in its slot");
         held[q] = -1;
-      } else if (uses[op.out] && last[op.out] == i + 1 && i + 1 < cut[j + 1] && !(op.flags & OP_A_LATE)) {
+      } else if (uses[op.out] && last[op.out] == i + 1 && last[op.out] < cut[j + 1] && !(op.flags & OP_A_LATE)) {
         fail("adjoint loaded before its last delivery");
       }
       for (int k = 0; k < op.nk; ++k) {
@@ -95,7 +96,7 @@ static void check(const Dag &dag, const std::vector<int> &order, int n_slots, in
         const bool first = (op.flags & (k == 0 ? OP_FIRST_KID0 : OP_FIRST_KID1)) != 0;
         if (first != (got[kid] == 0)) fail("first delivery");
         if (op.flags & (k == 0 ? OP_PASS_KID0 : OP_PASS_KID1)) {
-          const int q = pass_slot(op.flags, k);
+          const int q = walk_slot(op, k);
           ++handoffs;
           if (q >= n_slots || held[q] != (first ? -1 : kid)) fail("delivery to another row's slot");
           held[q] = kid;
