@@ -255,39 +255,28 @@ static void plan_budget(Engine &e) {
     }
     bp.rec_begin.push_back(static_cast<int>(rec.size()));
   }
-  bp.seg_root_begin.assign(1, 0);
+  // a segment is a launch: a slot hands on only what it made itself
+  std::vector<DevOp> adj = ops;
   for (int j = 0; j < bp.n_seg; ++j) {
-    for (size_t r = 0; r < e.root_slots.size(); ++r)
-      if (seg_of[e.root_slots[r]] == j) {
-        bp.root_phys.push_back(phys[e.root_slots[r]]);
-        bp.root_index.push_back(static_cast<int32_t>(r));
-      }
-    bp.seg_root_begin.push_back(static_cast<int>(bp.root_phys.size()));
+    const int b = bp.seg_chunk[j], n = bp.seg_chunk[j + 1] - b, r = bp.rec_begin[b];
+    assign_forward_slots(ops.data() + b, n, e.fwd_slots);
+    assign_forward_slots(rec.data() + r, bp.rec_begin[b + n] - r, e.fwd_slots);
+    assign_reverse_slots(adj.data() + b, n, e.adj_slots);
   }
-  if (e.walks()) {
-    // a segment is a launch: a slot hands on only what it made itself
-    std::vector<DevOp> adj = ops;
-    for (int j = 0; j < bp.n_seg; ++j) {
-      const int b = bp.seg_chunk[j], n = bp.seg_chunk[j + 1] - b, r = bp.rec_begin[b];
-      assign_forward_slots(ops.data() + b, n, e.fwd_slots);
-      assign_forward_slots(rec.data() + r, bp.rec_begin[b + n] - r, e.fwd_slots);
-      assign_reverse_slots(adj.data() + b, n, e.adj_slots);
-    }
-    upload(e.d_ops_b_adj, adj, e.stream);
-  }
+  upload(e.d_ops_b_adj, adj, e.stream);
   upload(e.d_ops_b, ops, e.stream);
   upload(e.d_ops_rec, rec, e.stream);
-  upload(e.d_root_phys, bp.root_phys, e.stream);
-  upload(e.d_root_index, bp.root_index, e.stream);
   resize_rows(e, bp.n_phys);
 }
 
+constexpr int AA_ADJ_WAVES = 8;  // waves of the 20-state reverse walk that a CU holds
 constexpr int CUS = 256, LDS_PER_CU = 160 * 1024, LDS_PER_GROUP = 64 * 1024;
 
-// LDS slots per wave of a walk of `waves` waves.
+// LDS slots per wave of a walk of `groups` workgroups, of which a CU's
+// registers hold at most `most_per_cu`.
 template <typename Lds>
-static int walk_slots(int64_t waves, Lds &&lds) {
-  const int per_cu = static_cast<int>(std::min<int64_t>(12, (waves + CUS - 1) / CUS));
+static int walk_slots(int64_t groups, Lds &&lds, int most_per_cu = 12) {
+  const int per_cu = static_cast<int>(std::min<int64_t>(most_per_cu, (groups + CUS - 1) / CUS));
   // (LDS is given out in pieces of 1280 bytes)
   const size_t most = std::min<size_t>(LDS_PER_CU / per_cu / 1280 * 1280, LDS_PER_GROUP);
   int n = 2;
@@ -295,13 +284,20 @@ static int walk_slots(int64_t waves, Lds &&lds) {
   return n;
 }
 
-// Granules and LDS slots per wave of the 4-state FP64 walks.  Four granules
+// Granules and LDS slots per wave of the FP64 walks.  4 states: four granules
 // share an op's fixed work best (41,345 patterns x 4 categories, gradient:
 // 0.66 ms, 0.92 with two, 1.00 with one); fewer once they would leave SIMDs
 // without a wave (8,719 patterns: 0.303 / 0.285 / 0.286 ms, 611 patterns, lnL:
 // 53.4 / 50.8 / 50.4 us).  As many slots as let the launch's waves, at most
-// three per SIMD, be resident together.
+// three per SIMD (two in the 20-state reverse walk), be resident together.
 static void choose_walk_shape(Engine &e) {
+  if (e.S == AA_STATES) {
+    const int64_t groups = e.L.n_sites_pad / AA_SITES;
+    e.rpw = TILE / AA_SITES;
+    e.fwd_slots = walk_slots(groups, [&](int n) { return forward_walk_lds_aa(e.C, n); }, std::max(1, 12 / e.C));
+    e.adj_slots = walk_slots(groups * e.C, [&](int n) { return adjoint_walk_lds_aa(n); }, AA_ADJ_WAVES);
+    return;
+  }
   const int64_t granules = e.L.n_sites_pad * e.C / 16;
   const int least = e.C == 8 ? 2 : 1;
   e.walk_nq = e.C == 8 ? 2 : 4;
@@ -388,34 +384,17 @@ static void build_schedule(Engine &e) {
     return op;
   };
 
-  // plain form: level chunks (one per pruning level), ops in slot order, one
-  // launch each; the 4-state walks take a depth-first order instead, each op
-  // a chunk
+  // the walks' depth-first order, each op a chunk
   e.ops_all.clear();
   e.chunks.clear();
-  if (e.walks())
-    for (int s : depth_first_order(e.dag, e.root_slots)) {
-      const int i = static_cast<int>(e.ops_all.size());
-      e.ops_all.push_back(make_op(s));
-      e.chunks.push_back(LevelChunk{e.dag.var[s].level, i, i + 1});
-    }
-  for (int l = 1; l <= max_level && !e.walks(); ++l) {
-    const auto &lv = e.level_ops[l];
-    if (lv.empty()) continue;
-    LevelChunk ch{};
-    ch.level = l;
-    ch.op_begin = static_cast<int>(e.ops_all.size());
-    for (int s : lv) e.ops_all.push_back(make_op(s));
-    ch.op_end = static_cast<int>(e.ops_all.size());
-    e.chunks.push_back(ch);
+  for (int s : depth_first_order(e.dag, e.root_slots)) {
+    const int i = static_cast<int>(e.ops_all.size());
+    e.ops_all.push_back(make_op(s));
+    e.chunks.push_back(LevelChunk{e.dag.var[s].level, i, i + 1});
   }
   {
-    // adjoint: chunks backwards, each chunk's runs in order, ops in index
-    // order (the runs are contiguous ranges of the chunk)
-    split_level_runs(e.ops_all, e.chunks, e.adj_runs, e.adj_run_begin);
-    std::vector<int> order;
-    for (auto it = e.chunks.rbegin(); it != e.chunks.rend(); ++it)
-      for (int i = it->op_begin; i < it->op_end; ++i) order.push_back(i);
+    std::vector<int> order;  // adjoint: backwards
+    for (int i = static_cast<int>(e.ops_all.size()) - 1; i >= 0; --i) order.push_back(i);
     set_adjoint_flags(e.ops_all, order, nv);
   }
 
@@ -431,11 +410,11 @@ static void build_schedule(Engine &e) {
   }
 
   // gradient rows, one per (op, child), numbered in the order this engine's
-  // adjoint walks the ops (plain form: levels top down; FP32 form: groups
+  // adjoint walks the ops (the walks: backwards; 20 states FP32: groups
   // backwards), so that a workgroup's consecutive ops write consecutive rows
   {
     std::vector<int> walk;  // indices into the form's op list
-    const bool grouped = e.opt.precision == NRX_FP32 && !e.walks();
+    const bool grouped = !e.walks();
     std::vector<DevOp> &ops = grouped ? e.ops_dfs : e.ops_all;
     if (grouped) {
       for (int g = static_cast<int>(e.group_begin.size()) - 2; g >= 0; --g)
@@ -493,14 +472,11 @@ static void build_schedule(Engine &e) {
   upload(e.d_class_dlogprob, e.class_dlogprob, e.stream);
   std::vector<int32_t> rs(e.root_slots.begin(), e.root_slots.end());
   upload(e.d_root_slots, rs, e.stream);
-  // gradient partials per site block: a wave of the walks (4 states), 64-site
-  // tiles of C waves (20 states FP64) or 32-site workgroups (FP32)
+  // gradient partials per site block: a wave of the walks, or the waves of a
+  // 32-site workgroup (20 states FP32)
   if (e.walks()) {
     e.gpw = 1;
-    e.gbpt = e.rpw;
-  } else if (e.opt.precision != NRX_FP32) {
-    e.gpw = TILE * e.C / 64;
-    e.gbpt = 1;
+    e.gbpt = e.S == AA_STATES ? e.rpw * e.C : e.rpw;
   } else {
     e.gpw = e.C;
     e.gbpt = TILE / AA_TILE;
@@ -748,48 +724,22 @@ static void forward(Engine &e, bool incremental) {
       all = false;
       break;
     }
-  // 4 states: one launch (a wave walks its sites through the ops); 20
-  // states: one launch per level (one op per workgroup, so a level fills
-  // the GPU)
+  // one launch: a wave walks its sites through the ops
   if (all) {
-    if (e.walks()) {
-      record_kernel_begin(e, 0);
-      launch_forward_walk(e, e.d_ops_fwd.as<DevOp>(), static_cast<int>(e.ops_all.size()));
-      record_kernel_end(e, 0);
-    } else {
-      for (const LevelChunk &ch : e.chunks) {
-        record_kernel_begin(e, 0);
-        launch_forward_level(e, e.d_ops.as<DevOp>() + ch.op_begin, ch.op_end - ch.op_begin, ch);
-        record_kernel_end(e, 0);
-      }
-    }
+    record_kernel_begin(e, 0);
+    launch_forward_walk(e, e.d_ops_fwd.as<DevOp>(), static_cast<int>(e.ops_all.size()));
+    record_kernel_end(e, 0);
   } else {
-    // only the invalid CLVs, level by level
+    // only the invalid CLVs
     std::vector<DevOp> dirty;
-    std::vector<LevelChunk> lv;
-    for (const LevelChunk &ch : e.chunks) {
-      LevelChunk d = ch;
-      d.op_begin = static_cast<int>(dirty.size());
-      for (int i = ch.op_begin; i < ch.op_end; ++i)
-        if (e.clv_dirty[e.ops_all[i].out]) dirty.push_back(e.ops_all[i]);
-      d.op_end = static_cast<int>(dirty.size());
-      if (d.op_end > d.op_begin) lv.push_back(d);
-    }
+    for (const DevOp &op : e.ops_all)
+      if (e.clv_dirty[op.out]) dirty.push_back(op);
     if (!dirty.empty()) {
-      if (e.walks())
-        assign_forward_slots(dirty.data(), static_cast<int>(dirty.size()), e.fwd_slots);
+      assign_forward_slots(dirty.data(), static_cast<int>(dirty.size()), e.fwd_slots);
       stage_upload(e, e.d_ops_dirty, dirty);
-      if (e.walks()) {
-        record_kernel_begin(e, 0);
-        launch_forward_walk(e, e.d_ops_dirty.as<DevOp>(), static_cast<int>(dirty.size()));
-        record_kernel_end(e, 0);
-      } else {
-        for (const LevelChunk &d : lv) {
-          record_kernel_begin(e, 0);
-          launch_forward_level(e, e.d_ops_dirty.as<DevOp>() + d.op_begin, d.op_end - d.op_begin, d);
-          record_kernel_end(e, 0);
-        }
-      }
+      record_kernel_begin(e, 0);
+      launch_forward_walk(e, e.d_ops_dirty.as<DevOp>(), static_cast<int>(dirty.size()));
+      record_kernel_end(e, 0);
     }
   }
   for (const DevOp &op : e.ops_all) e.clv_dirty[op.out] = 0;
@@ -827,66 +777,37 @@ static void fetch_results(Engine &e) {
   stream_sync(e);
 }
 
-// Reverse sweep of level chunks c_hi down to c_lo (plain form).  20
-// states: one launch per run of ops without a common child, one op per
-// workgroup, so that a level fills the GPU.  4 states: one launch for all
-// of them.
+// Reverse sweep of chunks c_hi down to c_lo (FP64 form), one launch.
 static void adjoint_chunks(Engine &e, int c_hi, int c_lo, const DevOp *ops, bool keep = false) {
-  if (e.S == AA_STATES) {
-    for (int c = c_hi; c >= c_lo; --c)
-      for (int r = e.adj_run_begin[c]; r < e.adj_run_begin[c + 1]; ++r) {
-        record_kernel_begin(e, 1);
-        launch_adjoint_level(e, e.adj_runs[r], ops);
-        record_kernel_end(e, 1);
-      }
-  } else if (c_hi >= c_lo) {
-    record_kernel_begin(e, 1);
-    launch_adjoint_walk(e, ops + e.chunks[c_lo].op_begin, e.chunks[c_hi].op_end - e.chunks[c_lo].op_begin, keep);
-    record_kernel_end(e, 1);
-  }
+  if (c_hi < c_lo) return;
+  record_kernel_begin(e, 1);
+  launch_adjoint_walk(e, ops + e.chunks[c_lo].op_begin, e.chunks[c_hi].op_end - e.chunks[c_lo].op_begin, keep);
+  record_kernel_end(e, 1);
 }
 
-// Forward pass, root sums and (with `gradient`) reverse sweep of the FP64
-// form under a memory budget; the mixture runs between the two.
-static void budget_forward(Engine &e, bool gradient) {
+// Forward pass with its root sums and (with `gradient`) reverse sweep of the
+// FP64 form under a memory budget; the mixture runs between the two.
+static void budget_forward(Engine &e) {
   const auto &bp = e.bp;
-  const DevOp *ops = e.d_ops_b.as<DevOp>();
   for (int j = 0; j < bp.n_seg; ++j) {
-    if (e.walks()) {
-      record_kernel_begin(e, 0);
-      launch_forward_walk(e, ops + bp.seg_chunk[j], bp.seg_chunk[j + 1] - bp.seg_chunk[j]);
-      record_kernel_end(e, 0);
-      continue;
-    }
-    for (int c = bp.seg_chunk[j]; c < bp.seg_chunk[j + 1]; ++c) {
-      const LevelChunk &ch = e.chunks[c];
-      record_kernel_begin(e, 0);
-      launch_forward_level(e, ops + ch.op_begin, ch.op_end - ch.op_begin, ch);
-      record_kernel_end(e, 0);
-    }
-    const int r0 = bp.seg_root_begin[j], nr = bp.seg_root_begin[j + 1] - r0;
-    launch_root_partials(e, gradient, e.d_root_phys.as<int32_t>() + r0, e.d_root_index.as<int32_t>() + r0, nr);
+    record_kernel_begin(e, 0);
+    launch_forward_walk(e, e.d_ops_b.as<DevOp>() + bp.seg_chunk[j], bp.seg_chunk[j + 1] - bp.seg_chunk[j]);
+    record_kernel_end(e, 0);
   }
 }
 
 static void budget_adjoint(Engine &e) {
   const auto &bp = e.bp;
-  const DevOp *ops = (e.walks() ? e.d_ops_b_adj : e.d_ops_b).as<DevOp>(), *rec = e.d_ops_rec.as<DevOp>();
+  const DevOp *rec = e.d_ops_rec.as<DevOp>();
   for (int j = bp.n_seg - 1; j >= 0; --j) {
     const int c0 = bp.seg_chunk[j], c1 = bp.seg_chunk[j + 1];
-    if (e.walks() && j < bp.n_seg - 1 && bp.rec_begin[c1] > bp.rec_begin[c0]) {
+    // (the last segment's pool still holds its CLVs)
+    if (j < bp.n_seg - 1 && bp.rec_begin[c1] > bp.rec_begin[c0]) {
       record_kernel_begin(e, 0);
       launch_forward_walk(e, rec + bp.rec_begin[c0], bp.rec_begin[c1] - bp.rec_begin[c0]);
       record_kernel_end(e, 0);
-    } else if (!e.walks() && j < bp.n_seg - 1)  // the last segment's pool still holds its CLVs
-      for (int c = bp.seg_chunk[j]; c < bp.seg_chunk[j + 1]; ++c) {
-        const int n = bp.rec_begin[c + 1] - bp.rec_begin[c];
-        if (n == 0) continue;
-        record_kernel_begin(e, 0);
-        launch_forward_level(e, rec + bp.rec_begin[c], n, e.chunks[c]);
-        record_kernel_end(e, 0);
-      }
-    adjoint_chunks(e, bp.seg_chunk[j + 1] - 1, bp.seg_chunk[j], ops);
+    }
+    adjoint_chunks(e, c1 - 1, c0, e.d_ops_b_adj.as<DevOp>());
   }
 }
 
@@ -1031,7 +952,7 @@ static int evaluate(Engine &e, int variant, bool incremental, bool update_pm, bo
     std::fill(e.clv_dirty.begin(), e.clv_dirty.end(), 0);
   } else if (e.bp.n_seg > 1) {
     // memory budget: segments forward, then the reverse sweep recomputing
-    budget_forward(e, gradient);
+    budget_forward(e);
     launch_mixture(e, variant, e.rpw);
     if (gradient) {
       budget_adjoint(e);
@@ -1040,12 +961,10 @@ static int evaluate(Engine &e, int variant, bool incremental, bool update_pm, bo
     std::fill(e.clv_dirty.begin(), e.clv_dirty.end(), 0);
   } else {
     forward(e, incremental);
-    if (!e.walks()) launch_root_partials(e, gradient);
     launch_mixture(e, variant, e.rpw);
     if (gradient) {
       e.d_adj.alloc(sizeof(double) * e.clv_elems_per_slot * e.dag.var.size());
-      adjoint_chunks(e, static_cast<int>(e.chunks.size()) - 1, 0, (e.walks() ? e.d_ops_adj : e.d_ops).as<DevOp>(),
-                     keep_adjoints);
+      adjoint_chunks(e, static_cast<int>(e.chunks.size()) - 1, 0, e.d_ops_adj.as<DevOp>(), keep_adjoints);
       launch_grad_reduce(e);
     }
   }
@@ -1674,6 +1593,7 @@ int nrx_create(const nrx_network_desc *net, const nrx_partition_desc *parts, int
     if (e->opt.precision == NRX_FP32) e->d_Qf.alloc(sizeof(float) * ss * e->C);
     const size_t pm = static_cast<size_t>(n_parts) * e->E * e->C * e->S * e->S;
     e->d_P.alloc(sizeof(double) * pm);
+    if (e->S == AA_STATES && !aa32) e->d_PA.alloc(sizeof(double) * 2 * pm);
     e->d_dP.alloc(sizeof(double) * pm);
     e->d_d2P.alloc(sizeof(double) * pm);
     e->clv_elems_per_slot = static_cast<size_t>(n) * e->C * e->S;
@@ -2411,7 +2331,7 @@ int nrx_get_stats(nrx_engine *eng, nrx_stats *out) {
     // 20-state FP32.
     const bool fp32 = e.opt.precision == NRX_FP32;
     const double aexp = fp32 ? (e.S == AA_STATES ? scl * e.C : scl) : 0.0;
-    const bool pass = e.S == 4;
+    const bool pass = e.walks();
     const std::vector<DevOp> &adj_ops = e.walks() ? e.ops_adj : fp32 ? e.ops_dfs : e.ops_all;
     out->n_lds_handoffs = 0;
     if (pass)

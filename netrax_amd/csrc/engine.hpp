@@ -23,6 +23,11 @@ constexpr int MAX_CATS = 8;
 constexpr int AA_STATES = 20;
 constexpr int AA_TILE = 32;
 constexpr int AA_TABLE = 64 * 12;
+// FP64: per (partition, edge, category) the tables of P and P^T
+constexpr int AA_MAT = AA_STATES * AA_STATES;
+constexpr int AA_MATS = 2 * AA_MAT;
+constexpr int AA_SITES = 16;                 // sites of a wave
+constexpr int AA_ROW = AA_SITES * AA_STATES;  // a wave's row: one category of its sites
 constexpr int AA_KINDS = 2;  // operand tables per (partition, edge, category): P, P^T
 
 // ---------------------------------------------------------------- model
@@ -257,6 +262,13 @@ constexpr size_t forward_walk_lds(int nq, int n_slots) { return static_cast<size
 constexpr size_t adjoint_walk_lds(int nq, int n_slots) {
   return sizeof(double) * GRAD_RING + static_cast<size_t>(n_slots) * nq * 512;
 }
+// (20 states: a wave per category of 16 sites)
+constexpr size_t forward_walk_lds_aa(int C, int n_slots) {
+  return static_cast<size_t>(n_slots) * C * (sizeof(double) * AA_ROW + 4 * AA_SITES);
+}
+constexpr size_t adjoint_walk_lds_aa(int n_slots) {
+  return sizeof(double) * (GRAD_RING + static_cast<size_t>(n_slots) * AA_ROW);
+}
 constexpr size_t forward_lds32(int C, int blocks, int n_slots) {
   return static_cast<size_t>(n_slots) * blocks * (1024 + 256 / C);
 }
@@ -266,19 +278,11 @@ constexpr size_t adjoint_lds32(int C, int blocks, int n_slots) {
 
 // Kernel launchers (kernels.hip)
 void launch_pmatrices(Engine &e);
-// 20 states: one level
-void launch_forward_level(Engine &e, const DevOp *ops, int n_ops, const LevelChunk &ch);
-// 4 states: ops in an order with children first, with their LDS slots
+// FP64: ops in an order with children first, with their LDS slots
 // assigned (assign_forward_slots); root site sums and seed factors included
 void launch_forward_walk(Engine &e, const DevOp *ops, int n_ops);
-void launch_root_partials(Engine &e, bool seeds);
-// root partials of n roots: physical rows `rows`, root indices `index`
-void launch_root_partials(Engine &e, bool seeds, const int32_t *rows, const int32_t *index, int n);
 void launch_mixture(Engine &e, int variant, int partials_per_tile);
-// 20 states: one run of ops, taken from `ops` (same positions as in the
-// op list)
-void launch_adjoint_level(Engine &e, const LevelChunk &ch, const DevOp *ops);
-// 4 states: the ops backwards (slots from assign_reverse_slots); keep: every
+// FP64: the ops backwards (slots from assign_reverse_slots); keep: every
 // adjoint is also stored in HBM
 void launch_adjoint_walk(Engine &e, const DevOp *ops, int n_ops, bool keep);
 void launch_grad_reduce(Engine &e);

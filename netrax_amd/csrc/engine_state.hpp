@@ -76,9 +76,6 @@ struct Engine : nrx_engine {
   // 4-state walks, with their LDS slots in the two lists the walks read
   std::vector<DevOp> ops_all, ops_fwd, ops_adj;
   std::vector<LevelChunk> chunks;
-  // plain form reverse sweep: runs of ops without a common child, per chunk
-  std::vector<LevelChunk> adj_runs;
-  std::vector<int> adj_run_begin;
   // FP32 form, 20 states: groups of independent ops in a depth-first-biased order
   std::vector<DevOp> ops_dfs;
   std::vector<int32_t> group_begin;  // [n_groups + 1] into ops_dfs
@@ -124,11 +121,8 @@ struct Engine : nrx_engine {
     int n_phys = 0, n_boundary = 0;
     std::vector<int> seg_chunk;         // [n_seg + 1] chunk ranges of the segments
     std::vector<int> rec_begin;         // [n_chunks + 1] ranges of ops_rec per chunk
-    std::vector<int32_t> root_phys;     // per segment, its roots' physical rows ...
-    std::vector<int32_t> root_index;    // ... and their root indices
-    std::vector<int> seg_root_begin;    // [n_seg + 1] ranges of the two above
   } bp;
-  DevBuf d_ops_b, d_ops_b_adj, d_ops_rec, d_root_phys, d_root_index;
+  DevBuf d_ops_b, d_ops_b_adj, d_ops_rec;
   hipGraphExec_t nr_graph = nullptr;
   int nr_graph_key[4] = {-1, -1, -1, -1};  // variant, mode, max_iters, paths
   const void *nr_graph_bufs[3] = {nullptr, nullptr, nullptr};
@@ -153,6 +147,7 @@ struct Engine : nrx_engine {
   DevBuf d_V, d_Vinv, d_eval, d_rates, d_freqs, d_brlen;
   DevBuf d_P, d_dP, d_d2P, d_Pf, d_PfT;
   DevBuf d_clv, d_scl, d_adj, d_adj_exp, d_Qf;
+  DevBuf d_PA;  // 20-state FP64 form: P and P^T in operand order
   DevBuf d_Pa;  // 20-state FP32 form: matrix-core operand tables
   DevBuf d_ops, d_ops_dirty, d_Qd;
   DevBuf d_ops_fwd, d_ops_adj;  // 4 states: the walks' op lists
@@ -183,7 +178,8 @@ struct Engine : nrx_engine {
   int n_k[2] = {0, 0};
   nrx_timing last_timing{};
 
-  bool walks() const { return S == 4; }
+  // passes by the depth-first walks (all but 20 states in single precision)
+  bool walks() const { return S == 4 || opt.precision == NRX_FP64; }
 
   ~Engine();
 };

@@ -198,20 +198,20 @@ __host__ __device__ __forceinline__ size_t grad_index(int64_t block, int n_uses,
   return (static_cast<size_t>(block) * n_uses + g) * pw + w;
 }
 
-// FP64 rows: S states of one (site, category).
-//   20 states  state pairs, each pair of a wave's 64 sites contiguous (a wave
-//              is one category of a 64-site tile, lane = site):
-//              [tile][category][pair 10][site 64][2], so a wave's 16-byte
-//              access is one span of 1 KiB
-//   4 states   granules of 64 doubles in the lane order of the matrix
-//              instruction (see k_forward_walk): [state 4][block 4][site 4],
-//              a block being one category of 4 sites.  A granule holds all
-//              categories of 16 / C sites (8 categories: half the categories
-//              of 4 sites, two granules in turn).
+// FP64 rows: S states of one (site, category), in the lane order of the
+// matrix instructions, so that an access of the walks is one 512-byte span:
+//   4 states   granules of 64 doubles (see k_forward_walk): [state 4][block
+//              4][site 4], a block being one category of 4 sites.  A granule
+//              holds all categories of 16 / C sites (8 categories: half the
+//              categories of 4 sites, two granules in turn).
+//   20 states  [16-site block][category][state 20][site 16]
+// Sumtables are kept in state pairs, each pair of a wave's 64 rows contiguous:
+//   4 states   [64 rows][pair 2][row 64][2]
+//   20 states  [64 sites][category][pair 10][site 64][2]
 // A row kept whole (32 or 160 bytes) would make every access of a wave touch
 // the lines of all its 64 rows and use 16 bytes of each.
 constexpr int PAIR_STRIDE = 128;  // doubles between a row's state pairs
-constexpr int STATE_STRIDE = 16;  // doubles between a 4-state row's entries
+constexpr int STATE_STRIDE = 16;  // doubles between a CLV row's entries
 template <int S, int C>
 __device__ __forceinline__ size_t pair_offset(int64_t site, int c) {
   if constexpr (S == 4) {
@@ -224,7 +224,7 @@ __device__ __forceinline__ size_t pair_offset(int64_t site, int c) {
 template <int S, int C>
 __device__ __forceinline__ size_t row_offset(int64_t site, int c) {
   if constexpr (S != 4) {
-    return pair_offset<S, C>(site, c);
+    return static_cast<size_t>(((site >> 4) * C + c) * (S * STATE_STRIDE) + (site & 15));
   } else if constexpr (C == 8) {
     return static_cast<size_t>(((site >> 2) * 2 + (c >> 2)) * 64 + (c & 3) * 4 + (site & 3));
   } else {
@@ -253,18 +253,8 @@ __device__ __forceinline__ void store_pairs(double *__restrict__ p, const double
 
 template <int S>
 __device__ __forceinline__ void load_clv(const double *__restrict__ p, double (&x)[S]) {
-  if constexpr (S == 4) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) x[i] = p[i * STATE_STRIDE];
-  } else {
-    load_pairs<S>(p, x);
-  }
-}
-
-template <int S>
-__device__ __forceinline__ void store_clv(double *__restrict__ p, const double (&x)[S]) {
-  static_assert(S != 4, "4-state rows are written by k_forward_walk and k_adjoint_level");
-  store_pairs<S>(p, x);
+  for (int i = 0; i < S; ++i) x[i] = p[i * STATE_STRIDE];
 }
 
 template <int S>
@@ -300,6 +290,12 @@ __device__ __forceinline__ void matvec_t(const double *__restrict__ M, const dou
 }
 
 // ------------------------------------------------------------- P matrices
+// Place of entry (i, k) of a matrix in its operand table: per chunk of four
+// columns, rows 0-15 as [column][row 16], then rows 16-19 as [column][row 4].
+__device__ __forceinline__ int aa_place(int i, int k) {
+  return (k >> 2) * 80 + (i < 16 ? (k & 3) * 16 + i : 64 + (k & 3) * 4 + (i & 3));
+}
+
 // P_{p,e,c} = V diag(exp(lambda r_c t_e)) V^-1, with first and second
 // derivatives in t (libpll's pll_update_prob_matrices computes the same
 // product from the same eigendecomposition).
@@ -308,7 +304,7 @@ __global__ void k_pmatrices(DevLayout L, const double *__restrict__ V,
                             const double *__restrict__ rates, const double *__restrict__ brlen,
                             double *__restrict__ P, double *__restrict__ dP,
                             double *__restrict__ d2P, float *__restrict__ Pf,
-                            float *__restrict__ PfT) {
+                            float *__restrict__ PfT, double *__restrict__ PA) {
   const int S = L.S, C = L.C;
   const int64_t total = static_cast<int64_t>(L.n_parts) * L.n_edges * C * S * S;
   const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -336,48 +332,10 @@ __global__ void k_pmatrices(DevLayout L, const double *__restrict__ V,
   d2P[idx] = a2;
   if (Pf) Pf[idx] = static_cast<float>(a0);
   if (PfT) PfT[idx - (i * S + j) + (j * S + i)] = static_cast<float>(a0);
-}
-
-// ---------------------------------------------------- root site sums (FP64)
-// partial[r][wave tile] = sum over the wave's sites of
-//   w_s * (log(sum_c (1/C) sum_i pi_i CLV[s,c,i]) + scaler_s * log(2^-256))
-// (pll_compute_root_loglikelihood semantics, ImprovedLoglikelihood.cpp:450).
-template <int S, int C>
-__global__ void __launch_bounds__(TILE *C)
-    k_root_partials(const int32_t *__restrict__ root_slots, int n_root, DevLayout L,
-                    const double *__restrict__ clv, const int32_t *__restrict__ scl,
-                    const double *__restrict__ freqs, const double *__restrict__ weights,
-                    const int32_t *__restrict__ tile_part, double *__restrict__ partials,
-                    double *__restrict__ seed, const int32_t *__restrict__ root_index) {
-  constexpr int PW = TILE * C / 64;
-  const int tile = blockIdx.x;
-  if (tile >= L.n_tiles) return;
-  const int c = threadIdx.x % C;
-  const int64_t site = static_cast<int64_t>(tile) * TILE + threadIdx.x / C;
-  const int part = tile_part[tile];
-  const int64_t n = L.n_sites_pad;
-  const size_t n_wt = static_cast<size_t>(L.n_tiles) * PW;
-  const int wt = tile * PW + threadIdx.x / 64;
-  const size_t slot = static_cast<size_t>(n) * (C * S), ro = row_offset<S, C>(site, c);
-  const double w = weights[site];
-  // one root CLV per workgroup (grid tiles x roots): the roots' site sums
-  // are independent, and a 2-D grid keeps every CU busy
-  for (int rr = blockIdx.y; rr < min(n_root, static_cast<int>(blockIdx.y) + 1); ++rr) {
-    const int root = root_slots[rr];
-    const int r = root_index ? root_index[rr] : rr;
-    double x[S];
-    load_clv<S>(clv + static_cast<size_t>(root) * slot + ro, x);
-    double t = 0.0;
-#pragma unroll
-    for (int i = 0; i < S; ++i) t = fma(freqs[part * S + i], x[i], t);
-    t = cat_sum<C>(t) * (1.0 / C);
-    // the adjoint's seed factor at this root and site, w / (C Ltilde)
-    if (seed && c == 0) seed[static_cast<size_t>(r) * n + site] = w != 0.0 ? w * (1.0 / C) / t : 0.0;
-    double val = 0.0;
-    if (c == 0 && w != 0.0)
-      val = w * (log(t) + scl[static_cast<size_t>(root) * n + site] * LOG_SCALE_THRESHOLD);
-    val = wave_sum(val);
-    if ((threadIdx.x & 63) == 0) partials[static_cast<size_t>(r) * n_wt + wt] = val;
+  if (PA) {
+    double *tab = PA + idx / AA_MAT * AA_MATS;
+    tab[aa_place(i, j)] = a0;
+    tab[AA_MAT + aa_place(j, i)] = a0;
   }
 }
 
@@ -1050,220 +1008,415 @@ __global__ void __launch_bounds__(64, 3)
   }
 }
 
-// ------------------------------------------- 20 states, FP64 plain form
-// One wavefront per rate category: lane l of wave c holds site l of the
-// 64-site tile in category c.  Every P (and r_c Q) element a wave reads is
-// then the same for all of its lanes, so the matrices come in through the
-// scalar data path as SGPR operands of the FMAs -- no vector load and no
-// LDS read per matrix element, which is what bounds a (site, category) per
-// lane mapping at 20 states (400 elements per matrix).  The per-site
-// quantity that spans categories (the scaling maximum) crosses the waves
-// through LDS.  The CLV layout is the same as every other FP64 kernel's.
-// A matrix the kernel only reads, addressed uniformly across the wave: in
-// the constant address space its loads are scalar loads.
-using cmat = const __attribute__((address_space(4))) double *;
-__device__ __forceinline__ cmat as_cmat(const double *p) { return (cmat)p; }
+// ------------------------------------------------ 20 states, FP64 plain form
+// The walks of the 4-state form at 20 states: a wave holds one rate category
+// of 16 sites, as five chunks of 64 entries (chunk j, lane l: state 4 j +
+// (l >> 4), site l & 15), which are both the columns that
+// v_mfma_f64_16x16x4 takes as its B operand over four states and the rows
+// that it returns; a product's rows 0-15 are five of those, its rows 16-19
+// five v_mfma_f64_4x4x4 whose blocks are the four 4-site groups.  So no entry
+// is padding (20 = 16 + 4 rows, 5 x 4 states summed over), a product's result
+// is the next one's operand, and the stored rows are these registers.
+// P comes from tables in the lane order of the A operands (k_pmatrices).
+typedef double f64x4 __attribute__((ext_vector_type(4)));
 
-// Workgroup (tile, op): the op's CLV rows of one 64-site tile, C waves.
-template <int C>
-__global__ void __launch_bounds__(TILE *C)
-    k_forward_level_aa(const DevOp *__restrict__ ops, DevLayout L, double *__restrict__ clv,
-                       int32_t *__restrict__ scl, const uint32_t *__restrict__ tips, const double *__restrict__ P,
-                       const int32_t *__restrict__ tile_part) {
-  constexpr int S = 20;
-  __shared__ double smax[C][64];
-  const int tile = blockIdx.x;
-  if (tile >= L.n_tiles) return;  // grid padded to a multiple of 8 tiles
-  const DevOp op = ops[blockIdx.y];
-  const int part = tile_part[tile];
-  const int c = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-  const int lane = threadIdx.x & 63;
-  const int64_t site = static_cast<int64_t>(tile) * TILE + lane;
-  const int64_t n = L.n_sites_pad;
-  const size_t slot = static_cast<size_t>(n) * (C * S), ro = row_offset<S, C>(site, c);
-  // loads of both children first; the tip mask and the scaler are loaded
-  // for every child (tip 0 and variant 0 stand in for the absent one): a
-  // value loaded on one path only would be copied at the join, which waits
-  // for every load issued so far
-  double x[2][S];
-  uint32_t tm[2];
-  int sk[2];
-  __builtin_amdgcn_s_setprio(1);  // see the note at wait_loads
+struct Mat20 {
+  double a[10];  // chunk j: rows 0-15 in a[2 j], rows 16-19 in a[2 j + 1]
+};
+
+// big, small: a lane's byte offsets within a chunk's two parts
+__device__ __forceinline__ void load_mat(const GAS double *tab, uint32_t big, uint32_t small, Mat20 &m) {
 #pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const int32_t kid = k < op.nk ? op.kid[k] : -1;
-    tm[k] = tips[static_cast<size_t>(kid < 0 ? -kid - 1 : 0) * n + site];
-    sk[k] = scl[static_cast<size_t>(kid < 0 ? 0 : kid) * n + site];
-    if (k < op.nk && kid >= 0) load_clv<S>(clv + static_cast<size_t>(kid) * slot + ro, x[k]);
+  for (int j = 0; j < 5; ++j) {
+    m.a[2 * j] = *at(tab, big + j * 640);
+    m.a[2 * j + 1] = *at(tab, small + j * 640);
   }
-  __builtin_amdgcn_s_setprio(0);
-  int sc = 0;
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    if (k < op.nk) {
-      if (op.kid[k] < 0)
-        tip_vec<S>(tm[k], x[k]);
-      else
-        sc += sk[k];
-    }
-  }
-  double v[S];
-#pragma unroll
-  for (int i = 0; i < S; ++i) v[i] = 1.0;
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    if (k < op.nk) {
-      const cmat Pk = as_cmat(P + ((static_cast<size_t>(part) * L.n_edges + op.edge[k]) * C + c) * (S * S));
-#pragma unroll
-      for (int i = 0; i < S; ++i) {
-        double s = 0.0;
-#pragma unroll
-        for (int jj = 0; jj < S; ++jj) s = fma(Pk[i * S + jj], x[k][jj], s);
-        v[i] *= s;
-      }
-    }
-  }
-  double m = v[0];
-#pragma unroll
-  for (int i = 1; i < S; ++i) m = fmax(m, v[i]);
-  smax[c][lane] = m;
-  __syncthreads();
-  double mm = smax[0][lane];
-#pragma unroll
-  for (int cc = 1; cc < C; ++cc) mm = fmax(mm, smax[cc][lane]);
-  if (mm < SCALE_THRESHOLD) {
-#pragma unroll
-    for (int i = 0; i < S; ++i) v[i] *= SCALE_FACTOR;
-    sc += 1;
-  }
-  store_clv<S>(clv + static_cast<size_t>(op.out) * slot + ro, v);
-  if (c == 0) scl[static_cast<size_t>(op.out) * n + site] = sc;
 }
 
-// Reverse sweep of one level (push form, as k_adjoint_level): one
-// workgroup per tile walks the level's ops in order; per op and child k,
-// z_k = Abar F y_other, dJ/dt_k += z_k . (r_c Q y_k), Abar_k += P_k^T z_k,
-// formed row by row of P so that z never has to be held whole.
+// y = M x + y
+__device__ __forceinline__ void mul20(const Mat20 &m, const double (&x)[5], double (&y)[5]) {
+  f64x4 d = {y[0], y[1], y[2], y[3]};
+#pragma unroll
+  for (int j = 0; j < 5; ++j) {
+    d = __builtin_amdgcn_mfma_f64_16x16x4f64(m.a[2 * j], x[j], d, 0, 0, 0);
+    y[4] = mfma4(m.a[2 * j + 1], x[j], y[4]);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) y[r] = d[r];
+}
+
+__device__ __forceinline__ void zero(double (&y)[5]) {
+#pragma unroll
+  for (int r = 0; r < 5; ++r) y[r] = 0.0;
+}
+
+// A lane's entries of a tip's 0/1 vectors; mask: of the lane's site.
+__device__ __forceinline__ void tip20(uint32_t mask, int quad, double (&x)[5]) {
+#pragma unroll
+  for (int r = 0; r < 5; ++r)
+    x[r] = __hiloint2double(-static_cast<int>((mask >> (4 * r + quad)) & 1u) & 0x3FF00000, 0);
+}
+
+// The waves of a workgroup meet, their LDS accesses done (accesses to global
+// memory stay in flight).
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+struct FwdIn20 {
+  Mat20 m[2];
+  double x[2][5];  // children read from HBM
+  uint32_t raw[2]; // the children's scaler words, or tip masks
+};
+
+// Workgroup: 16 sites, a wave per category; scaler words as in
+// k_forward_walk.  Per op the waves trade which of their sites are small
+// (and at a root the categories' likelihoods) through LDS, with one barrier.
+// Bound: each wave's chain of ops, the matrix cores busy two fifths of the
+// time (18,564 patterns x 4 categories, 73 ops: 0.40 ms, 0.45 with both
+// matrices an op ahead at two waves per SIMD; 0.72 in ten launches of a
+// thread per row and category with P in scalar registers, whose FMAs wait for
+// every row of it).
 template <int C>
-__global__ void __launch_bounds__(TILE *C)
-    k_adjoint_level_aa(const DevOp *__restrict__ ops, int n_ops, DevLayout L, const double *__restrict__ clv,
-                       const int32_t *__restrict__ scl, double *__restrict__ adj,
-                       const uint32_t *__restrict__ tips, const double *__restrict__ P,
-                       const double *__restrict__ Qd, const double *__restrict__ freqs,
-                       const double *__restrict__ seed, const int32_t *__restrict__ tile_part,
-                       const double *__restrict__ beta, int n_root, int n_uses,
-                       double *__restrict__ grad_partials) {
-  constexpr int S = 20;
-  constexpr int PW = TILE * C / 64;
-  const int tile = blockIdx.x;
-  if (tile >= L.n_tiles) return;  // grid padded to a multiple of 8 tiles
-  const int part = tile_part[tile];
+__global__ void __launch_bounds__(64 * C, 3)
+    k_forward_level_aa(const DevOp *__restrict__ ops_, int n_ops, int n_slots, DevLayout L, double *__restrict__ clv_,
+                      int32_t *__restrict__ scl_, const uint32_t *__restrict__ tips_, const double *__restrict__ PA_,
+                      const double *__restrict__ freqs, const double *__restrict__ weights,
+                      const int32_t *__restrict__ tile_part, double *__restrict__ root_partials,
+                      double *__restrict__ seed) {
+  __shared__ uint32_t small_sites[2][C];
+  __shared__ double site_like[2][C][AA_SITES];
+  const CAS DevOp *ops = to_constant(ops_);
   const int c = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-  const int lane = threadIdx.x & 63;
-  const int64_t site = static_cast<int64_t>(tile) * TILE + lane;
-  const int64_t n = L.n_sites_pad;
-  const size_t slot = static_cast<size_t>(n) * (C * S), ro = row_offset<S, C>(site, c);
-  const double *Qc = Qd + (static_cast<size_t>(part) * C + c) * (S * S);
-  // one op of the run (whose ops share no child) per workgroup
-  ops += blockIdx.y;
-  n_ops = min(n_ops - static_cast<int>(blockIdx.y), 1);
-  for (int j = 0; j < n_ops; ++j) {
-    const DevOp op = ops[j];
-    // load phase: every load issued whatever the op's kind (the adjoint
-    // row of an op without consumers, seed row 0, tip 0 and variant 0 stand
-    // in for absent inputs and are dropped below), so that no join copies a
-    // loaded register and waits for the loads issued before it
-    double araw[S], x[2][S];
-    __builtin_amdgcn_s_setprio(1);  // see the note at wait_loads
-    load_clv<S>(adj + static_cast<size_t>(op.out) * slot + ro, araw);
-    const int kq = scl[static_cast<size_t>(op.out) * n + site];
-    const double sd = seed[static_cast<size_t>(op.root >= 0 ? op.root : 0) * n + site];
-    uint32_t tm[2];
-    int sk[2];
+  const int lane = threadIdx.x & 63, quad = lane >> 4, col = lane & 15;
+  const uint64_t n = L.n_sites_pad, row = n * (C * AA_STATES);
+  const int64_t site0 = static_cast<int64_t>(blockIdx.x) * AA_SITES;
+  const int part = to_constant(tile_part)[site0 / TILE];
+  // [slot][chunk][lane], then the slots' scaler words
+  double *slots = dyn_lds<double>() + c * n_slots * AA_ROW;
+  uint32_t *slot_scl = reinterpret_cast<uint32_t *>(dyn_lds<double>() + C * n_slots * AA_ROW) + c * n_slots * AA_SITES;
+  GAS double *clv = to_global(clv_) + (static_cast<int64_t>(blockIdx.x) * C + c) * AA_ROW;
+  GAS int32_t *scl = to_global(scl_) + site0;
+  const GAS uint32_t *tips = to_global(tips_) + site0;
+  const GAS double *PA = to_global(PA_) + (static_cast<int64_t>(part) * L.n_edges * C + c) * AA_MATS;
+  const uint32_t off = lane * 8, soff = col * 4;
+  const uint32_t big = lane * 8, small = 512 + (quad * 4 + (lane & 3)) * 8;
+
+  auto load = [&](const OpRegs &op, FwdIn20 &in) {
+    const uint32_t o = opaque(off), so = opaque(soff);
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-      const int32_t kid = k < op.nk ? op.kid[k] : -1;
-      tm[k] = tips[static_cast<size_t>(kid < 0 ? -kid - 1 : 0) * n + site];
-      sk[k] = scl[static_cast<size_t>(kid < 0 ? 0 : kid) * n + site];
-      if (k < op.nk && kid >= 0) load_clv<S>(clv + static_cast<size_t>(kid) * slot + ro, x[k]);
-    }
-    __builtin_amdgcn_s_setprio(0);
-    const bool has_adj = (op.flags & OP_HAS_CONSUMERS) != 0;
-    double a[S];
+      // (a one-child op's second child stands for its first)
+      const int32_t kid = k < op.nk() ? op.kid(k) : op.kid(0);
+      const GAS char *tip = reinterpret_cast<const GAS char *>(tips) + static_cast<uint32_t>(~kid) * (n * 4);
+      const GAS char *word = reinterpret_cast<const GAS char *>(scl) + static_cast<uint32_t>(kid) * (n * 4);
+      in.raw[k] = *at(reinterpret_cast<const GAS uint32_t *>(kid < 0 ? tip : word), so);
+      if (op.has(OP_LOAD0, OP_LOAD1, k))
 #pragma unroll
-    for (int i = 0; i < S; ++i) a[i] = has_adj ? araw[i] : 0.0;
-    if (op.root >= 0) {
+        for (int r = 0; r < 5; ++r) in.x[k][r] = *at(clv + static_cast<uint32_t>(op.kid(k)) * row, o + r * 512);
+    }
+    load_mat(PA + static_cast<int64_t>(op.edge(0)) * (C * AA_MATS), opaque(big), opaque(small), in.m[0]);
+  };
+  auto child = [&](const OpRegs &op, FwdIn20 &in, int k, double (&y)[5], uint32_t &count) {
+    uint32_t below = in.raw[k] >> 1;
+    if (op.kid(k) < 0) {
+      tip20(in.raw[k], quad, in.x[k]);
+      below = 0;
+    }
+    if (op.has(OP_PASS_KID0, OP_PASS_KID1, k)) {
+      const int slot = op.slot(k);
+#pragma unroll
+      for (int r = 0; r < 5; ++r) in.x[k][r] = slots[slot * AA_ROW + r * 64 + lane];
+      below = slot_scl[slot * AA_SITES + col] >> 1;
+    }
+    count += below;
+    zero(y);
+    mul20(in.m[k], in.x[k], y);
+  };
+  auto step = [&](int t, const OpRegs &op, OpRegs &ahead, OpRegs &after, FwdIn20 &in, FwdIn20 &next) {
+    arrive(in.raw);
+    arrive(in.x[0]);
+    arrive(in.x[1]);
+    arrive(in.m[0].a);
+    arrive(ahead);
+    __builtin_amdgcn_sched_barrier(0);
+    // (the second child's matrix comes while the first is multiplied: one op
+    // ahead it would cost a third of the waves)
+    load_mat(PA + static_cast<int64_t>(op.edge(1)) * (C * AA_MATS), opaque(big), opaque(small), in.m[1]);
+    load(ahead, next);
+    after = fetch_op(ops, min(t + 2, n_ops - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    const uint32_t o = opaque(off);
+    double v[5];
+    uint32_t count = 0;
+    child(op, in, 0, v, count);
+    if (op.nk() == 2) {
+      double y[5];
+      child(op, in, 1, y, count);
+#pragma unroll
+      for (int r = 0; r < 5; ++r) v[r] *= y[r];
+    }
+    // a site is rescaled when its entries of every category are below the
+    // threshold
+    double m = v[0];
+#pragma unroll
+    for (int r = 1; r < 5; ++r) m = fmax(m, v[r]);
+    uint64_t low = __builtin_amdgcn_ballot_w64(m < SCALE_THRESHOLD);
+    low &= low >> 32;
+    uint32_t sites = static_cast<uint32_t>(low & (low >> 16)) & 0xFFFF;
+    double like = 0.0;
+    if (op.root() >= 0) {
+      // site likelihoods Ltilde = (1/C) sum_c pi . x
+#pragma unroll
+      for (int r = 0; r < 5; ++r) like = fma(freqs[part * AA_STATES + 4 * r + quad], v[r], like);
+      like += __shfl_xor(like, 16);
+      like += __shfl_xor(like, 32);
+    }
+    if constexpr (C > 1) {
+      // (two sets of cells in turn: one barrier separates a cell's readers
+      // from the op after next, which writes it again)
+      if (lane == 0) small_sites[t & 1][c] = sites;
+      if (op.root() >= 0 && lane < AA_SITES) site_like[t & 1][c][col] = like;
+      lds_barrier();
+#pragma unroll
+      for (int cc = 0; cc < C; ++cc) sites &= small_sites[t & 1][cc];
+      if (op.root() >= 0) {
+        like = 0.0;
+#pragma unroll
+        for (int cc = 0; cc < C; ++cc) like += site_like[t & 1][cc][col];
+      }
+    }
+    uint32_t word = count << 1;
+    const bool scaled = (sites >> col) & 1;
+    if (sites) {
+#pragma unroll
+      for (int r = 0; r < 5; ++r)
+        if (scaled) v[r] *= SCALE_FACTOR;
+      if (scaled) word += 3;
+    }
+#pragma unroll
+    for (int r = 0; r < 5; ++r) *at(clv + op.out() * row, o + r * 512) = v[r];
+    // (lanes of a site and the categories' waves store the same word)
+    *at(scl + op.out() * n, opaque(soff)) = static_cast<int32_t>(word);
+    if (op.flags() & OP_A_PASS) {
+      const int slot = op.slot(2);
+#pragma unroll
+      for (int r = 0; r < 5; ++r) slots[slot * AA_ROW + r * 64 + lane] = v[r];
+      slot_scl[slot * AA_SITES + col] = word;
+    }
+    if (op.root() >= 0 && c == 0) {
+      const double t_site = like * (scaled ? SCALE_FACTOR : 1.0) * (1.0 / C);
+      const double w = weights[site0 + col];
+      const double wk = lane < AA_SITES ? w : 0.0;
+      const double val = wk != 0.0 ? wk * (log(t_site) + static_cast<double>(word >> 1) * LOG_SCALE_THRESHOLD) : 0.0;
+      const double sum = wave_sum(val);
+      if (lane == 0) root_partials[static_cast<int64_t>(op.root()) * gridDim.x + blockIdx.x] = sum;
+      // the adjoint's seed factor at this root and site, w / (C Ltilde)
+      seed[op.root() * n + site0 + col] = w != 0.0 ? w * (1.0 / C) / t_site : 0.0;
+    }
+  };
+  OpRegs op0 = fetch_op(ops, 0), op1 = fetch_op(ops, min(1, n_ops - 1));
+  FwdIn20 a;
+  load(op0, a);
+  for (int t = 0; t < n_ops; t += 2) {
+    FwdIn20 b, d;  // what an op does not load stays undefined: nothing is carried over
+    OpRegs op2, op3;
+    step(t, op0, op1, op2, a, b);
+    if (t + 1 >= n_ops) break;
+    step(t + 1, op1, op2, op3, b, d);
+    a = d;
+    op0 = op2;
+    op1 = op3;
+  }
+}
+
+struct AdjIn20 {
+  Mat20 m[2];
+  double x[2][5];   // inner children
+  double a[5];      // own adjoint, where no slot holds it
+  uint32_t raw[2];  // tip children's masks
+  uint32_t word;    // own scaler word
+};
+
+// The reverse sweep of k_adjoint_level at 20 states.  A workgroup is one wave
+// (a category of 16 sites; nothing crosses the categories), categories in the
+// grid's slow direction, so that waves running together read the same tables.
+// Bound: as the forward walk, at two waves per SIMD (18,564 patterns x 4
+// categories: 0.75 ms; 1.79 in 18 launches of a thread per row, with every
+// adjoint through HBM).
+template <int C>
+__global__ void __launch_bounds__(64, 2)
+    k_adjoint_level_aa(const DevOp *__restrict__ ops_, int n_ops, int n_slots, DevLayout L,
+                      const double *__restrict__ clv_, const int32_t *__restrict__ scl_, double *__restrict__ adj_,
+                      const uint32_t *__restrict__ tips_, const double *__restrict__ PA_,
+                      const double *__restrict__ Qd, const double *__restrict__ freqs,
+                      const double *__restrict__ seed, const int32_t *__restrict__ tile_part,
+                      const double *__restrict__ beta, int n_root, int n_uses, double *__restrict__ grad_partials) {
+  const CAS DevOp *ops = to_constant(ops_);
+  const int lane = threadIdx.x, quad = lane >> 4, col = lane & 15;
+  const int n_blocks = L.n_tiles * (TILE / AA_SITES);
+  const int c = blockIdx.x / n_blocks, block = blockIdx.x % n_blocks;
+  const uint64_t n = L.n_sites_pad, row = n * (C * AA_STATES);
+  const int64_t site0 = static_cast<int64_t>(block) * AA_SITES;
+  const int part = to_constant(tile_part)[site0 / TILE];
+  double *ring = dyn_lds<double>();
+  double *slots = ring + GRAD_RING;  // [slot][chunk][lane]
+  const int64_t wave = static_cast<int64_t>(block) * C + c;
+  const GAS double *clv = to_global(clv_) + wave * AA_ROW;
+  GAS double *adj = to_global(adj_) + wave * AA_ROW;
+  const GAS int32_t *scl = to_global(scl_) + site0;
+  const GAS uint32_t *tips = to_global(tips_) + site0;
+  const GAS double *PA = to_global(PA_) + (static_cast<int64_t>(part) * L.n_edges * C + c) * AA_MATS;
+  GAS double *grad = to_global(grad_partials) + wave * n_uses;
+  const uint32_t off = lane * 8, soff = col * 4;
+  const uint32_t big = lane * 8, small = 512 + (quad * 4 + (lane & 3)) * 8;
+  Mat20 Q;
+#pragma unroll
+  for (int j = 0; j < 5; ++j) {
+    const double *Qc = Qd + (static_cast<size_t>(part) * C + c) * AA_MAT + 4 * j + quad;
+    Q.a[2 * j] = Qc[col * AA_STATES];
+    Q.a[2 * j + 1] = Qc[(16 + (lane & 3)) * AA_STATES];
+  }
+
+  auto load = [&](const OpRegs &op, AdjIn20 &in) {
+    const uint32_t o = opaque(off), so = opaque(soff);
+    in.word = static_cast<uint32_t>(*at(scl + op.out() * n, so));
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      // (a one-child op's second child stands for its first)
+      const int32_t kid = k < op.nk() ? op.kid(k) : op.kid(0);
+      if (kid < 0)
+        in.raw[k] = *at(tips + static_cast<uint32_t>(~kid) * n, so);
+      else if (k < op.nk())
+#pragma unroll
+        for (int r = 0; r < 5; ++r) in.x[k][r] = *at(clv + static_cast<uint32_t>(kid) * row, o + r * 512);
+    }
+    if ((op.flags() & (OP_HAS_CONSUMERS | OP_A_PASS | OP_A_LATE)) == OP_HAS_CONSUMERS)
+#pragma unroll
+      for (int r = 0; r < 5; ++r) in.a[r] = *at(adj + op.out() * row, o + r * 512);
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      load_mat(PA + static_cast<int64_t>(op.edge(k)) * (C * AA_MATS), opaque(big), opaque(small), in.m[k]);
+  };
+  int flushed = ops[n_ops - 1].gslot[0];  // the sweep's first gradient row
+  auto step = [&](int t, const OpRegs &op, OpRegs &ahead, OpRegs &after, AdjIn20 &in, AdjIn20 &next) {
+    arrive(in.raw);
+    asm volatile("" : "+v"(in.word));
+    arrive(in.x[0]);
+    arrive(in.x[1]);
+    arrive(in.a);
+    arrive(in.m[0].a);
+    arrive(in.m[1].a);
+    arrive(ahead);
+    __builtin_amdgcn_sched_barrier(0);
+    const uint32_t o = opaque(off);
+    // the transposes of the inner children's matrices, used after the products
+    Mat20 mt[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      if (k < op.nk() && op.kid(k) >= 0)
+        load_mat(PA + static_cast<int64_t>(op.edge(k)) * (C * AA_MATS) + AA_MAT, opaque(big), opaque(small), mt[k]);
+    __builtin_amdgcn_sched_barrier(0);
+    double (&a)[5] = in.a;
+    if (op.flags() & OP_A_PASS) {
+      const double *slot = slots + op.slot(2) * AA_ROW + lane;
+#pragma unroll
+      for (int r = 0; r < 5; ++r) a[r] = slot[r * 64];
+    } else if (op.flags() & OP_A_LATE) {
+#pragma unroll
+      for (int r = 0; r < 5; ++r) a[r] = *at(adj + op.out() * row, o + r * 512);
+    } else if (!(op.flags() & OP_HAS_CONSUMERS)) {
+      zero(a);
+    }
+    if (op.root() >= 0) {
       // seed beta * w * (1/C) pi_i / Ltilde at a displayed-tree root
-      const double f = beta[part * n_root + op.root] * sd;
+      const double f = beta[part * n_root + op.root()] * seed[op.root() * n + site0 + col];
 #pragma unroll
-      for (int i = 0; i < S; ++i) a[i] = fma(f, freqs[part * S + i], a[i]);
+      for (int r = 0; r < 5; ++r) a[r] = fma(f, freqs[part * AA_STATES + 4 * r + quad], a[r]);
     }
-    double y[2][S];
-    int ks = 0;
+    if (in.word & 1u)
+#pragma unroll
+      for (int r = 0; r < 5; ++r) a[r] *= SCALE_FACTOR;
+    double y[2][5];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-      if (k < op.nk) {
-        if (op.kid[k] < 0)
-          tip_vec<S>(tm[k], x[k]);
-        else
-          ks += sk[k];
-        const cmat Pk = as_cmat(P + ((static_cast<size_t>(part) * L.n_edges + op.edge[k]) * C + c) * (S * S));
-#pragma unroll
-        for (int i = 0; i < S; ++i) {
-          double s = 0.0;
-#pragma unroll
-          for (int jj = 0; jj < S; ++jj) s = fma(Pk[i * S + jj], x[k][jj], s);
-          y[k][i] = s;
-        }
-      }
+      if (k >= op.nk()) continue;
+      if (op.kid(k) < 0) tip20(in.raw[k], quad, in.x[k]);
+      zero(y[k]);
+      mul20(in.m[k], in.x[k], y[k]);
     }
-    const double F = (kq - ks) > 0 ? SCALE_FACTOR : 1.0;
+    __builtin_amdgcn_sched_barrier(0);
+    load(ahead, next);  // into the registers the products freed
+    after = fetch_op(ops, max(t - 2, 0));
+    __builtin_amdgcn_sched_barrier(0);
+    double g[2] = {0.0, 0.0};
+    auto use = [&](int k, const double (&z)[5]) {
+      const bool inner = op.kid(k) >= 0, pass = op.has(OP_PASS_KID0, OP_PASS_KID1, k);
+      double *slot = slots + op.slot(k) * AA_ROW + lane;
+      GAS double *dst = adj + static_cast<uint32_t>(op.kid(k)) * row;
+      double b[5];
+      zero(b);
+      // what the child's adjoint holds already (the deliveries before this
+      // op's are stores of this wave, so in order)
+      if (op.has(OP_ACC0, OP_ACC1, k)) {
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      if (k >= op.nk) continue;
-      const int32_t kid = op.kid[k];
-      cmat Pk = as_cmat(P + ((static_cast<size_t>(part) * L.n_edges + op.edge[k]) * C + c) * (S * S));
-      cmat Qk = as_cmat(Qc);
-      // opaque to the optimiser: the matrices are read again here, through
-      // the scalar cache, instead of being kept in (or hoisted out of the op
-      // loop into) 800 SGPRs each, which would spill
-      asm volatile("" : "+s"(Pk));
-      asm volatile("" : "+s"(Qk));
-      double back[S], gk = 0.0;
-      // one straight-line body per case (internal child or tip): a branch
-      // inside the row loop splits it into blocks across which the scalar
-      // registers holding matrix rows stay live and spill
-      auto rows = [&](auto with_back) {
+        for (int r = 0; r < 5; ++r) b[r] = *at(dst, o + r * 512);
+      } else if (inner && pass && !op.has(OP_FIRST_KID0, OP_FIRST_KID1, k)) {
 #pragma unroll
-        for (int i = 0; i < S; ++i) {
-          const double zi = a[i] * F * (op.nk == 2 ? y[1 - k][i] : 1.0);
-          double d = 0.0;
-#pragma unroll
-          for (int jj = 0; jj < S; ++jj) d = fma(Qk[i * S + jj], y[k][jj], d);
-          gk = fma(zi, d, gk);
-          if constexpr (decltype(with_back)::value) {
-#pragma unroll
-            for (int jj = 0; jj < S; ++jj) back[jj] = i == 0 ? Pk[jj] * zi : fma(Pk[i * S + jj], zi, back[jj]);
-          }
-        }
-      };
-      if (kid >= 0)
-        rows(std::true_type{});
-      else
-        rows(std::false_type{});
-      const double g = wave_sum(gk);
-      if (lane == 0) grad_partials[grad_index(tile, n_uses, op.gslot[k], PW, c)] = g;
-      if (kid >= 0) {
-        double *dst = adj + static_cast<size_t>(kid) * slot + ro;
-        if (!(op.flags & (k == 0 ? OP_FIRST_KID0 : OP_FIRST_KID1))) {
-          double acc[S];
-          load_clv<S>(dst, acc);
-#pragma unroll
-          for (int i = 0; i < S; ++i) back[i] += acc[i];
-        }
-        store_clv<S>(dst, back);
+        for (int r = 0; r < 5; ++r) b[r] = slot[r * 64];
       }
+      double q[5];
+      zero(q);
+      mul20(Q, y[k], q);
+#pragma unroll
+      for (int r = 0; r < 5; ++r) g[k] = fma(z[r], q[r], g[k]);
+      if (!inner) return;
+      mul20(mt[k], z, b);
+      if (pass) {
+#pragma unroll
+        for (int r = 0; r < 5; ++r) slot[r * 64] = b[r];
+      } else {
+#pragma unroll
+        for (int r = 0; r < 5; ++r) *at(dst, o + r * 512) = b[r];
+      }
+    };
+    double z[5];
+    if (op.nk() == 2) {
+#pragma unroll
+      for (int r = 0; r < 5; ++r) z[r] = a[r] * y[1][r];
+      use(0, z);
+#pragma unroll
+      for (int r = 0; r < 5; ++r) z[r] = a[r] * y[0][r];
+      use(1, z);
+    } else {
+      use(0, a);
     }
+    // rows are numbered in the order of the sweep: row r waits in ring[r %
+    // GRAD_RING], and 64 at a time leave as one store
+    const double total = pair_wave_sum(g[0], g[1]);
+    const int k = lane >> 5;
+    if ((lane & 31) == 31 && k < op.nk()) ring[(op.gslot() + k) % GRAD_RING] = total;
+    const int done = op.gslot() + op.nk();
+    if (done - flushed >= 64) {
+      grad[flushed + lane] = ring[(flushed + lane) % GRAD_RING];
+      flushed += 64;
+    }
+    if (t == 0 && lane < done - flushed) grad[flushed + lane] = ring[(flushed + lane) % GRAD_RING];
+  };
+  OpRegs op0 = fetch_op(ops, n_ops - 1), op1 = fetch_op(ops, max(n_ops - 2, 0));
+  AdjIn20 u;
+  load(op0, u);
+  for (int t = n_ops - 1; t >= 0; t -= 2) {
+    AdjIn20 v, w;  // what an op does not load stays undefined: nothing is carried over
+    OpRegs op2, op3;
+    step(t, op0, op1, op2, u, v);
+    if (t == 0) break;
+    step(t - 1, op1, op2, op3, v, w);
+    u = w;
+    op0 = op2;
+    op1 = op3;
   }
 }
 
@@ -2481,7 +2634,6 @@ __device__ __forceinline__ void stage_path_p(double *sPp, const PathStep *__rest
 // rescalings (FP64) or exponent (FP32) that a CLV's scaler word counts
 template <int S, typename T>
 __device__ __forceinline__ int scl_count(int32_t word) {
-  if constexpr (S != 4) return word;
   return std::is_same<T, double>::value ? word >> 1 : word_k(word);
 }
 // a thread's row in a CLV slot of either form (FP32 rows are kept whole)
@@ -3160,7 +3312,7 @@ void launch_pmatrices(Engine &e) {
   hipLaunchKernelGGL(k_pmatrices, dim3(nb), dim3(256), 0, e.stream, e.L, e.d_V.as<double>(),
                      e.d_Vinv.as<double>(), e.d_eval.as<double>(), e.d_rates.as<double>(),
                      e.d_brlen.as<double>(), e.d_P.as<double>(), e.d_dP.as<double>(),
-                     e.d_d2P.as<double>(), e.d_Pf.as<float>(), e.d_PfT.as<float>());
+                     e.d_d2P.as<double>(), e.d_Pf.as<float>(), e.d_PfT.as<float>(), e.d_PA.as<double>());
   NRX_HIP(hipGetLastError());
 }
 
@@ -3173,21 +3325,6 @@ void dispatch_c(int C, F &&f) {
     case 8: f(std::integral_constant<int, 8>{}); break;
     default: throw std::invalid_argument("unsupported number of rate categories");
   }
-}
-
-void launch_forward_level(Engine &e, const DevOp *ops, int n_ops, const LevelChunk &) {
-  if (n_ops == 0) return;
-  if (e.S == AA_STATES) {
-    dispatch_c(e.C, [&](auto c) {
-      constexpr int C = decltype(c)::value;
-      hipLaunchKernelGGL((k_forward_level_aa<C>), dim3(e.L.n_tiles_grid, n_ops), dim3(TILE * C), 0, e.stream,
-                         ops, e.L, e.d_clv.as<double>(), e.d_scl.as<int32_t>(), e.d_tips.as<uint32_t>(),
-                         e.d_P.as<double>(), e.d_tile_part.as<int32_t>());
-    });
-    NRX_HIP(hipGetLastError());
-    return;
-  }
-  throw std::logic_error("launch_forward_level: 4-state passes go through launch_forward_walk");
 }
 
 // Shapes of the 4-state FP64 walks: C categories, NQ granules per wave (8
@@ -3209,6 +3346,18 @@ static void dispatch_walk(int C, int NQ, F &&f) {
 void launch_forward_walk(Engine &e, const DevOp *ops, int n_ops) {
   if (n_ops == 0) return;
   const unsigned waves = static_cast<unsigned>(e.L.n_tiles) * e.rpw;
+  if (e.S == AA_STATES) {
+    dispatch_c(e.C, [&](auto c) {
+      constexpr int C = decltype(c)::value;
+      hipLaunchKernelGGL((k_forward_level_aa<C>), dim3(waves), dim3(64 * C), forward_walk_lds_aa(C, e.fwd_slots),
+                         e.stream, ops, n_ops, e.fwd_slots, e.L, e.d_clv.as<double>(), e.d_scl.as<int32_t>(),
+                         e.d_tips.as<uint32_t>(), e.d_PA.as<double>(), e.d_freqs.as<double>(),
+                         e.d_weights.as<double>(), e.d_tile_part.as<int32_t>(), e.d_root_partials.as<double>(),
+                         e.d_site_seed.as<double>());
+    });
+    NRX_HIP(hipGetLastError());
+    return;
+  }
   dispatch_walk(e.C, e.walk_nq, [&](auto c, auto nq) {
     constexpr int C = decltype(c)::value, NQ = decltype(nq)::value;
     hipLaunchKernelGGL((k_forward_walk<4, C, NQ>), dim3(waves), dim3(64), forward_walk_lds(NQ, e.fwd_slots), e.stream,
@@ -3217,23 +3366,6 @@ void launch_forward_walk(Engine &e, const DevOp *ops, int n_ops) {
                        e.d_tile_part.as<int32_t>(), e.d_root_partials.as<double>(), e.d_site_seed.as<double>());
   });
   NRX_HIP(hipGetLastError());
-}
-
-void launch_root_partials(Engine &e, bool seeds, const int32_t *rows, const int32_t *index, int n) {
-  if (n == 0) return;
-  if (e.S != AA_STATES) throw std::logic_error("launch_root_partials: the 4-state forward walk forms the root sums");
-  dispatch_c(e.C, [&](auto c) {
-    constexpr int S = AA_STATES, C = decltype(c)::value;
-    hipLaunchKernelGGL((k_root_partials<S, C>), dim3(e.L.n_tiles, n), dim3(TILE * C), 0, e.stream, rows, n, e.L,
-                       e.d_clv.as<double>(), e.d_scl.as<int32_t>(), e.d_freqs.as<double>(),
-                       e.d_weights.as<double>(), e.d_tile_part.as<int32_t>(), e.d_root_partials.as<double>(),
-                       seeds ? e.d_site_seed.as<double>() : nullptr, index);
-  });
-  NRX_HIP(hipGetLastError());
-}
-
-void launch_root_partials(Engine &e, bool seeds) {
-  launch_root_partials(e, seeds, e.d_root_slots.as<int32_t>(), nullptr, static_cast<int>(e.root_slots.size()));
 }
 
 void launch_mixture(Engine &e, int variant, int pw) {
@@ -3250,15 +3382,17 @@ void launch_mixture(Engine &e, int variant, int pw) {
   NRX_HIP(hipGetLastError());
 }
 
-void launch_adjoint_level(Engine &e, const LevelChunk &ch, const DevOp *ops) {
-  const int n_ops = ch.op_end - ch.op_begin;
+void launch_adjoint_walk(Engine &e, const DevOp *ops, int n_ops, bool keep) {
   if (n_ops == 0) return;
+  const unsigned waves = static_cast<unsigned>(e.L.n_tiles) * e.rpw;
   if (e.S == AA_STATES) {
+    // (rows kept for the model gradient are a 4-state matter)
+    if (keep) throw std::logic_error("launch_adjoint_walk: 20-state adjoints are not kept");
     dispatch_c(e.C, [&](auto c) {
       constexpr int C = decltype(c)::value;
-      hipLaunchKernelGGL((k_adjoint_level_aa<C>), dim3(e.L.n_tiles_grid, n_ops), dim3(TILE * C), 0, e.stream,
-                         ops + ch.op_begin, n_ops, e.L, e.d_clv.as<double>(), e.d_scl.as<int32_t>(),
-                         e.d_adj.as<double>(), e.d_tips.as<uint32_t>(), e.d_P.as<double>(), e.d_Qd.as<double>(),
+      hipLaunchKernelGGL((k_adjoint_level_aa<C>), dim3(waves * C), dim3(64), adjoint_walk_lds_aa(e.adj_slots), e.stream,
+                         ops, n_ops, e.adj_slots, e.L, e.d_clv.as<double>(), e.d_scl.as<int32_t>(),
+                         e.d_adj.as<double>(), e.d_tips.as<uint32_t>(), e.d_PA.as<double>(), e.d_Qd.as<double>(),
                          e.d_freqs.as<double>(), e.d_site_seed.as<double>(), e.d_tile_part.as<int32_t>(),
                          e.d_beta.as<double>(), static_cast<int>(e.root_slots.size()), e.n_uses,
                          e.d_grad_partials.as<double>());
@@ -3266,12 +3400,6 @@ void launch_adjoint_level(Engine &e, const LevelChunk &ch, const DevOp *ops) {
     NRX_HIP(hipGetLastError());
     return;
   }
-  throw std::logic_error("launch_adjoint_level: 4-state sweeps go through launch_adjoint_walk");
-}
-
-void launch_adjoint_walk(Engine &e, const DevOp *ops, int n_ops, bool keep) {
-  if (n_ops == 0) return;
-  const unsigned waves = static_cast<unsigned>(e.L.n_tiles) * e.rpw;
   dispatch_walk(e.C, e.walk_nq, [&](auto c, auto nq) {
     constexpr int C = decltype(c)::value, NQ = decltype(nq)::value;
     hipLaunchKernelGGL((k_adjoint_level<C, NQ>), dim3(waves), dim3(64), adjoint_walk_lds(NQ, e.adj_slots), e.stream,
