@@ -778,10 +778,10 @@ static void fetch_results(Engine &e) {
 }
 
 // Reverse sweep of chunks c_hi down to c_lo (FP64 form), one launch.
-static void adjoint_chunks(Engine &e, int c_hi, int c_lo, const DevOp *ops, bool keep = false) {
+static void adjoint_chunks(Engine &e, int c_hi, int c_lo, const DevOp *ops, bool model = false) {
   if (c_hi < c_lo) return;
   record_kernel_begin(e, 1);
-  launch_adjoint_walk(e, ops + e.chunks[c_lo].op_begin, e.chunks[c_hi].op_end - e.chunks[c_lo].op_begin, keep);
+  launch_adjoint_walk(e, ops + e.chunks[c_lo].op_begin, e.chunks[c_hi].op_end - e.chunks[c_lo].op_begin, model);
   record_kernel_end(e, 1);
 }
 
@@ -875,13 +875,37 @@ static int stage_invalid_ops(Engine &e, const NetDesc *&desc) {
   return n;
 }
 
+// Slices of a partition's waves that the model gradient's sums are formed in.
+constexpr int MODEL_SLICES = 8;
+// Doubles of the model gradient's workspaces, in launch_model_grad's order.
+static std::array<size_t, 4> model_sizes(const Engine &e) {
+  const size_t P = e.P, nl = e.C == 8 ? 128 : 64;
+  return {std::max(1, e.n_uses) * P * MODEL_SLICES * nl, std::max<size_t>(1, e.root_slots.size()) * P * MODEL_SLICES * 4,
+          P * e.E * (16 + e.C), P * (16 + e.C + 4)};
+}
+static double *model_buffer(const Engine &e, int which) {
+  const auto n = model_sizes(e);
+  double *p = e.d_mg_sums.as<double>();
+  for (int i = 0; i < which; ++i) p += n[i];
+  return p;
+}
+static void alloc_model_grad(Engine &e) {
+  const size_t waves = static_cast<size_t>(e.L.n_tiles) * e.rpw, nl = e.C == 8 ? 128 : 64;
+  e.d_mg_g.alloc(sizeof(double) * std::max(1, e.n_uses) * waves * nl);
+  e.d_mg_r.alloc(sizeof(double) * std::max<size_t>(1, e.root_slots.size()) * waves * 4);
+  const auto n = model_sizes(e);
+  e.d_mg_sums.alloc(sizeof(double) * (n[0] + n[1] + n[2] + n[3]));
+}
+static void enqueue_model_grad(Engine &e) {
+  launch_model_grad(e, model_buffer(e, 0), model_buffer(e, 1), model_buffer(e, 2), model_buffer(e, 3), MODEL_SLICES);
+}
+
 // `fetch` false: the results stay on the device (for a caller that reads
 // them there, such as the device Newton sweep) and no host wait is made;
 // the host copy is then stale, so the cache is marked invalid.
-// `keep_adjoints`: the reverse sweep of the 4-state FP64 form leaves every
-// CLV's adjoint in HBM (the model gradient reads them).
+// `model`: the model gradient's sums too (FP64 form, 4 states).
 static int evaluate(Engine &e, int variant, bool incremental, bool update_pm, bool gradient, bool fetch = true,
-                    bool keep_adjoints = false) {
+                    bool model = false) {
   check_ready(e);
   if (variant != NRX_AVERAGE_DISPLAYED_TREES && variant != NRX_BEST_DISPLAYED_TREE)
     throw std::invalid_argument("unknown likelihood variant");
@@ -964,8 +988,9 @@ static int evaluate(Engine &e, int variant, bool incremental, bool update_pm, bo
     launch_mixture(e, variant, e.rpw);
     if (gradient) {
       e.d_adj.alloc(sizeof(double) * e.clv_elems_per_slot * e.dag.var.size());
-      adjoint_chunks(e, static_cast<int>(e.chunks.size()) - 1, 0, e.d_ops_adj.as<DevOp>(), keep_adjoints);
+      adjoint_chunks(e, static_cast<int>(e.chunks.size()) - 1, 0, e.d_ops_adj.as<DevOp>(), model);
       launch_grad_reduce(e);
+      if (model) enqueue_model_grad(e);
     }
   }
   end_timing(e);
@@ -1977,25 +2002,17 @@ int nrx_model_gradient(nrx_engine *eng, int32_t variant, double *total, double *
     if (e.opt.precision != NRX_FP64 || e.S != 4)
       return fail(NRX_ERR_UNSUPPORTED, "model gradients are provided for the FP64 form with 4-state data");
     require_resident(e);
-    // CLVs, adjoints, mixture weights
-    const int rc = evaluate(e, variant, true, true, true, /*fetch=*/true, /*keep_adjoints=*/true);
+    // CLVs, adjoints, mixture weights, and per partition dJ/dQ, dJ/dr_c and
+    // the frequencies' direct share
+    check_ready(e);
+    alloc_model_grad(e);
+    const int rc = evaluate(e, variant, true, true, true, /*fetch=*/true, /*model=*/true);
     if (rc != NRX_OK) return rc;
     *total = e.cached_total;
     const int S = e.S, C = e.C, P = e.P, nr = S * (S - 1) / 2;
-    const int n_ops = static_cast<int>(e.ops_all.size());
-    const int n_root = static_cast<int>(e.root_slots.size());
-    // slices per partition so that the grid fills the GPU
-    int n_split = std::max(1, (2048 + n_ops * P - 1) / std::max(1, n_ops * P));
-    for (const PartInfo &pi : e.parts) n_split = std::min(n_split, std::max(1, pi.tile_end - pi.tile_begin));
-    const int nch = P * n_split;
-    const size_t ng = static_cast<size_t>(std::max(1, e.n_uses)) * nch * C * S * S;
-    const size_t nrr = static_cast<size_t>(std::max(1, n_root)) * nch * S;
-    e.d_mg_g.alloc(sizeof(double) * ng);
-    e.d_mg_r.alloc(sizeof(double) * nrr);
-    launch_model_grad(e, n_split, e.d_mg_g.as<double>(), e.d_mg_r.as<double>());
-    std::vector<double> G(ng), Rr(nrr);
-    NRX_HIP(hipMemcpyAsync(G.data(), e.d_mg_g.p, sizeof(double) * ng, hipMemcpyDeviceToHost, e.stream));
-    NRX_HIP(hipMemcpyAsync(Rr.data(), e.d_mg_r.p, sizeof(double) * nrr, hipMemcpyDeviceToHost, e.stream));
+    std::vector<double> sums(model_sizes(e)[3]);
+    NRX_HIP(hipMemcpyAsync(sums.data(), model_buffer(e, 3), sizeof(double) * sums.size(), hipMemcpyDeviceToHost,
+                           e.stream));
     stream_sync(e);
     for (int p = 0; p < P; ++p) {
       const PartInfo &pi = e.parts[p];
@@ -2016,74 +2033,7 @@ int nrx_model_gradient(nrx_engine *eng, int32_t variant, double *total, double *
         R[i * S + i] = -rowsum;
         mu += pf[i] * rowsum;
       }
-      std::vector<double> Q(S * S);
-      for (int q = 0; q < S * S; ++q) Q[q] = R[q] / mu;
-      // dJ/dQ through P_{e,c} = exp(Q r_c t_e) = V exp(L s) V^-1:
-      // dJ/dQ = V^-T ((V^T G V^-T) o Psi) V^T, Psi_kl = (e^{l_k s} - e^{l_l s}) / (l_k - l_l)
-      // (s e^{l_k s} for equal eigenvalues); dJ/dr_c = sum_e t_e tr(G^T Q P)
-      std::vector<double> dQ(S * S, 0.0), dr(C, 0.0), Gm(S * S), H(S * S), T1(S * S), Ps(S * S), QP(S * S);
-      for (int ed = 0; ed < e.E; ++ed) {
-        for (int c = 0; c < C; ++c) {
-          std::fill(Gm.begin(), Gm.end(), 0.0);
-          for (int i = e.edge_use_begin[ed]; i < e.edge_use_begin[ed + 1]; ++i) {
-            const int u = e.edge_use_list[i];
-            for (int sl = 0; sl < n_split; ++sl) {
-              const double *g = &G[((static_cast<size_t>(u) * nch + p * n_split + sl) * C + c) * S * S];
-              for (int q = 0; q < S * S; ++q) Gm[q] += g[q];
-            }
-          }
-          const double s = pi.rates[c] * e.brlen[ed];
-          // H = V^T G Vinv^T
-          for (int a = 0; a < S; ++a)
-            for (int j = 0; j < S; ++j) {
-              double acc = 0.0;
-              for (int i = 0; i < S; ++i) acc += m.V[i * S + a] * Gm[i * S + j];
-              T1[a * S + j] = acc;
-            }
-          for (int a = 0; a < S; ++a)
-            for (int b = 0; b < S; ++b) {
-              double acc = 0.0;
-              for (int j = 0; j < S; ++j) acc += T1[a * S + j] * m.Vinv[b * S + j];
-              H[a * S + b] = acc;
-            }
-          for (int a = 0; a < S; ++a)
-            for (int b = 0; b < S; ++b) {
-              const double la = m.eval[a], lb = m.eval[b];
-              const double psi = std::fabs(la - lb) > 1e-10 * std::max(1.0, std::fabs(la))
-                                     ? (std::exp(la * s) - std::exp(lb * s)) / (la - lb)
-                                     : s * std::exp(0.5 * (la + lb) * s);
-              H[a * S + b] *= psi;
-            }
-          // dQ += Vinv^T H V^T
-          for (int i = 0; i < S; ++i)
-            for (int b = 0; b < S; ++b) {
-              double acc = 0.0;
-              for (int a = 0; a < S; ++a) acc += m.Vinv[a * S + i] * H[a * S + b];
-              T1[i * S + b] = acc;
-            }
-          for (int i = 0; i < S; ++i)
-            for (int j = 0; j < S; ++j) {
-              double acc = 0.0;
-              for (int b = 0; b < S; ++b) acc += T1[i * S + b] * m.V[j * S + b];
-              dQ[i * S + j] += acc;
-            }
-          // tr(G^T Q P) with P = V exp(L s) Vinv
-          for (int i = 0; i < S; ++i)
-            for (int j = 0; j < S; ++j) {
-              double acc = 0.0;
-              for (int k = 0; k < S; ++k) acc += m.V[i * S + k] * std::exp(m.eval[k] * s) * m.Vinv[k * S + j];
-              Ps[i * S + j] = acc;
-            }
-          double tr = 0.0;
-          for (int i = 0; i < S; ++i)
-            for (int j = 0; j < S; ++j) {
-              double acc = 0.0;
-              for (int k = 0; k < S; ++k) acc += Q[i * S + k] * Ps[k * S + j];
-              tr += Gm[i * S + j] * acc;
-            }
-          dr[c] += e.brlen[ed] * tr;
-        }
-      }
+      const double *dQ = &sums[static_cast<size_t>(p) * (S * S + C + S)], *dr = dQ + S * S, *direct = dr + C;
       // chain to exchangeabilities and frequencies: Q = R / mu,
       // R_ij = rho_ij pi_j (i != j), R_ii = -sum_{j != i} R_ij,
       // mu = sum_i pi_i sum_{j != i} rho_ij pi_j
@@ -2107,10 +2057,7 @@ int nrx_model_gradient(nrx_engine *eng, int32_t variant, double *total, double *
           dmu_dpi += 2.0 * rho * pf[i];
         }
         g += dmu * dmu_dpi;
-        // the frequencies' direct share at the displayed-tree roots
-        for (int r = 0; r < n_root; ++r)
-          for (int sl = 0; sl < n_split; ++sl)
-            g += Rr[(static_cast<size_t>(r) * nch + p * n_split + sl) * S + kq];
+        g += direct[kq];  // at the displayed-tree roots
         d_freqs[static_cast<size_t>(p) * S + kq] = g;
       }
       if (d_rates)

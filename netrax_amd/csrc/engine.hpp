@@ -282,9 +282,9 @@ void launch_pmatrices(Engine &e);
 // assigned (assign_forward_slots); root site sums and seed factors included
 void launch_forward_walk(Engine &e, const DevOp *ops, int n_ops);
 void launch_mixture(Engine &e, int variant, int partials_per_tile);
-// FP64: the ops backwards (slots from assign_reverse_slots); keep: every
-// adjoint is also stored in HBM
-void launch_adjoint_walk(Engine &e, const DevOp *ops, int n_ops, bool keep);
+// FP64: the ops backwards (slots from assign_reverse_slots); model: with the
+// model gradient's sums per use and root (d_mg_g, d_mg_r; 4 states)
+void launch_adjoint_walk(Engine &e, const DevOp *ops, int n_ops, bool model);
 void launch_grad_reduce(Engine &e);
 // nets: a descriptor other than the engine's own (its invalid ops only)
 void launch_forward_persistent(Engine &e, const NetDesc *nets = nullptr);
@@ -293,10 +293,10 @@ void launch_mfma_tables(Engine &e);
 void launch_forward_mfma(Engine &e, const NetDesc *nets = nullptr);
 void launch_adjoint_mfma(Engine &e);
 void launch_sumtables(Engine &e, int n_paths, int max_steps);
-// FP64 4-state: per use, chunk and category the summed z x^T (dlnL/dP);
-// per root CLV and chunk the frequencies' direct share (a chunk is one of
-// n_split slices of a partition's tiles, chunk = partition * n_split + slice)
-void launch_model_grad(Engine &e, int n_split, double *g_out, double *r_out);
+// FP64 4-state: from the walk's sums per partition dJ/dQ [16], dJ/drates [C]
+// and the frequencies' direct share [4] into out; the others are workspaces:
+// g_sum [uses][P][slices][64 or 128], r_sum [roots][P][slices][4], edge_out [P][E][16 + C]
+void launch_model_grad(Engine &e, double *g_sum, double *r_sum, double *edge_out, double *out, int n_slice);
 // Newton-Raphson of a branch length on the device: `rounds` rounds of
 // (evaluate the sumtables at the state's length, reduce, Newton step; no-ops
 // once the state is done or has taken its max_iters steps), then the

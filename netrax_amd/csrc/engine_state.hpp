@@ -108,7 +108,7 @@ struct Engine : nrx_engine {
   // device Newton-Raphson: state, class table, tree lnLs; its captured
   // sequence, valid while the sumtable buffers keep their addresses
   DevBuf d_nr_state, d_nr_cls;
-  DevBuf d_mg_g, d_mg_r;  // model gradient partials
+  DevBuf d_mg_g, d_mg_r, d_mg_sums;  // model gradient: the walk's sums per use and root, and what is made of them
   // Memory budget of the FP64 form: with n_seg > 1 the CLV, adjoint and
   // scaler rows live in n_phys physical rows.  The level chunks are cut into
   // n_seg segments; a CLV consumed in a later segment than its own keeps a

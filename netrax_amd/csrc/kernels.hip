@@ -819,14 +819,22 @@ struct AdjIn4 {
 // Bound: HBM (every inner child's CLV once per use; 50 taxa, 41,345 patterns:
 // 1.6 GB in 0.363 ms, 4.5 TB/s; with P in LDS and every adjoint through HBM
 // 2.99 GB in 0.648 ms).
-template <int C, int NQ>
-__global__ void __launch_bounds__(64, 3)
-    k_adjoint_level(const DevOp *__restrict__ ops_, int n_ops, int n_slots, int keep, DevLayout L,
-                    const double *__restrict__ clv_, const int32_t *__restrict__ scl_, double *__restrict__ adj_,
-                    const uint8_t *__restrict__ tips_, const double *__restrict__ P_, const double *__restrict__ Qd,
-                    const double *__restrict__ freqs, const double *__restrict__ seed,
-                    const int32_t *__restrict__ tile_part, const double *__restrict__ beta, int n_root, int n_uses,
-                    double *__restrict__ grad_partials) {
+//
+// MODEL: also, per use, the sums over the wave's sites of z x^T (dJ/dP), one
+// entry per lane of a granule (G, [use][wave][NA][64]), and per root those of
+// the frequencies' direct share, f x with f = beta w / (C Ltilde)
+// (r_part, [root][wave][4]).  Both are products over sites: z and x are
+// transposed by a product with the identity, which is exact, and multiplied
+// (41,345 patterns, 138 ops: 0.44 ms against 0.32 without, and 0.08 for
+// k_model_reduce; a pass of its own over stored adjoints and CLVs took 0.85
+// ms, and storing the adjoints 0.10).
+template <int C, int NQ, bool MODEL>
+__device__ __forceinline__ void adjoint_walk4(
+    const DevOp *__restrict__ ops_, int n_ops, const DevLayout &L, const double *__restrict__ clv_,
+    const int32_t *__restrict__ scl_, double *__restrict__ adj_, const uint8_t *__restrict__ tips_,
+    const double *__restrict__ P_, const double *__restrict__ Qd, const double *__restrict__ freqs,
+    const double *__restrict__ seed, const int32_t *__restrict__ tile_part, const double *__restrict__ beta, int n_root,
+    int n_uses, double *__restrict__ grad_partials, double *__restrict__ G_, double *__restrict__ r_part) {
   using W = Quad<C, NQ>;
   constexpr int NA = W::NA, SPW = W::SPW;
   const CAS DevOp *ops = to_constant(ops_);
@@ -853,6 +861,8 @@ __global__ void __launch_bounds__(64, 3)
     Q[h] = Qd[part * (C * 16) + aoff[h] / 8];
   }
   const double pi = freqs[part * 4 + state];
+  const double eye = (lane & 3) == state ? 1.0 : 0.0;
+  GAS double *G = to_global(G_) + static_cast<int64_t>(blockIdx.x) * (NA * 64);
 
   auto load = [&](const OpRegs &op, AdjIn4<C, NQ> &in) {
     const uint32_t o = opaque(off);
@@ -948,12 +958,20 @@ __global__ void __launch_bounds__(64, 3)
     if (op.root() >= 0) {
       // seed beta * w * (1/C) pi_i / Ltilde at a displayed-tree root
       const double f = beta[part * n_root + op.root()] * in.sd[0];
+      if constexpr (MODEL) {
+        double r = 0.0;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+          r = fma(__shfl(f, W::site(lane, q)), *at(clv + op.out() * row, off + q * 512), r);
+        r += dpp<0x121>(r);  // over the 16 lanes of a state: row_ror 1, 2, 4, 8
+        r += dpp<0x122>(r);
+        r += dpp<0x124>(r);
+        r += dpp<0x128>(r);
+        if ((lane & 15) == 0) r_part[(static_cast<int64_t>(op.root()) * gridDim.x + blockIdx.x) * 4 + state] = r;
+      }
 #pragma unroll
       for (int q = 0; q < NQ; ++q) a[q] = fma(__shfl(f, W::site(lane, q)), pi, a[q]);
     }
-    if (keep)  // the model gradient reads every adjoint
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) *at(adj + op.out() * row, off + q * 512) = a[q];
     const uint64_t scaled = __builtin_amdgcn_ballot_w64(lane < SPW && (in.word[0] & 1u));
     if (scaled)
 #pragma unroll
@@ -963,6 +981,17 @@ __global__ void __launch_bounds__(64, 3)
     auto use = [&](int k) {
 #pragma unroll
       for (int q = 0; q < NQ; ++q) g[k] = fma(z[q], mfma4(Q[W::half(q)], y[k][q], 0.0), g[k]);
+      if constexpr (MODEL) {
+        double m[NA];
+#pragma unroll
+        for (int h = 0; h < NA; ++h) m[h] = 0.0;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+          m[W::half(q)] = mfma4(mfma4(z[q], eye, 0.0), mfma4(in.x[k * NQ + q], eye, 0.0), m[W::half(q)]);
+        GAS double *dst = G + static_cast<int64_t>(op.gslot() + k) * gridDim.x * (NA * 64);
+#pragma unroll
+        for (int h = 0; h < NA; ++h) *at(dst, opaque(off) + h * 512) = m[h];
+      }
       if (op.kid(k) >= 0) deliver(op, in, k, z, acc[k]);
     };
     product(op, in, 0, y[0]);
@@ -1006,6 +1035,29 @@ __global__ void __launch_bounds__(64, 3)
     op0 = op2;
     op1 = op3;
   }
+}
+
+template <int C, int NQ>
+__global__ void __launch_bounds__(64, 3)
+    k_adjoint_level(const DevOp *__restrict__ ops, int n_ops, DevLayout L, const double *__restrict__ clv,
+                    const int32_t *__restrict__ scl, double *__restrict__ adj, const uint8_t *__restrict__ tips,
+                    const double *__restrict__ P, const double *__restrict__ Qd, const double *__restrict__ freqs,
+                    const double *__restrict__ seed, const int32_t *__restrict__ tile_part,
+                    const double *__restrict__ beta, int n_root, int n_uses, double *__restrict__ grad_partials) {
+  adjoint_walk4<C, NQ, false>(ops, n_ops, L, clv, scl, adj, tips, P, Qd, freqs, seed, tile_part, beta, n_root, n_uses,
+                              grad_partials, nullptr, nullptr);
+}
+
+template <int C, int NQ>
+__global__ void __launch_bounds__(64, 3)
+    k_model_adjoint(const DevOp *__restrict__ ops, int n_ops, DevLayout L, const double *__restrict__ clv,
+                    const int32_t *__restrict__ scl, double *__restrict__ adj, const uint8_t *__restrict__ tips,
+                    const double *__restrict__ P, const double *__restrict__ Qd, const double *__restrict__ freqs,
+                    const double *__restrict__ seed, const int32_t *__restrict__ tile_part,
+                    const double *__restrict__ beta, int n_root, int n_uses, double *__restrict__ grad_partials,
+                    double *__restrict__ G, double *__restrict__ r_part) {
+  adjoint_walk4<C, NQ, true>(ops, n_ops, L, clv, scl, adj, tips, P, Qd, freqs, seed, tile_part, beta, n_root, n_uses,
+                             grad_partials, G, r_part);
 }
 
 // ------------------------------------------------ 20 states, FP64 plain form
@@ -1421,130 +1473,137 @@ __global__ void __launch_bounds__(64, 2)
 }
 
 // ---------------------------------------------- model gradient (FP64)
-// dlnL / dP_{e,c} for every (op, child) use: G = sum over sites of z (x)^T
-// with z the adjoint of y = P x (recomputed from the op's stored adjoint
-// and its children, as k_adjoint_level forms it) and x the child's CLV; and, at displayed-tree roots, the direct
-// dependence of lnL on the frequencies, sum_s beta w (1/C) x_i / Ltilde.
-// Grid (op, chunk): a chunk is a 1/n_split slice of one partition's tiles,
-// so every partial belongs to one partition; a workgroup walks its tiles
-// and reduces its threads' sums once, in a fixed order.
-template <int S, int C>
-__global__ void __launch_bounds__(TILE *C)
-    k_model_grad(const DevOp *__restrict__ ops, DevLayout L, const double *__restrict__ clv,
-                 const int32_t *__restrict__ scl, const double *__restrict__ adj,
-                 const typename TipType<S>::type *__restrict__ tips, const double *__restrict__ P,
-                 const double *__restrict__ freqs, const double *__restrict__ weights,
-                 const double *__restrict__ beta, int n_root, const int32_t *__restrict__ part_tile_begin,
-                 int n_split, int n_uses, double *__restrict__ g_out, double *__restrict__ r_out) {
-  __shared__ double red[TILE * C / 64][2 * S * S + S];
-  const DevOp op = ops[blockIdx.x];
-  const int chunk = blockIdx.y;
-  const int part = chunk / n_split, slice = chunk % n_split;
-  const int tb = part_tile_begin[part], te = part_tile_begin[part + 1];
-  const int t0 = tb + (te - tb) * slice / n_split, t1 = tb + (te - tb) * (slice + 1) / n_split;
-  const int c = threadIdx.x % C;
-  const int64_t n = L.n_sites_pad;
-  const size_t slot = static_cast<size_t>(n) * (C * S);
-  const double *Pk[2];
-#pragma unroll
-  for (int k = 0; k < 2; ++k)
-    Pk[k] = P + ((static_cast<size_t>(part) * L.n_edges + (k < op.nk ? op.edge[k] : 0)) * C + c) * (S * S);
-  double g[2][S * S], rr[S];
-#pragma unroll
-  for (int q = 0; q < S * S; ++q) g[0][q] = g[1][q] = 0.0;
-#pragma unroll
-  for (int i = 0; i < S; ++i) rr[i] = 0.0;
-  const double bt = op.root >= 0 ? beta[part * n_root + op.root] : 0.0;
-  for (int tile = t0; tile < t1; ++tile) {
-    const int64_t site = static_cast<int64_t>(tile) * TILE + threadIdx.x / C;
-    const size_t ro = row_offset<S, C>(site, c);
-    const double w = weights[site];
-    double a[S], x[2][S], y[2][S];
-#pragma unroll
-    for (int i = 0; i < S; ++i) a[i] = 0.0;
-    load_clv<S>(adj + static_cast<size_t>(op.out) * slot + ro, a);
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      if (k >= op.nk) continue;
-      const int32_t kid = op.kid[k];
-      if (kid >= 0) {
-        load_clv<S>(clv + static_cast<size_t>(kid) * slot + ro, x[k]);
-      } else {
-        tip_vec<S>(tips[static_cast<size_t>(-kid - 1) * n + site], x[k]);
-      }
-      matvec<S>(Pk[k], x[k], y[k]);
-    }
-    if (op.root >= 0) {
-      // the frequencies' direct share beta w (1/C) x_i / Ltilde
-      double xr[S];
-      load_clv<S>(clv + static_cast<size_t>(op.out) * slot + ro, xr);
-      double t = 0.0;
-#pragma unroll
-      for (int i = 0; i < S; ++i) t = fma(freqs[part * S + i], xr[i], t);
-      t = cat_sum<C>(t) * (1.0 / C);
-      const double f = w != 0.0 ? bt * w * (1.0 / C) / t : 0.0;
-#pragma unroll
-      for (int i = 0; i < S; ++i) rr[i] = fma(f, xr[i], rr[i]);
-    }
-    const double F = (scl[static_cast<size_t>(op.out) * n + site] & 1) ? SCALE_FACTOR : 1.0;
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      if (k >= op.nk) continue;
-#pragma unroll
-      for (int i = 0; i < S; ++i) {
-        const double z = a[i] * F * (op.nk == 2 ? y[1 - k][i] : 1.0);
-#pragma unroll
-        for (int j = 0; j < S; ++j) g[k][i * S + j] = fma(z, x[k][j], g[k][i * S + j]);
-      }
-    }
+// dJ/dP of every use from the walks' sums G: per (use, partition, slice of the
+// partition's waves) the sum over the slice, [use][partition][slice][nl]; the
+// rows after the uses are the roots' sums r_part ([root][wave][4]) likewise.
+// A workgroup holds 256 / nl waves' entries at once and adds them in order.
+__global__ void __launch_bounds__(256)
+    k_model_reduce(const double *__restrict__ G, const double *__restrict__ r_part, int n_uses, int nl, int n_waves,
+                   int waves_per_tile, const int32_t *__restrict__ part_tile_begin, int P, int n_slice,
+                   double *__restrict__ g_sum, double *__restrict__ r_sum) {
+  __shared__ double sh[256];
+  const bool root = static_cast<int>(blockIdx.x) >= n_uses;
+  const int row = root ? blockIdx.x - n_uses : blockIdx.x, width = root ? 4 : nl;
+  const int p = blockIdx.y / n_slice, slice = blockIdx.y % n_slice;
+  const int wb = part_tile_begin[p] * waves_per_tile, we = part_tile_begin[p + 1] * waves_per_tile;
+  const int w0 = wb + static_cast<int>(static_cast<int64_t>(we - wb) * slice / n_slice);
+  const int w1 = wb + static_cast<int>(static_cast<int64_t>(we - wb) * (slice + 1) / n_slice);
+  const int i = threadIdx.x % width, lead = threadIdx.x / width, step = 256 / width;
+  const double *in = (root ? r_part : G) + static_cast<size_t>(row) * n_waves * width + i;
+  double s = 0.0;
+  for (int w = w0 + lead; w < w1; w += step) s += in[static_cast<size_t>(w) * width];
+  sh[threadIdx.x] = s;
+  __syncthreads();
+  if (lead == 0) {
+    for (int j = 1; j < step; ++j) s += sh[j * width + i];
+    (root ? r_sum : g_sum)[((static_cast<size_t>(row) * P + p) * n_slice + slice) * width + i] = s;
   }
-  // sums over the sites of each category: lanes of one category are C apart
-  const int wave = threadIdx.x / 64, lane = threadIdx.x & 63;
-  auto site_sum = [&](double v) {
+}
+
+// Per (edge, partition): G_c = sum over the edge's uses, and through P_c =
+// exp(Q r_c t) = V exp(L s) V^-1 (s = r_c t) the edge's part of
+//   dJ/dQ   = sum_c V^-T ((V^T G_c V^-T) o Psi) V^T,
+//             Psi_kl = (e^{l_k s} - e^{l_l s}) / (l_k - l_l), s e^{l_k s} for equal eigenvalues
+//   dJ/dr_c = t tr(G_c^T Q P_c)
+// into out[partition][edge][16 + C] (on the host, 84,000 exponentials for 110
+// edges, it took 0.6 ms).  Lane (c & 3, i, j) holds entry (i, j) of
+// category c; with 8 categories the lanes take two in turn.
+template <int C>
+__global__ void __launch_bounds__(64)
+    k_model_chain(DevLayout L, const double *__restrict__ g_sum, int n_slice,
+                  const int32_t *__restrict__ edge_use_begin, const int32_t *__restrict__ edge_use_list,
+                  const double *__restrict__ V_, const double *__restrict__ Vinv_, const double *__restrict__ ev_,
+                  const double *__restrict__ rates, const double *__restrict__ brlen, double *__restrict__ out) {
+  constexpr int NA = C == 8 ? 2 : 1, NL = 64 * NA, SB = C >= 4 ? 1 : 4 / C;
+  __shared__ double raw[NL], m0[64], m1[64], sums[64];
+  const int edge = blockIdx.x, p = blockIdx.y, lane = threadIdx.x;
+  const int i = (lane >> 2) & 3, j = lane & 3;
+  const double *V = V_ + p * 16, *W = Vinv_ + p * 16, *ev = ev_ + p * 4;
+  double total[NA];
 #pragma unroll
-    for (int off = C; off < 64; off <<= 1) v += __shfl_xor(v, off);
-    return v;
-  };
-#pragma unroll
-  for (int k = 0; k < 2; ++k)
-#pragma unroll
-    for (int q = 0; q < S * S; ++q) g[k][q] = site_sum(g[k][q]);
-  // lane c (< C) of every wave now holds its category's wave sums; combine
-  // the waves through LDS in wave order, one category at a time
-  for (int cc = 0; cc < C; ++cc) {
-    if (lane == cc) {
-#pragma unroll
-      for (int k = 0; k < 2; ++k)
-#pragma unroll
-        for (int q = 0; q < S * S; ++q) red[wave][k * S * S + q] = g[k][q];
-    }
-    __syncthreads();
-    if (threadIdx.x < 2 * S * S) {
-      const int k = threadIdx.x / (S * S), q = threadIdx.x % (S * S);
-      double sum = 0.0;
-      for (int wv = 0; wv < TILE * C / 64; ++wv) sum += red[wv][threadIdx.x];
-      if (k < op.nk)
-        g_out[((static_cast<size_t>(op.gslot[k]) * gridDim.y + chunk) * C + cc) * (S * S) + q] = sum;
-    }
-    __syncthreads();
+  for (int h = 0; h < NA; ++h) {
+    double s = 0.0;
+    for (int u = edge_use_begin[edge]; u < edge_use_begin[edge + 1]; ++u)
+#pragma unroll 8
+      for (int sl = 0; sl < n_slice; ++sl)
+        s += g_sum[((static_cast<size_t>(edge_use_list[u]) * L.n_parts + p) * n_slice + sl) * NL + h * 64 + lane];
+    raw[h * 64 + lane] = s;  // [half][row i][block][column j]
   }
-  if (op.root >= 0) {
+  __syncthreads();
+  const double t = brlen[edge];
+  double *dst = out + (static_cast<size_t>(p) * L.n_edges + edge) * (16 + C);
+  double dq = 0.0;
 #pragma unroll
-    for (int i = 0; i < S; ++i) {
-      double v = rr[i];
+  for (int h = 0; h < NA; ++h) {
+    const int c = (lane >> 4) + 4 * h, cc = min(c, C - 1), base = (lane >> 4) * 16;
+    const bool mine = c < C;
+    double g = 0.0;
 #pragma unroll
-      for (int off = 1; off < 64; off <<= 1) v += __shfl_xor(v, off);
-      rr[i] = v;
-    }
-    if (lane == 0)
+    for (int b = 0; b < SB; ++b) g += mine ? raw[h * 64 + i * 16 + ((lane >> 4) * SB + b) % 4 * 4 + j] : 0.0;
+    const double s = rates[p * C + cc] * t;
+    double qp = 0.0;  // Q P_c = V L exp(L s) V^-1
 #pragma unroll
-      for (int i = 0; i < S; ++i) red[wave][2 * S * S + i] = rr[i];
+    for (int k = 0; k < 4; ++k) qp = fma(V[i * 4 + k] * (ev[k] * exp(ev[k] * s)), W[k * 4 + j], qp);
+    sums[lane] = g * qp;
+    m0[lane] = g;
     __syncthreads();
-    if (threadIdx.x < S) {
-      double sum = 0.0;
-      for (int wv = 0; wv < TILE * C / 64; ++wv) sum += red[wv][2 * S * S + threadIdx.x];
-      r_out[(static_cast<size_t>(op.root) * gridDim.y + chunk) * S + threadIdx.x] = sum;
+    if ((lane & 15) == 0 && mine) {
+      double tr = 0.0;
+      for (int k = 0; k < 16; ++k) tr += sums[base + k];
+      dst[16 + c] = t * tr;
     }
+    auto product = [&](const double *src, double *to, auto &&left, bool times_left) {
+      double acc = 0.0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        acc = times_left ? fma(left(i, k), src[base + k * 4 + j], acc) : fma(src[base + i * 4 + k], left(k, j), acc);
+      to[lane] = acc;
+      __syncthreads();
+      return acc;
+    };
+    product(m0, m1, [&](int a, int k) { return V[k * 4 + a]; }, true);             // V^T G
+    const double hv = product(m1, m0, [&](int k, int b) { return W[b * 4 + k]; }, false);  // (V^T G) V^-T
+    const double la = ev[i], lb = ev[j];
+    const double psi = fabs(la - lb) > 1e-10 * fmax(1.0, fabs(la)) ? (exp(la * s) - exp(lb * s)) / (la - lb)
+                                                                   : s * exp(0.5 * (la + lb) * s);
+    __syncthreads();
+    m0[lane] = hv * psi;
+    __syncthreads();
+    product(m0, m1, [&](int a, int k) { return W[k * 4 + a]; }, true);             // V^-T H
+    dq += product(m1, m0, [&](int k, int b) { return V[b * 4 + k]; }, false);      // (V^-T H) V^T
+    total[h] = mine ? dq : 0.0;
+  }
+  sums[lane] = total[NA - 1];
+  __syncthreads();
+  if (lane < 16) {
+    double d = 0.0;
+    for (int c = 0; c < (C < 4 ? C : 4); ++c) d += sums[c * 16 + lane];
+    dst[lane] = d;
+  }
+}
+
+// Per partition the sums over the edges and, of the roots' shares, over roots
+// and slices: out[partition][16 + C + 4].  Eight groups of 32 threads take
+// every eighth term.
+__global__ void __launch_bounds__(256)
+    k_model_total(int n_edges, int C, int n_root, int n_slice, int P, const double *__restrict__ edge_out,
+                  const double *__restrict__ r_sum, double *__restrict__ out) {
+  __shared__ double sh[8][32];
+  const int p = blockIdx.x, i = threadIdx.x & 31, group = threadIdx.x >> 5, width = 16 + C;
+  double s = 0.0;
+  if (i < width) {
+#pragma unroll 4
+    for (int e = group; e < n_edges; e += 8) s += edge_out[(static_cast<size_t>(p) * n_edges + e) * width + i];
+  } else if (i < width + 4) {
+#pragma unroll 4
+    for (int t = group; t < n_root * n_slice; t += 8)
+      s += r_sum[((static_cast<size_t>(t / n_slice) * P + p) * n_slice + t % n_slice) * 4 + i - width];
+  }
+  sh[group][i] = s;
+  __syncthreads();
+  if (threadIdx.x < width + 4) {
+    for (int g = 1; g < 8; ++g) s += sh[g][i];
+    out[p * (width + 4) + i] = s;
   }
 }
 
@@ -3382,12 +3441,11 @@ void launch_mixture(Engine &e, int variant, int pw) {
   NRX_HIP(hipGetLastError());
 }
 
-void launch_adjoint_walk(Engine &e, const DevOp *ops, int n_ops, bool keep) {
+void launch_adjoint_walk(Engine &e, const DevOp *ops, int n_ops, bool model) {
   if (n_ops == 0) return;
   const unsigned waves = static_cast<unsigned>(e.L.n_tiles) * e.rpw;
   if (e.S == AA_STATES) {
-    // (rows kept for the model gradient are a 4-state matter)
-    if (keep) throw std::logic_error("launch_adjoint_walk: 20-state adjoints are not kept");
+    if (model) throw std::logic_error("launch_adjoint_walk: model gradients are built for 4-state data");
     dispatch_c(e.C, [&](auto c) {
       constexpr int C = decltype(c)::value;
       hipLaunchKernelGGL((k_adjoint_level_aa<C>), dim3(waves * C), dim3(64), adjoint_walk_lds_aa(e.adj_slots), e.stream,
@@ -3402,12 +3460,17 @@ void launch_adjoint_walk(Engine &e, const DevOp *ops, int n_ops, bool keep) {
   }
   dispatch_walk(e.C, e.walk_nq, [&](auto c, auto nq) {
     constexpr int C = decltype(c)::value, NQ = decltype(nq)::value;
-    hipLaunchKernelGGL((k_adjoint_level<C, NQ>), dim3(waves), dim3(64), adjoint_walk_lds(NQ, e.adj_slots), e.stream,
-                       ops, n_ops, e.adj_slots, keep ? 1 : 0, e.L, e.d_clv.as<double>(), e.d_scl.as<int32_t>(),
-                       e.d_adj.as<double>(), e.d_tips.as<uint8_t>(), e.d_P.as<double>(), e.d_Qd.as<double>(),
-                       e.d_freqs.as<double>(), e.d_site_seed.as<double>(), e.d_tile_part.as<int32_t>(),
-                       e.d_beta.as<double>(), static_cast<int>(e.root_slots.size()), e.n_uses,
-                       e.d_grad_partials.as<double>());
+    auto go = [&](auto kernel, auto... extra) {
+      hipLaunchKernelGGL(kernel, dim3(waves), dim3(64), adjoint_walk_lds(NQ, e.adj_slots), e.stream, ops, n_ops, e.L,
+                         e.d_clv.as<double>(), e.d_scl.as<int32_t>(), e.d_adj.as<double>(), e.d_tips.as<uint8_t>(),
+                         e.d_P.as<double>(), e.d_Qd.as<double>(), e.d_freqs.as<double>(), e.d_site_seed.as<double>(),
+                         e.d_tile_part.as<int32_t>(), e.d_beta.as<double>(), static_cast<int>(e.root_slots.size()),
+                         e.n_uses, e.d_grad_partials.as<double>(), extra...);
+    };
+    if (model)
+      go(k_model_adjoint<C, NQ>, e.d_mg_g.as<double>(), e.d_mg_r.as<double>());
+    else
+      go(k_adjoint_level<C, NQ>);
   });
   NRX_HIP(hipGetLastError());
 }
@@ -3589,17 +3652,22 @@ void launch_deriv_fused(Engine &e, const PathStep *steps, const int32_t *path_be
   NRX_HIP(hipGetLastError());
 }
 
-void launch_model_grad(Engine &e, int n_split, double *g_out, double *r_out) {
-  if (e.S != 4) throw std::invalid_argument("model gradients are built for 4-state data");
+void launch_model_grad(Engine &e, double *g_sum, double *r_sum, double *edge_out, double *out, int n_slice) {
+  const int n_root = static_cast<int>(e.root_slots.size()), nl = e.C == 8 ? 128 : 64;
+  hipLaunchKernelGGL(k_model_reduce, dim3(e.n_uses + n_root, e.P * n_slice), dim3(256), 0, e.stream,
+                     e.d_mg_g.as<double>(), e.d_mg_r.as<double>(), e.n_uses, nl, e.L.n_tiles * e.rpw, e.rpw,
+                     e.d_part_tile_begin.as<int32_t>(), e.P, n_slice, g_sum, r_sum);
+  NRX_HIP(hipGetLastError());
   dispatch_c(e.C, [&](auto c) {
     constexpr int C = decltype(c)::value;
-    hipLaunchKernelGGL((k_model_grad<4, C>), dim3(static_cast<unsigned>(e.ops_all.size()), e.P * n_split),
-                       dim3(TILE * C), 0, e.stream, e.d_ops.as<DevOp>(), e.L, e.d_clv.as<double>(),
-                       e.d_scl.as<int32_t>(), e.d_adj.as<double>(), e.d_tips.as<uint8_t>(), e.d_P.as<double>(),
-                       e.d_freqs.as<double>(), e.d_weights.as<double>(), e.d_beta.as<double>(),
-                       static_cast<int>(e.root_slots.size()), e.d_part_tile_begin.as<int32_t>(), n_split, e.n_uses,
-                       g_out, r_out);
+    hipLaunchKernelGGL((k_model_chain<C>), dim3(e.E, e.P), dim3(64), 0, e.stream, e.L, g_sum, n_slice,
+                       e.d_edge_use_begin.as<int32_t>(), e.d_edge_use_list.as<int32_t>(), e.d_V.as<double>(),
+                       e.d_Vinv.as<double>(), e.d_eval.as<double>(), e.d_rates.as<double>(), e.d_brlen.as<double>(),
+                       edge_out);
   });
+  NRX_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_model_total, dim3(e.P), dim3(256), 0, e.stream, e.E, e.C, n_root, n_slice, e.P, edge_out, r_sum,
+                     out);
   NRX_HIP(hipGetLastError());
 }
 
