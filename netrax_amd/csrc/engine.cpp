@@ -269,7 +269,8 @@ static void plan_budget(Engine &e) {
   resize_rows(e, bp.n_phys);
 }
 
-constexpr int AA_ADJ_WAVES = 8;  // waves of the 20-state reverse walk that a CU holds
+// waves of the 20-state walks that a CU holds
+constexpr int AA_ADJ_WAVES = 8, AA_FWD32_WAVES = 16, AA_ADJ32_WAVES = 12;
 constexpr int CUS = 256, LDS_PER_CU = 160 * 1024, LDS_PER_GROUP = 64 * 1024;
 
 // LDS slots per wave of a walk of `groups` workgroups, of which a CU's
@@ -294,6 +295,11 @@ static void choose_walk_shape(Engine &e) {
   if (e.S == AA_STATES) {
     const int64_t groups = e.L.n_sites_pad / AA_SITES;
     e.rpw = TILE / AA_SITES;
+    if (e.opt.precision == NRX_FP32) {
+      e.fwd_slots = walk_slots(groups, [&](int n) { return forward_lds_aa32(e.C, n); }, AA_FWD32_WAVES / e.C);
+      e.adj_slots = walk_slots(groups * e.C, [&](int n) { return adjoint_lds_aa32(n); }, AA_ADJ32_WAVES);
+      return;
+    }
     e.fwd_slots = walk_slots(groups, [&](int n) { return forward_walk_lds_aa(e.C, n); }, std::max(1, 12 / e.C));
     e.adj_slots = walk_slots(groups * e.C, [&](int n) { return adjoint_walk_lds_aa(n); }, AA_ADJ_WAVES);
     return;
@@ -398,45 +404,23 @@ static void build_schedule(Engine &e) {
     set_adjoint_flags(e.ops_all, order, nv);
   }
 
-  // 20 states FP32: groups of up to tune_group independent ops in
-  // depth-first priority
-  e.ops_dfs.clear();
-  e.group_begin.assign(1, 0);
-  if (!e.walks()) {
-    std::vector<DevOp> proto(nv);
-    for (int v = 0; v < nv; ++v)
-      if (e.needed[v]) proto[v] = make_op(v);
-    build_batched_order(e.dag, e.root_slots, proto, e.tune_group, e.ops_dfs, e.group_begin);
-  }
-
   // gradient rows, one per (op, child), numbered in the order this engine's
-  // adjoint walks the ops (the walks: backwards; 20 states FP32: groups
-  // backwards), so that a workgroup's consecutive ops write consecutive rows
+  // adjoint walks the ops (backwards), so that a wave's consecutive ops write
+  // consecutive rows
   {
-    std::vector<int> walk;  // indices into the form's op list
-    const bool grouped = !e.walks();
-    std::vector<DevOp> &ops = grouped ? e.ops_dfs : e.ops_all;
-    if (grouped) {
-      for (int g = static_cast<int>(e.group_begin.size()) - 2; g >= 0; --g)
-        for (int i = e.group_begin[g]; i < e.group_begin[g + 1]; ++i) walk.push_back(i);
-    } else {
-      for (auto it = e.chunks.rbegin(); it != e.chunks.rend(); ++it)
-        for (int i = it->op_begin; i < it->op_end; ++i) walk.push_back(i);
-    }
     std::vector<std::array<int32_t, 2>> gslot(nv, {0, 0});
     std::vector<std::vector<int>> by_edge(e.E);
     e.n_uses = 0;
-    for (int i : walk) {
-      const DevOp &op = ops[i];
+    for (auto it = e.ops_all.rbegin(); it != e.ops_all.rend(); ++it) {
+      const DevOp &op = *it;
       for (int k = 0; k < op.nk; ++k) {
         gslot[op.out][k] = e.n_uses;
         by_edge[op.edge[k]].push_back(e.n_uses);
         e.n_uses++;
       }
     }
-    for (std::vector<DevOp> *list : {&e.ops_all, &e.ops_dfs})
-      for (DevOp &op : *list)
-        for (int k = 0; k < op.nk; ++k) op.gslot[k] = gslot[op.out][k];
+    for (DevOp &op : e.ops_all)
+      for (int k = 0; k < op.nk; ++k) op.gslot[k] = gslot[op.out][k];
     e.edge_use_begin.assign(e.E + 1, 0);
     e.edge_use_list.clear();
     for (int ed = 0; ed < e.E; ++ed) {
@@ -453,34 +437,24 @@ static void build_schedule(Engine &e) {
     dc[k].use = e.class_use[k];
   }
   upload(e.d_ops, e.ops_all, e.stream);
-  if (e.walks()) {
-    if (e.opt.precision == NRX_FP64) {
-      choose_walk_shape(e);
-    } else {
-      const int64_t blocks = e.L.n_sites_pad * e.C / 64;
-      // (a single 64-site tile of 1 category is one block)
-      e.walk_blocks = e.C == 1 ? 1 : walk_blocks_of(e.tune_group, blocks);
-      choose_slots32(e, blocks);
-    }
-    assign_walk_slots(e);
+  if (e.opt.precision == NRX_FP64 || e.S == AA_STATES) {
+    choose_walk_shape(e);
+  } else {
+    const int64_t blocks = e.L.n_sites_pad * e.C / 64;
+    // (a single 64-site tile of 1 category is one block)
+    e.walk_blocks = e.C == 1 ? 1 : walk_blocks_of(e.tune_group, blocks);
+    choose_slots32(e, blocks);
   }
-  upload(e.d_ops_dfs, e.ops_dfs, e.stream);
-  upload(e.d_group_begin, e.group_begin, e.stream);
+  assign_walk_slots(e);
   upload(e.d_edge_use_begin, e.edge_use_begin, e.stream);
   upload(e.d_edge_use_list, e.edge_use_list, e.stream);
   upload(e.d_classes, dc, e.stream);
   upload(e.d_class_dlogprob, e.class_dlogprob, e.stream);
   std::vector<int32_t> rs(e.root_slots.begin(), e.root_slots.end());
   upload(e.d_root_slots, rs, e.stream);
-  // gradient partials per site block: a wave of the walks, or the waves of a
-  // 32-site workgroup (20 states FP32)
-  if (e.walks()) {
-    e.gpw = 1;
-    e.gbpt = e.S == AA_STATES ? e.rpw * e.C : e.rpw;
-  } else {
-    e.gpw = e.C;
-    e.gbpt = TILE / AA_TILE;
-  }
+  // gradient partials per wave
+  e.gpw = 1;
+  e.gbpt = e.S == AA_STATES ? e.rpw * e.C : e.rpw;
   if (e.gpw * e.gbpt < e.rpw) throw std::logic_error("gradient partial layout does not cover the tile");
   const size_t n_wt = static_cast<size_t>(e.L.n_tiles) * e.rpw;
   const size_t n_gwt = static_cast<size_t>(e.L.n_tiles) * e.gpw * e.gbpt;
@@ -501,9 +475,6 @@ static void build_schedule(Engine &e) {
 NetDesc make_netdesc(const Engine &e) {
   NetDesc d{};
   d.L = e.L;
-  d.ops = e.d_ops_dfs.as<DevOp>();
-  d.group_begin = e.d_group_begin.as<int32_t>();
-  d.n_groups = static_cast<int32_t>(e.group_begin.size()) - 1;
   d.n_root = static_cast<int32_t>(e.root_slots.size());
   d.n_uses = e.n_uses;
   d.ops_fwd = e.d_ops_fwd.as<DevOp>();
@@ -530,9 +501,8 @@ NetDesc make_netdesc(const Engine &e) {
   // every buffer the persistent kernels read must exist before its address
   // is handed to the device
   const bool aa = e.S == AA_STATES;
-  const void *need[] = {aa ? d.ops : d.ops_fwd, aa ? static_cast<const void *>(d.group_begin) : d.ops_adj,
-                        d.clv, d.scl, d.adj, d.adj_exp, d.tips, aa ? static_cast<const void *>(d.Pa) : d.Pf,
-                        aa ? static_cast<const void *>(d.Pa) : d.PfT, d.Qf, d.tile_part, d.freqs, d.weights, d.beta,
+  const void *need[] = {d.ops_fwd, d.ops_adj, d.clv, d.scl, d.adj, d.adj_exp, d.tips, aa ? d.Pa : d.Pf,
+                        aa ? d.Pa : d.PfT, d.Qf, d.tile_part, d.freqs, d.weights, d.beta,
                         d.root_partials, d.grad_partials, d.seed};
   for (const void *p : need)
     if (!p) throw std::logic_error("device descriptor built before its buffers were allocated");
@@ -543,8 +513,8 @@ static void upload_netdesc(Engine &e) {
   if (e.opt.precision != NRX_FP32) return;
   std::vector<NetDesc> nd{make_netdesc(e)};
   upload(e.d_netdesc, nd, e.stream);
-  // work items: the walks' waves, or tiles of 32 sites for 20-state data
-  const int n_work = e.L.n_tiles * (e.S == AA_STATES ? TILE / AA_TILE : e.rpw);
+  // work items: the walks' waves
+  const int n_work = e.L.n_tiles * e.rpw;
   std::vector<WorkItem> work(n_work);
   for (int t = 0; t < n_work; ++t) work[t] = WorkItem{0, t};
   upload(e.d_work, work, e.stream);
@@ -665,7 +635,6 @@ static bool stage_pmatrices(Engine &e, bool do_update) {
 
 static void enqueue_pmatrices(Engine &e) {
   launch_pmatrices(e);
-  if (e.opt.precision == NRX_FP32 && e.S == AA_STATES) launch_mfma_tables(e);
 }
 
 static void record_kernel_begin(Engine &e, int kind) {
@@ -811,8 +780,10 @@ static void budget_adjoint(Engine &e) {
   }
 }
 
-// FP32 form, 4 states, incremental evaluation: the ops whose CLVs are invalid
-// in walk order, with slots of their own.  Returns as stage_invalid_ops.
+// FP32 form, incremental evaluation: the ops whose CLVs are invalid in walk
+// order, with slots of their own, as a device descriptor.  Returns their
+// number, or -1 when every op is invalid (the full list, and its graph, is
+// used instead); `desc` points to the staged descriptor.
 static int stage_invalid_walk(Engine &e, const NetDesc *&desc) {
   std::vector<DevOp> ops;
   for (const DevOp &op : e.ops_all)
@@ -825,51 +796,6 @@ static int stage_invalid_walk(Engine &e, const NetDesc *&desc) {
   NetDesc d = make_netdesc(e);
   d.ops_fwd = e.d_ops_inc.as<DevOp>();
   d.n_fwd = n;
-  stage_upload(e, e.d_netdesc_inc, std::vector<NetDesc>{d});
-  desc = e.d_netdesc_inc.as<NetDesc>();
-  return n;
-}
-
-// FP32 form, 20 states, incremental evaluation: the ops whose CLVs are invalid, in the
-// forward order and groups of the full list (a subset of a group of
-// independent ops is independent), as a device descriptor of their own.
-// A group is flagged independent of the one before it when it reads none of
-// that group's outputs, as the kernels' early-load rule requires.  Returns
-// the number of groups (0: nothing to recompute), or -1 when every op is
-// invalid (the full list, and its graph, is used instead); `desc` points to
-// the staged descriptor.
-static int stage_invalid_ops(Engine &e, const NetDesc *&desc) {
-  const int ng = static_cast<int>(e.group_begin.size()) - 1;
-  std::vector<DevOp> ops;
-  std::vector<int32_t> gb(1, 0);
-  std::vector<int32_t> prev, cur;
-  for (int g = 0; g < ng; ++g) {
-    cur.clear();
-    const size_t first = ops.size();
-    for (int i = e.group_begin[g]; i < e.group_begin[g + 1]; ++i) {
-      const DevOp &op = e.ops_dfs[i];
-      if (!e.clv_dirty[op.out]) continue;
-      ops.push_back(op);
-      cur.push_back(op.out);
-    }
-    if (cur.empty()) continue;
-    bool indep = !prev.empty();
-    for (size_t i = first; i < ops.size() && indep; ++i)
-      for (int k = 0; k < ops[i].nk; ++k)
-        if (std::find(prev.begin(), prev.end(), ops[i].kid[k]) != prev.end()) indep = false;
-    ops[first].flags = indep ? (ops[first].flags | OP_GROUP_INDEP) : (ops[first].flags & ~OP_GROUP_INDEP);
-    gb.push_back(static_cast<int32_t>(ops.size()));
-    prev.swap(cur);
-  }
-  if (ops.size() == e.ops_dfs.size()) return -1;
-  const int n = static_cast<int>(gb.size()) - 1;
-  if (n == 0) return 0;
-  stage_upload(e, e.d_ops_inc, ops);
-  stage_upload(e, e.d_group_begin_inc, gb);
-  NetDesc d = make_netdesc(e);
-  d.ops = e.d_ops_inc.as<DevOp>();
-  d.group_begin = e.d_group_begin_inc.as<int32_t>();
-  d.n_groups = n;
   stage_upload(e, e.d_netdesc_inc, std::vector<NetDesc>{d});
   desc = e.d_netdesc_inc.as<NetDesc>();
   return n;
@@ -929,13 +855,12 @@ static int evaluate(Engine &e, int variant, bool incremental, bool update_pm, bo
     // runs the invalid ops only, through a descriptor of their own, eagerly
     const bool aa32 = e.S == AA_STATES;
     const NetDesc *inc = nullptr;
-    int n_inc_groups = -1;
-    if (incremental) n_inc_groups = e.walks() ? stage_invalid_walk(e, inc) : stage_invalid_ops(e, inc);
-    const bool partial = n_inc_groups >= 0;
-    auto enqueue = [&e, aa32, variant, gradient, pm_in_graph, inc, n_inc_groups](bool timed) {
+    const int n_inc = incremental ? stage_invalid_walk(e, inc) : -1;
+    const bool partial = n_inc >= 0;
+    auto enqueue = [&e, aa32, variant, gradient, pm_in_graph, inc, n_inc](bool timed) {
       if (pm_in_graph) enqueue_pmatrices(e);
       if (timed) record_kernel_begin(e, 0);
-      if (n_inc_groups == 0) {
+      if (n_inc == 0) {
         // no CLV to recompute (a probability change, or a repeated call)
       } else if (aa32) {
         launch_forward_mfma(e, inc);
@@ -1526,9 +1451,8 @@ int nrx_create(const nrx_network_desc *net, const nrx_partition_desc *parts, int
     if (e->opt.precision == NRX_FP32 && !aa32 &&
         sizeof(float) * (static_cast<size_t>(e->E) + 1) * e->C * 16 > 65536)
       return fail(NRX_ERR_UNSUPPORTED, "network too large for the FP32 form's LDS tables");
-    // site-sum partials per 64-site tile: one per wave (the 20-state FP32
-    // form runs two 32-site workgroups of C waves per tile)
-    e->pw = aa32 ? 2 * e->C : TILE * e->C / 64;
+    // site-sum partials per 64-site tile: one per wave
+    e->pw = TILE * e->C / 64;
     e->rpw = e->pw;
     e->parts.resize(n_parts);
     int64_t off = 0;
@@ -1627,14 +1551,16 @@ int nrx_create(const nrx_network_desc *net, const nrx_partition_desc *parts, int
     e->d_clv.alloc(real_b * e->clv_elems_per_slot * std::max<size_t>(nv, 1));
     e->d_scl.alloc(sizeof(int32_t) * static_cast<size_t>(n) * std::max<size_t>(nv, 1));
     if (e->opt.precision == NRX_FP32) {
-      e->d_Pf.alloc(sizeof(float) * pm);
-      if (!aa32) e->d_PfT.alloc(sizeof(float) * pm);
+      if (!aa32) {
+        e->d_Pf.alloc(sizeof(float) * pm);
+        e->d_PfT.alloc(sizeof(float) * pm);
+      }
       e->d_adj.alloc(sizeof(float) * e->clv_elems_per_slot * std::max<size_t>(nv, 1));
       // adjoint exponents: per site (4 states) or per (site, category) (20 states)
       const size_t per_slot = aa32 ? static_cast<size_t>(n) * e->C : static_cast<size_t>(n);
       e->d_adj_exp.alloc(sizeof(int32_t) * per_slot * std::max<size_t>(nv, 1));
       if (aa32)
-        e->d_Pa.alloc(sizeof(float) * static_cast<size_t>(n_parts) * e->E * e->C * AA_KINDS * AA_TABLE);
+        e->d_Pa.alloc(sizeof(float) * 2 * pm);
     }
 
     const int nc = static_cast<int>(e->dag.classes.size());
@@ -2258,44 +2184,40 @@ int nrx_get_stats(nrx_engine *eng, nrx_stats *out) {
     const double scl = 4.0 * sites;            // one scaler row
     const double tip_b = (e.S == 4 ? 1.0 : 4.0) * sites;
     double fwd_ops = 0.0;
-    for (const DevOp &op : e.walks() ? e.ops_fwd : e.ops_all) {
+    for (const DevOp &op : e.ops_fwd) {
       for (int k = 0; k < op.nk; ++k) {
-        if (e.walks() && (op.flags & (k == 0 ? OP_PASS_KID0 : OP_PASS_KID1))) continue;  // handed over in LDS
+        if (op.flags & (k == 0 ? OP_PASS_KID0 : OP_PASS_KID1)) continue;  // handed over in LDS
         fwd_ops += op.kid[k] >= 0 ? row + scl : tip_b;
       }
       fwd_ops += row + scl;  // parent CLV and scaler written
     }
     // the walks form the root sums in place and write the seed factors
-    const double root = e.root_slots.size() * ((e.walks() ? 0.0 : row + scl) + 8.0 * sites);
+    const double root = e.root_slots.size() * 8.0 * sites;
     const double pm = static_cast<double>(e.P) * e.E * e.C * e.S * e.S * b;
-    // push-form adjoint, over the op list and flags of the engine's form:
-    // per op read its scaler, its adjoint (when accumulated) and its children
-    // with their scalers; per inner child write the delivered adjoint, and
-    // read it back first when another consumer delivered before.  A root op
-    // reads the seed factor (plain form, 8 bytes per site) or its own CLV
-    // (FP32 form).  Adjoints handed over through LDS (FP32, 4 states) move no
-    // HBM bytes.  Adjoint exponents: per site, or per (site, category) for
-    // 20-state FP32.
+    // push-form adjoint: per op read its scaler, its adjoint (when
+    // accumulated) and its children; per inner child write the delivered
+    // adjoint, and read it back first when another consumer delivered before.
+    // A root op reads the seed factor (8 bytes per site).  Adjoints handed
+    // over through LDS move no HBM bytes.  Adjoint exponents (FP32): per site,
+    // or per (site, category) of 20-state data.
     const bool fp32 = e.opt.precision == NRX_FP32;
     const double aexp = fp32 ? (e.S == AA_STATES ? scl * e.C : scl) : 0.0;
-    const bool pass = e.walks();
-    const std::vector<DevOp> &adj_ops = e.walks() ? e.ops_adj : fp32 ? e.ops_dfs : e.ops_all;
+    const std::vector<DevOp> &adj_ops = e.ops_adj;
     out->n_lds_handoffs = 0;
-    if (pass)
-      for (const DevOp &op : adj_ops)
-        out->n_lds_handoffs += ((op.flags & OP_PASS_KID0) != 0) + ((op.flags & OP_PASS_KID1) != 0);
+    for (const DevOp &op : adj_ops)
+      out->n_lds_handoffs += ((op.flags & OP_PASS_KID0) != 0) + ((op.flags & OP_PASS_KID1) != 0);
     double adj = 0.0;
     for (const DevOp &op : adj_ops) {
       adj += scl;
-      if ((op.flags & OP_HAS_CONSUMERS) && !(pass && (op.flags & OP_A_PASS))) adj += row + aexp;
-      if (op.root >= 0) adj += fp32 && !e.walks() ? row : 8.0 * sites;
+      if ((op.flags & OP_HAS_CONSUMERS) && !(op.flags & OP_A_PASS)) adj += row + aexp;
+      if (op.root >= 0) adj += 8.0 * sites;
       for (int k = 0; k < op.nk; ++k) {
         if (op.kid[k] < 0) {
           adj += tip_b;
           continue;
         }
-        adj += e.walks() ? row : row + scl;  // child CLV and scaler (the walks read only their own CLV's)
-        if (pass && (op.flags & (k == 0 ? OP_PASS_KID0 : OP_PASS_KID1))) continue;
+        adj += row;  // child CLV
+        if (op.flags & (k == 0 ? OP_PASS_KID0 : OP_PASS_KID1)) continue;
         adj += row + aexp;  // delivered adjoint
         if (!(op.flags & (k == 0 ? OP_FIRST_KID0 : OP_FIRST_KID1))) adj += row + aexp;
       }
@@ -2412,10 +2334,9 @@ int nrx_batch_optimize(nrx_batch *batch, int32_t variant, int32_t mode, const in
 
 namespace nrx {
 
-// Shapes of the FP32 form's kernels.  20-state data has 32 sites per
-// workgroup and tunes the group width g.  For 4-state data g chooses the row
-// blocks of a wave (walk_blocks_of); ts and h are part of a shape's name and
-// choose nothing.
+// Shapes of the FP32 form's kernels.  For 4-state data g chooses the row
+// blocks of a wave (walk_blocks_of); ts and h, and all of a shape of 20-state
+// data, are part of its name and choose nothing.
 struct Shape {
   int g, ts, h;
   bool operator==(const Shape &o) const { return g == o.g && ts == o.ts && h == o.h; }
@@ -2489,14 +2410,13 @@ int nrx_autotune(nrx_engine *eng, int32_t variant, int32_t reps, nrx_tuning *bes
     int rc = NRX_OK;
     try {
       for (size_t i = 0; i < cands.size() && rc == NRX_OK; ++i) {
-        if (e.walks()) {  // shapes that run the same kernels are timed once
-          const int64_t blocks = e.L.n_sites_pad * e.C / 64;
-          size_t j = 0;
-          while (walk_blocks_of(cands[j].g, blocks) != walk_blocks_of(cands[i].g, blocks)) ++j;
-          if (j < i) {
-            ms[i] = ms[j];
-            continue;
-          }
+        // shapes that run the same kernels are timed once
+        const int64_t blocks = e.L.n_sites_pad * e.C / 64;
+        size_t j = 0;
+        while (e.S != AA_STATES && walk_blocks_of(cands[j].g, blocks) != walk_blocks_of(cands[i].g, blocks)) ++j;
+        if (j < i) {
+          ms[i] = ms[j];
+          continue;
         }
         apply_shape(e, cands[i]);
         rc = evaluate(e, variant, false, true, true);  // warm-up (and graph capture)

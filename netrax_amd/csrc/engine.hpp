@@ -16,19 +16,15 @@ namespace nrx {
 constexpr int TILE = 64;
 constexpr int MAX_CATS = 8;
 
-// FP32 form for 20-state data (matrix cores): a workgroup handles a 32-site
-// tile, CLVs and adjoints are stored per tile as [C][20][32], and each
-// (partition, edge, category) has three operand tables (P, P^T, P') of
-// 64 lanes x 12 floats in the lane order of the matrix instruction.
+// 20-state data (matrix cores): a wave holds one category of 16 sites, and
+// each (partition, edge, category) has tables of P and P^T in the order of the
+// matrix instructions' operands.
 constexpr int AA_STATES = 20;
-constexpr int AA_TILE = 32;
-constexpr int AA_TABLE = 64 * 12;
-// FP64: per (partition, edge, category) the tables of P and P^T
+constexpr int AA_TILE = 32;  // tile_sites of a kernel shape's name
 constexpr int AA_MAT = AA_STATES * AA_STATES;
 constexpr int AA_MATS = 2 * AA_MAT;
 constexpr int AA_SITES = 16;                 // sites of a wave
 constexpr int AA_ROW = AA_SITES * AA_STATES;  // a wave's row: one category of its sites
-constexpr int AA_KINDS = 2;  // operand tables per (partition, edge, category): P, P^T
 
 // ---------------------------------------------------------------- model
 struct EigenModel {
@@ -188,12 +184,9 @@ struct DevLayout {
 // score one network or a batch of them.
 struct NetDesc {
   DevLayout L;
-  const DevOp *ops;
-  const int32_t *group_begin;
-  int32_t n_groups;
   int32_t n_root;
   int32_t n_uses;  // gradient rows
-  // 4-state walks: op lists (forward and reverse) and LDS slots per wave
+  // op lists (forward and reverse) and LDS slots per wave
   const DevOp *ops_fwd, *ops_adj;
   int32_t n_fwd, n_adj, fwd_slots, adj_slots;
   double *seed;      // root seed factors [root][site]
@@ -205,7 +198,7 @@ struct NetDesc {
   const uint8_t *tips;
   const float *Pf;
   const float *Qf;
-  const float *Pa;  // 20-state data: operand tables [part][edge][C][kind][AA_TABLE]
+  const float *Pa;  // 20-state data: operand tables [part][edge][C][P, P^T][AA_MAT]
   const int32_t *tile_part;
   const double *freqs;
   const double *weights;
@@ -269,6 +262,12 @@ constexpr size_t forward_walk_lds_aa(int C, int n_slots) {
 constexpr size_t adjoint_walk_lds_aa(int n_slots) {
   return sizeof(double) * (GRAD_RING + static_cast<size_t>(n_slots) * AA_ROW);
 }
+constexpr size_t forward_lds_aa32(int C, int n_slots) {
+  return static_cast<size_t>(n_slots) * C * 4 * (AA_ROW + AA_SITES);
+}
+constexpr size_t adjoint_lds_aa32(int n_slots) {
+  return sizeof(double) * GRAD_RING + forward_lds_aa32(1, n_slots);
+}
 constexpr size_t forward_lds32(int C, int blocks, int n_slots) {
   return static_cast<size_t>(n_slots) * blocks * (1024 + 256 / C);
 }
@@ -289,7 +288,6 @@ void launch_grad_reduce(Engine &e);
 // nets: a descriptor other than the engine's own (its invalid ops only)
 void launch_forward_persistent(Engine &e, const NetDesc *nets = nullptr);
 void launch_adjoint_persistent(Engine &e);
-void launch_mfma_tables(Engine &e);
 void launch_forward_mfma(Engine &e, const NetDesc *nets = nullptr);
 void launch_adjoint_mfma(Engine &e);
 void launch_sumtables(Engine &e, int n_paths, int max_steps);

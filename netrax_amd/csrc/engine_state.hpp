@@ -76,9 +76,6 @@ struct Engine : nrx_engine {
   // 4-state walks, with their LDS slots in the two lists the walks read
   std::vector<DevOp> ops_all, ops_fwd, ops_adj;
   std::vector<LevelChunk> chunks;
-  // FP32 form, 20 states: groups of independent ops in a depth-first-biased order
-  std::vector<DevOp> ops_dfs;
-  std::vector<int32_t> group_begin;  // [n_groups + 1] into ops_dfs
   std::vector<int32_t> edge_use_begin, edge_use_list;  // gradient rows per edge
   int n_uses = 0;
   int pw = 1;   // site-sum partials per tile (one per wave)
@@ -148,13 +145,13 @@ struct Engine : nrx_engine {
   DevBuf d_P, d_dP, d_d2P, d_Pf, d_PfT;
   DevBuf d_clv, d_scl, d_adj, d_adj_exp, d_Qf;
   DevBuf d_PA;  // 20-state FP64 form: P and P^T in operand order
-  DevBuf d_Pa;  // 20-state FP32 form: matrix-core operand tables
+  DevBuf d_Pa;  // 20-state FP32 form: likewise
   DevBuf d_ops, d_ops_dirty, d_Qd;
   DevBuf d_ops_fwd, d_ops_adj;  // 4 states: the walks' op lists
   // FP32 form, incremental evaluation: the invalid ops, their groups (20
   // states) and their descriptor
-  DevBuf d_ops_inc, d_group_begin_inc, d_netdesc_inc;
-  DevBuf d_ops_dfs, d_group_begin, d_edge_use_begin, d_edge_use_list;
+  DevBuf d_ops_inc, d_netdesc_inc;
+  DevBuf d_edge_use_begin, d_edge_use_list;
   DevBuf d_netdesc, d_work;  // FP32 form: this engine's NetDesc and (0, tile) work table
   DevBuf d_classes, d_class_dlogprob, d_root_slots;
   DevBuf d_root_partials, d_beta, d_grad_partials, d_root_sums, d_use_sums;
@@ -177,9 +174,6 @@ struct Engine : nrx_engine {
   std::vector<hipEvent_t> ev_k[2];
   int n_k[2] = {0, 0};
   nrx_timing last_timing{};
-
-  // passes by the depth-first walks (all but 20 states in single precision)
-  bool walks() const { return S == 4 || opt.precision == NRX_FP64; }
 
   ~Engine();
 };

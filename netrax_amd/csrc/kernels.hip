@@ -296,6 +296,15 @@ __device__ __forceinline__ int aa_place(int i, int k) {
   return (k >> 2) * 80 + (i < 16 ? (k & 3) * 16 + i : 64 + (k & 3) * 4 + (i & 3));
 }
 
+// The same for FP32, where a step's four columns are 4 q + r (r < 4, q < 4) or
+// 16 + q: rows 0-15 as [lane 16 q + row][step r], then [lane] of the last
+// step; then rows 16-19 as [4 q + row][r] and [4 q + row].
+__device__ __forceinline__ int aa_place32(int i, int k) {
+  const int q = k < 16 ? k >> 2 : k - 16, r = k < 16 ? k & 3 : 4;
+  const int lane = i < 16 ? 16 * q + i : 4 * q + (i - 16), base = i < 16 ? 0 : 320, lanes = i < 16 ? 64 : 16;
+  return base + (r < 4 ? lane * 4 + r : 4 * lanes + lane);
+}
+
 // P_{p,e,c} = V diag(exp(lambda r_c t_e)) V^-1, with first and second
 // derivatives in t (libpll's pll_update_prob_matrices computes the same
 // product from the same eigendecomposition).
@@ -304,7 +313,7 @@ __global__ void k_pmatrices(DevLayout L, const double *__restrict__ V,
                             const double *__restrict__ rates, const double *__restrict__ brlen,
                             double *__restrict__ P, double *__restrict__ dP,
                             double *__restrict__ d2P, float *__restrict__ Pf,
-                            float *__restrict__ PfT, double *__restrict__ PA) {
+                            float *__restrict__ PfT, double *__restrict__ PA, float *__restrict__ Pa) {
   const int S = L.S, C = L.C;
   const int64_t total = static_cast<int64_t>(L.n_parts) * L.n_edges * C * S * S;
   const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -336,6 +345,11 @@ __global__ void k_pmatrices(DevLayout L, const double *__restrict__ V,
     double *tab = PA + idx / AA_MAT * AA_MATS;
     tab[aa_place(i, j)] = a0;
     tab[AA_MAT + aa_place(j, i)] = a0;
+  }
+  if (Pa) {
+    float *tab = Pa + idx / AA_MAT * AA_MATS;
+    tab[aa_place32(i, j)] = static_cast<float>(a0);
+    tab[AA_MAT + aa_place32(j, i)] = static_cast<float>(a0);
   }
 }
 
@@ -2217,433 +2231,432 @@ __global__ void __launch_bounds__(WG, 3)
                                    static_cast<int64_t>(wi.tile) * Rows<C, row_blocks<G>>::SPW);
 }
 
-// ============================================= FP32 form, 20 states (MFMA)
-// CLV x P runs on the matrix cores.  For one rate category c and a tile of
-// 32 sites, D = P_c X is a chain of 10 v_mfma_f32_32x32x2f32 (M = parent
-// state, 20 padded to 32 with zero rows of P; K = child state, 2 per step;
-// N = site).  Operand layout of that instruction, lane l, h = l / 32,
-// col = l % 32:
-//   A (32 x 2)   lane l holds A[col][h]
-//   B (2 x 32)   lane l holds B[h][col]
-//   D (32 x 32)  lane l, register r holds D[8 (r / 4) + 4 h + r % 4][col]
-// CLVs and adjoints are stored per tile as [C][20 states][32 sites], so the
-// B operand of step t (state 2t + h) and every D register (one state per
-// half wave) is one coalesced pair of 128-byte rows; no transpose is
-// needed between a CLV's producer and its consumers.  The A operands (P
-// and P^T per partition, edge and category) are laid out in lane order by
-// k_mfma_tables; r_c Q, the same for every edge, is read once per sweep.  A workgroup is C waves, wave c = rate
-// category c of one 32-site tile.  CLV scalers are per site, as in the
-// 4-state form: the waves combine their site maxima through LDS once per
-// group of independent ops.  Adjoint exponents are per (site, category),
-// so the reverse sweep only synchronises the waves at displayed-tree roots.
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-constexpr int AA_STEPS = 10;   // K = 20 states, 2 per instruction
-constexpr int AA_ROWS = 12;    // D registers holding real states (rows < 20 for h = 0)
+// ==================================================== FP32 form, 20 states
+// The walks of the 20-state FP64 form in FP32: a wave holds one rate category
+// of 16 sites, lane l the states 4 q + r (r < 4) and 16 + q of site l & 15, q
+// = l >> 4.  Rows 0-15 of a product are five v_mfma_f32_16x16x4 (step r takes
+// the four states 4 q + r, the last one 16 + q; register i of D is row 4 q +
+// i); rows 16-19 are five v_mfma_f32_4x4x1, whose 16 blocks are (q, 4-site
+// group) and each sum their q's states, then summed over q and dealt out to
+// the lanes that hold them.  So no entry is padding, and a product's result
+// is the next one's operand and the stored row, [lane 64][4] then [lane 64].
+// Tables of P and P^T in operand order come from k_pmatrices; r_c Q, the same
+// for every edge, is read once per sweep.
+//
+// CLVs are renormalised per site as in the 4-state form (scaler words too);
+// adjoint exponents are per (site, category), so the reverse walk's waves
+// never meet.
+struct Mat20f {
+  f32x4 big, small;  // steps 0-3 of rows 0-15, of rows 16-19
+  float big4, small4;
+};
 
-__device__ __forceinline__ int aa_row(int r, int h) { return 8 * (r >> 2) + 4 * h + (r & 3); }
-__device__ __forceinline__ bool aa_valid(int r, int h) { return r < 8 || h == 0; }
+struct Row20f {
+  f32x4 v;  // states 4 q + r
+  float e;  // state 16 + q
+};
 
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+__device__ __forceinline__ void arrive(Mat20f &m) {
+  arrive(m.big);
+  arrive(m.small);
+  asm volatile("" : "+v"(m.big4), "+v"(m.small4));
+}
+__device__ __forceinline__ void arrive(Row20f &x) {
+  arrive(x.v);
+  asm volatile("" : "+v"(x.e));
 }
 
-__device__ __forceinline__ void load_a(const GAS float *__restrict__ tab, int lane, float (&a)[AA_STEPS]) {
-  const GAS float4 *p = reinterpret_cast<const GAS float4 *>(tab + lane * (AA_TABLE / 64));
-  const float4 v0 = p[0], v1 = p[1], v2 = p[2];
-  a[0] = v0.x; a[1] = v0.y; a[2] = v0.z; a[3] = v0.w;
-  a[4] = v1.x; a[5] = v1.y; a[6] = v1.z; a[7] = v1.w;
-  a[8] = v2.x; a[9] = v2.y;
+// lane16, small16: a lane's byte offsets among the 16-byte parts
+__device__ __forceinline__ void load_mat(const GAS float *tab_, uint32_t lane16, uint32_t small16, Mat20f &m) {
+  const GAS char *tab = reinterpret_cast<const GAS char *>(tab_);
+  m.big = *reinterpret_cast<const GAS f32x4 *>(tab + lane16);
+  m.big4 = *reinterpret_cast<const GAS float *>(tab + 1024 + (lane16 >> 2));
+  m.small = *reinterpret_cast<const GAS f32x4 *>(tab + 1280 + small16);
+  m.small4 = *reinterpret_cast<const GAS float *>(tab + 1536 + (small16 >> 2));
 }
 
-// B operand of a child: rows 2t + h of column col ([20][32] block of one
-// category), or the 0/1 vector of a tip's state mask
-__device__ __forceinline__ void load_b(const GAS float *__restrict__ blk, int h, float (&b)[AA_STEPS]) {
+__device__ __forceinline__ Row20f load_row(const GAS char *p, uint32_t lane16) {
+  Row20f x;
+  x.v = *reinterpret_cast<const GAS f32x4 *>(p + lane16);
+  x.e = *reinterpret_cast<const GAS float *>(p + 1024 + (lane16 >> 2));
+  return x;
+}
+__device__ __forceinline__ void store_row(GAS char *p, uint32_t lane16, const Row20f &x) {
+  *reinterpret_cast<GAS f32x4 *>(p + lane16) = x.v;
+  *reinterpret_cast<GAS float *>(p + 1024 + (lane16 >> 2)) = x.e;
+}
+__device__ __forceinline__ Row20f slot_row(const float *slot, int lane) {
+  return Row20f{*reinterpret_cast<const f32x4 *>(slot + lane * 4), slot[256 + lane]};
+}
+__device__ __forceinline__ void slot_store(float *slot, int lane, const Row20f &x) {
+  *reinterpret_cast<f32x4 *>(slot + lane * 4) = x.v;
+  slot[256 + lane] = x.e;
+}
+
+// y = M x
+__device__ __forceinline__ Row20f mul20(const Mat20f &m, const Row20f &x) {
+  f32x4 d = {0.f, 0.f, 0.f, 0.f}, t = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int t = 0; t < AA_STEPS; ++t) b[t] = blk[(2 * t + h) * AA_TILE];
-}
-__device__ __forceinline__ void tip_b(uint32_t mask, int h, float (&b)[AA_STEPS]) {
-#pragma unroll
-  for (int t = 0; t < AA_STEPS; ++t) b[t] = ((mask >> (2 * t + h)) & 1u) ? 1.0f : 0.0f;
-}
-
-__device__ __forceinline__ f32x16 mfma_chain(const float (&a)[AA_STEPS], const float (&b)[AA_STEPS]) {
-  f32x16 acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int t = 0; t < AA_STEPS; ++t) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t], b[t], acc, 0, 0, 0);
-  return acc;
-}
-
-// Operand tables: Pa[((p E + e) C + c) 3 + kind][lane][12], entry t < 10 of
-// lane (h, col) = M[col][2t + h] with M = P (kind 0), P^T (1); zero
-// for col >= 20 and t >= 10.
-__global__ void k_mfma_tables(DevLayout L, const double *__restrict__ P, float *__restrict__ Pa) {
-  const int64_t total = static_cast<int64_t>(L.n_parts) * L.n_edges * L.C * AA_KINDS * AA_TABLE;
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (idx >= total) return;
-  const int t = idx % 12;
-  const int lane = (idx / 12) % 64;
-  const int kind = (idx / AA_TABLE) % AA_KINDS;
-  const int64_t mat = idx / (AA_TABLE * AA_KINDS);  // (p E + e) C + c
-  const int h = lane >> 5, col = lane & 31;
-  float v = 0.0f;
-  if (t < AA_STEPS && col < AA_STATES) {
-    const int k = 2 * t + h;
-    const double *M = P + mat * (AA_STATES * AA_STATES);
-    v = static_cast<float>(kind == 1 ? M[k * AA_STATES + col] : M[col * AA_STATES + k]);
+  for (int r = 0; r < 4; ++r) {
+    d = __builtin_amdgcn_mfma_f32_16x16x4f32(m.big[r], x.v[r], d, 0, 0, 0);
+    t = __builtin_amdgcn_mfma_f32_4x4x1f32(m.small[r], x.v[r], t, 0, 0, 0);
   }
-  Pa[idx] = v;
+  d = __builtin_amdgcn_mfma_f32_16x16x4f32(m.big4, x.e, d, 0, 0, 0);
+  t = __builtin_amdgcn_mfma_f32_4x4x1f32(m.small4, x.e, t, 0, 0, 0);
+  // t[i] of quad q: row 16 + i over q's states; quad i gets the sum over the quads
+  auto add = [](auto s) { return __uint_as_float(s[0]) + __uint_as_float(s[1]); };
+  const float a = add(__builtin_amdgcn_permlane32_swap(__float_as_uint(t[0]), __float_as_uint(t[2]), false, false));
+  const float b = add(__builtin_amdgcn_permlane32_swap(__float_as_uint(t[1]), __float_as_uint(t[3]), false, false));
+  return Row20f{d, add(__builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false))};
 }
 
+// A lane's entries of a tip's 0/1 vector; mask: of the lane's site.
+__device__ __forceinline__ Row20f tip20f(uint32_t mask, int quad) {
+  return Row20f{tip_row(mask >> (4 * quad)),
+                __int_as_float(-static_cast<int>((mask >> (16 + quad)) & 1u) & 0x3F800000)};
+}
+
+__device__ __forceinline__ Row20f scale_row(const Row20f &x, int e) { return Row20f{scale4(x.v, e), ldexpf(x.e, e)}; }
+
+// Maximum over the states of a site of values >= 0 (see site_max).
+__device__ __forceinline__ float quad_max(float m) {
+  const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+  const int u = max(static_cast<int>(s[0]), static_cast<int>(s[1]));
+  const auto t = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  return __int_as_float(max(static_cast<int>(t[0]), static_cast<int>(t[1])));
+}
+
+struct FwdIn20f {
+  Mat20f m[2];
+  Row20f x[2];      // children read from HBM
+  uint32_t raw[2];  // the children's scaler words, or tip masks
+  __device__ __forceinline__ void arrive_all() {
+    arrive(raw);
+    arrive(x[0]);
+    arrive(x[1]);
+    arrive(m[0]);
+    arrive(m[1]);
+  }
+};
+
+// Workgroup: 16 sites, a wave per category, as k_forward_level_aa.
+// Bound: each wave's chain of ops (18,564 patterns x 4 categories, 73 ops:
+// 0.22 ms; 0.35 with 32-site waves of v_mfma_f32_32x32x2, whose 12 of 32 rows
+// are padding, a group of four ops at a time and every CLV through HBM).
 template <int C, int G>
-__device__ __forceinline__ void forward_mfma_body(
-    const CAS DevOp *__restrict__ ops, const CAS int32_t *__restrict__ group_begin, int n_groups,
-    const DevLayout L, GAS float *__restrict__ clv, GAS int32_t *__restrict__ scl,
-    const GAS uint32_t *__restrict__ tips, const GAS double *__restrict__ freqs,
-    const GAS int32_t *__restrict__ tile_part, const GAS float *__restrict__ Pa_all,
-    const GAS double *__restrict__ weights, GAS double *__restrict__ root_partials,
-    int tile /* 32-site tile */) {
-  __shared__ float smax[2][G][C][AA_TILE];
-  __shared__ double ssum[2][G][C][AA_TILE];
-  const int part = tile_part[tile >> 1];
-  const int c = threadIdx.x >> 6, lane = threadIdx.x & 63, h = lane >> 5, col = lane & 31;
-  const int64_t n = L.n_sites_pad;
-  const int64_t site = static_cast<int64_t>(tile) * AA_TILE + col;
-  const size_t slot_stride = static_cast<size_t>(n) * C * AA_STATES;
-  const size_t tile_off = static_cast<size_t>(tile) * (C * AA_STATES * AA_TILE) +
-                          static_cast<size_t>(c) * (AA_STATES * AA_TILE) + col;
-  const GAS float *__restrict__ Pa =
-      Pa_all + static_cast<size_t>(part) * L.n_edges * C * AA_KINDS * AA_TABLE;
-  const double w = weights[site];
-  const size_t n_wt = static_cast<size_t>(L.n_tiles) * 2 * C;
-  const size_t wt = static_cast<size_t>(tile) * C + c;
-  for (int gi = 0; gi < n_groups; ++gi) {
-    const int buf = gi & 1;
-    const int g0 = group_begin[gi];
-    const int nb = group_begin[gi + 1] - g0;
-    float v[G][AA_ROWS];
-    int ks[G];
+__global__ void __launch_bounds__(64 * C, 4)
+    k_forward_mfma(const NetDesc *__restrict__ nets) {
+  static_assert(G == 4, "group widths name one kernel");
+  __shared__ float site_most[2][C][AA_SITES];
+  __shared__ double site_like[2][C][AA_SITES];
+  const NetDesc &nd = nets[0];
+  const CAS DevOp *ops = to_constant(nd.ops_fwd);
+  const int n_slots = nd.fwd_slots;
+  const int c = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int lane = threadIdx.x & 63, quad = lane >> 4, col = lane & 15;
+  const uint64_t n = nd.L.n_sites_pad, row = n * (C * AA_STATES * 4);  // bytes of a CLV
+  const int64_t site0 = static_cast<int64_t>(blockIdx.x) * AA_SITES;
+  const int part = to_constant(nd.tile_part)[site0 / TILE];
+  // [slot][row], then the slots' scaler words
+  float *slots = dyn_lds<float>() + c * n_slots * AA_ROW;
+  int32_t *slot_scl = reinterpret_cast<int32_t *>(dyn_lds<float>() + C * n_slots * AA_ROW) + c * n_slots * AA_SITES;
+  GAS char *clv = reinterpret_cast<GAS char *>(to_global(nd.clv) + (static_cast<int64_t>(blockIdx.x) * C + c) * AA_ROW);
+  GAS char *scl = reinterpret_cast<GAS char *>(to_global(nd.scl) + site0);
+  const GAS char *tips = reinterpret_cast<const GAS char *>(to_global(nd.tips)) + site0 * 4;
+  const GAS float *Pa = to_global(nd.Pa) + (static_cast<int64_t>(part) * nd.L.n_edges * C + c) * AA_MATS;
+  const GAS double *freqs = to_global(nd.freqs) + part * AA_STATES;
+  const uint32_t off = lane * 16, soff = col * 4, small = (quad * 4 + (lane & 3)) * 16;
+
+  auto load = [&](const OpRegs &op, FwdIn20f &in) {
+    const uint32_t o = opaque(off), so = opaque(soff), sm = opaque(small);
 #pragma unroll
-    for (int j = 0; j < G; ++j) {
-      ks[j] = 0;
-      if (j < nb) {
-        const DevOp op = ops[g0 + j];
+    for (int k = 0; k < 2; ++k) {
+      // (a one-child op's second child stands for its first)
+      const int32_t kid = k < op.nk() ? op.kid(k) : op.kid(0);
+      const GAS char *tip = tips + static_cast<uint32_t>(~kid) * (n * 4);
+      const GAS char *word = scl + static_cast<uint32_t>(kid) * (n * 4);
+      in.raw[k] = *reinterpret_cast<const GAS uint32_t *>((kid < 0 ? tip : word) + so);
+      if (op.has(OP_LOAD0, OP_LOAD1, k)) in.x[k] = load_row(clv + static_cast<uint32_t>(op.kid(k)) * row, o);
+    }
 #pragma unroll
-        for (int r = 0; r < AA_ROWS; ++r) v[j][r] = 1.0f;
-        // both children's operands as raw values first, then the chains
-        float a[2][AA_STEPS], b[2][AA_STEPS];
-        int sk[2];
-        uint32_t tm[2];
+    for (int k = 0; k < 2; ++k) load_mat(Pa + static_cast<int64_t>(op.edge(k)) * (C * AA_MATS), o, sm, in.m[k]);
+  };
+  auto child = [&](const OpRegs &op, FwdIn20f &in, int k, int &ks) {
+    if (op.kid(k) < 0) {
+      in.x[k] = tip20f(in.raw[k], quad);
+      in.raw[k] = 0;
+    }
+    if (op.has(OP_PASS_KID0, OP_PASS_KID1, k)) {
+      in.x[k] = slot_row(slots + op.slot(k) * AA_ROW, lane);
+      in.raw[k] = slot_scl[op.slot(k) * AA_SITES + col];
+    }
+    ks += word_k(static_cast<int32_t>(in.raw[k]));
+    return mul20(in.m[k], in.x[k]);
+  };
+  int turn = 0;
+  auto step = [&](const OpRegs &op, FwdIn20f &in, Nothing) {
+    int ks = 0;
+    Row20f v = child(op, in, 0, ks);
+    if (op.nk() == 2) {
+      const Row20f y = child(op, in, 1, ks);
+      v.v *= y.v;
+      v.e *= y.e;
+    }
+    // (products of values >= 0; a negative rounding error loses to any
+    // positive value, see site_max)
+    float m = quad_max(fmaxf(fmaxf(fmaxf(v.v[0], v.v[1]), fmaxf(v.v[2], v.v[3])), v.e));
+    double like = 0.0;
+    if (op.root() >= 0) {
+      // site likelihoods Ltilde = (1/C) sum_c pi . x
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-          // the tip mask and the scaler are loaded for every child (tip 0
-          // and variant 0 stand in for the absent one): a value loaded on
-          // one path only would be copied at the join, which waits for
-          // every load issued so far
-          const int32_t kid = kk < op.nk ? op.kid[kk] : -1;
-          tm[kk] = tips[static_cast<size_t>(kid < 0 ? -kid - 1 : 0) * n + site];
-          sk[kk] = scl[static_cast<size_t>(kid < 0 ? 0 : kid) * n + site];
-          if (kk < op.nk) {
-            load_a(Pa + (static_cast<size_t>(op.edge[kk]) * C + c) * AA_KINDS * AA_TABLE, lane, a[kk]);
-            if (kid >= 0) load_b(clv + kid * slot_stride + tile_off, h, b[kk]);
-          }
-        }
+      for (int r = 0; r < 4; ++r) like = fma(freqs[4 * quad + r], static_cast<double>(v.v[r]), like);
+      like = fma(freqs[16 + quad], static_cast<double>(v.e), like);
+      like += __shfl_xor(like, 16);
+      like += __shfl_xor(like, 32);
+    }
+    if constexpr (C > 1) {
+      // (two sets of cells in turn: one barrier separates a cell's readers
+      // from the op after next, which writes it again)
+      if (lane < AA_SITES) site_most[turn][c][col] = m;
+      if (op.root() >= 0 && lane < AA_SITES) site_like[turn][c][col] = like;
+      lds_barrier();
+      int most = 0;
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-          if (kk < op.nk) {
-            if (op.kid[kk] < 0) tip_b(tm[kk], h, b[kk]);
-            ks[j] += op.kid[kk] < 0 ? 0 : sk[kk];
-            const f32x16 d = mfma_chain(a[kk], b[kk]);
+      for (int cc = 0; cc < C; ++cc) most = max(most, __float_as_int(site_most[turn][cc][col]));
+      m = __int_as_float(most);
+      if (op.root() >= 0) {
+        like = 0.0;
 #pragma unroll
-            for (int r = 0; r < AA_ROWS; ++r) v[j][r] *= d[r];
-          }
-        }
-        float m = 0.0f;
-#pragma unroll
-        for (int r = 0; r < AA_ROWS; ++r) m = fmaxf(m, v[j][r]);
-        m = fmaxf(m, __shfl_xor(m, 32));
-        if (h == 0) smax[buf][j][c][col] = m;
-        if (op.root >= 0) {
-          double s = 0.0;
-#pragma unroll
-          for (int r = 0; r < AA_ROWS; ++r)
-            if (aa_valid(r, h)) s = fma(freqs[part * AA_STATES + aa_row(r, h)], static_cast<double>(v[j][r]), s);
-          s += __shfl_xor(s, 32);
-          if (h == 0) ssum[buf][j][c][col] = s;
-        }
+        for (int cc = 0; cc < C; ++cc) like += site_like[turn][cc][col];
       }
+      turn ^= 1;
     }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < G; ++j) {
-      if (j < nb) {
-        const DevOp op = ops[g0 + j];
-        float m = 0.0f;
-#pragma unroll
-        for (int cc = 0; cc < C; ++cc) m = fmaxf(m, smax[buf][j][cc][col]);
-        int e = 0;
-        if (m > 0.f) (void)frexpf(m, &e);
-        const int k = ks[j] - e;
-        GAS float *dst = clv + op.out * slot_stride + tile_off;
-#pragma unroll
-        for (int r = 0; r < AA_ROWS; ++r)
-          if (aa_valid(r, h)) dst[aa_row(r, h) * AA_TILE] = ldexpf(v[j][r], -e);
-        if (c == 0 && h == 0) scl[static_cast<size_t>(op.out) * n + site] = k;
-        if (op.root >= 0) {
-          double t = 0.0;
-#pragma unroll
-          for (int cc = 0; cc < C; ++cc) t += ssum[buf][j][cc][col];
-          t = ldexp(t, -e) * (1.0 / C);
-          double val = (c == 0 && h == 0 && w != 0.0) ? w * (log(t) - k * LN2) : 0.0;
-          val = wave_sum(val);
-          if (lane == 0) root_partials[static_cast<size_t>(op.root) * n_wt + wt] = val;
-        }
-      }
+    const int e = m > 0.f ? __builtin_amdgcn_frexp_expf(m) : 0;
+    v = scale_row(v, -e);
+    const int32_t word = ((ks - e) << 9) | (e & 511);
+    store_row(clv + op.out() * row, opaque(off), v);
+    // (lanes of a site and the categories' waves store the same word)
+    *reinterpret_cast<GAS int32_t *>(scl + op.out() * (n * 4) + opaque(soff)) = word;
+    if (op.flags() & OP_A_PASS) {
+      slot_store(slots + op.slot(2) * AA_ROW, lane, v);
+      slot_scl[op.slot(2) * AA_SITES + col] = word;
     }
-  }
+    if (op.root() >= 0 && c == 0) {
+      const double t = ldexp(like, -e) * (1.0 / C), w = to_global(nd.weights)[site0 + col];
+      const double val = lane < AA_SITES && w != 0.0 ? w * (log(t) - word_k(word) * LN2) : 0.0;
+      const double sum = wave_sum(val);
+      if (lane == 0) to_global(nd.root_partials)[op.root() * static_cast<int64_t>(gridDim.x) + blockIdx.x] = sum;
+      // the adjoint's seed factor at this root and site, w / (C Ltilde)
+      to_global(nd.seed)[op.root() * static_cast<int64_t>(n) + site0 + col] = w != 0.0 ? w / (C * t) : 0.0;
+    }
+  };
+  walk_ops<FwdIn20f>(ops, nd.n_fwd, false, load, [](const OpRegs &) { return Nothing{}; }, step);
 }
 
-template <int C, int G>
-__global__ void __launch_bounds__(64 * C)
-    k_forward_mfma(const NetDesc *__restrict__ nets, const WorkItem *__restrict__ work) {
-  const WorkItem wi = work[blockIdx.x];
-  const NetDesc &nd = nets[wi.net];
-  forward_mfma_body<C, G>(to_constant(nd.ops), to_constant(nd.group_begin), nd.n_groups, nd.L,
-                          to_global(nd.clv), to_global(nd.scl),
-                          to_global(reinterpret_cast<const uint32_t *>(nd.tips)), to_global(nd.freqs),
-                          to_global(nd.tile_part), to_global(nd.Pa), to_global(nd.weights),
-                          to_global(nd.root_partials), wi.tile);
+__device__ __forceinline__ int align_add(Row20f &x, int ex, const Row20f &y, int ey) {
+  const int e = max(ex, ey);
+  const float sx = ldexpf(1.0f, ex - e), sy = ldexpf(1.0f, ey - e);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) x.v[i] = fmaf(x.v[i], sx, y.v[i] * sy);
+  x.e = fmaf(x.e, sx, y.e * sy);
+  return e;
 }
 
-// Adjoint delivery to a child (push form) with one exponent per (site,
-// category): lanes l and l ^ 32 hold the two halves of a site's states.
-__device__ __forceinline__ void deliver_adjoint_mfma(GAS float *__restrict__ dst_m, GAS int32_t *__restrict__ dst_e,
-                                                     bool first, int h, float (&b)[AA_ROWS], int eb) {
-  float mb = 0.0f;
-#pragma unroll
-  for (int r = 0; r < AA_ROWS; ++r) mb = fmaxf(mb, fabsf(b[r]));
-  mb = fmaxf(mb, __shfl_xor(mb, 32));
-  if (!(mb > 0.f)) eb = EXP_EMPTY;
-  if (!first) {
-    float acc[AA_ROWS];
-#pragma unroll
-    for (int r = 0; r < AA_ROWS; ++r) acc[r] = aa_valid(r, h) ? dst_m[aa_row(r, h) * AA_TILE] : 0.0f;
-    const int ea = *dst_e;
-    if (ea > eb) {
-#pragma unroll
-      for (int r = 0; r < AA_ROWS; ++r) b[r] = acc[r] + ldexpf(b[r], eb - ea);
-      eb = ea;
-    } else {
-#pragma unroll
-      for (int r = 0; r < AA_ROWS; ++r) b[r] += ldexpf(acc[r], ea - eb);
-    }
-    mb = 0.0f;
-#pragma unroll
-    for (int r = 0; r < AA_ROWS; ++r) mb = fmaxf(mb, fabsf(b[r]));
-    mb = fmaxf(mb, __shfl_xor(mb, 32));
+struct AdjIn20f {
+  Mat20f m[2];
+  Row20f x[2], a;   // inner children; own adjoint, where no slot holds it
+  double sd[1];     // seed factor of a displayed-tree root
+  uint32_t raw[2];  // tip children's masks
+  int32_t ea[1], word[1];
+  __device__ __forceinline__ void arrive_all() {
+    arrive(raw);
+    arrive(ea);
+    arrive(word);
+    arrive(sd);
+    arrive(a);
+    arrive(x[0]);
+    arrive(x[1]);
+    arrive(m[0]);
+    arrive(m[1]);
   }
-  if (mb > 0.f) {
-    int e;
-    (void)frexpf(mb, &e);
-#pragma unroll
-    for (int r = 0; r < AA_ROWS; ++r) b[r] = ldexpf(b[r], -e);
-    eb += e;
-  } else {
-    eb = EXP_EMPTY;
-  }
-#pragma unroll
-  for (int r = 0; r < AA_ROWS; ++r)
-    if (aa_valid(r, h)) dst_m[aa_row(r, h) * AA_TILE] = b[r];
-  if (h == 0) *dst_e = eb;
-}
+};
+// What the op reads while its products run: the inner children's transposed
+// matrices, and what their adjoints hold already, where no slot does.
+struct Held20f {
+  Mat20f mt[2];
+  Row20f m[2];
+  int32_t e[2];
+};
 
-// Reverse sweep of the 20-state FP32 form (push form, as k_adjoint_persistent):
-// y_k = P_k x_k from the child's B operand; P'_k x_k = r_c Q y_k and
-// P_k^T z_k (z_k = Abar * y_other) take y_k and z_k from the D layout into
-// B operands through wave-private LDS blocks, and P_k^T z_k is delivered to
-// the child.
+// The reverse sweep (as k_adjoint_persistent) of one category of 16 sites,
+// categories in the grid's slow direction, so that waves running together
+// read the same tables.  The sums over sites of dJ/dt are FP64.  Bound: as the
+// forward walk, at three waves per SIMD (same shape: 0.40 ms; 0.69 with
+// 32-site waves, products reordered through LDS).
 template <int C>
-__device__ __forceinline__ void adjoint_mfma_body(
-    const CAS DevOp *__restrict__ ops, const CAS int32_t *__restrict__ group_begin, int n_groups,
-    const DevLayout L, const GAS float *__restrict__ clv, const GAS int32_t *__restrict__ scl,
-    GAS float *__restrict__ adj, GAS int32_t *__restrict__ adj_exp,
-    const GAS uint32_t *__restrict__ tips, const GAS double *__restrict__ freqs,
-    const GAS int32_t *__restrict__ tile_part, const GAS float *__restrict__ Pa_all,
-    const GAS float *__restrict__ Qf, const GAS double *__restrict__ weights, const GAS double *__restrict__ beta,
-    int n_root, int n_uses, GAS double *__restrict__ grad_partials, int tile) {
-  __shared__ double rsum[2][C][AA_TILE];
-  __shared__ float zb[C][2][AA_STATES * AA_TILE];
-  const int part = tile_part[tile >> 1];
-  const int c = threadIdx.x >> 6, lane = threadIdx.x & 63, h = lane >> 5, col = lane & 31;
-  const int64_t n = L.n_sites_pad;
-  const int64_t site = static_cast<int64_t>(tile) * AA_TILE + col;
-  const size_t slot_stride = static_cast<size_t>(n) * C * AA_STATES;
-  const size_t tile_off = static_cast<size_t>(tile) * (C * AA_STATES * AA_TILE) +
-                          static_cast<size_t>(c) * (AA_STATES * AA_TILE) + col;
-  // adjoint exponents: [slot][tile][C][32]
-  const size_t exp_stride = static_cast<size_t>(n) * C;
-  const size_t exp_off = static_cast<size_t>(tile) * (C * AA_TILE) + static_cast<size_t>(c) * AA_TILE + col;
-  const GAS float *__restrict__ Pa =
-      Pa_all + static_cast<size_t>(part) * L.n_edges * C * AA_KINDS * AA_TABLE;
-  const double w = weights[site];
-  float *zw = zb[c][0], *yw = zb[c][1];
-  // A operand of r_c Q (the partition's and this wave's category), held for
-  // the whole sweep: P' x = r_c Q (P x) reuses y = P x instead of a P' table
-  float qa[AA_STEPS];
+__global__ void __launch_bounds__(64, 3)
+    k_adjoint_mfma(const NetDesc *__restrict__ nets) {
+  const NetDesc &nd = nets[0];
+  const CAS DevOp *ops = to_constant(nd.ops_adj);
+  const int n_ops = nd.n_adj;
+  const int lane = threadIdx.x, quad = lane >> 4, col = lane & 15;
+  const int n_blocks = nd.L.n_tiles * (TILE / AA_SITES);
+  const int c = blockIdx.x / n_blocks, block = blockIdx.x % n_blocks;
+  const uint64_t n = nd.L.n_sites_pad, row = n * (C * AA_STATES * 4);
+  const int64_t site0 = static_cast<int64_t>(block) * AA_SITES;
+  const int part = to_constant(nd.tile_part)[site0 / TILE];
+  double *ring = dyn_lds<double>();
+  float *slots = reinterpret_cast<float *>(ring + GRAD_RING);  // [slot][row], then the slots' exponents
+  int32_t *slot_e = reinterpret_cast<int32_t *>(slots + nd.adj_slots * AA_ROW) + col;
+  const int64_t wave = static_cast<int64_t>(block) * C + c;
+  const GAS char *clv = reinterpret_cast<const GAS char *>(to_global(nd.clv) + wave * AA_ROW);
+  GAS char *adj = reinterpret_cast<GAS char *>(to_global(nd.adj) + wave * AA_ROW);
+  GAS char *adj_exp = reinterpret_cast<GAS char *>(to_global(nd.adj_exp) + wave * AA_SITES);  // [slot][wave][site]
+  const GAS char *scl = reinterpret_cast<const GAS char *>(to_global(nd.scl) + site0);
+  const GAS char *tips = reinterpret_cast<const GAS char *>(to_global(nd.tips)) + site0 * 4;
+  const GAS float *Pa = to_global(nd.Pa) + (static_cast<int64_t>(part) * nd.L.n_edges * C + c) * AA_MATS;
+  const GAS double *freqs = to_global(nd.freqs) + part * AA_STATES;
+  const GAS double *seed = to_global(nd.seed) + site0 + col;
+  const GAS double *beta = to_global(nd.beta) + part * nd.n_root;
+  GAS double *grad = to_global(nd.grad_partials) + wave * nd.n_uses;
+  const uint32_t off = lane * 16, soff = col * 4, small = (quad * 4 + (lane & 3)) * 16;
+  Mat20f Q;
   {
-    const GAS float *q = Qf + (static_cast<size_t>(part) * C + c) * (AA_STATES * AA_STATES);
+    const GAS float *q = to_global(nd.Qf) + (static_cast<size_t>(part) * C + c) * AA_MAT;
 #pragma unroll
-    for (int t = 0; t < AA_STEPS; ++t) qa[t] = col < AA_STATES ? q[col * AA_STATES + 2 * t + h] : 0.0f;
-  }
-  int rb = 0;
-  for (int gi = n_groups - 1; gi >= 0; --gi) {
-    const int g0 = group_begin[gi];
-    const int g1 = group_begin[gi + 1];
-    for (int oi = g0; oi < g1; ++oi) {
-      const DevOp op = ops[oi];
-      const int kq = scl[static_cast<size_t>(op.out) * n + site];
-      float a[AA_ROWS];
-      int ea = EXP_EMPTY;
-      if (op.flags & OP_HAS_CONSUMERS) {
-        const GAS float *src = adj + op.out * slot_stride + tile_off;
-#pragma unroll
-        for (int r = 0; r < AA_ROWS; ++r) a[r] = aa_valid(r, h) ? src[aa_row(r, h) * AA_TILE] : 0.0f;
-        ea = adj_exp[op.out * exp_stride + exp_off];
-      } else {
-#pragma unroll
-        for (int r = 0; r < AA_ROWS; ++r) a[r] = 0.0f;
-      }
-      float b[2][AA_STEPS];
-      int skraw[2];
-      uint32_t tm[2];
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
-        // the tip mask and the scaler are loaded for every child (tip 0 and
-        // variant 0 stand in for the absent one): a value loaded on one
-        // path only would be copied at the join, which waits for every
-        // load issued so far
-        const int32_t kid = kk < op.nk ? op.kid[kk] : -1;
-        tm[kk] = tips[static_cast<size_t>(kid < 0 ? -kid - 1 : 0) * n + site];
-        skraw[kk] = scl[static_cast<size_t>(kid < 0 ? 0 : kid) * n + site];
-        if (kk < op.nk && kid >= 0) load_b(clv + kid * slot_stride + tile_off, h, b[kk]);
-      }
-      // every A operand of the op (P and, for inner children, P^T) is
-      // requested here with the op's other loads, so the chains below wait
-      // for one round trip per op instead of one per table
-      float pa[2][AA_STEPS], pt[2][AA_STEPS];
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
-        if (kk < op.nk) {
-          const GAS float *tab = Pa + (static_cast<size_t>(op.edge[kk]) * C + c) * AA_KINDS * AA_TABLE;
-          load_a(tab, lane, pa[kk]);
-          if (op.kid[kk] >= 0) load_a(tab + AA_TABLE, lane, pt[kk]);
-        }
-      }
-      int sk[2] = {0, 0};
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
-        if (kk < op.nk) {
-          if (op.kid[kk] < 0)
-            tip_b(tm[kk], h, b[kk]);
-          else
-            sk[kk] = skraw[kk];
-        }
-      }
-      const int ks = sk[0] + sk[1];
-      if (op.root >= 0) {
-        // seed beta * w * (1/C) pi_i / Ltilde, Ltilde = (1/C) sum_c pi . x_c
-        const GAS float *xq = clv + op.out * slot_stride + tile_off;
-        double s = 0.0;
-#pragma unroll
-        for (int r = 0; r < AA_ROWS; ++r)
-          if (aa_valid(r, h))
-            s = fma(freqs[part * AA_STATES + aa_row(r, h)], static_cast<double>(xq[aa_row(r, h) * AA_TILE]), s);
-        s += __shfl_xor(s, 32);
-        if (h == 0) rsum[rb][c][col] = s;
-        __syncthreads();
-        double t = 0.0;
-#pragma unroll
-        for (int cc = 0; cc < C; ++cc) t += rsum[rb][cc][col];
-        t *= 1.0 / C;
-        rb ^= 1;
-        const double bw = beta[part * n_root + op.root] * w;
-        int ef = EXP_EMPTY;
-        float sd[AA_ROWS];
-        double mf = 0.0;
-        if (bw != 0.0) mf = frexp(bw / (C * t), &ef);
-#pragma unroll
-        for (int r = 0; r < AA_ROWS; ++r)
-          sd[r] = aa_valid(r, h) ? static_cast<float>(mf * freqs[part * AA_STATES + aa_row(r, h)]) : 0.0f;
-        if (ef > ea) {
-#pragma unroll
-          for (int r = 0; r < AA_ROWS; ++r) a[r] = sd[r] + ldexpf(a[r], ea - ef);
-          ea = ef;
-        } else {
-#pragma unroll
-          for (int r = 0; r < AA_ROWS; ++r) a[r] += ldexpf(sd[r], ef - ea);
-        }
-      }
-      f32x16 y[2];
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk)
-        if (kk < op.nk) y[kk] = mfma_chain(pa[kk], b[kk]);
-      const int ez = ea + kq - ks;
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
-        if (kk < op.nk) {
-          float z[AA_ROWS];
-#pragma unroll
-          for (int r = 0; r < AA_ROWS; ++r) z[r] = op.nk == 2 ? a[r] * y[1 - kk][r] : a[r];
-          // y_k from the D layout into a B operand (rows 2t + h) through the
-          // wave's LDS block, then P'_k x_k = r_c Q y_k
-#pragma unroll
-          for (int r = 0; r < AA_ROWS; ++r)
-            if (aa_valid(r, h)) yw[aa_row(r, h) * AA_TILE + col] = y[kk][r];
-          wave_sync();
-          float yb[AA_STEPS];
-#pragma unroll
-          for (int t = 0; t < AA_STEPS; ++t) yb[t] = yw[(2 * t + h) * AA_TILE + col];
-          wave_sync();
-          const f32x16 dy = mfma_chain(qa, yb);
-          float gd = 0.0f;
-#pragma unroll
-          for (int r = 0; r < AA_ROWS; ++r) gd = fmaf(z[r], dy[r], gd);
-          const double gv = wave_sum(ldexp(static_cast<double>(gd), ez));
-          if (lane == 0) grad_partials[grad_index(tile, n_uses, op.gslot[kk], C, c)] = gv;
-          const int32_t kid = op.kid[kk];
-          if (kid >= 0) {
-#pragma unroll
-            for (int r = 0; r < AA_ROWS; ++r)
-              if (aa_valid(r, h)) zw[aa_row(r, h) * AA_TILE + col] = z[r];
-            wave_sync();
-            float bz[AA_STEPS];
-#pragma unroll
-            for (int t = 0; t < AA_STEPS; ++t) bz[t] = zw[(2 * t + h) * AA_TILE + col];
-            wave_sync();
-            const f32x16 bk = mfma_chain(pt[kk], bz);
-            float back[AA_ROWS];
-#pragma unroll
-            for (int r = 0; r < AA_ROWS; ++r) back[r] = bk[r];
-            deliver_adjoint_mfma(adj + kid * slot_stride + tile_off, adj_exp + kid * exp_stride + exp_off,
-                                 (op.flags & (kk == 0 ? OP_FIRST_KID0 : OP_FIRST_KID1)) != 0, h, back, ez);
-          }
-        }
-      }
+    for (int r = 0; r < 4; ++r) {
+      Q.big[r] = q[col * AA_STATES + 4 * quad + r];
+      Q.small[r] = q[(16 + (lane & 3)) * AA_STATES + 4 * quad + r];
     }
+    Q.big4 = q[col * AA_STATES + 16 + quad];
+    Q.small4 = q[(16 + (lane & 3)) * AA_STATES + 16 + quad];
   }
-}
 
-template <int C>
-__global__ void __launch_bounds__(64 * C)
-    k_adjoint_mfma(const NetDesc *__restrict__ nets, const WorkItem *__restrict__ work) {
-  const WorkItem wi = work[blockIdx.x];
-  const NetDesc &nd = nets[wi.net];
-  adjoint_mfma_body<C>(to_constant(nd.ops), to_constant(nd.group_begin), nd.n_groups, nd.L,
-                       to_global(nd.clv), to_global(nd.scl), to_global(nd.adj), to_global(nd.adj_exp),
-                       to_global(reinterpret_cast<const uint32_t *>(nd.tips)), to_global(nd.freqs),
-                       to_global(nd.tile_part), to_global(nd.Pa), to_global(nd.Qf), to_global(nd.weights),
-                       to_global(nd.beta), nd.n_root, nd.n_uses, to_global(nd.grad_partials), wi.tile);
+  auto load = [&](const OpRegs &op, AdjIn20f &in) {
+    const uint32_t o = opaque(off), so = opaque(soff), sm = opaque(small);
+    in.word[0] = *reinterpret_cast<const GAS int32_t *>(scl + op.out() * (n * 4) + so);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      // (a one-child op's second child stands for its first)
+      const int32_t kid = k < op.nk() ? op.kid(k) : op.kid(0);
+      if (kid < 0)
+        in.raw[k] = *reinterpret_cast<const GAS uint32_t *>(tips + static_cast<uint32_t>(~kid) * (n * 4) + so);
+      else if (k < op.nk())
+        in.x[k] = load_row(clv + static_cast<uint32_t>(kid) * row, o);
+    }
+    if ((op.flags() & (OP_HAS_CONSUMERS | OP_A_PASS | OP_A_LATE)) == OP_HAS_CONSUMERS) {
+      in.a = load_row(adj + op.out() * row, o);
+      in.ea[0] = *reinterpret_cast<const GAS int32_t *>(adj_exp + op.out() * (n * (C * 4)) + so);
+    }
+    if (op.root() >= 0) in.sd[0] = seed[op.root() * static_cast<int64_t>(n)];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) load_mat(Pa + static_cast<int64_t>(op.edge(k)) * (C * AA_MATS), o, sm, in.m[k]);
+  };
+  auto early = [&](const OpRegs &op) {
+    Held20f held;
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      if (k < op.nk() && op.kid(k) >= 0)
+        load_mat(Pa + static_cast<int64_t>(op.edge(k)) * (C * AA_MATS) + AA_MAT, opaque(off), opaque(small),
+                 held.mt[k]);
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      if (op.has(OP_ACC0, OP_ACC1, k)) {
+        const uint64_t kid = static_cast<uint32_t>(op.kid(k));
+        held.m[k] = load_row(adj + kid * row, opaque(off));
+        held.e[k] = *reinterpret_cast<const GAS int32_t *>(adj_exp + kid * (n * (C * 4)) + opaque(soff));
+      }
+    return held;
+  };
+  // Delivers b (exponent ez) to child k's adjoint (as the 4-state walk).
+  auto deliver = [&](const OpRegs &op, int k, Row20f b, int ez, Held20f &held) {
+    const bool pass = op.has(OP_PASS_KID0, OP_PASS_KID1, k);
+    float *slot = slots + op.slot(k) * AA_ROW;
+    int32_t *se = slot_e + op.slot(k) * AA_SITES;
+    if (!op.has(OP_FIRST_KID0, OP_FIRST_KID1, k)) {
+      if (pass) {
+        held.m[k] = slot_row(slot, lane);
+        held.e[k] = *se;
+      }
+      ez = align_add(b, ez, held.m[k], held.e[k]);
+    }
+    if (pass) {
+      slot_store(slot, lane, b);
+      *se = ez;  // (the lanes of a site store the same exponent)
+    } else {
+      const uint64_t kid = static_cast<uint32_t>(op.kid(k));
+      store_row(adj + kid * row, opaque(off), b);
+      *reinterpret_cast<GAS int32_t *>(adj_exp + kid * (n * (C * 4)) + opaque(soff)) = ez;
+    }
+  };
+  int flushed = ops[n_ops - 1].gslot[0];  // the sweep's first gradient row
+  const int rows_end = nd.n_uses;
+  auto step = [&](const OpRegs &op, AdjIn20f &in, Held20f &held) {
+    Row20f &a = in.a;
+    int &ez = in.ea[0];
+    if (op.flags() & OP_A_PASS) {
+      a = slot_row(slots + op.slot(2) * AA_ROW, lane);
+      ez = slot_e[op.slot(2) * AA_SITES];
+    } else if (op.flags() & OP_A_LATE) {
+      a = load_row(adj + op.out() * row, off);
+      ez = *reinterpret_cast<const GAS int32_t *>(adj_exp + op.out() * (n * (C * 4)) + soff);
+      wait_loads();
+    } else if (!(op.flags() & OP_HAS_CONSUMERS)) {
+      a = Row20f{{0.f, 0.f, 0.f, 0.f}, 0.f};
+      ez = EXP_EMPTY;
+    }
+    if (op.root() >= 0) {
+      // seed beta * w * (1/C) pi_i / Ltilde at a displayed-tree root
+      int ef = EXP_EMPTY;
+      Row20f sd = {{0.f, 0.f, 0.f, 0.f}, 0.f};
+      const double f = beta[op.root()] * in.sd[0];
+      if (f != 0.0) {
+        const double mf = frexp(f, &ef);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sd.v[r] = static_cast<float>(mf * freqs[4 * quad + r]);
+        sd.e = static_cast<float>(mf * freqs[16 + quad]);
+      }
+      ez = align_add(a, ez, sd, ef);
+    }
+    // (renormalised and its exponent made z's as in the 4-state walk)
+    const float m = quad_max(
+        fmaxf(fmaxf(fmaxf(fabsf(a.v[0]), fabsf(a.v[1])), fmaxf(fabsf(a.v[2]), fabsf(a.v[3]))), fabsf(a.e)));
+    const int e = __builtin_amdgcn_frexp_expf(m);  // 0 of 0
+    a = scale_row(a, -e);
+    ez = m > 0.f ? ez + e - word_step(in.word[0]) : EXP_EMPTY;
+    Row20f y[2];
+    double g[2] = {0.0, 0.0};
+    auto product = [&](int k) {
+      if (op.kid(k) < 0) in.x[k] = tip20f(in.raw[k], quad);
+      y[k] = mul20(in.m[k], in.x[k]);
+    };
+    auto use = [&](int k, const Row20f &z) {
+      const Row20f d = mul20(Q, y[k]);
+      const float gd =
+          fmaf(z.e, d.e, fmaf(z.v[3], d.v[3], fmaf(z.v[2], d.v[2], fmaf(z.v[1], d.v[1], z.v[0] * d.v[0]))));
+      g[k] = ldexp(static_cast<double>(gd), ez);
+      if (op.kid(k) >= 0) deliver(op, k, mul20(held.mt[k], z), ez, held);
+    };
+    product(0);
+    if (op.nk() == 2) {
+      product(1);
+      use(0, Row20f{a.v * y[1].v, a.e * y[1].e});
+      use(1, Row20f{a.v * y[0].v, a.e * y[0].e});
+    } else {
+      use(0, a);
+    }
+    // (rows leave as in k_adjoint_level)
+    const double total = pair_wave_sum(g[0], g[1]);
+    const int k = lane >> 5;
+    if ((lane & 31) == 31 && k < op.nk()) ring[(op.gslot() + k) % GRAD_RING] = total;
+    const int done = op.gslot() + op.nk();
+    if (done - flushed >= 64) {
+      grad[flushed + lane] = ring[(flushed + lane) % GRAD_RING];
+      flushed += 64;
+    }
+    if (done == rows_end && lane < done - flushed) grad[flushed + lane] = ring[(flushed + lane) % GRAD_RING];
+  };
+  walk_ops<AdjIn20f>(ops, n_ops, true, load, early, step);
 }
 
 // ===================================================== branch derivatives
@@ -3371,7 +3384,8 @@ void launch_pmatrices(Engine &e) {
   hipLaunchKernelGGL(k_pmatrices, dim3(nb), dim3(256), 0, e.stream, e.L, e.d_V.as<double>(),
                      e.d_Vinv.as<double>(), e.d_eval.as<double>(), e.d_rates.as<double>(),
                      e.d_brlen.as<double>(), e.d_P.as<double>(), e.d_dP.as<double>(),
-                     e.d_d2P.as<double>(), e.d_Pf.as<float>(), e.d_PfT.as<float>(), e.d_PA.as<double>());
+                     e.d_d2P.as<double>(), e.d_Pf.as<float>(), e.d_PfT.as<float>(), e.d_PA.as<double>(),
+                     e.d_Pa.as<float>());
   NRX_HIP(hipGetLastError());
 }
 
@@ -3526,38 +3540,20 @@ void launch_adjoint_persistent_multi(hipStream_t stream, int C, int blocks, cons
   NRX_HIP(hipGetLastError());
 }
 
-void launch_mfma_tables(Engine &e) {
-  const int64_t total = static_cast<int64_t>(e.P) * e.E * e.C * AA_KINDS * AA_TABLE;
-  const int nb = static_cast<int>((total + 255) / 256);
-  hipLaunchKernelGGL(k_mfma_tables, dim3(nb), dim3(256), 0, e.stream, e.L, e.d_P.as<double>(),
-                     e.d_Pa.as<float>());
-  NRX_HIP(hipGetLastError());
-}
-
-// one workgroup per 32-site tile: the work table holds 2 n_tiles items
 void launch_forward_mfma(Engine &e, const NetDesc *nets) {
   dispatch_c(e.C, [&](auto c) {
-    constexpr int CC = decltype(c)::value;
-    auto go = [&](auto g) {
-      constexpr int GG = decltype(g)::value;
-      hipLaunchKernelGGL((k_forward_mfma<CC, GG>), dim3(2 * e.L.n_tiles), dim3(64 * CC), 0,
-                         e.stream, nets ? nets : e.d_netdesc.as<NetDesc>(), e.d_work.as<WorkItem>());
-    };
-    switch (e.tune_group) {
-      case 1: go(std::integral_constant<int, 1>{}); break;
-      case 2: go(std::integral_constant<int, 2>{}); break;
-      case 4: go(std::integral_constant<int, 4>{}); break;
-      default: throw std::invalid_argument("unsupported group width for 20-state data");
-    }
+    constexpr int C = decltype(c)::value;
+    hipLaunchKernelGGL((k_forward_mfma<C, 4>), dim3(e.L.n_tiles * e.rpw), dim3(64 * C), forward_lds_aa32(C, e.fwd_slots),
+                       e.stream, nets ? nets : e.d_netdesc.as<NetDesc>());
   });
   NRX_HIP(hipGetLastError());
 }
 
 void launch_adjoint_mfma(Engine &e) {
   dispatch_c(e.C, [&](auto c) {
-    constexpr int CC = decltype(c)::value;
-    hipLaunchKernelGGL((k_adjoint_mfma<CC>), dim3(2 * e.L.n_tiles), dim3(64 * CC), 0, e.stream,
-                       e.d_netdesc.as<NetDesc>(), e.d_work.as<WorkItem>());
+    constexpr int C = decltype(c)::value;
+    hipLaunchKernelGGL((k_adjoint_mfma<C>), dim3(e.L.n_tiles * e.rpw * C), dim3(64), adjoint_lds_aa32(e.adj_slots),
+                       e.stream, e.d_netdesc.as<NetDesc>());
   });
   NRX_HIP(hipGetLastError());
 }
