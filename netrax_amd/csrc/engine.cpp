@@ -452,18 +452,15 @@ static void build_schedule(Engine &e) {
   upload(e.d_class_dlogprob, e.class_dlogprob, e.stream);
   std::vector<int32_t> rs(e.root_slots.begin(), e.root_slots.end());
   upload(e.d_root_slots, rs, e.stream);
-  // gradient partials per wave
-  e.gpw = 1;
-  e.gbpt = e.S == AA_STATES ? e.rpw * e.C : e.rpw;
-  if (e.gpw * e.gbpt < e.rpw) throw std::logic_error("gradient partial layout does not cover the tile");
+  e.gwpt = e.S == AA_STATES ? e.rpw * e.C : e.rpw;
   const size_t n_wt = static_cast<size_t>(e.L.n_tiles) * e.rpw;
-  const size_t n_gwt = static_cast<size_t>(e.L.n_tiles) * e.gpw * e.gbpt;
+  const size_t n_gwt = static_cast<size_t>(e.L.n_tiles) * e.gwpt;
   e.d_root_partials.alloc(sizeof(double) * std::max<size_t>(1, rs.size()) * n_wt);
   e.d_beta.alloc(sizeof(double) * std::max<size_t>(1, rs.size()) * e.P);
   e.d_grad_partials.alloc(sizeof(double) * std::max(1, e.n_uses) * n_gwt);
   e.d_site_seed.alloc(sizeof(double) * std::max<size_t>(1, rs.size()) * e.L.n_sites_pad);
   e.d_root_sums.alloc(sizeof(double) * std::max<size_t>(1, rs.size()) * e.P);
-  e.d_use_sums.alloc(sizeof(double) * std::max(1, e.n_uses) * static_cast<size_t>(e.P));
+  e.d_use_sums.alloc(sizeof(double) * std::max(1, e.n_uses) * static_cast<size_t>(e.P) * GRAD_SLICES);
   stream_sync(e);
   upload_netdesc(e);
   plan_budget(e);
@@ -1117,7 +1114,7 @@ struct Batch {
   DevBuf d_nets, d_work, d_small, d_offsets, d_out;
   double *h_out = nullptr;
   std::vector<int64_t> offsets;
-  int n_work = 0, C = 0, max_pm = 0, max_root_rows = 0, max_use_rows = 0, max_edges = 0,
+  int n_work = 0, C = 0, max_pm = 0, max_root_rows = 0, max_uses = 0, max_parts = 0, max_edges = 0,
       max_res = 0;
   int fwd_slots = 0, adj_slots = 0;  // the most any engine has
   bool use_graph = false;
@@ -1171,8 +1168,7 @@ static SmallDesc make_smalldesc(const Engine &e) {
   d.rl_part_dbrlen = e.rl.part_dbrlen;
   d.rl_dprob = e.rl.dprob;
   d.pw = e.rpw;
-  d.gpw = e.gpw;
-  d.gbpt = e.gbpt;
+  d.gwpt = e.gwpt;
   const void *need[] = {d.V, d.Vinv, d.ev, d.rates, d.brlen, d.P, d.dP, d.d2P, d.Pf, d.PfT,
                         d.part_tile_begin, d.classes, d.class_dlogprob, d.root_partials,
                         d.root_sums, d.grad_partials, d.use_sums, d.beta, d.edge_use_begin,
@@ -1191,7 +1187,7 @@ static void build_batch(Batch &b) {
   std::vector<SmallDesc> small(n);
   std::vector<std::pair<int, int>> order;  // (cost, engine)
   b.offsets.assign(n + 1, 0);
-  b.max_pm = b.max_root_rows = b.max_use_rows = b.max_edges = b.max_res = 0;
+  b.max_pm = b.max_root_rows = b.max_uses = b.max_parts = b.max_edges = b.max_res = 0;
   b.fwd_slots = b.adj_slots = 0;
   b.versions.resize(n);
   b.G = b.engines[0]->tune_group;
@@ -1217,7 +1213,7 @@ static void build_batch(Batch &b) {
     e->fwd_slots = std::min(fwd, e->fwd_slots);
     e->adj_slots = std::min(adj, e->adj_slots);
     if (reshaped) {  // the root sums and gradient rows are per wave
-      e->gbpt = e->rpw;
+      e->gwpt = e->rpw;
       std::fill(e->clv_dirty.begin(), e->clv_dirty.end(), 1);
       e->cache_valid = false;
     } else if (e->fwd_slots == fwd && e->adj_slots == adj) {
@@ -1237,7 +1233,8 @@ static void build_batch(Batch &b) {
     b.offsets[i + 1] = b.offsets[i] + e.rl.size;
     b.max_pm = std::max(b.max_pm, e.P * e.E * e.C * e.S * e.S);
     b.max_root_rows = std::max(b.max_root_rows, static_cast<int>(e.root_slots.size()) * e.P);
-    b.max_use_rows = std::max(b.max_use_rows, e.n_uses * e.P);
+    b.max_uses = std::max(b.max_uses, e.n_uses);
+    b.max_parts = std::max(b.max_parts, e.P);
     b.max_edges = std::max(b.max_edges, e.E);
     b.max_res = std::max(b.max_res, e.rl.size);
     b.fwd_slots = std::max(b.fwd_slots, e.fwd_slots);
@@ -1336,7 +1333,7 @@ int nrx_batch_evaluate(nrx_batch *batch, int32_t variant, double *lnl, double *d
       if (grad) {
         launch_adjoint_persistent_multi(b.stream, b.C, b.blocks, b.d_nets.as<NetDesc>(),
                                         b.d_work.as<WorkItem>(), b.n_work, b.adj_slots);
-        launch_grad_reduce_multi(b.stream, sd, n, b.max_use_rows, b.max_edges);
+        launch_grad_reduce_multi(b.stream, sd, n, b.max_uses, b.max_parts, b.max_edges);
       }
       launch_gather_results(b.stream, sd, n, b.d_offsets.as<int64_t>(), b.d_out.as<double>(),
                             b.max_res);

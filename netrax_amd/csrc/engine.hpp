@@ -230,7 +230,7 @@ struct SmallDesc {
   int32_t rl_total, rl_per_part, rl_root_logl, rl_tree_logl, rl_alpha, rl_dbrlen,
       rl_part_dbrlen, rl_dprob;
   int32_t pw;           // root partials per 64-site tile
-  int32_t gpw, gbpt, pad;  // gradient partials: waves per site block, blocks per tile
+  int32_t gwpt, pad[2];  // gradient partials per 64-site tile: its waves
 };
 
 struct Engine;
@@ -239,7 +239,7 @@ struct Engine;
 void launch_pmatrices_multi(hipStream_t s, const SmallDesc *d, int n, int max_elems);
 void launch_root_reduce_multi(hipStream_t s, const SmallDesc *d, int n, int max_rows);
 void launch_mixture_multi(hipStream_t s, const SmallDesc *d, int n, int variant);
-void launch_grad_reduce_multi(hipStream_t s, const SmallDesc *d, int n, int max_rows, int max_edges);
+void launch_grad_reduce_multi(hipStream_t s, const SmallDesc *d, int n, int max_uses, int max_parts, int max_edges);
 void launch_gather_results(hipStream_t s, const SmallDesc *d, int n, const int64_t *offsets,
                            double *out, int max_size);
 // blocks: 64-row blocks per wave (1 or 2)
@@ -251,6 +251,8 @@ void launch_adjoint_persistent_multi(hipStream_t stream, int C, int blocks, cons
 // Dynamic LDS of the 4-state walks: the reverse walk's ring of gradient sums
 // on their way to HBM, and n_slots rows with their scaler words or exponents.
 constexpr int GRAD_RING = 128;
+// Slices of a partition's waves that a gradient row is summed in.
+constexpr int GRAD_SLICES = 32;
 constexpr size_t forward_walk_lds(int nq, int n_slots) { return static_cast<size_t>(n_slots) * (nq * 512 + 256); }
 constexpr size_t adjoint_walk_lds(int nq, int n_slots) {
   return sizeof(double) * GRAD_RING + static_cast<size_t>(n_slots) * nq * 512;

@@ -83,8 +83,7 @@ struct Engine : nrx_engine {
   // 4-state walks: LDS slots per wave, and granules per wave (FP64)
   int walk_nq = 4, fwd_slots = 4, adj_slots = 4;
   int walk_blocks = 1;  // 64-row blocks per wave (FP32)
-  // gradient partials [site block][row][wave]: waves per block, blocks per tile
-  int gpw = 1, gbpt = 1;
+  int gwpt = 1;  // gradient partials [wave][row]: waves per tile
   // FP32 form shape (nrx_autotune / nrx_set_tuning): ops per group of the
   // 20-state kernels; for 4 states see walk_blocks_of.  The other two are
   // part of a shape's name only.

@@ -174,6 +174,45 @@ __device__ __forceinline__ double wave_sum(double v) {
 }
 
 // Deterministic workgroup sum; result valid in thread 0.
+// Sum over the 64 lanes, in every lane.
+__device__ __forceinline__ double lane_sum(double v) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+  return v;
+}
+
+// Sums that carry their rounding errors along (Knuth's two-sum): the trees'
+// log-likelihoods, large and nearly equal, are compared by their exponentials.
+struct Exact {
+  double s = 0.0, e = 0.0;
+  __device__ __forceinline__ void add(double v) {
+    const double t = s + v, b = t - s;
+    e += (s - (t - b)) + (v - b);
+    s = t;
+  }
+  // over the 64 lanes, in every lane
+  __device__ __forceinline__ double lanes() {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      const double v = __shfl_xor(s, off), w = __shfl_xor(e, off);
+      add(v);
+      e += w;
+    }
+    return value();
+  }
+  __device__ __forceinline__ double value() const { return fabs(s) < INFINITY ? s + e : s; }
+};
+// over the 256 threads, in thread 0
+__device__ __forceinline__ double block_sum_exact(Exact x) {
+  __shared__ double sh[4];
+  const double v = x.lanes();
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+  __syncthreads();
+  Exact sum;
+  for (int i = 0; i < 4; ++i) sum.add(sh[i]);
+  return sum.value();
+}
+
 template <int NT>
 __device__ __forceinline__ double block_sum(double v, double *sh) {
   v = wave_sum(v);
@@ -187,15 +226,6 @@ __device__ __forceinline__ double block_sum(double v, double *sh) {
   }
   __syncthreads();
   return r;
-}
-
-// Gradient partials: one value per (site block, gradient row, wave of the
-// block), stored [block][row][wave].  Rows are numbered in the order the
-// adjoint walks the ops, so a workgroup's waves fill whole cache lines of
-// their own block instead of scattering 8-byte writes over rows shared with
-// other workgroups (partial-line writes cost a read-modify-write in HBM).
-__host__ __device__ __forceinline__ size_t grad_index(int64_t block, int n_uses, int g, int pw, int w) {
-  return (static_cast<size_t>(block) * n_uses + g) * pw + w;
 }
 
 // FP64 rows: S states of one (site, category), in the lane order of the
@@ -366,6 +396,7 @@ __global__ void k_pmatrices(DevLayout L, const double *__restrict__ V,
 // otherwise the same code runs on the global arrays.  The arithmetic and
 // its order are the same either way.
 constexpr int MIX_LDS_DOUBLES = 6144;  // 48 KiB
+constexpr int MIX_PARTIALS = 2048;  // see launch_mixture
 __host__ __device__ inline int mixture_lds_doubles(int n_root, int nc, int R, int P) {
   return n_root * P + 2 * nc + nc * P + nc * R;
 }
@@ -374,8 +405,7 @@ __device__ void mixture_body(const DevLayout &L, int n_root, int nc, int R, int 
                              const double *__restrict__ class_dlogprob,
                              const double *__restrict__ root_sums, double *__restrict__ beta,
                              double *__restrict__ res, const ResultLayout &rl) {
-  __shared__ double best[64], ssum[64];
-  __shared__ int arg[64];
+  __shared__ double per_part[64];
   const int P = L.n_parts;  // <= 64 (checked on the host)
   const bool staged = mixture_lds_doubles(n_root, nc, R, P) <= MIX_LDS_DOUBLES;
   // class k: log-probability lp[k], root index ri[k], use flag cu[k]
@@ -416,64 +446,65 @@ __device__ void mixture_body(const DevLayout &L, int n_root, int nc, int R, int 
     const int r = root_of(k);
     res[rl.tree_logl + p * nc + k] = r >= 0 ? rs[r * P + p] : 0.0;
   }
-  // best class per partition (first maximum in class order)
-  for (int p = threadIdx.x; p < P; p += blockDim.x) {
-    double bv = -INFINITY;
-    int ba = -1;
-    for (int k = 0; k < nc; ++k) {
-      if (!used(k)) continue;
-      const double v = logprob(k) + rs[root_of(k) * P + p];
-      if (v > bv) {
-        bv = v;
-        ba = k;
+  // a wave per partition, lanes over the classes
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, n_waves = blockDim.x >> 6;
+  for (int p = wave; p < P; p += n_waves) {
+    // best class (first maximum in class order)
+    double best = -INFINITY;
+    int arg = -1;
+    for (int k = lane; k < nc; k += 64) {
+      const double v = used(k) ? logprob(k) + rs[root_of(k) * P + p] : -INFINITY;
+      if (v > best) {
+        best = v;
+        arg = k;
       }
     }
-    best[p] = bv;
-    arg[p] = ba;
-  }
-  __syncthreads();
-  for (int idx = threadIdx.x; idx < nc * P; idx += blockDim.x) {
-    const int p = idx / nc, k = idx % nc;
-    double a = 0.0;
-    if (variant == 1)
-      a = k == arg[p] ? 1.0 : 0.0;
-    else if (used(k) && best[p] > -INFINITY)
-      a = exp(logprob(k) + rs[root_of(k) * P + p] - best[p]);
-    alpha[p * nc + k] = a;
-  }
-  __syncthreads();
-  for (int p = threadIdx.x; p < P; p += blockDim.x) {
-    double sacc = 0.0;
-    for (int k = 0; k < nc; ++k) sacc += alpha[p * nc + k];
-    ssum[p] = sacc;
-    res[rl.per_part + p] = variant == 1 ? best[p] : best[p] + log(sacc);
-  }
-  __syncthreads();
-  if (variant != 1)
-    for (int idx = threadIdx.x; idx < nc * P; idx += blockDim.x) {
-      const int p = idx / nc;
-      alpha[idx] = ssum[p] > 0.0 ? alpha[idx] / ssum[p] : 0.0;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      const double v = __shfl_xor(best, off);
+      const int k = __shfl_xor(arg, off);
+      if (v > best || (v == best && k >= 0 && (arg < 0 || k < arg))) {
+        best = v;
+        arg = k;
+      }
     }
+    double sum = 0.0;
+    for (int k = lane; k < nc; k += 64) {
+      double a = 0.0;
+      if (variant == 1)
+        a = k == arg ? 1.0 : 0.0;
+      else if (used(k) && best > -INFINITY)
+        a = exp(logprob(k) + rs[root_of(k) * P + p] - best);
+      alpha[p * nc + k] = a;
+      sum += a;
+    }
+    sum = lane_sum(sum);
+    if (variant != 1)
+      for (int k = lane; k < nc; k += 64) alpha[p * nc + k] = sum > 0.0 ? alpha[p * nc + k] / sum : 0.0;
+    if (lane == 0) {
+      per_part[p] = variant == 1 ? best : best + log(sum);
+      res[rl.per_part + p] = per_part[p];
+    }
+  }
   __syncthreads();
   if (staged)
     for (int idx = threadIdx.x; idx < nc * P; idx += blockDim.x) res[rl.alpha + idx] = alpha[idx];
   for (int idx = threadIdx.x; idx < n_root * P; idx += blockDim.x) {
     const int p = idx / n_root, r = idx % n_root;
     double b = 0.0;
-    for (int k = 0; k < nc; ++k)
-      if (root_of(k) == r) b += alpha[p * nc + k];
+#pragma unroll 8
+    for (int k = 0; k < nc; ++k) b += root_of(k) == r ? alpha[p * nc + k] : 0.0;
     beta[p * n_root + r] = b;
   }
-  for (int r = threadIdx.x; r < R; r += blockDim.x) {
+  for (int r = wave; r < R; r += n_waves) {
     double g = 0.0;
-    for (int p = 0; p < P; ++p)
-      for (int k = 0; k < nc; ++k)
-        g += alpha[p * nc + k] * cdl[static_cast<size_t>(k) * R + r];
-    res[rl.dprob + r] = g;
+    for (int idx = lane; idx < nc * P; idx += 64) g += alpha[idx] * cdl[static_cast<size_t>(idx % nc) * R + r];
+    g = lane_sum(g);
+    if (lane == 0) res[rl.dprob + r] = g;
   }
   if (threadIdx.x == 0) {
     double tot = 0.0;
-    for (int p = 0; p < P; ++p) tot += res[rl.per_part + p];
+    for (int p = 0; p < P; ++p) tot += per_part[p];
     res[rl.total] = tot;
   }
 }
@@ -481,8 +512,25 @@ __device__ void mixture_body(const DevLayout &L, int n_root, int nc, int R, int 
 __global__ void __launch_bounds__(256)
     k_mixture(DevLayout L, int n_root, int nc, int R, int variant,
               const DevClass *__restrict__ classes, const double *__restrict__ class_dlogprob,
-              const double *__restrict__ root_sums, double *__restrict__ beta,
-              double *__restrict__ res, ResultLayout rl) {
+              double *__restrict__ root_sums, double *__restrict__ beta,
+              double *__restrict__ res, ResultLayout rl, const double *__restrict__ root_partials, int pw,
+              const int32_t *__restrict__ part_tile_begin) {
+  if (root_partials) {
+    // few partials: summed here, a wave per (root CLV, partition)
+    const int P = L.n_parts, lane = threadIdx.x & 63;
+    for (int i = threadIdx.x >> 6; i < n_root * P; i += blockDim.x >> 6) {
+      const int p = i % P;
+      const double *in = root_partials + static_cast<int64_t>(i / P) * L.n_tiles * pw;
+      const int t1 = part_tile_begin[p + 1] * pw;
+      Exact sum;
+#pragma unroll 8
+      for (int t = part_tile_begin[p] * pw + lane; t < t1; t += 64) sum.add(in[t]);
+      const double s = sum.lanes();
+      if (lane == 0) root_sums[i] = s;
+    }
+    __threadfence_block();
+    __syncthreads();
+  }
   mixture_body(L, n_root, nc, R, variant, classes, class_dlogprob, root_sums, beta, res, rl);
 }
 
@@ -1626,38 +1674,76 @@ __global__ void __launch_bounds__(256)
 // (partials_per_tile per tile, tiles of a partition are contiguous).  One
 // workgroup per (row, partition): coalesced strided loads, fixed tree
 // order, so the sums are deterministic.
+__device__ void reduce_segments_body(const double *__restrict__ in, size_t row_stride, int pw,
+                                     const int32_t *__restrict__ ptb, int P, int row, int p,
+                                     double *__restrict__ out) {
+  const double *r = in + static_cast<size_t>(row) * row_stride;
+  const int t0 = ptb[p] * pw, t1 = ptb[p + 1] * pw;
+  Exact sum;
+  for (int t = t0 + threadIdx.x; t < t1; t += 256) sum.add(r[t]);
+  const double s = block_sum_exact(sum);
+  if (threadIdx.x == 0) out[static_cast<size_t>(row) * P + p] = s;
+}
+
 __global__ void __launch_bounds__(256)
     k_reduce_segments(const double *__restrict__ in, size_t row_stride, int pw,
                       const int32_t *__restrict__ part_tile_begin, int P,
                       double *__restrict__ out) {
-  __shared__ double sh[4];
-  const int row = blockIdx.x / P, p = blockIdx.x % P;
-  const double *r = in + static_cast<size_t>(row) * row_stride;
-  const int t0 = part_tile_begin[p] * pw, t1 = part_tile_begin[p + 1] * pw;
-  double s = 0.0;
-  for (int t = t0 + threadIdx.x; t < t1; t += 256) s += r[t];
-  s = block_sum<256>(s, sh);
-  if (threadIdx.x == 0) out[static_cast<size_t>(row) * P + p] = s;
+  reduce_segments_body(in, row_stride, pw, part_tile_begin, P, blockIdx.x / P, blockIdx.x % P, out);
 }
 
-// part_dbrlen[p][e] = sum over the uses of edge e of use_sums[u][p];
-// dbrlen[e] = sum over partitions.
-__global__ void k_grad_total(DevLayout L, const int32_t *__restrict__ edge_use_begin,
-                             const int32_t *__restrict__ edge_use_list,
-                             const double *__restrict__ use_sums, double *__restrict__ res,
-                             ResultLayout rl) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= L.n_edges) return;
-  const int P = L.n_parts;
-  double tot = 0.0;
-  for (int p = 0; p < P; ++p) {
+// Per gradient row and slice of a partition's waves the sum of their partials
+// ([wave][row]): out[row][partition][slice].  A workgroup takes 64 rows, so
+// that what it reads are whole lines (a workgroup per row read 8 bytes of each
+// line: 41,345 patterns, 248 rows, with k_grad_total 16 us against 9).
+__device__ void reduce_grad_body(const double *__restrict__ in, int n_uses, int waves_per_tile,
+                                 const int32_t *__restrict__ ptb, int P, double *__restrict__ out) {
+  __shared__ double sh[4][64];
+  const int lane = threadIdx.x & 63, quarter = threadIdx.x >> 6;
+  const int row = blockIdx.x * 64 + lane, p = blockIdx.y / GRAD_SLICES, slice = blockIdx.y % GRAD_SLICES;
+  const int64_t wb = static_cast<int64_t>(ptb[p]) * waves_per_tile, n = static_cast<int64_t>(ptb[p + 1]) * waves_per_tile - wb;
+  const int64_t w0 = wb + n * slice / GRAD_SLICES, w1 = wb + n * (slice + 1) / GRAD_SLICES;
+  const bool mine = row < n_uses;
+  double s = 0.0;
+#pragma unroll 8
+  for (int64_t w = w0 + quarter; w < w1; w += 4) s += mine ? in[w * n_uses + row] : 0.0;
+  sh[quarter][lane] = s;
+  __syncthreads();
+  if (quarter == 0 && mine)
+    out[(static_cast<int64_t>(row) * P + p) * GRAD_SLICES + slice] = s + sh[1][lane] + sh[2][lane] + sh[3][lane];
+}
+
+// part_dbrlen[p][e] = sum over the uses of edge e, dbrlen[e] = over the
+// partitions too.  A workgroup per edge, a wave per partition in turn.
+__device__ void grad_total_body(int n_edges, int P, const int32_t *__restrict__ edge_use_begin,
+                                const int32_t *__restrict__ edge_use_list, const double *__restrict__ use_sums,
+                                double *__restrict__ part_dbrlen, double *__restrict__ dbrlen) {
+  __shared__ double sh[64];  // P <= 64 (checked on the host)
+  const int e = blockIdx.x, lane = threadIdx.x & 63;
+  const int u0 = edge_use_begin[e], n = (edge_use_begin[e + 1] - u0) * GRAD_SLICES;
+  for (int p = threadIdx.x >> 6; p < P; p += blockDim.x >> 6) {
     double s = 0.0;
-    for (int i = edge_use_begin[e]; i < edge_use_begin[e + 1]; ++i)
-      s += use_sums[static_cast<size_t>(edge_use_list[i]) * P + p];
-    res[rl.part_dbrlen + p * L.n_edges + e] = s;
-    tot += s;
+    for (int i = lane; i < n; i += 64)
+      s += use_sums[(static_cast<int64_t>(edge_use_list[u0 + i / GRAD_SLICES]) * P + p) * GRAD_SLICES + i % GRAD_SLICES];
+    s = lane_sum(s);
+    if (lane == 0) {
+      sh[p] = s;
+      part_dbrlen[p * n_edges + e] = s;
+    }
   }
-  res[rl.dbrlen + e] = tot;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double tot = 0.0;
+    for (int p = 0; p < P; ++p) tot += sh[p];
+    dbrlen[e] = tot;
+  }
+}
+
+__global__ void __launch_bounds__(256)
+    k_grad_total(int n_edges, int P, const int32_t *__restrict__ edge_use_begin,
+                 const int32_t *__restrict__ edge_use_list, const double *__restrict__ use_sums,
+                 double *__restrict__ res, ResultLayout rl) {
+  grad_total_body(n_edges, P, edge_use_begin, edge_use_list, use_sums, res + rl.part_dbrlen, res + rl.dbrlen);
 }
 
 // ==================================================== FP32 form, 4 states
@@ -3262,18 +3348,6 @@ __global__ void k_pmatrices_multi(const SmallDesc *__restrict__ descs) {
   d.PfT[idx - (i * S + j) + (j * S + i)] = static_cast<float>(a0);
 }
 
-__device__ void reduce_segments_body(const double *__restrict__ in, size_t row_stride, int pw,
-                                     const int32_t *__restrict__ ptb, int P, int row, int p,
-                                     double *__restrict__ out) {
-  __shared__ double sh[4];
-  const double *r = in + static_cast<size_t>(row) * row_stride;
-  const int t0 = ptb[p] * pw, t1 = ptb[p + 1] * pw;
-  double s = 0.0;
-  for (int t = t0 + threadIdx.x; t < t1; t += 256) s += r[t];
-  s = block_sum<256>(s, sh);
-  if (threadIdx.x == 0) out[static_cast<size_t>(row) * P + p] = s;
-}
-
 __global__ void __launch_bounds__(256) k_root_reduce_multi(const SmallDesc *__restrict__ descs) {
   const SmallDesc &d = descs[blockIdx.y];
   const int P = d.L.n_parts;
@@ -3282,34 +3356,17 @@ __global__ void __launch_bounds__(256) k_root_reduce_multi(const SmallDesc *__re
                        d.part_tile_begin, P, blockIdx.x / P, blockIdx.x % P, d.root_sums);
 }
 
-// out[g][p] = sum of the gradient partials of row g over the site blocks of
-// partition p and their waves (layout [block][row][wave], gbpt blocks per
-// 64-site tile, gpw waves per block), in a fixed order
-__device__ void reduce_grad_body(const double *__restrict__ in, int n_uses, int gpw, int gbpt,
-                                 const int32_t *__restrict__ ptb, int P, int g, int p,
-                                 double *__restrict__ out) {
-  __shared__ double sh[4];
-  const int64_t q1 = static_cast<int64_t>(ptb[p + 1] - ptb[p]) * gbpt * gpw;
-  const int64_t b0 = static_cast<int64_t>(ptb[p]) * gbpt;
-  double s = 0.0;
-  for (int64_t q = threadIdx.x; q < q1; q += 256)
-    s += in[grad_index(b0 + q / gpw, n_uses, g, gpw, static_cast<int>(q % gpw))];
-  s = block_sum<256>(s, sh);
-  if (threadIdx.x == 0) out[static_cast<size_t>(g) * P + p] = s;
-}
-
 __global__ void __launch_bounds__(256)
-    k_reduce_grad(const double *__restrict__ in, int n_uses, int gpw, int gbpt,
-                  const int32_t *__restrict__ ptb, int P, double *__restrict__ out) {
-  reduce_grad_body(in, n_uses, gpw, gbpt, ptb, P, blockIdx.x / P, blockIdx.x % P, out);
+    k_reduce_grad(const double *__restrict__ in, int n_uses, int waves_per_tile, const int32_t *__restrict__ ptb, int P,
+                  double *__restrict__ out) {
+  reduce_grad_body(in, n_uses, waves_per_tile, ptb, P, out);
 }
 
 __global__ void __launch_bounds__(256) k_use_reduce_multi(const SmallDesc *__restrict__ descs) {
-  const SmallDesc &d = descs[blockIdx.y];
+  const SmallDesc &d = descs[blockIdx.z];
   const int P = d.L.n_parts;
-  if (static_cast<int>(blockIdx.x) >= d.n_uses * P) return;
-  reduce_grad_body(d.grad_partials, d.n_uses, d.gpw, d.gbpt, d.part_tile_begin, P, blockIdx.x / P,
-                   blockIdx.x % P, d.use_sums);
+  if (static_cast<int>(blockIdx.x) * 64 >= d.n_uses || static_cast<int>(blockIdx.y) >= P * GRAD_SLICES) return;
+  reduce_grad_body(d.grad_partials, d.n_uses, d.gwpt, d.part_tile_begin, P, d.use_sums);
 }
 
 __global__ void __launch_bounds__(256) k_mixture_multi(const SmallDesc *__restrict__ descs,
@@ -3328,20 +3385,11 @@ __global__ void __launch_bounds__(256) k_mixture_multi(const SmallDesc *__restri
                d.beta, d.res, rl);
 }
 
-__global__ void k_grad_total_multi(const SmallDesc *__restrict__ descs) {
+__global__ void __launch_bounds__(256) k_grad_total_multi(const SmallDesc *__restrict__ descs) {
   const SmallDesc &d = descs[blockIdx.y];
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= d.L.n_edges) return;
-  const int P = d.L.n_parts;
-  double tot = 0.0;
-  for (int p = 0; p < P; ++p) {
-    double s = 0.0;
-    for (int i = d.edge_use_begin[e]; i < d.edge_use_begin[e + 1]; ++i)
-      s += d.use_sums[static_cast<size_t>(d.edge_use_list[i]) * P + p];
-    d.res[d.rl_part_dbrlen + p * d.L.n_edges + e] = s;
-    tot += s;
-  }
-  d.res[d.rl_dbrlen + e] = tot;
+  if (static_cast<int>(blockIdx.x) >= d.L.n_edges) return;
+  grad_total_body(d.L.n_edges, d.L.n_parts, d.edge_use_begin, d.edge_use_list, d.use_sums, d.res + d.rl_part_dbrlen,
+                  d.res + d.rl_dbrlen);
 }
 
 // Copies every network's result block next to each other for one D2H copy.
@@ -3443,15 +3491,21 @@ void launch_forward_walk(Engine &e, const DevOp *ops, int n_ops) {
 
 void launch_mixture(Engine &e, int variant, int pw) {
   const int nr = static_cast<int>(e.root_slots.size());
-  hipLaunchKernelGGL(k_reduce_segments, dim3(nr * e.P), dim3(256), 0, e.stream,
-                     e.d_root_partials.as<double>(), static_cast<size_t>(e.L.n_tiles) * pw, pw,
-                     e.d_part_tile_begin.as<int32_t>(), e.P, e.d_root_sums.as<double>());
-  NRX_HIP(hipGetLastError());
+  // root sums of few partials are formed by the mixture's workgroup, which
+  // saves a launch (4.8 us with the gap); it adds about 500 partials per us
+  const int64_t n_wt = static_cast<int64_t>(e.L.n_tiles) * pw;
+  const bool fused = nr * n_wt <= MIX_PARTIALS;
+  if (!fused) {
+    hipLaunchKernelGGL(k_reduce_segments, dim3(nr * e.P), dim3(256), 0, e.stream, e.d_root_partials.as<double>(),
+                       static_cast<size_t>(n_wt), pw, e.d_part_tile_begin.as<int32_t>(), e.P,
+                       e.d_root_sums.as<double>());
+    NRX_HIP(hipGetLastError());
+  }
   hipLaunchKernelGGL(k_mixture, dim3(1), dim3(256), sizeof(double) * MIX_LDS_DOUBLES, e.stream, e.L, nr,
                      static_cast<int>(e.dag.classes.size()), e.R, variant,
                      e.d_classes.as<DevClass>(), e.d_class_dlogprob.as<double>(),
-                     e.d_root_sums.as<double>(), e.d_beta.as<double>(), e.d_result.as<double>(),
-                     e.rl);
+                     e.d_root_sums.as<double>(), e.d_beta.as<double>(), e.d_result.as<double>(), e.rl,
+                     fused ? e.d_root_partials.as<double>() : nullptr, pw, e.d_part_tile_begin.as<int32_t>());
   NRX_HIP(hipGetLastError());
 }
 
@@ -3490,16 +3544,14 @@ void launch_adjoint_walk(Engine &e, const DevOp *ops, int n_ops, bool model) {
 }
 
 void launch_grad_reduce(Engine &e) {
-  hipLaunchKernelGGL(k_reduce_grad, dim3(e.n_uses * e.P), dim3(256), 0, e.stream, e.d_grad_partials.as<double>(),
-                     e.n_uses, e.gpw, e.gbpt, e.d_part_tile_begin.as<int32_t>(), e.P, e.d_use_sums.as<double>());
+  hipLaunchKernelGGL(k_reduce_grad, dim3((e.n_uses + 63) / 64, e.P * GRAD_SLICES), dim3(256), 0, e.stream,
+                     e.d_grad_partials.as<double>(), e.n_uses, e.gwpt, e.d_part_tile_begin.as<int32_t>(), e.P,
+                     e.d_use_sums.as<double>());
   NRX_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_grad_total, dim3((e.E + 255) / 256), dim3(256), 0, e.stream, e.L,
-                     e.d_edge_use_begin.as<int32_t>(), e.d_edge_use_list.as<int32_t>(),
-                     e.d_use_sums.as<double>(), e.d_result.as<double>(), e.rl);
+  hipLaunchKernelGGL(k_grad_total, dim3(e.E), dim3(256), 0, e.stream, e.E, e.P, e.d_edge_use_begin.as<int32_t>(),
+                     e.d_edge_use_list.as<int32_t>(), e.d_use_sums.as<double>(), e.d_result.as<double>(), e.rl);
   NRX_HIP(hipGetLastError());
 }
-
-
 
 // Shapes of the 4-state FP32 walks: C categories, one or two row blocks.
 template <typename F>
@@ -3712,11 +3764,10 @@ void launch_mixture_multi(hipStream_t s, const SmallDesc *d, int n, int variant)
   NRX_HIP(hipGetLastError());
 }
 
-void launch_grad_reduce_multi(hipStream_t s, const SmallDesc *d, int n, int max_rows,
-                              int max_edges) {
-  hipLaunchKernelGGL(k_use_reduce_multi, dim3(max_rows, n), dim3(256), 0, s, d);
+void launch_grad_reduce_multi(hipStream_t s, const SmallDesc *d, int n, int max_uses, int max_parts, int max_edges) {
+  hipLaunchKernelGGL(k_use_reduce_multi, dim3((max_uses + 63) / 64, max_parts * GRAD_SLICES, n), dim3(256), 0, s, d);
   NRX_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_grad_total_multi, dim3((max_edges + 255) / 256, n), dim3(256), 0, s, d);
+  hipLaunchKernelGGL(k_grad_total_multi, dim3(max_edges, n), dim3(256), 0, s, d);
   NRX_HIP(hipGetLastError());
 }
 
