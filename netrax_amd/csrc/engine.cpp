@@ -106,7 +106,6 @@ Engine::~Engine() {
   if (h_stage) (void)hipHostFree(h_stage);
   if (h_result) (void)hipHostFree(h_result);
   if (h_brlen) (void)hipHostFree(h_brlen);
-  if (ev_brlen) (void)hipEventDestroy(ev_brlen);
   if (ev_begin) (void)hipEventDestroy(ev_begin);
   if (ev_end) (void)hipEventDestroy(ev_end);
   for (auto &v : ev_k)
@@ -603,15 +602,10 @@ static void upload_models(Engine &e) {
   upload(e.d_freqs, fr, e.stream);
 }
 
-// P matrices for changed edges / models; marks dependent CLVs invalid.
-// Branch lengths to the device through the engine's pinned staging buffer,
-// asynchronously on stream s (no host round trip per evaluation).  The
-// buffer is rewritten only once the previous copy out of it has finished.
-static void upload_brlen(Engine &e, hipStream_t s) {
-  NRX_HIP(hipEventSynchronize(e.ev_brlen));
+// Branch lengths to the pinned copy that the next launch of the P kernels reads.
+static void stage_brlen(Engine &e) {
+  if (e.brlen_in_flight) stream_sync(e);
   std::copy(e.brlen.begin(), e.brlen.end(), e.h_brlen);
-  NRX_HIP(hipMemcpyAsync(e.d_brlen.p, e.h_brlen, sizeof(double) * e.E, hipMemcpyHostToDevice, s));
-  NRX_HIP(hipEventRecord(e.ev_brlen, s));
 }
 
 // Host side of a P-matrix update: marks the CLVs the changed edges and
@@ -624,7 +618,7 @@ static bool stage_pmatrices(Engine &e, bool do_update) {
   mark_clv_dirty_for_edges(e);
   if (!do_update) return false;
   if (e.model_dirty) upload_models(e);
-  upload_brlen(e, e.stream);
+  stage_brlen(e);
   e.model_dirty = false;
   std::fill(e.edge_dirty.begin(), e.edge_dirty.end(), 0);
   return true;
@@ -632,6 +626,7 @@ static bool stage_pmatrices(Engine &e, bool do_update) {
 
 static void enqueue_pmatrices(Engine &e) {
   launch_pmatrices(e);
+  e.brlen_in_flight = true;
 }
 
 static void record_kernel_begin(Engine &e, int kind) {
@@ -657,6 +652,7 @@ static void record_kernel_end(Engine &e, int kind) {
 // staging memory has then been read, so the staging starts over.
 static void stream_sync(Engine &e) {
   NRX_HIP(hipStreamSynchronize(e.stream));
+  e.brlen_in_flight = false;
   e.h_stage_off = 0;
 }
 
@@ -737,10 +733,16 @@ static void end_timing(Engine &e) {
   e.last_timing = t;
 }
 
-static void fetch_results(Engine &e) {
-  NRX_HIP(hipMemcpyAsync(e.h_result, e.d_result.p, sizeof(double) * e.rl.size,
-                         hipMemcpyDeviceToHost, e.stream));
-  stream_sync(e);
+// Results of up to this many doubles are written into host memory by the
+// kernels that form them (a copy after them costs a small evaluation a tenth of
+// its time); larger blocks are copied.
+constexpr int HOST_RESULTS = 16384;
+static double *host_results(const Engine &e, bool fetch) {
+  return fetch && e.rl.size <= HOST_RESULTS ? e.h_result_dev : nullptr;
+}
+static void copy_results(Engine &e) {
+  if (e.rl.size > HOST_RESULTS)
+    NRX_HIP(hipMemcpyAsync(e.h_result, e.d_result.p, sizeof(double) * e.rl.size, hipMemcpyDeviceToHost, e.stream));
 }
 
 // Reverse sweep of chunks c_hi down to c_lo (FP64 form), one launch.
@@ -844,6 +846,9 @@ static int evaluate(Engine &e, int variant, bool incremental, bool update_pm, bo
     end_timing(e);
     return NRX_OK;  // nothing changed since the last evaluation
   }
+  // (a graph always hands its results on)
+  const bool graphed = e.opt.precision == NRX_FP32 && e.opt.use_graph;
+  double *host = host_results(e, fetch || graphed);
   bool results_copied = false;
   if (e.opt.precision == NRX_FP32) {
     // batched form: the op list in one persistent launch, root site sums
@@ -854,7 +859,7 @@ static int evaluate(Engine &e, int variant, bool incremental, bool update_pm, bo
     const NetDesc *inc = nullptr;
     const int n_inc = incremental ? stage_invalid_walk(e, inc) : -1;
     const bool partial = n_inc >= 0;
-    auto enqueue = [&e, aa32, variant, gradient, pm_in_graph, inc, n_inc](bool timed) {
+    auto enqueue = [&e, aa32, variant, gradient, pm_in_graph, inc, n_inc, host](bool timed) {
       if (pm_in_graph) enqueue_pmatrices(e);
       if (timed) record_kernel_begin(e, 0);
       if (n_inc == 0) {
@@ -865,7 +870,7 @@ static int evaluate(Engine &e, int variant, bool incremental, bool update_pm, bo
         launch_forward_persistent(e, inc);
       }
       if (timed) record_kernel_end(e, 0);
-      launch_mixture(e, variant, e.rpw);
+      launch_mixture(e, variant, e.rpw, host);
       if (gradient) {
         if (timed) record_kernel_begin(e, 1);
         if (aa32)
@@ -873,7 +878,7 @@ static int evaluate(Engine &e, int variant, bool incremental, bool update_pm, bo
         else
           launch_adjoint_persistent(e);
         if (timed) record_kernel_end(e, 1);
-        launch_grad_reduce(e);
+        launch_grad_reduce(e, host);
       }
     };
     if (e.opt.use_graph && !partial) {
@@ -886,10 +891,9 @@ static int evaluate(Engine &e, int variant, bool incremental, bool update_pm, bo
       if (!ge)
         ge = capture_graph(e.stream, [&]() {
           enqueue(false);
-          // the result block comes back inside the graph (a copy node)
-          NRX_HIP(hipMemcpyAsync(e.h_result, e.d_result.p, sizeof(double) * e.rl.size, hipMemcpyDeviceToHost,
-                                 e.stream));
+          copy_results(e);
         });
+      e.brlen_in_flight |= pm_in_graph;
       NRX_HIP(hipGraphLaunch(ge, e.stream));
       results_copied = true;
     } else {
@@ -899,19 +903,19 @@ static int evaluate(Engine &e, int variant, bool incremental, bool update_pm, bo
   } else if (e.bp.n_seg > 1) {
     // memory budget: segments forward, then the reverse sweep recomputing
     budget_forward(e);
-    launch_mixture(e, variant, e.rpw);
+    launch_mixture(e, variant, e.rpw, host);
     if (gradient) {
       budget_adjoint(e);
-      launch_grad_reduce(e);
+      launch_grad_reduce(e, host);
     }
     std::fill(e.clv_dirty.begin(), e.clv_dirty.end(), 0);
   } else {
     forward(e, incremental);
-    launch_mixture(e, variant, e.rpw);
+    launch_mixture(e, variant, e.rpw, host);
     if (gradient) {
       e.d_adj.alloc(sizeof(double) * e.clv_elems_per_slot * e.dag.var.size());
       adjoint_chunks(e, static_cast<int>(e.chunks.size()) - 1, 0, e.d_ops_adj.as<DevOp>(), model);
-      launch_grad_reduce(e);
+      launch_grad_reduce(e, host);
       if (model) enqueue_model_grad(e);
     }
   }
@@ -921,10 +925,8 @@ static int evaluate(Engine &e, int variant, bool incremental, bool update_pm, bo
     e.cache_valid = false;
     return NRX_OK;
   }
-  if (results_copied)
-    stream_sync(e);
-  else
-    fetch_results(e);
+  if (!results_copied) copy_results(e);
+  stream_sync(e);
   e.probs_dirty = false;
   e.cache_valid = true;
   e.cache_variant = variant;
@@ -1111,8 +1113,8 @@ struct Batch {
   std::vector<int> versions;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  DevBuf d_nets, d_work, d_small, d_offsets, d_out;
-  double *h_out = nullptr;
+  DevBuf d_nets, d_work, d_small, d_offsets;
+  double *h_out = nullptr, *h_out_dev = nullptr;  // pinned, and its device address
   std::vector<int64_t> offsets;
   int n_work = 0, C = 0, max_pm = 0, max_root_rows = 0, max_uses = 0, max_parts = 0, max_edges = 0,
       max_res = 0;
@@ -1138,6 +1140,7 @@ static SmallDesc make_smalldesc(const Engine &e) {
   d.Vinv = e.d_Vinv.as<double>();
   d.ev = e.d_eval.as<double>();
   d.rates = e.d_rates.as<double>();
+  d.host_brlen = e.h_brlen_dev;
   d.brlen = e.d_brlen.as<double>();
   d.P = e.d_P.as<double>();
   d.dP = e.d_dP.as<double>();
@@ -1169,7 +1172,7 @@ static SmallDesc make_smalldesc(const Engine &e) {
   d.rl_dprob = e.rl.dprob;
   d.pw = e.rpw;
   d.gwpt = e.gwpt;
-  const void *need[] = {d.V, d.Vinv, d.ev, d.rates, d.brlen, d.P, d.dP, d.d2P, d.Pf, d.PfT,
+  const void *need[] = {d.V, d.Vinv, d.ev, d.rates, d.host_brlen, d.brlen, d.P, d.dP, d.d2P, d.Pf, d.PfT,
                         d.part_tile_begin, d.classes, d.class_dlogprob, d.root_partials,
                         d.root_sums, d.grad_partials, d.use_sums, d.beta, d.edge_use_begin,
                         d.edge_use_list, d.res};
@@ -1252,10 +1255,10 @@ static void build_batch(Batch &b) {
   upload(b.d_small, small, b.stream);
   upload(b.d_work, work, b.stream);
   upload(b.d_offsets, b.offsets, b.stream);
-  b.d_out.alloc(sizeof(double) * b.offsets[n]);
   if (b.h_out) NRX_HIP(hipHostFree(b.h_out));
   NRX_HIP(hipHostMalloc(reinterpret_cast<void **>(&b.h_out), sizeof(double) * b.offsets[n],
                         hipHostMallocDefault));
+  NRX_HIP(hipHostGetDevicePointer(reinterpret_cast<void **>(&b.h_out_dev), b.h_out, 0));
 }
 
 }  // namespace nrx
@@ -1316,12 +1319,18 @@ int nrx_batch_evaluate(nrx_batch *batch, int32_t variant, double *lnl, double *d
       check_ready(e);
       // models and branch lengths of every engine, as update_pmatrices does
       if (e.model_dirty) upload_models(e);
-      upload_brlen(e, b.stream);  // ordered before the batch's kernels
+      stage_brlen(e);
       e.model_dirty = false;
       std::fill(e.edge_dirty.begin(), e.edge_dirty.end(), 0);
       rebuild |= b.versions[i] != e.schedule_version;
     }
     if (rebuild) build_batch(b);
+    // the batch's kernels read the engines' pinned lengths: they have ended
+    // whichever way this call ends
+    struct Drain {
+      hipStream_t s;
+      ~Drain() { (void)hipStreamSynchronize(s); }
+    } drain{b.stream};
     const bool grad = dbrlen != nullptr;
     auto enqueue = [&]() {
       const SmallDesc *sd = b.d_small.as<SmallDesc>();
@@ -1335,8 +1344,7 @@ int nrx_batch_evaluate(nrx_batch *batch, int32_t variant, double *lnl, double *d
                                         b.d_work.as<WorkItem>(), b.n_work, b.adj_slots);
         launch_grad_reduce_multi(b.stream, sd, n, b.max_uses, b.max_parts, b.max_edges);
       }
-      launch_gather_results(b.stream, sd, n, b.d_offsets.as<int64_t>(), b.d_out.as<double>(),
-                            b.max_res);
+      launch_gather_results(b.stream, sd, n, b.d_offsets.as<int64_t>(), b.h_out_dev, b.max_res);
     };
     hipGraphExec_t *ge = nullptr;
     if (b.use_graph) {
@@ -1349,8 +1357,6 @@ int nrx_batch_evaluate(nrx_batch *batch, int32_t variant, double *lnl, double *d
     else
       enqueue();
     NRX_HIP(hipEventRecord(b.ev1, b.stream));
-    NRX_HIP(hipMemcpyAsync(b.h_out, b.d_out.p, sizeof(double) * b.offsets[n],
-                           hipMemcpyDeviceToHost, b.stream));
     NRX_HIP(hipStreamSynchronize(b.stream));
     if (device_ms) {
       float ms = 0.f;
@@ -1481,7 +1487,6 @@ int nrx_create(const nrx_network_desc *net, const nrx_partition_desc *parts, int
     NRX_HIP(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
     NRX_HIP(hipEventCreate(&e->ev_begin));
     NRX_HIP(hipEventCreate(&e->ev_end));
-    NRX_HIP(hipEventCreateWithFlags(&e->ev_brlen, hipEventDisableTiming));
 
     // tips, weights, tile -> partition
     const int64_t n = L.n_sites_pad;
@@ -1535,6 +1540,7 @@ int nrx_create(const nrx_network_desc *net, const nrx_partition_desc *parts, int
     e->d_brlen.alloc(sizeof(double) * e->E);
     NRX_HIP(hipHostMalloc(reinterpret_cast<void **>(&e->h_brlen), sizeof(double) * std::max(1, e->E),
                           hipHostMallocDefault));
+    NRX_HIP(hipHostGetDevicePointer(reinterpret_cast<void **>(&e->h_brlen_dev), e->h_brlen, 0));
     e->d_Qd.alloc(sizeof(double) * ss * e->C);
     if (e->opt.precision == NRX_FP32) e->d_Qf.alloc(sizeof(float) * ss * e->C);
     const size_t pm = static_cast<size_t>(n_parts) * e->E * e->C * e->S * e->S;
@@ -1582,6 +1588,7 @@ int nrx_create(const nrx_network_desc *net, const nrx_partition_desc *parts, int
     e->d_result.alloc(sizeof(double) * rl.size);
     NRX_HIP(hipHostMalloc(reinterpret_cast<void **>(&e->h_result), sizeof(double) * rl.size,
                           hipHostMallocDefault));
+    NRX_HIP(hipHostGetDevicePointer(reinterpret_cast<void **>(&e->h_result_dev), e->h_result, 0));
 
     e->brlen.assign(e->E, 0.1);
     e->probs.assign(e->R, 0.5);

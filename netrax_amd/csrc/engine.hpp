@@ -216,7 +216,8 @@ struct WorkItem {
 struct SmallDesc {
   DevLayout L;
   // P matrices
-  const double *V, *Vinv, *ev, *rates, *brlen;
+  const double *V, *Vinv, *ev, *rates, *host_brlen;  // lengths: pinned host memory
+  double *brlen;
   double *P, *dP, *d2P;
   float *Pf, *PfT;
   // reductions and mixture
@@ -282,11 +283,12 @@ void launch_pmatrices(Engine &e);
 // FP64: ops in an order with children first, with their LDS slots
 // assigned (assign_forward_slots); root site sums and seed factors included
 void launch_forward_walk(Engine &e, const DevOp *ops, int n_ops);
-void launch_mixture(Engine &e, int variant, int partials_per_tile);
+// host: pinned memory that the results go to as well, or null
+void launch_mixture(Engine &e, int variant, int partials_per_tile, double *host);
 // FP64: the ops backwards (slots from assign_reverse_slots); model: with the
 // model gradient's sums per use and root (d_mg_g, d_mg_r; 4 states)
 void launch_adjoint_walk(Engine &e, const DevOp *ops, int n_ops, bool model);
-void launch_grad_reduce(Engine &e);
+void launch_grad_reduce(Engine &e, double *host);
 // nets: a descriptor other than the engine's own (its invalid ops only)
 void launch_forward_persistent(Engine &e, const NetDesc *nets = nullptr);
 void launch_adjoint_persistent(Engine &e);

@@ -157,8 +157,11 @@ struct Engine : nrx_engine {
   DevBuf d_site_seed;  // plain form: adjoint seed factor w / (C Ltilde) [root][site]
   DevBuf d_result;
   double *h_result = nullptr;  // pinned
-  double *h_brlen = nullptr;   // pinned staging of the branch lengths
-  hipEvent_t ev_brlen = nullptr;  // the last copy out of h_brlen
+  double *h_result_dev = nullptr;  // its device address
+  // branch lengths as the P kernels read them: pinned, with its device address;
+  // in flight from a launch to the next wait for the stream
+  double *h_brlen = nullptr, *h_brlen_dev = nullptr;
+  bool brlen_in_flight = false;
   ResultLayout rl{};
   size_t clv_elems_per_slot = 0;  // n_sites_pad * C * S
 

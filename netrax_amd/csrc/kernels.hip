@@ -340,8 +340,8 @@ __device__ __forceinline__ int aa_place32(int i, int k) {
 // product from the same eigendecomposition).
 __global__ void k_pmatrices(DevLayout L, const double *__restrict__ V,
                             const double *__restrict__ Vinv, const double *__restrict__ ev,
-                            const double *__restrict__ rates, const double *__restrict__ brlen,
-                            double *__restrict__ P, double *__restrict__ dP,
+                            const double *__restrict__ rates, const double *__restrict__ in_brlen,
+                            double *__restrict__ brlen, double *__restrict__ P, double *__restrict__ dP,
                             double *__restrict__ d2P, float *__restrict__ Pf,
                             float *__restrict__ PfT, double *__restrict__ PA, float *__restrict__ Pa) {
   const int S = L.S, C = L.C;
@@ -354,7 +354,8 @@ __global__ void k_pmatrices(DevLayout L, const double *__restrict__ V,
   const int e = (idx / (S * S * C)) % L.n_edges;
   const int p = idx / (static_cast<int64_t>(S) * S * C * L.n_edges);
   const double rt = rates[p * C + c];
-  const double t = brlen[e];
+  const double t = in_brlen[e];
+  if (brlen && p == 0 && idx % (C * S * S) == 0) brlen[e] = t;
   const double *Vp = V + static_cast<size_t>(p) * S * S;
   const double *Wp = Vinv + static_cast<size_t>(p) * S * S;
   const double *lp = ev + static_cast<size_t>(p) * S;
@@ -404,8 +405,13 @@ __device__ void mixture_body(const DevLayout &L, int n_root, int nc, int R, int 
                              const DevClass *__restrict__ classes,
                              const double *__restrict__ class_dlogprob,
                              const double *__restrict__ root_sums, double *__restrict__ beta,
-                             double *__restrict__ res, const ResultLayout &rl) {
+                             double *__restrict__ res, double *__restrict__ host, const ResultLayout &rl) {
   __shared__ double per_part[64];
+  // results, for the device and (unless null) straight into the host's pinned block
+  auto put = [&](int i, double v) {
+    res[i] = v;
+    if (host) host[i] = v;
+  };
   const int P = L.n_parts;  // <= 64 (checked on the host)
   const bool staged = mixture_lds_doubles(n_root, nc, R, P) <= MIX_LDS_DOUBLES;
   // class k: log-probability lp[k], root index ri[k], use flag cu[k]
@@ -439,12 +445,12 @@ __device__ void mixture_body(const DevLayout &L, int n_root, int nc, int R, int 
   // per-(root CLV, partition) tree lnL and per-class copies
   for (int idx = threadIdx.x; idx < n_root * P; idx += blockDim.x) {
     const int r = idx / P, p = idx % P;
-    res[rl.root_logl + p * n_root + r] = rs[idx];
+    put(rl.root_logl + p * n_root + r, rs[idx]);
   }
   for (int idx = threadIdx.x; idx < nc * P; idx += blockDim.x) {
     const int p = idx / nc, k = idx % nc;
     const int r = root_of(k);
-    res[rl.tree_logl + p * nc + k] = r >= 0 ? rs[r * P + p] : 0.0;
+    put(rl.tree_logl + p * nc + k, r >= 0 ? rs[r * P + p] : 0.0);
   }
   // a wave per partition, lanes over the classes
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, n_waves = blockDim.x >> 6;
@@ -483,12 +489,11 @@ __device__ void mixture_body(const DevLayout &L, int n_root, int nc, int R, int 
       for (int k = lane; k < nc; k += 64) alpha[p * nc + k] = sum > 0.0 ? alpha[p * nc + k] / sum : 0.0;
     if (lane == 0) {
       per_part[p] = variant == 1 ? best : best + log(sum);
-      res[rl.per_part + p] = per_part[p];
+      put(rl.per_part + p, per_part[p]);
     }
   }
   __syncthreads();
-  if (staged)
-    for (int idx = threadIdx.x; idx < nc * P; idx += blockDim.x) res[rl.alpha + idx] = alpha[idx];
+  for (int idx = threadIdx.x; idx < nc * P; idx += blockDim.x) put(rl.alpha + idx, alpha[idx]);
   for (int idx = threadIdx.x; idx < n_root * P; idx += blockDim.x) {
     const int p = idx / n_root, r = idx % n_root;
     double b = 0.0;
@@ -500,12 +505,12 @@ __device__ void mixture_body(const DevLayout &L, int n_root, int nc, int R, int 
     double g = 0.0;
     for (int idx = lane; idx < nc * P; idx += 64) g += alpha[idx] * cdl[static_cast<size_t>(idx % nc) * R + r];
     g = lane_sum(g);
-    if (lane == 0) res[rl.dprob + r] = g;
+    if (lane == 0) put(rl.dprob + r, g);
   }
   if (threadIdx.x == 0) {
     double tot = 0.0;
     for (int p = 0; p < P; ++p) tot += per_part[p];
-    res[rl.total] = tot;
+    put(rl.total, tot);
   }
 }
 
@@ -513,7 +518,8 @@ __global__ void __launch_bounds__(256)
     k_mixture(DevLayout L, int n_root, int nc, int R, int variant,
               const DevClass *__restrict__ classes, const double *__restrict__ class_dlogprob,
               double *__restrict__ root_sums, double *__restrict__ beta,
-              double *__restrict__ res, ResultLayout rl, const double *__restrict__ root_partials, int pw,
+              double *__restrict__ res, double *__restrict__ host, ResultLayout rl,
+              const double *__restrict__ root_partials, int pw,
               const int32_t *__restrict__ part_tile_begin) {
   if (root_partials) {
     // few partials: summed here, a wave per (root CLV, partition)
@@ -531,7 +537,7 @@ __global__ void __launch_bounds__(256)
     __threadfence_block();
     __syncthreads();
   }
-  mixture_body(L, n_root, nc, R, variant, classes, class_dlogprob, root_sums, beta, res, rl);
+  mixture_body(L, n_root, nc, R, variant, classes, class_dlogprob, root_sums, beta, res, host, rl);
 }
 
 // ------------------------------------------------ 4 states, FP64 plain form
@@ -1717,7 +1723,8 @@ __device__ void reduce_grad_body(const double *__restrict__ in, int n_uses, int 
 // partitions too.  A workgroup per edge, a wave per partition in turn.
 __device__ void grad_total_body(int n_edges, int P, const int32_t *__restrict__ edge_use_begin,
                                 const int32_t *__restrict__ edge_use_list, const double *__restrict__ use_sums,
-                                double *__restrict__ part_dbrlen, double *__restrict__ dbrlen) {
+                                double *__restrict__ part_dbrlen, double *__restrict__ dbrlen,
+                                double *__restrict__ host_part_dbrlen, double *__restrict__ host_dbrlen) {
   __shared__ double sh[64];  // P <= 64 (checked on the host)
   const int e = blockIdx.x, lane = threadIdx.x & 63;
   const int u0 = edge_use_begin[e], n = (edge_use_begin[e + 1] - u0) * GRAD_SLICES;
@@ -1729,6 +1736,7 @@ __device__ void grad_total_body(int n_edges, int P, const int32_t *__restrict__ 
     if (lane == 0) {
       sh[p] = s;
       part_dbrlen[p * n_edges + e] = s;
+      if (host_part_dbrlen) host_part_dbrlen[p * n_edges + e] = s;
     }
   }
   __syncthreads();
@@ -1736,14 +1744,16 @@ __device__ void grad_total_body(int n_edges, int P, const int32_t *__restrict__ 
     double tot = 0.0;
     for (int p = 0; p < P; ++p) tot += sh[p];
     dbrlen[e] = tot;
+    if (host_dbrlen) host_dbrlen[e] = tot;
   }
 }
 
 __global__ void __launch_bounds__(256)
     k_grad_total(int n_edges, int P, const int32_t *__restrict__ edge_use_begin,
                  const int32_t *__restrict__ edge_use_list, const double *__restrict__ use_sums,
-                 double *__restrict__ res, ResultLayout rl) {
-  grad_total_body(n_edges, P, edge_use_begin, edge_use_list, use_sums, res + rl.part_dbrlen, res + rl.dbrlen);
+                 double *__restrict__ res, double *__restrict__ host, ResultLayout rl) {
+  grad_total_body(n_edges, P, edge_use_begin, edge_use_list, use_sums, res + rl.part_dbrlen, res + rl.dbrlen,
+                  host ? host + rl.part_dbrlen : nullptr, host ? host + rl.dbrlen : nullptr);
 }
 
 // ==================================================== FP32 form, 4 states
@@ -3332,7 +3342,8 @@ __global__ void k_pmatrices_multi(const SmallDesc *__restrict__ descs) {
   const int e = (idx / (S * S * C)) % L.n_edges;
   const int p = idx / (static_cast<int64_t>(S) * S * C * L.n_edges);
   const double rt = d.rates[p * C + c];
-  const double t = d.brlen[e];
+  const double t = d.host_brlen[e];
+  if (p == 0 && idx % (C * S * S) == 0) d.brlen[e] = t;
   double a0 = 0.0, a1 = 0.0, a2 = 0.0;
   for (int k = 0; k < S; ++k) {
     const double lr = d.ev[p * S + k] * rt;
@@ -3382,14 +3393,14 @@ __global__ void __launch_bounds__(256) k_mixture_multi(const SmallDesc *__restri
   rl.part_dbrlen = d.rl_part_dbrlen;
   rl.dprob = d.rl_dprob;
   mixture_body(d.L, d.n_root, d.nc, d.R, variant, d.classes, d.class_dlogprob, d.root_sums,
-               d.beta, d.res, rl);
+               d.beta, d.res, nullptr, rl);
 }
 
 __global__ void __launch_bounds__(256) k_grad_total_multi(const SmallDesc *__restrict__ descs) {
   const SmallDesc &d = descs[blockIdx.y];
   if (static_cast<int>(blockIdx.x) >= d.L.n_edges) return;
   grad_total_body(d.L.n_edges, d.L.n_parts, d.edge_use_begin, d.edge_use_list, d.use_sums, d.res + d.rl_part_dbrlen,
-                  d.res + d.rl_dbrlen);
+                  d.res + d.rl_dbrlen, nullptr, nullptr);
 }
 
 // Copies every network's result block next to each other for one D2H copy.
@@ -3426,12 +3437,20 @@ void dispatch_sc(int S, int C, F &&f) {
 
 }  // namespace
 
+constexpr int64_t PM_DIRECT_WAVES = 4096;
 void launch_pmatrices(Engine &e) {
   const int64_t total = static_cast<int64_t>(e.P) * e.E * e.C * e.S * e.S;
   const int nb = static_cast<int>((total + 255) / 256);
+  // the kernel reads the lengths in the host's pinned memory (and leaves them
+  // in d_brlen): a copy ahead of it takes 4 us and a gap.  Every wave's read
+  // crosses the bus, so many waves get the copy.
+  const bool direct = total <= 64 * PM_DIRECT_WAVES;
+  if (!direct)
+    NRX_HIP(hipMemcpyAsync(e.d_brlen.p, e.h_brlen, sizeof(double) * e.E, hipMemcpyHostToDevice, e.stream));
   hipLaunchKernelGGL(k_pmatrices, dim3(nb), dim3(256), 0, e.stream, e.L, e.d_V.as<double>(),
                      e.d_Vinv.as<double>(), e.d_eval.as<double>(), e.d_rates.as<double>(),
-                     e.d_brlen.as<double>(), e.d_P.as<double>(), e.d_dP.as<double>(),
+                     direct ? e.h_brlen_dev : e.d_brlen.as<double>(), direct ? e.d_brlen.as<double>() : nullptr,
+                     e.d_P.as<double>(), e.d_dP.as<double>(),
                      e.d_d2P.as<double>(), e.d_Pf.as<float>(), e.d_PfT.as<float>(), e.d_PA.as<double>(),
                      e.d_Pa.as<float>());
   NRX_HIP(hipGetLastError());
@@ -3489,7 +3508,7 @@ void launch_forward_walk(Engine &e, const DevOp *ops, int n_ops) {
   NRX_HIP(hipGetLastError());
 }
 
-void launch_mixture(Engine &e, int variant, int pw) {
+void launch_mixture(Engine &e, int variant, int pw, double *host) {
   const int nr = static_cast<int>(e.root_slots.size());
   // root sums of few partials are formed by the mixture's workgroup, which
   // saves a launch (4.8 us with the gap); it adds about 500 partials per us
@@ -3504,7 +3523,7 @@ void launch_mixture(Engine &e, int variant, int pw) {
   hipLaunchKernelGGL(k_mixture, dim3(1), dim3(256), sizeof(double) * MIX_LDS_DOUBLES, e.stream, e.L, nr,
                      static_cast<int>(e.dag.classes.size()), e.R, variant,
                      e.d_classes.as<DevClass>(), e.d_class_dlogprob.as<double>(),
-                     e.d_root_sums.as<double>(), e.d_beta.as<double>(), e.d_result.as<double>(), e.rl,
+                     e.d_root_sums.as<double>(), e.d_beta.as<double>(), e.d_result.as<double>(), host, e.rl,
                      fused ? e.d_root_partials.as<double>() : nullptr, pw, e.d_part_tile_begin.as<int32_t>());
   NRX_HIP(hipGetLastError());
 }
@@ -3543,13 +3562,13 @@ void launch_adjoint_walk(Engine &e, const DevOp *ops, int n_ops, bool model) {
   NRX_HIP(hipGetLastError());
 }
 
-void launch_grad_reduce(Engine &e) {
+void launch_grad_reduce(Engine &e, double *host) {
   hipLaunchKernelGGL(k_reduce_grad, dim3((e.n_uses + 63) / 64, e.P * GRAD_SLICES), dim3(256), 0, e.stream,
                      e.d_grad_partials.as<double>(), e.n_uses, e.gwpt, e.d_part_tile_begin.as<int32_t>(), e.P,
                      e.d_use_sums.as<double>());
   NRX_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_grad_total, dim3(e.E), dim3(256), 0, e.stream, e.E, e.P, e.d_edge_use_begin.as<int32_t>(),
-                     e.d_edge_use_list.as<int32_t>(), e.d_use_sums.as<double>(), e.d_result.as<double>(), e.rl);
+                     e.d_edge_use_list.as<int32_t>(), e.d_use_sums.as<double>(), e.d_result.as<double>(), host, e.rl);
   NRX_HIP(hipGetLastError());
 }
 
