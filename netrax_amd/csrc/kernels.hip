@@ -235,22 +235,12 @@ __device__ __forceinline__ double block_sum(double v, double *sh) {
 //              holds all categories of 16 / C sites (8 categories: half the
 //              categories of 4 sites, two granules in turn).
 //   20 states  [16-site block][category][state 20][site 16]
-// Sumtables are kept in state pairs, each pair of a wave's 64 rows contiguous:
-//   4 states   [64 rows][pair 2][row 64][2]
-//   20 states  [64 sites][category][pair 10][site 64][2]
+// Sumtables of 4 states have the same order, of 20 states they are kept in
+// pairs: [64 sites][category][pair 10][site 64][2].
 // A row kept whole (32 or 160 bytes) would make every access of a wave touch
 // the lines of all its 64 rows and use 16 bytes of each.
 constexpr int PAIR_STRIDE = 128;  // doubles between a row's state pairs
 constexpr int STATE_STRIDE = 16;  // doubles between a CLV row's entries
-template <int S, int C>
-__device__ __forceinline__ size_t pair_offset(int64_t site, int c) {
-  if constexpr (S == 4) {
-    const int64_t r = site * C + c;
-    return static_cast<size_t>((r >> 6) * (2 * PAIR_STRIDE) + (r & 63) * 2);
-  } else {
-    return static_cast<size_t>(((site >> 6) * C + c) * (S / 2 * PAIR_STRIDE) + (site & 63) * 2);
-  }
-}
 template <int S, int C>
 __device__ __forceinline__ size_t row_offset(int64_t site, int c) {
   if constexpr (S != 4) {
@@ -265,26 +255,36 @@ __device__ __forceinline__ size_t row_offset(int64_t site, int c) {
 }
 
 template <int S>
-__device__ __forceinline__ void load_pairs(const double *__restrict__ p, double (&x)[S]) {
-#pragma unroll
-  for (int i = 0; i < S / 2; ++i) {
-    const double2 v = *reinterpret_cast<const double2 *>(p + i * PAIR_STRIDE);
-    x[2 * i] = v.x;
-    x[2 * i + 1] = v.y;
-  }
-}
-
-template <int S>
-__device__ __forceinline__ void store_pairs(double *__restrict__ p, const double (&x)[S]) {
-#pragma unroll
-  for (int i = 0; i < S / 2; ++i)
-    *reinterpret_cast<double2 *>(p + i * PAIR_STRIDE) = make_double2(x[2 * i], x[2 * i + 1]);
-}
-
-template <int S>
 __device__ __forceinline__ void load_clv(const double *__restrict__ p, double (&x)[S]) {
 #pragma unroll
   for (int i = 0; i < S; ++i) x[i] = p[i * STATE_STRIDE];
+}
+
+// a sumtable row of (site, category)
+template <int S, int C>
+__device__ __forceinline__ size_t st_offset(int64_t site, int c) {
+  if constexpr (S == 4)
+    return row_offset<S, C>(site, c);
+  else
+    return static_cast<size_t>(((site >> 6) * C + c) * (S / 2 * PAIR_STRIDE) + (site & 63) * 2);
+}
+template <int S>
+__device__ __forceinline__ void load_st(const double *__restrict__ p, double (&x)[S]) {
+  if constexpr (S == 4) {
+    load_clv<S>(p, x);
+  } else {
+#pragma unroll
+    for (int i = 0; i < S / 2; ++i) {
+      const double2 v = *reinterpret_cast<const double2 *>(p + i * PAIR_STRIDE);
+      x[2 * i] = v.x;
+      x[2 * i + 1] = v.y;
+    }
+  }
+}
+template <int S>
+__device__ __forceinline__ void store_st(double *__restrict__ p, const double (&x)[S]) {
+#pragma unroll
+  for (int i = 0; i < S; ++i) p[S == 4 ? i * STATE_STRIDE : i / 2 * PAIR_STRIDE + i % 2] = x[i];
 }
 
 template <int S>
@@ -2903,6 +2903,108 @@ __device__ __forceinline__ void path_sumtable(const PathStep *__restrict__ steps
   }
 }
 
+// The same on the matrix cores, for 4 states in FP64 (see k_forward_walk for
+// the granules): a wave walks one path for its four granules, a step being
+// y = P_sib x_sib, z = a F y, a' = P_child^T z.  Bound: the siblings' rows
+// through L2 (16 paths, 41,345 patterns: 68 us, 116 with a thread per row and
+// P in LDS, 32 reads of it per row and step).
+constexpr int PATH_BATCH = 4;  // steps whose loads are issued together
+template <int C>
+__device__ __forceinline__ void path_sumtable4(const PathStep *__restrict__ steps_, int n_steps, const DevLayout &L,
+                                               int part, int64_t site0, const double *__restrict__ clv_,
+                                               const int32_t *__restrict__ scl_, const uint8_t *__restrict__ tips_,
+                                               const double *__restrict__ P_, const double *__restrict__ V,
+                                               const double *__restrict__ Vinv, const double *__restrict__ freqs,
+                                               double *__restrict__ st_) {
+  constexpr int NQ = 4;
+  using W = Quad<C, NQ>;
+  constexpr int NA = W::NA, SPW = W::SPW;
+  const CAS PathStep *steps = to_constant(steps_);
+  const int lane = threadIdx.x & 63, state = lane >> 4;
+  const uint64_t n = L.n_sites_pad, row = n * (C * 4);
+  const GAS double *clv = to_global(clv_) + site0 * (C * 4);
+  const GAS int32_t *scl = to_global(scl_) + site0;
+  const GAS uint8_t *tips = to_global(tips_) + site0;
+  const GAS double *P = to_global(P_) + static_cast<int64_t>(part) * L.n_edges * (C * 16);
+  const uint32_t off = lane * 8, soff = (lane % SPW) * 4, woff = (lane % W::NW) * 4;
+  const int tip_shift = 8 * (lane & 3) + state;
+  uint32_t aoff[NA], toff[NA];
+#pragma unroll
+  for (int h = 0; h < NA; ++h) {
+    aoff[h] = (W::cat(lane, h) * 16 + (lane & 3) * 4 + state) * 8;
+    toff[h] = (W::cat(lane, h) * 16 + state * 4 + (lane & 3)) * 8;
+  }
+  auto load_row = [&](int32_t kid, double (&x)[NQ], uint32_t &raw) {
+    if (kid < 0)
+      raw = *at(reinterpret_cast<const GAS uint32_t *>(tips + static_cast<uint32_t>(~kid) * n), woff);
+    else
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) x[q] = *at(clv + static_cast<uint32_t>(kid) * row, off + q * 512);
+  };
+  auto tip_row = [&](int32_t kid, double (&x)[NQ], uint32_t raw) {
+    if (kid < 0)
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) x[q] = tip_entry<C, NQ>(raw, q, lane, tip_shift);
+  };
+  const int32_t low = steps[n_steps - 1].child;
+  double a[NQ], xc[NQ];
+  uint32_t rawc = 0;
+  load_row(steps[0].out, a, rawc);
+  load_row(low, xc, rawc);
+  const double pi = freqs[part * 4 + state], pi_c = pi * (1.0 / C);
+  // the seed (1/C) pi_i / Ltilde at the root
+#pragma unroll
+  for (int q = 0; q < NQ; q += NA) {
+    double t = mfma4(pi_c, a[q], 0.0);
+    if constexpr (C == 8) t += mfma4(pi_c, a[q + 1], 0.0);
+    if constexpr (C >= 4) t += dpp<0x124>(t);  // row_ror:4
+    if constexpr (C >= 2) t += dpp<0x128>(t);  // row_ror:8
+#pragma unroll
+    for (int h = 0; h < NA; ++h) a[q + h] = pi / (C * t);
+  }
+  for (int s0 = 0; s0 < n_steps; s0 += PATH_BATCH) {
+    double x[PATH_BATCH][NQ], A[PATH_BATCH][NA], AT[PATH_BATCH][NA];
+    uint32_t raw[PATH_BATCH], word[PATH_BATCH];
+#pragma unroll
+    for (int u = 0; u < PATH_BATCH; ++u) {
+      if (s0 + u >= n_steps) continue;
+      const CAS PathStep &ps = steps[s0 + u];
+      word[u] = *at(scl + static_cast<uint32_t>(ps.out) * n, soff);
+#pragma unroll
+      for (int h = 0; h < NA; ++h) AT[u][h] = *at(P + static_cast<int64_t>(ps.edge_child) * (C * 16), toff[h]);
+      if (ps.nk == 2) {
+        load_row(ps.sib, x[u], raw[u]);
+#pragma unroll
+        for (int h = 0; h < NA; ++h) A[u][h] = *at(P + static_cast<int64_t>(ps.edge_sib) * (C * 16), aoff[h]);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < PATH_BATCH; ++u) {
+      if (s0 + u >= n_steps) continue;
+      const CAS PathStep &ps = steps[s0 + u];
+      const uint64_t scaled = __builtin_amdgcn_ballot_w64(lane < SPW && (word[u] & 1u));
+      if (scaled)
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+          if ((scaled >> W::site(lane, q)) & 1) a[q] *= SCALE_FACTOR;
+      if (ps.nk == 2) {
+        tip_row(ps.sib, x[u], raw[u]);
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) a[q] *= mfma4(A[u][W::half(q)], x[u][q], 0.0);
+      }
+      if (s0 + u + 1 < n_steps)
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) a[q] = mfma4(AT[u][W::half(q)], a[q], 0.0);
+    }
+  }
+  // st_k = (z^T V)_k (V^-1 x)_k
+  tip_row(low, xc, rawc);
+  const double vt = V[part * 16 + state * 4 + (lane & 3)], wi = Vinv[part * 16 + (lane & 3) * 4 + state];
+  GAS double *st = to_global(st_) + site0 * (C * 4);
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) *at(st, off + q * 512) = mfma4(vt, a[q], 0.0) * mfma4(wi, xc[q], 0.0);
+}
+
 template <int S, int C, typename T>
 __global__ void __launch_bounds__(TILE *C)
     k_sumtables(const PathStep *__restrict__ steps, const int32_t *__restrict__ path_begin,
@@ -2912,6 +3014,18 @@ __global__ void __launch_bounds__(TILE *C)
                 const double *__restrict__ P, const double *__restrict__ V,
                 const double *__restrict__ Vinv, const double *__restrict__ freqs,
                 double *__restrict__ st) {
+  if constexpr (S == 4 && std::is_same<T, double>::value) {
+    // the paths of eight tiles in turn, one tile per XCD: what they have in
+    // common (siblings' rows) is read from its L2
+    const int group = blockIdx.x / (8 * n_paths), r = blockIdx.x % (8 * n_paths);
+    const int tile = group * 8 + r % 8, path = r / 8;
+    if (tile >= L.n_tiles) return;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    path_sumtable4<C>(steps + path_begin[path], path_begin[path + 1] - path_begin[path], L, tile_part[tile],
+                      static_cast<int64_t>(tile) * TILE + wave * Quad<C, 4>::SPW, clv, scl, tips, P, V, Vinv, freqs,
+                      st + static_cast<int64_t>(path) * L.n_sites_pad * (C * 4));
+    return;
+  } else {
   double *sPp = dyn_lds<double>();
   const int tile = blockIdx.x;
   const int part = tile_part[tile];
@@ -2927,7 +3041,8 @@ __global__ void __launch_bounds__(TILE *C)
   double stv[S];
   path_sumtable<S, C, T>(steps, b0, b1, sPp, n_staged, L, part, site, c, clv, scl, scale_unit, tips, P, V, Vinv,
                          freqs, stv);
-  store_pairs<S>(st + static_cast<size_t>(j) * L.n_sites_pad * (C * S) + pair_offset<S, C>(site, c), stv);
+  store_st<S>(st + static_cast<size_t>(j) * L.n_sites_pad * (C * S) + st_offset<S, C>(site, c), stv);
+  }
 }
 
 // Per displayed tree j and wave: sums over sites of w log rho(b),
@@ -2995,7 +3110,7 @@ __global__ void __launch_bounds__(TILE *C)
   const int c = threadIdx.x % C;
   const int64_t site = static_cast<int64_t>(tile) * TILE + threadIdx.x / C;
   const int64_t n = L.n_sites_pad;
-  const size_t slot = static_cast<size_t>(n) * (C * S), ro = pair_offset<S, C>(site, c);
+  const size_t slot = static_cast<size_t>(n) * (C * S), ro = st_offset<S, C>(site, c);
   const size_t n_wt = static_cast<size_t>(L.n_tiles) * PW;
   const int wt = tile * PW + threadIdx.x / 64;
   const double w = weights[site];
@@ -3004,7 +3119,7 @@ __global__ void __launch_bounds__(TILE *C)
   // one path per workgroup (grid tiles x paths)
   for (int j = blockIdx.y; j < min(n_paths, static_cast<int>(blockIdx.y) + 1); ++j) {
     double stv[S], v[3];
-    load_pairs<S>(st + static_cast<size_t>(j) * slot + ro, stv);
+    load_st<S>(st + static_cast<size_t>(j) * slot + ro, stv);
     sumtable_partials<S, C>(stv, ex, lr, w, c, v);
     if ((threadIdx.x & 63) == 0)
 #pragma unroll
@@ -3036,7 +3151,7 @@ __global__ void __launch_bounds__(TILE *C)
   const int c = threadIdx.x % C;
   const int64_t site = static_cast<int64_t>(tile) * TILE + threadIdx.x / C;
   const int64_t n = L.n_sites_pad;
-  const size_t slot = static_cast<size_t>(n) * (C * S), ro = pair_offset<S, C>(site, c);
+  const size_t slot = static_cast<size_t>(n) * (C * S), ro = st_offset<S, C>(site, c);
   const size_t n_wt = static_cast<size_t>(L.n_tiles) * PW;
   const int wt = tile * PW + threadIdx.x / 64;
   const double w = weights[site];
@@ -3045,7 +3160,7 @@ __global__ void __launch_bounds__(TILE *C)
   // one path per workgroup (grid tiles x the largest path count)
   for (int j = blockIdx.y; j < min(n_paths, static_cast<int>(blockIdx.y) + 1); ++j) {
     double stv[S], v[3];
-    load_pairs<S>(st + static_cast<size_t>(j) * slot + ro, stv);
+    load_st<S>(st + static_cast<size_t>(j) * slot + ro, stv);
     sumtable_partials<S, C>(stv, ex, lr, w, c, v);
     if ((threadIdx.x & 63) == 0)
 #pragma unroll
@@ -3643,7 +3758,9 @@ void launch_sumtables(Engine &e, int n_paths, int max_steps) {
                          e.d_P.as<double>(), e.d_V.as<double>(), e.d_Vinv.as<double>(),
                          e.d_freqs.as<double>(), e.d_st.as<double>());
     } else {
-      hipLaunchKernelGGL((k_sumtables<S, C, double>), dim3(e.L.n_tiles, n_paths), dim3(TILE * C), lds,
+      // (4 states: see the kernel)
+      const dim3 grid = S == 4 ? dim3((e.L.n_tiles + 7) / 8 * 8 * n_paths) : dim3(e.L.n_tiles, n_paths);
+      hipLaunchKernelGGL((k_sumtables<S, C, double>), grid, dim3(TILE * C), S == 4 ? 0 : lds,
                          e.stream, e.d_steps.as<PathStep>(), e.d_path_begin.as<int32_t>(), n_paths,
                          e.L, e.d_tile_part.as<int32_t>(),
                          e.d_clv.as<double>(), e.d_scl.as<int32_t>(), 256, e.d_tips.as<TT>(),
