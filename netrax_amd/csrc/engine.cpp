@@ -1143,8 +1143,6 @@ static SmallDesc make_smalldesc(const Engine &e) {
   d.host_brlen = e.h_brlen_dev;
   d.brlen = e.d_brlen.as<double>();
   d.P = e.d_P.as<double>();
-  d.dP = e.d_dP.as<double>();
-  d.d2P = e.d_d2P.as<double>();
   d.Pf = e.d_Pf.as<float>();
   d.PfT = e.d_PfT.as<float>();
   d.n_root = static_cast<int32_t>(e.root_slots.size());
@@ -1172,7 +1170,7 @@ static SmallDesc make_smalldesc(const Engine &e) {
   d.rl_dprob = e.rl.dprob;
   d.pw = e.rpw;
   d.gwpt = e.gwpt;
-  const void *need[] = {d.V, d.Vinv, d.ev, d.rates, d.host_brlen, d.brlen, d.P, d.dP, d.d2P, d.Pf, d.PfT,
+  const void *need[] = {d.V, d.Vinv, d.ev, d.rates, d.host_brlen, d.brlen, d.P, d.Pf, d.PfT,
                         d.part_tile_begin, d.classes, d.class_dlogprob, d.root_partials,
                         d.root_sums, d.grad_partials, d.use_sums, d.beta, d.edge_use_begin,
                         d.edge_use_list, d.res};
@@ -1546,8 +1544,6 @@ int nrx_create(const nrx_network_desc *net, const nrx_partition_desc *parts, int
     const size_t pm = static_cast<size_t>(n_parts) * e->E * e->C * e->S * e->S;
     e->d_P.alloc(sizeof(double) * pm);
     if (e->S == AA_STATES && !aa32) e->d_PA.alloc(sizeof(double) * 2 * pm);
-    e->d_dP.alloc(sizeof(double) * pm);
-    e->d_d2P.alloc(sizeof(double) * pm);
     e->clv_elems_per_slot = static_cast<size_t>(n) * e->C * e->S;
     const size_t nv = e->dag.var.size();
     const size_t real_b = e->opt.precision == NRX_FP32 ? sizeof(float) : sizeof(double);

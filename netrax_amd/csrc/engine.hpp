@@ -218,7 +218,7 @@ struct SmallDesc {
   // P matrices
   const double *V, *Vinv, *ev, *rates, *host_brlen;  // lengths: pinned host memory
   double *brlen;
-  double *P, *dP, *d2P;
+  double *P;
   float *Pf, *PfT;
   // reductions and mixture
   int32_t n_root, nc, R, n_uses;

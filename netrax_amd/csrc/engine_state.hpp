@@ -141,7 +141,7 @@ struct Engine : nrx_engine {
   hipStream_t stream = nullptr;
   DevBuf d_tips, d_weights, d_tile_part, d_part_tile_begin;
   DevBuf d_V, d_Vinv, d_eval, d_rates, d_freqs, d_brlen;
-  DevBuf d_P, d_dP, d_d2P, d_Pf, d_PfT;
+  DevBuf d_P, d_Pf, d_PfT;
   DevBuf d_clv, d_scl, d_adj, d_adj_exp, d_Qf;
   DevBuf d_PA;  // 20-state FP64 form: P and P^T in operand order
   DevBuf d_Pa;  // 20-state FP32 form: likewise
