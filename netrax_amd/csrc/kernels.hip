@@ -326,12 +326,13 @@ __device__ __forceinline__ int aa_place(int i, int k) {
   return (k >> 2) * 80 + (i < 16 ? (k & 3) * 16 + i : 64 + (k & 3) * 4 + (i & 3));
 }
 
-// The same for FP32, where a step's four columns are 4 q + r (r < 4, q < 4) or
-// 16 + q: rows 0-15 as [lane 16 q + row][step r], then [lane] of the last
-// step; then rows 16-19 as [4 q + row][r] and [4 q + row].
+// The same for FP32 (see mul20 there): rows 0-15 as [lane 16 q + m][step r] of
+// column 4 r + q, then [lane] of the last step, m = 4 (i & 3) + (i >> 2); then
+// rows 16-19 as [4 q + row][r] and [4 q + row].
 __device__ __forceinline__ int aa_place32(int i, int k) {
-  const int q = k < 16 ? k >> 2 : k - 16, r = k < 16 ? k & 3 : 4;
-  const int lane = i < 16 ? 16 * q + i : 4 * q + (i - 16), base = i < 16 ? 0 : 320, lanes = i < 16 ? 64 : 16;
+  const int q = k & 3, r = k >> 2;
+  const int lane = i < 16 ? 16 * q + 4 * (i & 3) + (i >> 2) : 4 * q + (i - 16);
+  const int base = i < 16 ? 0 : 320, lanes = i < 16 ? 64 : 16;
   return base + (r < 4 ? lane * 4 + r : 4 * lanes + lane);
 }
 
@@ -2346,13 +2347,15 @@ __global__ void __launch_bounds__(WG, 3)
 
 // ==================================================== FP32 form, 20 states
 // The walks of the 20-state FP64 form in FP32: a wave holds one rate category
-// of 16 sites, lane l the states 4 q + r (r < 4) and 16 + q of site l & 15, q
-// = l >> 4.  Rows 0-15 of a product are five v_mfma_f32_16x16x4 (step r takes
-// the four states 4 q + r, the last one 16 + q; register i of D is row 4 q +
-// i); rows 16-19 are five v_mfma_f32_4x4x1, whose 16 blocks are (q, 4-site
-// group) and each sum their q's states, then summed over q and dealt out to
-// the lanes that hold them.  So no entry is padding, and a product's result
-// is the next one's operand and the stored row, [lane 64][4] then [lane 64].
+// of 16 sites, lane l the states 4 r + q (r <= 4) of site l & 15, q = l >> 4.
+// Rows 0-15 of a product are a chain of five v_mfma_f32_16x16x4, over the
+// states in order; row m = 4 a + b of it is state 4 b + a, so register b of
+// lane group a of its result is the next product's operand.  Rows 16-19 are
+// another such chain in the forward walk (its rows 0, 4, 8, 12; the others are
+// not used), 320 cycles a product in all; in the reverse walk they are five
+// v_mfma_f32_4x4x1 whose blocks sum a quarter of the states each, 230 cycles.
+// (Summed that way forward, lnL rounds differently, by 1e-9 of its value.)
+// Rows are stored as [lane 64][4] then [lane 64].
 // Tables of P and P^T in operand order come from k_pmatrices; r_c Q, the same
 // for every edge, is read once per sweep.
 //
@@ -2365,7 +2368,7 @@ struct Mat20f {
 };
 
 struct Row20f {
-  f32x4 v;  // states 4 q + r
+  f32x4 v;  // states 4 r + q
   float e;  // state 16 + q
 };
 
@@ -2406,16 +2409,20 @@ __device__ __forceinline__ void slot_store(float *slot, int lane, const Row20f &
   slot[256 + lane] = x.e;
 }
 
-// y = M x
+// y = M x.  BLOCKS: rows 16-19 in blocks (lanes hold row 16 + (l & 3) of them),
+// else in a chain (row 16 + (l & 15) / 4).
+template <bool BLOCKS>
 __device__ __forceinline__ Row20f mul20(const Mat20f &m, const Row20f &x) {
   f32x4 d = {0.f, 0.f, 0.f, 0.f}, t = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    d = __builtin_amdgcn_mfma_f32_16x16x4f32(m.big[r], x.v[r], d, 0, 0, 0);
-    t = __builtin_amdgcn_mfma_f32_4x4x1f32(m.small[r], x.v[r], t, 0, 0, 0);
+  for (int r = 0; r < 5; ++r) {
+    const float xr = r < 4 ? x.v[r & 3] : x.e, big = r < 4 ? m.big[r & 3] : m.big4;
+    const float low = r < 4 ? m.small[r & 3] : m.small4;
+    d = __builtin_amdgcn_mfma_f32_16x16x4f32(big, xr, d, 0, 0, 0);
+    t = BLOCKS ? __builtin_amdgcn_mfma_f32_4x4x1f32(low, xr, t, 0, 0, 0)
+               : __builtin_amdgcn_mfma_f32_16x16x4f32(low, xr, t, 0, 0, 0);
   }
-  d = __builtin_amdgcn_mfma_f32_16x16x4f32(m.big4, x.e, d, 0, 0, 0);
-  t = __builtin_amdgcn_mfma_f32_4x4x1f32(m.small4, x.e, t, 0, 0, 0);
+  if constexpr (!BLOCKS) return Row20f{d, t[0]};
   // t[i] of quad q: row 16 + i over q's states; quad i gets the sum over the quads
   auto add = [](auto s) { return __uint_as_float(s[0]) + __uint_as_float(s[1]); };
   const float a = add(__builtin_amdgcn_permlane32_swap(__float_as_uint(t[0]), __float_as_uint(t[2]), false, false));
@@ -2425,8 +2432,11 @@ __device__ __forceinline__ Row20f mul20(const Mat20f &m, const Row20f &x) {
 
 // A lane's entries of a tip's 0/1 vector; mask: of the lane's site.
 __device__ __forceinline__ Row20f tip20f(uint32_t mask, int quad) {
-  return Row20f{tip_row(mask >> (4 * quad)),
-                __int_as_float(-static_cast<int>((mask >> (16 + quad)) & 1u) & 0x3F800000)};
+  Row20f x;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) x.v[r] = __int_as_float(-static_cast<int>((mask >> (4 * r + quad)) & 1u) & 0x3F800000);
+  x.e = __int_as_float(-static_cast<int>((mask >> (16 + quad)) & 1u) & 0x3F800000);
+  return x;
 }
 
 __device__ __forceinline__ Row20f scale_row(const Row20f &x, int e) { return Row20f{scale4(x.v, e), ldexpf(x.e, e)}; }
@@ -2454,7 +2464,7 @@ struct FwdIn20f {
 
 // Workgroup: 16 sites, a wave per category, as k_forward_level_aa.
 // Bound: each wave's chain of ops (18,564 patterns x 4 categories, 73 ops:
-// 0.22 ms; 0.35 with 32-site waves of v_mfma_f32_32x32x2, whose 12 of 32 rows
+// 0.24 ms; 0.35 with 32-site waves of v_mfma_f32_32x32x2, whose 12 of 32 rows
 // are padding, a group of four ops at a time and every CLV through HBM).
 template <int C, int G>
 __global__ void __launch_bounds__(64 * C, 4)
@@ -2478,7 +2488,7 @@ __global__ void __launch_bounds__(64 * C, 4)
   const GAS char *tips = reinterpret_cast<const GAS char *>(to_global(nd.tips)) + site0 * 4;
   const GAS float *Pa = to_global(nd.Pa) + (static_cast<int64_t>(part) * nd.L.n_edges * C + c) * AA_MATS;
   const GAS double *freqs = to_global(nd.freqs) + part * AA_STATES;
-  const uint32_t off = lane * 16, soff = col * 4, small = (quad * 4 + (lane & 3)) * 16;
+  const uint32_t off = lane * 16, soff = col * 4, small = (quad * 4 + (col >> 2)) * 16;
 
   auto load = [&](const OpRegs &op, FwdIn20f &in) {
     const uint32_t o = opaque(off), so = opaque(soff), sm = opaque(small);
@@ -2504,7 +2514,7 @@ __global__ void __launch_bounds__(64 * C, 4)
       in.raw[k] = slot_scl[op.slot(k) * AA_SITES + col];
     }
     ks += word_k(static_cast<int32_t>(in.raw[k]));
-    return mul20(in.m[k], in.x[k]);
+    return mul20<false>(in.m[k], in.x[k]);
   };
   int turn = 0;
   auto step = [&](const OpRegs &op, FwdIn20f &in, Nothing) {
@@ -2522,7 +2532,7 @@ __global__ void __launch_bounds__(64 * C, 4)
     if (op.root() >= 0) {
       // site likelihoods Ltilde = (1/C) sum_c pi . x
 #pragma unroll
-      for (int r = 0; r < 4; ++r) like = fma(freqs[4 * quad + r], static_cast<double>(v.v[r]), like);
+      for (int r = 0; r < 4; ++r) like = fma(freqs[4 * r + quad], static_cast<double>(v.v[r]), like);
       like = fma(freqs[16 + quad], static_cast<double>(v.e), like);
       like += __shfl_xor(like, 16);
       like += __shfl_xor(like, 32);
@@ -2635,14 +2645,15 @@ __global__ void __launch_bounds__(64, 3)
   const uint32_t off = lane * 16, soff = col * 4, small = (quad * 4 + (lane & 3)) * 16;
   Mat20f Q;
   {
-    const GAS float *q = to_global(nd.Qf) + (static_cast<size_t>(part) * C + c) * AA_MAT;
+    const GAS float *q = to_global(nd.Qf) + (static_cast<size_t>(part) * C + c) * AA_MAT + quad;
+    const GAS float *big = q + (4 * (col & 3) + (col >> 2)) * AA_STATES, *low = q + (16 + (lane & 3)) * AA_STATES;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      Q.big[r] = q[col * AA_STATES + 4 * quad + r];
-      Q.small[r] = q[(16 + (lane & 3)) * AA_STATES + 4 * quad + r];
+      Q.big[r] = big[4 * r];
+      Q.small[r] = low[4 * r];
     }
-    Q.big4 = q[col * AA_STATES + 16 + quad];
-    Q.small4 = q[(16 + (lane & 3)) * AA_STATES + 16 + quad];
+    Q.big4 = big[16];
+    Q.small4 = low[16];
   }
 
   auto load = [&](const OpRegs &op, AdjIn20f &in) {
@@ -2726,7 +2737,7 @@ __global__ void __launch_bounds__(64, 3)
       if (f != 0.0) {
         const double mf = frexp(f, &ef);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) sd.v[r] = static_cast<float>(mf * freqs[4 * quad + r]);
+        for (int r = 0; r < 4; ++r) sd.v[r] = static_cast<float>(mf * freqs[4 * r + quad]);
         sd.e = static_cast<float>(mf * freqs[16 + quad]);
       }
       ez = align_add(a, ez, sd, ef);
@@ -2741,14 +2752,14 @@ __global__ void __launch_bounds__(64, 3)
     double g[2] = {0.0, 0.0};
     auto product = [&](int k) {
       if (op.kid(k) < 0) in.x[k] = tip20f(in.raw[k], quad);
-      y[k] = mul20(in.m[k], in.x[k]);
+      y[k] = mul20<true>(in.m[k], in.x[k]);
     };
     auto use = [&](int k, const Row20f &z) {
-      const Row20f d = mul20(Q, y[k]);
+      const Row20f d = mul20<true>(Q, y[k]);
       const float gd =
           fmaf(z.e, d.e, fmaf(z.v[3], d.v[3], fmaf(z.v[2], d.v[2], fmaf(z.v[1], d.v[1], z.v[0] * d.v[0]))));
       g[k] = ldexp(static_cast<double>(gd), ez);
-      if (op.kid(k) >= 0) deliver(op, k, mul20(held.mt[k], z), ez, held);
+      if (op.kid(k) >= 0) deliver(op, k, mul20<true>(held.mt[k], z), ez, held);
     };
     product(0);
     if (op.nk() == 2) {
