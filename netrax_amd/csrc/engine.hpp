@@ -122,8 +122,7 @@ constexpr int PASS_SHIFT = 12;  // slot of use u (0, 1: children, 2: own) in bit
 constexpr int32_t PASS_BITS = 0x1FF << PASS_SHIFT;
 inline __host__ __device__ int pass_slot(int32_t flags, int u) { return (flags >> (PASS_SHIFT + 3 * u)) & 7; }
 
-// Plain form: the ops [op_begin, op_end), one pruning level of 20-state data
-// (a launch), or one op of the 4-state walk (where a memory budget may cut it).
+// The ops [op_begin, op_end): one op of the walk (where a memory budget may cut it).
 struct LevelChunk {
   int level, op_begin, op_end;
 };

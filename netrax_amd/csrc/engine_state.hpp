@@ -72,8 +72,8 @@ struct Engine : nrx_engine {
   std::vector<std::vector<int>> level_ops;  // variant slots per level (needed only)
   std::vector<int> root_slots;              // distinct displayed-tree-root CLVs
   std::vector<int> class_root_index;        // [nc]
-  // ops in level order (20 states), or in the depth-first order of the
-  // 4-state walks, with their LDS slots in the two lists the walks read
+  // ops in the depth-first order of the walks, with their LDS slots in the two
+  // lists the walks read
   std::vector<DevOp> ops_all, ops_fwd, ops_adj;
   std::vector<LevelChunk> chunks;
   std::vector<int32_t> edge_use_begin, edge_use_list;  // gradient rows per edge
@@ -84,9 +84,8 @@ struct Engine : nrx_engine {
   int walk_nq = 4, fwd_slots = 4, adj_slots = 4;
   int walk_blocks = 1;  // 64-row blocks per wave (FP32)
   int gwpt = 1;  // gradient partials [wave][row]: waves per tile
-  // FP32 form shape (nrx_autotune / nrx_set_tuning): ops per group of the
-  // 20-state kernels; for 4 states see walk_blocks_of.  The other two are
-  // part of a shape's name only.
+  // FP32 form shape (nrx_autotune / nrx_set_tuning): for the first, see
+  // walk_blocks_of (4 states); the others are part of a shape's name only.
   int tune_group = 4;
   int tune_tile = TILE;
   int tune_lanes = 1;
@@ -106,7 +105,7 @@ struct Engine : nrx_engine {
   DevBuf d_nr_state, d_nr_cls;
   DevBuf d_mg_g, d_mg_r, d_mg_sums;  // model gradient: the walk's sums per use and root, and what is made of them
   // Memory budget of the FP64 form: with n_seg > 1 the CLV, adjoint and
-  // scaler rows live in n_phys physical rows.  The level chunks are cut into
+  // scaler rows live in n_phys physical rows.  The ops are cut into
   // n_seg segments; a CLV consumed in a later segment than its own keeps a
   // fixed row (the boundary rows), the others share the rows of a pool that
   // each segment reuses.  The forward pass runs the segments in order; the
@@ -146,9 +145,8 @@ struct Engine : nrx_engine {
   DevBuf d_PA;  // 20-state FP64 form: P and P^T in operand order
   DevBuf d_Pa;  // 20-state FP32 form: likewise
   DevBuf d_ops, d_ops_dirty, d_Qd;
-  DevBuf d_ops_fwd, d_ops_adj;  // 4 states: the walks' op lists
-  // FP32 form, incremental evaluation: the invalid ops, their groups (20
-  // states) and their descriptor
+  DevBuf d_ops_fwd, d_ops_adj;  // the walks' op lists
+  // FP32 form, incremental evaluation: the invalid ops and their descriptor
   DevBuf d_ops_inc, d_netdesc_inc;
   DevBuf d_edge_use_begin, d_edge_use_list;
   DevBuf d_netdesc, d_work;  // FP32 form: this engine's NetDesc and (0, tile) work table

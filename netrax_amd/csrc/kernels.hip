@@ -2,17 +2,15 @@
 //
 // Data layout in HBM (one engine):
 //   CLV arena   one row of S values per (variant, site, category): FP64 in the
-//               order of row_offset, FP32 4 states [n_sites_pad][C][4],
-//               FP32 20 states per 32-site tile (see the matrix-core kernels)
-//   scalers     int32 [n_variants][n_sites_pad]
+//               order of row_offset, FP32 in the lane order of the walks
+//               (Rows; Row20f)
+//   scalers     int32 [n_variants][n_sites_pad], words as the walks describe
 //   adjoints    as the CLVs
 //   tips        uint8 (S <= 8) or uint32 (S = 20) state masks [n_tips][n_sites_pad]
-//   P, P', P''  real  [n_parts][n_edges][C][S][S]
-// The FP64 kernels of 20 states and the path kernels work on tiles of TILE =
-// 64 sites with TILE * C threads; the 20-state launches cover (tile, op) with
-// the tile count rounded up to a multiple of 8, so a tile always goes to the
-// same XCD (round-robin over workgroup ids) and its children's CLVs stay in
-// that XCD's L2.
+//   P           real  [n_parts][n_edges][C][S][S], 20 states also in operand order
+// Forward and reverse passes are walks of one wave (20 states forward: one per
+// category) through the whole op list; the path kernels of the branch
+// derivatives work on tiles of TILE = 64 sites with TILE * C threads.
 #include <cfloat>
 #include <cmath>
 #include <map>

@@ -1,4 +1,4 @@
-// Schedules of the op DAG for the persistent FP32 kernels (see schedule.hpp).
+// Schedules of the op DAG (see schedule.hpp).
 #include "schedule.hpp"
 
 #include <algorithm>

@@ -1,6 +1,8 @@
-// Schedules of the op DAG for the persistent FP32 kernels: the grouped op
-// order and the per-op flags the reverse sweep reads (first deliveries,
-// early read-backs, LDS pass slots).  Host code only, no HIP calls, so the
+// Schedules of the op DAG: the depth-first order of the walks, the flags the
+// reverse walk reads and the LDS slots; and the level runs and groups of
+// independent ops (split_level_runs, set_acc_early, set_pass_slots,
+// build_batched_order), which no pass of the engine takes and
+// tests/schedule_check.cpp replays.  Host code only, no HIP calls, so the
 // schedules can be built and checked without a GPU.
 #pragma once
 
@@ -23,7 +25,7 @@ void set_adjoint_flags(std::vector<DevOp> &ops, const std::vector<int> &adj_orde
 void split_level_runs(std::vector<DevOp> &ops, const std::vector<LevelChunk> &chunks, std::vector<LevelChunk> &runs,
                       std::vector<int> &run_begin);
 
-// 4-state walks: every variant the roots need, children first, each
+// Walks: every variant the roots need, children first, each
 // root's subtrees depth first and the child that needs more rows at once
 // before the other, so that few rows are held at a time.
 std::vector<int> depth_first_order(const Dag &dag, const std::vector<int> &root_slots);
