@@ -834,6 +834,12 @@ static int evaluate(Engine &e, int variant, bool incremental, bool update_pm, bo
   check_ready(e);
   if (variant != NRX_AVERAGE_DISPLAYED_TREES && variant != NRX_BEST_DISPLAYED_TREE)
     throw std::invalid_argument("unknown likelihood variant");
+  if (e.ops_all.empty()) {
+    // every displayed tree falls below min_tree_logprob: there is no op to
+    // walk (the walks take at least one) and no tree to sum over
+    e.cache_valid = false;
+    return fail(NRX_ERR_NEGINF, "Invalid network likelihood: negative infinity");
+  }
   begin_timing(e);
   const bool pm = stage_pmatrices(e, update_pm);
   // an FP32 evaluation replayed from a graph runs the P kernels inside it
@@ -1246,8 +1252,10 @@ static void build_batch(Batch &b) {
                      return x.first > y.first;
                    });
   std::vector<WorkItem> work;
-  for (const auto &o : order)
+  for (const auto &o : order) {
+    if (o.first == 0) continue;  // no displayed tree counts: nothing to walk, lnL is -infinity
     for (int t = 0; t < b.engines[o.second]->L.n_tiles * b.engines[o.second]->rpw; ++t) work.push_back({o.second, t});
+  }
   b.n_work = static_cast<int>(work.size());
   upload(b.d_nets, nets, b.stream);
   upload(b.d_small, small, b.stream);

@@ -3728,6 +3728,7 @@ void launch_adjoint_persistent(Engine &e) {
 
 void launch_forward_persistent_multi(hipStream_t stream, int C, int blocks, const NetDesc *nets, const WorkItem *work,
                                      int n_work, int max_slots) {
+  if (n_work == 0) return;
   dispatch_walk32(C, blocks, [&](auto c, auto g) {
     hipLaunchKernelGGL((k_forward_persistent<decltype(c)::value, decltype(g)::value, 64>), dim3(n_work), dim3(64),
                        forward_lds32(C, blocks, max_slots), stream, nets, work);
@@ -3737,6 +3738,7 @@ void launch_forward_persistent_multi(hipStream_t stream, int C, int blocks, cons
 
 void launch_adjoint_persistent_multi(hipStream_t stream, int C, int blocks, const NetDesc *nets, const WorkItem *work,
                                      int n_work, int max_slots) {
+  if (n_work == 0) return;
   dispatch_walk32(C, blocks, [&](auto c, auto g) {
     hipLaunchKernelGGL((k_adjoint_persistent<decltype(c)::value, decltype(g)::value, 64>), dim3(n_work), dim3(64),
                        adjoint_lds32(C, blocks, max_slots), stream, nets, work);
@@ -3909,6 +3911,7 @@ void launch_pmatrices_multi(hipStream_t s, const SmallDesc *d, int n, int max_el
 }
 
 void launch_root_reduce_multi(hipStream_t s, const SmallDesc *d, int n, int max_rows) {
+  if (max_rows == 0) return;
   hipLaunchKernelGGL(k_root_reduce_multi, dim3(max_rows, n), dim3(256), 0, s, d);
   NRX_HIP(hipGetLastError());
 }
@@ -3919,8 +3922,10 @@ void launch_mixture_multi(hipStream_t s, const SmallDesc *d, int n, int variant)
 }
 
 void launch_grad_reduce_multi(hipStream_t s, const SmallDesc *d, int n, int max_uses, int max_parts, int max_edges) {
-  hipLaunchKernelGGL(k_use_reduce_multi, dim3((max_uses + 63) / 64, max_parts * GRAD_SLICES, n), dim3(256), 0, s, d);
-  NRX_HIP(hipGetLastError());
+  if (max_uses > 0) {
+    hipLaunchKernelGGL(k_use_reduce_multi, dim3((max_uses + 63) / 64, max_parts * GRAD_SLICES, n), dim3(256), 0, s, d);
+    NRX_HIP(hipGetLastError());
+  }
   hipLaunchKernelGGL(k_grad_total_multi, dim3(max_edges, n), dim3(256), 0, s, d);
   NRX_HIP(hipGetLastError());
 }
