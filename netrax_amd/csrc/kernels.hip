@@ -878,6 +878,10 @@ __global__ void __launch_bounds__(64, 3)
   }
 }
 
+// The factor that a displayed-tree root seeds at a site: beta w / (C Ltilde).
+// A tree without weight seeds nothing, also where its likelihood is zero.
+__device__ __forceinline__ double root_seed(double beta, double factor) { return beta != 0.0 ? beta * factor : 0.0; }
+
 // Reverse pruning in push form.  For op q with children k (edge e_k, CLV
 // x_k, y_k = P_k x_k) and rescale factor F = 2^256 where q was rescaled:
 //   z_k      = Abar_q * F * prod_{j != k} y_j
@@ -1041,7 +1045,7 @@ __device__ __forceinline__ void adjoint_walk4(
     }
     if (op.root() >= 0) {
       // seed beta * w * (1/C) pi_i / Ltilde at a displayed-tree root
-      const double f = beta[part * n_root + op.root()] * in.sd[0];
+      const double f = root_seed(beta[part * n_root + op.root()], in.sd[0]);
       if constexpr (MODEL) {
         double r = 0.0;
 #pragma unroll
@@ -1468,7 +1472,7 @@ __global__ void __launch_bounds__(64, 2)
     }
     if (op.root() >= 0) {
       // seed beta * w * (1/C) pi_i / Ltilde at a displayed-tree root
-      const double f = beta[part * n_root + op.root()] * seed[op.root() * n + site0 + col];
+      const double f = root_seed(beta[part * n_root + op.root()], seed[op.root() * n + site0 + col]);
 #pragma unroll
       for (int r = 0; r < 5; ++r) a[r] = fma(f, freqs[part * AA_STATES + 4 * r + quad], a[r]);
     }
@@ -2247,7 +2251,7 @@ __device__ __forceinline__ void adjoint_walk32(const NetDesc &nd, float *lds, in
       for (int r = 0; r < NR; ++r) {
         int ef = EXP_EMPTY;
         f32x4 sd = {0.f, 0.f, 0.f, 0.f};
-        const double f = bt * in.sd[r];
+        const double f = root_seed(bt, in.sd[r]);
         if (f != 0.0) {
           const double mf = frexp(f, &ef);
 #pragma unroll
@@ -2731,7 +2735,7 @@ __global__ void __launch_bounds__(64, 3)
       // seed beta * w * (1/C) pi_i / Ltilde at a displayed-tree root
       int ef = EXP_EMPTY;
       Row20f sd = {{0.f, 0.f, 0.f, 0.f}, 0.f};
-      const double f = beta[op.root()] * in.sd[0];
+      const double f = root_seed(beta[op.root()], in.sd[0]);
       if (f != 0.0) {
         const double mf = frexp(f, &ef);
 #pragma unroll
