@@ -274,7 +274,7 @@ constexpr size_t forward_lds32(int C, int blocks, int n_slots) {
   return static_cast<size_t>(n_slots) * blocks * (1024 + 256 / C);
 }
 constexpr size_t adjoint_lds32(int C, int blocks, int n_slots) {
-  return sizeof(float) * GRAD_RING + forward_lds32(C, blocks, n_slots);
+  return sizeof(double) * GRAD_RING + forward_lds32(C, blocks, n_slots);
 }
 
 // Kernel launchers (kernels.hip)

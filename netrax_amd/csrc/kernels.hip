@@ -1788,8 +1788,9 @@ __global__ void __launch_bounds__(256)
 // CLVs are renormalised at every op by an exact power of two so the site
 // maximum lies in [0.5, 1); the per-site exponent k (true = stored * 2^-k) is
 // carried as an int32.  Site sums, the mixture and the gradient reduction
-// across waves are FP64; inside a wave the gradient's per-(site, category)
-// shares (each of order weight / branch length) are summed in FP32.
+// across row blocks are FP64; inside a block of 64 rows the gradient's
+// per-(site, category) shares (each of order weight / branch length) are
+// summed in FP32.
 constexpr double LN2 = 0.69314718055994530941723212145818;
 constexpr int EXP_EMPTY = -(1 << 28);  // exponent of an all-zero adjoint
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -2109,7 +2110,7 @@ __device__ __forceinline__ void adjoint_walk32(const NetDesc &nd, float *lds, in
   const uint64_t n = nd.L.n_sites_pad, row = n * (C * 16);
   const int part = to_constant(nd.tile_part)[site0 / TILE];
   const int n_slots = nd.adj_slots;
-  float *ring = lds;
+  double *ring = reinterpret_cast<double *>(lds);
   f32x4 *slots = reinterpret_cast<f32x4 *>(ring + GRAD_RING);  // [slot][block][lane], then exponents [slot][block][site]
   int32_t *slot_e = reinterpret_cast<int32_t *>(slots + n_slots * (NR * 64));
   const int sl = W::site(lane);
@@ -2272,7 +2273,9 @@ __device__ __forceinline__ void adjoint_walk32(const NetDesc &nd, float *lds, in
       ez[r] = m > 0.f ? ez[r] + e - word_step(in.word[r]) : EXP_EMPTY;
     }
     f32x4 y[2][NR];
-    float g[2] = {0.f, 0.f};
+    float g[NR][2];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) g[r][1] = 0.f;
     auto product = [&](int k) {
 #pragma unroll
       for (int r = 0; r < NR; ++r) {
@@ -2286,7 +2289,7 @@ __device__ __forceinline__ void adjoint_walk32(const NetDesc &nd, float *lds, in
         const f32x4 d = product4(Q, y[k][r]);
         const float gd = fmaf(z[r][3], d[3], fmaf(z[r][2], d[2], fmaf(z[r][1], d[1], z[r][0] * d[0])));
         // the site's share of dlnL/dt is O(weight / t): FP32 holds it
-        g[k] += ldexpf(gd, ez[r]);
+        g[r][k] = ldexpf(gd, ez[r]);
       }
       if (op.kid(k) >= 0) {
 #pragma unroll
@@ -2310,7 +2313,9 @@ __device__ __forceinline__ void adjoint_walk32(const NetDesc &nd, float *lds, in
       use(0, z);
     }
     // (rows leave as in k_adjoint_level)
-    const float total = pair_wave_sum_f32(g[0], g[1]);
+    double total = pair_wave_sum_f32(g[0][0], g[0][1]);
+#pragma unroll
+    for (int r = 1; r < NR; ++r) total += pair_wave_sum_f32(g[r][0], g[r][1]);
     const int k = lane >> 5;
     if ((lane & 31) == 31 && k < op.nk()) ring[(op.gslot() + k) % GRAD_RING] = total;
     const int done = op.gslot() + op.nk();
