@@ -322,11 +322,18 @@ static int walk_blocks_of(int tune_group, int64_t blocks) {
   return blocks / 2 >= 8 * CUS ? 2 : 1;
 }
 
-// LDS slots of the FP32 walks for a launch of `blocks` 64-row blocks.
-static void choose_slots32(Engine &e, int64_t blocks) {
-  e.rpw = e.C / e.walk_blocks;
-  e.fwd_slots = walk_slots(blocks / e.walk_blocks, [&](int n) { return forward_lds32(e.C, e.walk_blocks, n); });
-  e.adj_slots = walk_slots(blocks / e.walk_blocks, [&](int n) { return adjoint_lds32(e.C, e.walk_blocks, n); });
+// Shape of the 4-state FP32 walks of a launch of `blocks` 64-row blocks: blocks
+// per wave and LDS slots.
+struct Shape32 {
+  int blocks, fwd_slots, adj_slots;
+};
+static Shape32 shape32(int C, int tune_group, int64_t blocks) {
+  Shape32 s{};
+  // (a single 64-site tile of 1 category is one block)
+  s.blocks = C == 1 ? 1 : walk_blocks_of(tune_group, blocks);
+  s.fwd_slots = walk_slots(blocks / s.blocks, [&](int n) { return forward_lds32(C, s.blocks, n); });
+  s.adj_slots = walk_slots(blocks / s.blocks, [&](int n) { return adjoint_lds32(C, s.blocks, n); });
+  return s;
 }
 
 // The walks' two op lists with their slots.
@@ -337,6 +344,13 @@ static void assign_walk_slots(Engine &e) {
   assign_reverse_slots(e.ops_adj.data(), n, e.adj_slots);
   upload(e.d_ops_fwd, e.ops_fwd, e.stream);
   upload(e.d_ops_adj, e.ops_adj, e.stream);
+}
+
+// Deliveries that a reverse walk's ops hand over in LDS.
+static int lds_handoffs(const DevOp *ops, size_t n) {
+  int h = 0;
+  for (size_t i = 0; i < n; ++i) h += ((ops[i].flags & OP_PASS_KID0) != 0) + ((ops[i].flags & OP_PASS_KID1) != 0);
+  return h;
 }
 
 // Builds the level schedule, the batched order, root CLV set and gradient
@@ -438,11 +452,14 @@ static void build_schedule(Engine &e) {
   upload(e.d_ops, e.ops_all, e.stream);
   if (e.opt.precision == NRX_FP64 || e.S == AA_STATES) {
     choose_walk_shape(e);
+    e.gwpt = e.S == AA_STATES ? e.rpw * e.C : e.rpw;
   } else {
-    const int64_t blocks = e.L.n_sites_pad * e.C / 64;
-    // (a single 64-site tile of 1 category is one block)
-    e.walk_blocks = e.C == 1 ? 1 : walk_blocks_of(e.tune_group, blocks);
-    choose_slots32(e, blocks);
+    const Shape32 s = shape32(e.C, e.tune_group, e.L.n_sites_pad * e.C / 64);
+    e.walk_blocks = s.blocks;
+    e.fwd_slots = s.fwd_slots;
+    e.adj_slots = s.adj_slots;
+    e.rpw = e.C;
+    e.gwpt = e.C / s.blocks;
   }
   assign_walk_slots(e);
   upload(e.d_edge_use_begin, e.edge_use_begin, e.stream);
@@ -451,7 +468,6 @@ static void build_schedule(Engine &e) {
   upload(e.d_class_dlogprob, e.class_dlogprob, e.stream);
   std::vector<int32_t> rs(e.root_slots.begin(), e.root_slots.end());
   upload(e.d_root_slots, rs, e.stream);
-  e.gwpt = e.S == AA_STATES ? e.rpw * e.C : e.rpw;
   const size_t n_wt = static_cast<size_t>(e.L.n_tiles) * e.rpw;
   const size_t n_gwt = static_cast<size_t>(e.L.n_tiles) * e.gwpt;
   e.d_root_partials.alloc(sizeof(double) * std::max<size_t>(1, rs.size()) * n_wt);
@@ -509,8 +525,8 @@ static void upload_netdesc(Engine &e) {
   if (e.opt.precision != NRX_FP32) return;
   std::vector<NetDesc> nd{make_netdesc(e)};
   upload(e.d_netdesc, nd, e.stream);
-  // work items: the walks' waves
-  const int n_work = e.L.n_tiles * e.rpw;
+  // work items: the walks' waves (4 states; 20-state walks have no list)
+  const int n_work = e.L.n_tiles * e.gwpt;
   std::vector<WorkItem> work(n_work);
   for (int t = 0; t < n_work; ++t) work[t] = WorkItem{0, t};
   upload(e.d_work, work, e.stream);
@@ -1119,15 +1135,15 @@ struct Batch {
   std::vector<int> versions;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  DevBuf d_nets, d_work, d_small, d_offsets;
+  DevBuf d_nets, d_work, d_small, d_offsets, d_ops;
   double *h_out = nullptr, *h_out_dev = nullptr;  // pinned, and its device address
   std::vector<int64_t> offsets;
   int n_work = 0, C = 0, max_pm = 0, max_root_rows = 0, max_uses = 0, max_parts = 0, max_edges = 0,
       max_res = 0;
-  int fwd_slots = 0, adj_slots = 0;  // the most any engine has
   bool use_graph = false;
-  int G = 4, TS = TILE, H = 1;  // shape of the persistent kernels, shared by all engines
-  int blocks = 1;               // 64-row blocks per wave, likewise
+  int G = 4, TS = TILE, H = 1;  // tuned shape, shared by all engines
+  Shape32 shape{1, 2, 2};       // of the batch's launches; an engine alone keeps its own
+  std::vector<std::shared_ptr<int>> handoffs;  // per engine, of the batch's op list
   hipGraphExec_t graph_exec[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};  // [variant][gradient]
   ~Batch() {
     if (stream) (void)hipStreamSynchronize(stream);
@@ -1139,7 +1155,7 @@ struct Batch {
   }
 };
 
-static SmallDesc make_smalldesc(const Engine &e) {
+static SmallDesc make_smalldesc(const Engine &e, int gwpt) {
   SmallDesc d{};
   d.L = e.L;
   d.V = e.d_V.as<double>();
@@ -1175,7 +1191,7 @@ static SmallDesc make_smalldesc(const Engine &e) {
   d.rl_part_dbrlen = e.rl.part_dbrlen;
   d.rl_dprob = e.rl.dprob;
   d.pw = e.rpw;
-  d.gwpt = e.gwpt;
+  d.gwpt = gwpt;
   const void *need[] = {d.V, d.Vinv, d.ev, d.rates, d.host_brlen, d.brlen, d.P, d.Pf, d.PfT,
                         d.part_tile_begin, d.classes, d.class_dlogprob, d.root_partials,
                         d.root_sums, d.grad_partials, d.use_sums, d.beta, d.edge_use_begin,
@@ -1185,8 +1201,13 @@ static SmallDesc make_smalldesc(const Engine &e) {
   return d;
 }
 
-// Descriptors and the (network, tile) work table; tiles of networks with
-// longer op lists come first so the longest workgroups start earliest.
+// Descriptors, op lists and the (network, wave) work table; waves of networks
+// with longer op lists come first so the longest workgroups start earliest.
+// A batch launch holds far more waves than one engine's, so it has a shape of
+// its own: two blocks per wave earlier, and only as many LDS slots as let its
+// waves be resident (a row without a slot goes through HBM).  The engines'
+// buffers serve both: CLVs and root sums do not depend on the shape, and what
+// does (gradient partials) is never more than an engine alone needs.
 static void build_batch(Batch &b) {
   const int n = static_cast<int>(b.engines.size());
   destroy_graphs(b.graph_exec);  // they hold the old tables' addresses
@@ -1195,7 +1216,6 @@ static void build_batch(Batch &b) {
   std::vector<std::pair<int, int>> order;  // (cost, engine)
   b.offsets.assign(n + 1, 0);
   b.max_pm = b.max_root_rows = b.max_uses = b.max_parts = b.max_edges = b.max_res = 0;
-  b.fwd_slots = b.adj_slots = 0;
   b.versions.resize(n);
   b.G = b.engines[0]->tune_group;
   b.TS = b.engines[0]->tune_tile;
@@ -1203,38 +1223,32 @@ static void build_batch(Batch &b) {
   for (const Engine *e : b.engines)
     if (e->tune_group != b.G || e->tune_tile != b.TS || e->tune_lanes != b.H)
       throw std::invalid_argument("batch engines must share the FP32 kernel shape (nrx_set_tuning)");
-  // One batch launch holds far more waves than one engine's: its engines take
-  // the wave shape of the whole (never back to one block, so that batches
-  // with an engine in common settle), and each keeps only as many LDS slots
-  // as let the launch's waves be resident (a row without a slot goes through
-  // HBM); their own graphs then re-capture.
   int64_t blocks = 0;
   for (const Engine *e : b.engines) blocks += e->L.n_sites_pad * e->C / 64;
-  b.blocks = b.C == 1 ? 1 : walk_blocks_of(b.G, blocks);
-  for (const Engine *e : b.engines) b.blocks = std::max(b.blocks, e->walk_blocks);
-  for (Engine *e : b.engines) {
-    const bool reshaped = e->walk_blocks != b.blocks;
-    const int fwd = reshaped ? WALK_SLOTS : e->fwd_slots, adj = reshaped ? WALK_SLOTS : e->adj_slots;
-    e->walk_blocks = b.blocks;
-    choose_slots32(*e, blocks);
-    e->fwd_slots = std::min(fwd, e->fwd_slots);
-    e->adj_slots = std::min(adj, e->adj_slots);
-    if (reshaped) {  // the root sums and gradient rows are per wave
-      e->gwpt = e->rpw;
-      std::fill(e->clv_dirty.begin(), e->clv_dirty.end(), 1);
-      e->cache_valid = false;
-    } else if (e->fwd_slots == fwd && e->adj_slots == adj) {
-      continue;
-    }
-    assign_walk_slots(*e);
-    upload_netdesc(*e);
-    NRX_HIP(hipStreamSynchronize(e->stream));
-    e->schedule_version++;
+  b.shape = shape32(b.C, b.G, blocks);
+  const int gwpt = b.C / b.shape.blocks;
+  std::vector<DevOp> ops;  // per engine its forward, then its reverse list
+  for (int i = 0; i < n; ++i) {
+    Engine &e = *b.engines[i];
+    if (e.gwpt < gwpt) throw std::logic_error("batch waves exceed the engine's gradient partials");
+    const size_t at = ops.size(), n_ops = e.ops_all.size();
+    ops.insert(ops.end(), e.ops_all.begin(), e.ops_all.end());
+    ops.insert(ops.end(), e.ops_all.begin(), e.ops_all.end());
+    assign_forward_slots(ops.data() + at, static_cast<int>(n_ops), b.shape.fwd_slots);
+    assign_reverse_slots(ops.data() + at + n_ops, static_cast<int>(n_ops), b.shape.adj_slots);
+    *b.handoffs[i] = lds_handoffs(ops.data() + at + n_ops, n_ops);
   }
+  upload(b.d_ops, ops, b.stream);
+  size_t first_op = 0;
   for (int i = 0; i < n; ++i) {
     const Engine &e = *b.engines[i];
     nets[i] = make_netdesc(e);
-    small[i] = make_smalldesc(e);
+    nets[i].ops_fwd = b.d_ops.as<DevOp>() + first_op;
+    nets[i].ops_adj = nets[i].ops_fwd + e.ops_all.size();
+    nets[i].fwd_slots = b.shape.fwd_slots;
+    nets[i].adj_slots = b.shape.adj_slots;
+    first_op += 2 * e.ops_all.size();
+    small[i] = make_smalldesc(e, gwpt);
     b.versions[i] = e.schedule_version;
     order.push_back({static_cast<int>(e.ops_all.size()), i});
     b.offsets[i + 1] = b.offsets[i] + e.rl.size;
@@ -1244,8 +1258,6 @@ static void build_batch(Batch &b) {
     b.max_parts = std::max(b.max_parts, e.P);
     b.max_edges = std::max(b.max_edges, e.E);
     b.max_res = std::max(b.max_res, e.rl.size);
-    b.fwd_slots = std::max(b.fwd_slots, e.fwd_slots);
-    b.adj_slots = std::max(b.adj_slots, e.adj_slots);
   }
   std::stable_sort(order.begin(), order.end(),
                    [](const std::pair<int, int> &x, const std::pair<int, int> &y) {
@@ -1254,7 +1266,7 @@ static void build_batch(Batch &b) {
   std::vector<WorkItem> work;
   for (const auto &o : order) {
     if (o.first == 0) continue;  // no displayed tree counts: nothing to walk, lnL is -infinity
-    for (int t = 0; t < b.engines[o.second]->L.n_tiles * b.engines[o.second]->rpw; ++t) work.push_back({o.second, t});
+    for (int t = 0; t < b.engines[o.second]->L.n_tiles * gwpt; ++t) work.push_back({o.second, t});
   }
   b.n_work = static_cast<int>(work.size());
   upload(b.d_nets, nets, b.stream);
@@ -1296,6 +1308,12 @@ int nrx_batch_create(nrx_engine *const *engines, int32_t n_engines, nrx_batch **
     NRX_HIP(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
     NRX_HIP(hipEventCreate(&b->ev0));
     NRX_HIP(hipEventCreate(&b->ev1));
+    for (Engine *e : b->engines) {
+      b->handoffs.push_back(std::make_shared<int>(0));
+      auto &all = e->batch_handoffs;
+      all.erase(std::remove_if(all.begin(), all.end(), [](const auto &h) { return h.expired(); }), all.end());
+      all.push_back(b->handoffs.back());
+    }
     build_batch(*b);
     *out = reinterpret_cast<nrx_batch *>(b.release());
     return NRX_OK;
@@ -1341,13 +1359,13 @@ int nrx_batch_evaluate(nrx_batch *batch, int32_t variant, double *lnl, double *d
     auto enqueue = [&]() {
       const SmallDesc *sd = b.d_small.as<SmallDesc>();
       launch_pmatrices_multi(b.stream, sd, n, b.max_pm);
-      launch_forward_persistent_multi(b.stream, b.C, b.blocks, b.d_nets.as<NetDesc>(),
-                                      b.d_work.as<WorkItem>(), b.n_work, b.fwd_slots);
+      launch_forward_persistent_multi(b.stream, b.C, b.shape.blocks, b.d_nets.as<NetDesc>(),
+                                      b.d_work.as<WorkItem>(), b.n_work, b.shape.fwd_slots);
       launch_root_reduce_multi(b.stream, sd, n, b.max_root_rows);
       launch_mixture_multi(b.stream, sd, n, variant);
       if (grad) {
-        launch_adjoint_persistent_multi(b.stream, b.C, b.blocks, b.d_nets.as<NetDesc>(),
-                                        b.d_work.as<WorkItem>(), b.n_work, b.adj_slots);
+        launch_adjoint_persistent_multi(b.stream, b.C, b.shape.blocks, b.d_nets.as<NetDesc>(),
+                                        b.d_work.as<WorkItem>(), b.n_work, b.shape.adj_slots);
         launch_grad_reduce_multi(b.stream, sd, n, b.max_uses, b.max_parts, b.max_edges);
       }
       launch_gather_results(b.stream, sd, n, b.d_offsets.as<int64_t>(), b.h_out_dev, b.max_res);
@@ -2211,9 +2229,9 @@ int nrx_get_stats(nrx_engine *eng, nrx_stats *out) {
     const bool fp32 = e.opt.precision == NRX_FP32;
     const double aexp = fp32 ? (e.S == AA_STATES ? scl * e.C : scl) : 0.0;
     const std::vector<DevOp> &adj_ops = e.ops_adj;
-    out->n_lds_handoffs = 0;
-    for (const DevOp &op : adj_ops)
-      out->n_lds_handoffs += ((op.flags & OP_PASS_KID0) != 0) + ((op.flags & OP_PASS_KID1) != 0);
+    out->n_lds_handoffs = lds_handoffs(adj_ops.data(), adj_ops.size());
+    for (const auto &h : e.batch_handoffs)
+      if (const auto in_batch = h.lock()) out->n_lds_handoffs = std::min(out->n_lds_handoffs, *in_batch);
     double adj = 0.0;
     for (const DevOp &op : adj_ops) {
       adj += scl;

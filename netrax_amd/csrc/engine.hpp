@@ -242,11 +242,11 @@ void launch_mixture_multi(hipStream_t s, const SmallDesc *d, int n, int variant)
 void launch_grad_reduce_multi(hipStream_t s, const SmallDesc *d, int n, int max_uses, int max_parts, int max_edges);
 void launch_gather_results(hipStream_t s, const SmallDesc *d, int n, const int64_t *offsets,
                            double *out, int max_size);
-// blocks: 64-row blocks per wave (1 or 2)
+// blocks: 64-row blocks per wave (1 or 2); slots: LDS slots, as every network's descriptor has them
 void launch_forward_persistent_multi(hipStream_t stream, int C, int blocks, const NetDesc *nets, const WorkItem *work,
-                                     int n_work, int max_slots);
+                                     int n_work, int slots);
 void launch_adjoint_persistent_multi(hipStream_t stream, int C, int blocks, const NetDesc *nets, const WorkItem *work,
-                                     int n_work, int max_slots);
+                                     int n_work, int slots);
 
 // Dynamic LDS of the 4-state walks: the reverse walk's ring of gradient sums
 // on their way to HBM, and n_slots rows with their scaler words or exponents.

@@ -84,6 +84,8 @@ struct Engine : nrx_engine {
   int walk_nq = 4, fwd_slots = 4, adj_slots = 4;
   int walk_blocks = 1;  // 64-row blocks per wave (FP32)
   int gwpt = 1;  // gradient partials [wave][row]: waves per tile
+  // hand-offs in LDS of the batches that this engine is in (nrx_stats)
+  std::vector<std::weak_ptr<const int>> batch_handoffs;
   // FP32 form shape (nrx_autotune / nrx_set_tuning): for the first, see
   // walk_blocks_of (4 states); the others are part of a shape's name only.
   int tune_group = 4;

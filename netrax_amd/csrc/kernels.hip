@@ -1974,9 +1974,9 @@ __device__ __forceinline__ void forward_walk32(const NetDesc &nd, float *lds, in
   for (int r = 0; r < NR; ++r) w[r] = to_global(nd.weights)[site0 + r * W::SPB + sl];
 #pragma unroll
   for (int i = 0; i < 4; ++i) pi[i] = to_global(nd.freqs)[part * 4 + i];
-  GAS double *root_partials = to_global(nd.root_partials) + site0 / W::SPW;
+  GAS double *root_partials = to_global(nd.root_partials) + site0 / W::SPB;  // [root][block]
   GAS double *seed = to_global(nd.seed) + site0 + sl;
-  const int64_t n_waves = static_cast<int64_t>(n) / W::SPW;
+  const int64_t n_blocks = static_cast<int64_t>(n) / W::SPB;
 
   auto load = [&](const OpRegs &op, FwdIn32<C, NR> &in) {
     const uint32_t o = opaque(off), so = opaque(soff), tip_o = opaque(sl), ao = opaque(aoff);
@@ -2056,19 +2056,20 @@ __device__ __forceinline__ void forward_walk32(const NetDesc &nd, float *lds, in
       }
     }
     if (op.root() >= 0) {
-      double val = 0.0;
+      // (a sum per block, whatever the number of blocks of a wave: an engine
+      // and a batch that it is in leave each other the same sums)
 #pragma unroll
       for (int r = 0; r < NR; ++r) {
         double t = 0.0;
 #pragma unroll
         for (int i = 0; i < 4; ++i) t = fma(pi[i], static_cast<double>(v[r][i]), t);
         t = site_total<C>(t) * (1.0 / C);
-        if (W::cat(lane) == 0 && w[r] != 0.0) val += w[r] * (log(t) - word_k(word[r]) * LN2);
+        const bool counts = W::cat(lane) == 0 && w[r] != 0.0;
+        const double val = wave_sum(counts ? w[r] * (log(t) - word_k(word[r]) * LN2) : 0.0);
+        if (lane == 0) root_partials[op.root() * n_blocks + r] = val;
         // the adjoint's seed factor at this root and site, w / (C Ltilde)
         seed[op.root() * static_cast<int64_t>(n) + r * W::SPB] = w[r] != 0.0 ? w[r] / (C * t) : 0.0;
       }
-      val = wave_sum(val);
-      if (lane == 0) root_partials[op.root() * n_waves] = val;
     }
   };
   walk_ops<FwdIn32<C, NR>>(to_constant(nd.ops_fwd), nd.n_fwd, false, load,
@@ -3727,30 +3728,30 @@ static void dispatch_walk32(int C, int blocks, F &&f) {
 
 void launch_forward_persistent(Engine &e, const NetDesc *nets) {
   launch_forward_persistent_multi(e.stream, e.C, e.walk_blocks, nets ? nets : e.d_netdesc.as<NetDesc>(),
-                                  e.d_work.as<WorkItem>(), e.L.n_tiles * e.rpw, e.fwd_slots);
+                                  e.d_work.as<WorkItem>(), e.L.n_tiles * e.gwpt, e.fwd_slots);
 }
 
 void launch_adjoint_persistent(Engine &e) {
   launch_adjoint_persistent_multi(e.stream, e.C, e.walk_blocks, e.d_netdesc.as<NetDesc>(), e.d_work.as<WorkItem>(),
-                                  e.L.n_tiles * e.rpw, e.adj_slots);
+                                  e.L.n_tiles * e.gwpt, e.adj_slots);
 }
 
 void launch_forward_persistent_multi(hipStream_t stream, int C, int blocks, const NetDesc *nets, const WorkItem *work,
-                                     int n_work, int max_slots) {
+                                     int n_work, int slots) {
   if (n_work == 0) return;
   dispatch_walk32(C, blocks, [&](auto c, auto g) {
     hipLaunchKernelGGL((k_forward_persistent<decltype(c)::value, decltype(g)::value, 64>), dim3(n_work), dim3(64),
-                       forward_lds32(C, blocks, max_slots), stream, nets, work);
+                       forward_lds32(C, blocks, slots), stream, nets, work);
   });
   NRX_HIP(hipGetLastError());
 }
 
 void launch_adjoint_persistent_multi(hipStream_t stream, int C, int blocks, const NetDesc *nets, const WorkItem *work,
-                                     int n_work, int max_slots) {
+                                     int n_work, int slots) {
   if (n_work == 0) return;
   dispatch_walk32(C, blocks, [&](auto c, auto g) {
     hipLaunchKernelGGL((k_adjoint_persistent<decltype(c)::value, decltype(g)::value, 64>), dim3(n_work), dim3(64),
-                       adjoint_lds32(C, blocks, max_slots), stream, nets, work);
+                       adjoint_lds32(C, blocks, slots), stream, nets, work);
   });
   NRX_HIP(hipGetLastError());
 }
