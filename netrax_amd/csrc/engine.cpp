@@ -1339,16 +1339,20 @@ int nrx_batch_evaluate(nrx_batch *batch, int32_t variant, double *lnl, double *d
     const int n = static_cast<int>(b.engines.size());
     bool rebuild = false;
     for (int i = 0; i < n; ++i) {
-      Engine &e = *b.engines[i];
-      check_ready(e);
+      check_ready(*b.engines[i]);
+      rebuild |= b.versions[i] != b.engines[i]->schedule_version;
+    }
+    if (rebuild) build_batch(b);
+    for (Engine *engine : b.engines) {
       // models and branch lengths of every engine, as update_pmatrices does
+      // (once nothing can refuse the batch any more: an engine whose lengths
+      // count as taken over must get its P matrices)
+      Engine &e = *engine;
       if (e.model_dirty) upload_models(e);
       stage_brlen(e);
       e.model_dirty = false;
       std::fill(e.edge_dirty.begin(), e.edge_dirty.end(), 0);
-      rebuild |= b.versions[i] != e.schedule_version;
     }
-    if (rebuild) build_batch(b);
     // the batch's kernels read the engines' pinned lengths: they have ended
     // whichever way this call ends
     struct Drain {

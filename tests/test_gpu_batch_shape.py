@@ -76,3 +76,24 @@ def test_two_batches_share_an_engine():
     big.close()
     for a in anns[1:]:
         a.close()
+
+
+def test_refused_batch_leaves_the_engines_their_changes():
+    """A batch that is refused (its engines' shapes differ by now) has not
+    taken over the lengths set before: the engines alone evaluate at them."""
+    print("refused batch", flush=True)
+    anns = engines([300, 500])
+    batch = NetworkBatch(anns)
+    batch.evaluate(0)
+    for a in anns:
+        a.set_branch_lengths(a.network.brlen * 1.7)
+    anns[1].set_tuning(3, 64, 1)
+    with pytest.raises(_lib.NrxError):
+        batch.evaluate(0)
+    fresh = engines([300, 500])
+    for a, f in zip(anns, fresh):
+        f.set_branch_lengths(a.network.brlen)
+        assert a.loglikelihood() == f.loglikelihood(0)
+    batch.close()
+    for a in anns + fresh:
+        a.close()
