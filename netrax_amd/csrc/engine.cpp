@@ -268,22 +268,6 @@ static void plan_budget(Engine &e) {
   resize_rows(e, bp.n_phys);
 }
 
-// waves of the 20-state walks that a CU holds
-constexpr int AA_ADJ_WAVES = 8, AA_FWD32_WAVES = 16, AA_ADJ32_WAVES = 12;
-constexpr int CUS = 256, LDS_PER_CU = 160 * 1024, LDS_PER_GROUP = 64 * 1024;
-
-// LDS slots per wave of a walk of `groups` workgroups, of which a CU's
-// registers hold at most `most_per_cu`.
-template <typename Lds>
-static int walk_slots(int64_t groups, Lds &&lds, int most_per_cu = 12) {
-  const int per_cu = static_cast<int>(std::min<int64_t>(most_per_cu, (groups + CUS - 1) / CUS));
-  // (LDS is given out in pieces of 1280 bytes)
-  const size_t most = std::min<size_t>(LDS_PER_CU / per_cu / 1280 * 1280, LDS_PER_GROUP);
-  int n = 2;
-  while (n < WALK_SLOTS && lds(n + 1) <= most) ++n;
-  return n;
-}
-
 // Granules and LDS slots per wave of the FP64 walks.  4 states: four granules
 // share an op's fixed work best (41,345 patterns x 4 categories, gradient:
 // 0.66 ms, 0.92 with two, 1.00 with one); fewer once they would leave SIMDs
@@ -292,15 +276,10 @@ static int walk_slots(int64_t groups, Lds &&lds, int most_per_cu = 12) {
 // three per SIMD (two in the 20-state reverse walk), be resident together.
 static void choose_walk_shape(Engine &e) {
   if (e.S == AA_STATES) {
-    const int64_t groups = e.L.n_sites_pad / AA_SITES;
+    const AaSlots s = aa_walk_slots(e.C, e.opt.precision == NRX_FP32, e.L.n_sites_pad);
     e.rpw = TILE / AA_SITES;
-    if (e.opt.precision == NRX_FP32) {
-      e.fwd_slots = walk_slots(groups, [&](int n) { return forward_lds_aa32(e.C, n); }, AA_FWD32_WAVES / e.C);
-      e.adj_slots = walk_slots(groups * e.C, [&](int n) { return adjoint_lds_aa32(n); }, AA_ADJ32_WAVES);
-      return;
-    }
-    e.fwd_slots = walk_slots(groups, [&](int n) { return forward_walk_lds_aa(e.C, n); }, std::max(1, 12 / e.C));
-    e.adj_slots = walk_slots(groups * e.C, [&](int n) { return adjoint_walk_lds_aa(n); }, AA_ADJ_WAVES);
+    e.fwd_slots = s.fwd;
+    e.adj_slots = s.adj;
     return;
   }
   const int64_t granules = e.L.n_sites_pad * e.C / 16;

@@ -261,6 +261,9 @@ constexpr size_t adjoint_walk_lds(int nq, int n_slots) {
 constexpr size_t forward_walk_lds_aa(int C, int n_slots) {
   return static_cast<size_t>(n_slots) * C * (sizeof(double) * AA_ROW + 4 * AA_SITES);
 }
+// (what the forward kernels declare besides: the cells that the categories' waves trade)
+constexpr size_t forward_fixed_lds_aa(int C) { return C > 1 ? 2 * C * (4 + 8 * AA_SITES) : 0; }
+constexpr size_t forward_fixed_lds_aa32(int C) { return C > 1 ? 2 * C * (4 + 8) * AA_SITES : 0; }
 constexpr size_t adjoint_walk_lds_aa(int n_slots) {
   return sizeof(double) * (GRAD_RING + static_cast<size_t>(n_slots) * AA_ROW);
 }

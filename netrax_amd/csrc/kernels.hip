@@ -1228,6 +1228,7 @@ __global__ void __launch_bounds__(64 * C, 3)
                       double *__restrict__ seed) {
   __shared__ uint32_t small_sites[2][C];
   __shared__ double site_like[2][C][AA_SITES];
+  static_assert(C == 1 || sizeof(small_sites) + sizeof(site_like) == forward_fixed_lds_aa(C));
   const CAS DevOp *ops = to_constant(ops_);
   const int c = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63, quad = lane >> 4, col = lane & 15;
@@ -2480,6 +2481,7 @@ __global__ void __launch_bounds__(64 * C, 4)
   static_assert(G == 4, "group widths name one kernel");
   __shared__ float site_most[2][C][AA_SITES];
   __shared__ double site_like[2][C][AA_SITES];
+  static_assert(C == 1 || sizeof(site_most) + sizeof(site_like) == forward_fixed_lds_aa32(C));
   const NetDesc &nd = nets[0];
   const CAS DevOp *ops = to_constant(nd.ops_fwd);
   const int n_slots = nd.fwd_slots;

@@ -101,6 +101,18 @@ std::vector<int> depth_first_order(const Dag &dag, const std::vector<int> &root_
   return order;
 }
 
+AaSlots aa_walk_slots(int C, bool fp32, int64_t sites) {
+  // waves of the walks that a CU's registers hold
+  constexpr int FWD = 12, ADJ = 8, FWD32 = 16, ADJ32 = 12;
+  const int64_t groups = sites / AA_SITES;
+  if (fp32)
+    return {walk_slots(groups, [&](int n) { return forward_lds_aa32(C, n); }, FWD32 / C, forward_fixed_lds_aa32(C)),
+            walk_slots(groups * C, [&](int n) { return adjoint_lds_aa32(n); }, ADJ32)};
+  return {walk_slots(groups, [&](int n) { return forward_walk_lds_aa(C, n); }, std::max(1, FWD / C),
+                     forward_fixed_lds_aa(C)),
+          walk_slots(groups * C, [&](int n) { return adjoint_walk_lds_aa(n); }, ADJ)};
+}
+
 // The row with the furthest next read gives up its slot (it was stored in
 // HBM anyway), which keeps the most reads in LDS.
 void assign_forward_slots(DevOp *ops, int n, int n_slots) {

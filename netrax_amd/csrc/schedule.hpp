@@ -6,6 +6,7 @@
 // schedules can be built and checked without a GPU.
 #pragma once
 
+#include <algorithm>
 #include <cstdint>
 #include <vector>
 
@@ -43,6 +44,28 @@ void assign_forward_slots(DevOp *ops, int n, int n_slots);
 // An op's own adjoint, where HBM holds it, is read one op early unless
 // OP_A_LATE.
 void assign_reverse_slots(DevOp *ops, int n, int n_slots);
+
+constexpr int CUS = 256, LDS_PER_CU = 160 * 1024, LDS_PER_GROUP = 64 * 1024;
+constexpr int LDS_PIECE = 1280;  // LDS is given out in pieces of this
+
+// LDS slots per wave of a walk of `groups` workgroups, of which a CU's
+// registers hold at most `most_per_cu`: as many as let the workgroups that a CU
+// gets be resident together.  lds(n): a workgroup's dynamic LDS with n slots;
+// fixed: what its kernel declares besides.
+template <typename Lds>
+int walk_slots(int64_t groups, Lds &&lds, int most_per_cu = 12, size_t fixed = 0) {
+  const int per_cu = static_cast<int>(std::min<int64_t>(most_per_cu, (groups + CUS - 1) / CUS));
+  const size_t most = std::min<size_t>(LDS_PER_CU / per_cu / LDS_PIECE * LDS_PIECE - fixed, LDS_PER_GROUP);
+  int n = 2;
+  while (n < WALK_SLOTS && lds(n + 1) <= most) ++n;
+  return n;
+}
+
+// LDS slots of the 20-state walks over `sites` padded sites.
+struct AaSlots {
+  int fwd, adj;
+};
+AaSlots aa_walk_slots(int C, bool fp32, int64_t sites);
 
 // OP_ACC_EARLY* for the FP32 reverse sweep (groups backwards).
 void set_acc_early(std::vector<DevOp> &ops, const std::vector<int32_t> &group_begin, int nv);
