@@ -206,10 +206,12 @@ int nrx_brlen_derivatives_noalloc(nrx_engine *eng, int32_t variant, int32_t edge
  * the numerical model optimisation raxml-ng runs through the pll-modules
  * hook (src/optimization/ModelOptimization.cpp:25-97, likelihood target
  * network_logl_wrapper, src/RaxmlWrapper.cpp:21-26, 647-648) with analytic
- * derivatives.  One forward and one adjoint pass, then a pass that forms
- * dlnL/dP per (edge, category) from the adjoints, chained through the
- * eigendecomposition of the rate matrix on the host.  FP64 form, 4-state
- * data (NRX_ERR_UNSUPPORTED otherwise). */
+ * derivatives.  One forward and one adjoint pass, which forms dlnL/dP per
+ * (edge, category) on the way and leaves its sums in the adjoint rows; they
+ * are added up and chained through the eigendecomposition of the rate matrix
+ * on the device.  The engine keeps workspaces of a few MB for it, which do not
+ * grow with the number of sites but for 32 bytes per displayed tree's root and
+ * wave.  FP64 form, 4-state data (NRX_ERR_UNSUPPORTED otherwise). */
 int nrx_model_gradient(nrx_engine *eng, int32_t variant, double *total, double *d_subst,
                        double *d_freqs, double *d_alpha, double *d_rates);
 

@@ -740,7 +740,8 @@ static void copy_results(Engine &e) {
     NRX_HIP(hipMemcpyAsync(e.h_result, e.d_result.p, sizeof(double) * e.rl.size, hipMemcpyDeviceToHost, e.stream));
 }
 
-// Reverse sweep of chunks c_hi down to c_lo (FP64 form), one launch.
+// Reverse sweep of chunks c_hi down to c_lo (FP64 form), one launch; model:
+// for the model gradient's sums, in a shape of its own.
 static void adjoint_chunks(Engine &e, int c_hi, int c_lo, const DevOp *ops, bool model = false) {
   if (c_hi < c_lo) return;
   record_kernel_begin(e, 1);
@@ -795,13 +796,14 @@ static int stage_invalid_walk(Engine &e, const NetDesc *&desc) {
   return n;
 }
 
-// Slices of a partition's waves that the model gradient's sums are formed in.
-constexpr int MODEL_SLICES = 8;
+// Slices of a partition's waves that the model gradient's sums are formed in:
+// few partitions are cut so that a row is the work of several workgroups.
+static int model_slices(const Engine &e) { return std::min(8, std::max(1, 16 / e.P)); }
 // Doubles of the model gradient's workspaces, in launch_model_grad's order.
 static std::array<size_t, 4> model_sizes(const Engine &e) {
-  const size_t P = e.P, nl = e.C == 8 ? 128 : 64;
-  return {std::max(1, e.n_uses) * P * MODEL_SLICES * nl, std::max<size_t>(1, e.root_slots.size()) * P * MODEL_SLICES * 4,
-          P * e.E * (16 + e.C), P * (16 + e.C + 4)};
+  const size_t P = e.P, nl = e.C == 8 ? 128 : 64, PS = P * model_slices(e);
+  return {std::max(1, e.n_uses) * PS * nl, std::max<size_t>(1, e.root_slots.size()) * PS * 4, P * e.E * (16 + e.C),
+          P * (16 + e.C + 4)};
 }
 static double *model_buffer(const Engine &e, int which) {
   const auto n = model_sizes(e);
@@ -809,21 +811,39 @@ static double *model_buffer(const Engine &e, int which) {
   for (int i = 0; i < which; ++i) p += n[i];
   return p;
 }
-static void alloc_model_grad(Engine &e) {
-  const size_t waves = static_cast<size_t>(e.L.n_tiles) * e.rpw, nl = e.C == 8 ? 128 : 64;
-  e.d_mg_g.alloc(sizeof(double) * std::max(1, e.n_uses) * waves * nl);
+// Op list, tables and workspaces of the model gradient.
+static void prepare_model_grad(Engine &e) {
+  const size_t waves = static_cast<size_t>(e.L.n_tiles) * e.model_wpt();
   e.d_mg_r.alloc(sizeof(double) * std::max<size_t>(1, e.root_slots.size()) * waves * 4);
   const auto n = model_sizes(e);
   e.d_mg_sums.alloc(sizeof(double) * (n[0] + n[1] + n[2] + n[3]));
+  if (e.model_version == e.schedule_version) return;
+  std::vector<int32_t> use_row(std::max(1, e.n_uses), 0);
+  for (const DevOp &op : e.ops_all)
+    for (int k = 0; k < op.nk; ++k) use_row[op.gslot[k]] = 2 * op.out + k;
+  upload(e.d_use_row, use_row, e.stream);
+  e.model_slots = e.adj_slots;
+  if (e.model_nq() != e.walk_nq) {
+    // (8 categories: two waves per SIMD, by registers)
+    e.model_slots = walk_slots(waves, [&](int k) { return adjoint_walk_lds(e.model_nq(), k); }, e.C == 8 ? 8 : 12);
+    std::vector<DevOp> ops = e.ops_all;
+    assign_reverse_slots(ops.data(), static_cast<int>(ops.size()), e.model_slots);
+    upload(e.d_ops_model, ops, e.stream);
+  }
+  e.model_version = e.schedule_version;
+}
+static const DevOp *model_ops(const Engine &e) {
+  return (e.model_nq() != e.walk_nq ? e.d_ops_model : e.d_ops_adj).as<DevOp>();
 }
 static void enqueue_model_grad(Engine &e) {
-  launch_model_grad(e, model_buffer(e, 0), model_buffer(e, 1), model_buffer(e, 2), model_buffer(e, 3), MODEL_SLICES);
+  launch_model_grad(e, model_buffer(e, 0), model_buffer(e, 1), model_buffer(e, 2), model_buffer(e, 3), model_slices(e));
 }
 
 // `fetch` false: the results stay on the device (for a caller that reads
 // them there, such as the device Newton sweep) and no host wait is made;
 // the host copy is then stale, so the cache is marked invalid.
-// `model`: the model gradient's sums too (FP64 form, 4 states).
+// `model`: the model gradient's sums in place of the branches' (FP64 form, 4
+// states).
 static int evaluate(Engine &e, int variant, bool incremental, bool update_pm, bool gradient, bool fetch = true,
                     bool model = false) {
   check_ready(e);
@@ -915,9 +935,11 @@ static int evaluate(Engine &e, int variant, bool incremental, bool update_pm, bo
     launch_mixture(e, variant, e.rpw, host);
     if (gradient) {
       e.d_adj.alloc(sizeof(double) * e.clv_elems_per_slot * e.dag.var.size());
-      adjoint_chunks(e, static_cast<int>(e.chunks.size()) - 1, 0, e.d_ops_adj.as<DevOp>(), model);
-      launch_grad_reduce(e, host);
-      if (model) enqueue_model_grad(e);
+      adjoint_chunks(e, static_cast<int>(e.chunks.size()) - 1, 0, model ? model_ops(e) : e.d_ops_adj.as<DevOp>(), model);
+      if (model)
+        enqueue_model_grad(e);
+      else
+        launch_grad_reduce(e, host);
     }
   }
   end_timing(e);
@@ -1940,7 +1962,7 @@ int nrx_model_gradient(nrx_engine *eng, int32_t variant, double *total, double *
     // CLVs, adjoints, mixture weights, and per partition dJ/dQ, dJ/dr_c and
     // the frequencies' direct share
     check_ready(e);
-    alloc_model_grad(e);
+    prepare_model_grad(e);
     const int rc = evaluate(e, variant, true, true, true, /*fetch=*/true, /*model=*/true);
     if (rc != NRX_OK) return rc;
     *total = e.cached_total;

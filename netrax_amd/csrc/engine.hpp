@@ -287,8 +287,8 @@ void launch_pmatrices(Engine &e);
 void launch_forward_walk(Engine &e, const DevOp *ops, int n_ops);
 // host: pinned memory that the results go to as well, or null
 void launch_mixture(Engine &e, int variant, int partials_per_tile, double *host);
-// FP64: the ops backwards (slots from assign_reverse_slots); model: with the
-// model gradient's sums per use and root (d_mg_g, d_mg_r; 4 states)
+// FP64: the ops backwards (slots from assign_reverse_slots); model: for the
+// model gradient's sums per use (in the adjoint rows) and root (d_mg_r; 4 states)
 void launch_adjoint_walk(Engine &e, const DevOp *ops, int n_ops, bool model);
 void launch_grad_reduce(Engine &e, double *host);
 // nets: a descriptor other than the engine's own (its invalid ops only)

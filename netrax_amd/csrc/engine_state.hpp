@@ -105,7 +105,15 @@ struct Engine : nrx_engine {
   // device Newton-Raphson: state, class table, tree lnLs; its captured
   // sequence, valid while the sumtable buffers keep their addresses
   DevBuf d_nr_state, d_nr_cls;
-  DevBuf d_mg_g, d_mg_r, d_mg_sums;  // model gradient: the walk's sums per use and root, and what is made of them
+  // model gradient (FP64, 4 states): its reverse walk's granules per wave (as
+  // many as make a wave's part of an adjoint row hold an op's sums), waves per
+  // tile, LDS slots and op list (of schedule model_version, where the shape is
+  // not the gradient's); the sums per root, and what is made of the sums
+  int model_nq() const { return C == 8 ? 4 : walk_nq < 2 ? 2 : walk_nq; }
+  int model_wpt() const { return TILE * C / (16 * model_nq()); }
+  int model_slots = 0, model_version = -1;
+  DevBuf d_ops_model, d_use_row;  // use_row: adjoint row and child of each use
+  DevBuf d_mg_r, d_mg_sums;
   // Memory budget of the FP64 form: with n_seg > 1 the CLV, adjoint and
   // scaler rows live in n_phys physical rows.  The ops are cut into
   // n_seg segments; a CLV consumed in a later segment than its own keeps a

@@ -908,23 +908,27 @@ struct AdjIn4 {
 // 1.6 GB in 0.363 ms, 4.5 TB/s; with P in LDS and every adjoint through HBM
 // 2.99 GB in 0.648 ms).
 //
-// MODEL: also, per use, the sums over the wave's sites of z x^T (dJ/dP), one
-// entry per lane of a granule (G, [use][wave][NA][64]), and per root those of
-// the frequencies' direct share, f x with f = beta w / (C Ltilde)
-// (r_part, [root][wave][4]).  Both are products over sites: z and x are
-// transposed by a product with the identity, which is exact, and multiplied
-// (41,345 patterns, 138 ops: 0.44 ms against 0.32 without, and 0.08 for
-// k_model_reduce; a pass of its own over stored adjoints and CLVs took 0.85
-// ms, and storing the adjoints 0.10).
+// MODEL: instead of the gradient's shares, per use, the sums over the wave's
+// sites of z x^T (dJ/dP), one entry per lane of a granule, and per root those of
+// the frequencies' direct share, f x with f = beta w / (C Ltilde) (r_part,
+// [root][wave][4]).  Both are products over sites: z and x are transposed by a
+// product with the identity, which is exact, and multiplied (41,345 patterns,
+// 138 ops: 0.44 ms against 0.32 without, and 0.08 for k_model_reduce; a pass of
+// its own over stored adjoints and CLVs took 0.85 ms, and storing the adjoints
+// 0.10).  The sums of
+// child k go to [k][NA][64] of the wave's part of the op's own adjoint row: no
+// one reads that any more, it holds both (NQ >= 2 NA), and they take no memory
+// of their own (a buffer for them was a quarter of the CLVs and adjoints).
 template <int C, int NQ, bool MODEL>
 __device__ __forceinline__ void adjoint_walk4(
     const DevOp *__restrict__ ops_, int n_ops, const DevLayout &L, const double *__restrict__ clv_,
     const int32_t *__restrict__ scl_, double *__restrict__ adj_, const uint8_t *__restrict__ tips_,
     const double *__restrict__ P_, const double *__restrict__ Qd, const double *__restrict__ freqs,
     const double *__restrict__ seed, const int32_t *__restrict__ tile_part, const double *__restrict__ beta, int n_root,
-    int n_uses, double *__restrict__ grad_partials, double *__restrict__ G_, double *__restrict__ r_part) {
+    int n_uses, double *__restrict__ grad_partials, double *__restrict__ r_part) {
   using W = Quad<C, NQ>;
   constexpr int NA = W::NA, SPW = W::SPW;
+  static_assert(!MODEL || NQ >= 2 * NA);
   const CAS DevOp *ops = to_constant(ops_);
   const int lane = threadIdx.x, state = lane >> 4;
   const uint64_t n = L.n_sites_pad, row = n * (C * 4);
@@ -949,8 +953,6 @@ __device__ __forceinline__ void adjoint_walk4(
     Q[h] = Qd[part * (C * 16) + aoff[h] / 8];
   }
   const double pi = freqs[part * 4 + state];
-  const double eye = (lane & 3) == state ? 1.0 : 0.0;
-  GAS double *G = to_global(G_) + static_cast<int64_t>(blockIdx.x) * (NA * 64);
 
   auto load = [&](const OpRegs &op, AdjIn4<C, NQ> &in) {
     const uint32_t o = opaque(off);
@@ -1037,7 +1039,7 @@ __device__ __forceinline__ void adjoint_walk4(
       for (int q = 0; q < NQ; ++q) a[q] = slot[q * 64];
     } else if (op.flags() & OP_A_LATE) {
 #pragma unroll
-      for (int q = 0; q < NQ; ++q) a[q] = *at(adj + op.out() * row, off + q * 512);
+      for (int q = 0; q < NQ; ++q) a[q] = *at(adj + op.out() * row, opaque(off) + q * 512);
       wait_loads();
     } else if (!(op.flags() & OP_HAS_CONSUMERS)) {
 #pragma unroll
@@ -1055,7 +1057,7 @@ __device__ __forceinline__ void adjoint_walk4(
         r += dpp<0x122>(r);
         r += dpp<0x124>(r);
         r += dpp<0x128>(r);
-        if ((lane & 15) == 0) r_part[(static_cast<int64_t>(op.root()) * gridDim.x + blockIdx.x) * 4 + state] = r;
+        if ((lane & 15) == 0) *at(to_global(r_part) + (static_cast<int64_t>(op.root()) * gridDim.x + blockIdx.x) * 4, opaque(state) * 8) = r;
       }
 #pragma unroll
       for (int q = 0; q < NQ; ++q) a[q] = fma(__shfl(f, W::site(lane, q)), pi, a[q]);
@@ -1067,16 +1069,19 @@ __device__ __forceinline__ void adjoint_walk4(
         if ((scaled >> W::site(lane, q)) & 1) a[q] *= SCALE_FACTOR;
     double y[2][NQ], z[NQ], g[2] = {0.0, 0.0};
     auto use = [&](int k) {
+      if constexpr (!MODEL) {
 #pragma unroll
-      for (int q = 0; q < NQ; ++q) g[k] = fma(z[q], mfma4(Q[W::half(q)], y[k][q], 0.0), g[k]);
-      if constexpr (MODEL) {
+        for (int q = 0; q < NQ; ++q) g[k] = fma(z[q], mfma4(Q[W::half(q)], y[k][q], 0.0), g[k]);
+      } else {
+        const uint32_t l = opaque(lane);
+        const double eye = (l & 3) == l >> 4 ? 1.0 : 0.0;
         double m[NA];
 #pragma unroll
         for (int h = 0; h < NA; ++h) m[h] = 0.0;
 #pragma unroll
         for (int q = 0; q < NQ; ++q)
           m[W::half(q)] = mfma4(mfma4(z[q], eye, 0.0), mfma4(in.x[k * NQ + q], eye, 0.0), m[W::half(q)]);
-        GAS double *dst = G + static_cast<int64_t>(op.gslot() + k) * gridDim.x * (NA * 64);
+        GAS double *dst = adj + op.out() * row + k * (NA * 64);
 #pragma unroll
         for (int h = 0; h < NA; ++h) *at(dst, opaque(off) + h * 512) = m[h];
       }
@@ -1096,6 +1101,7 @@ __device__ __forceinline__ void adjoint_walk4(
       for (int q = 0; q < NQ; ++q) z[q] = a[q];
       use(0);
     }
+    if constexpr (MODEL) return;
     // rows are numbered in the order of the sweep: row r waits in ring[r %
     // GRAD_RING], and 64 at a time leave as one store
     const double total = pair_wave_sum(g[0], g[1]);
@@ -1133,19 +1139,18 @@ __global__ void __launch_bounds__(64, 3)
                     const double *__restrict__ seed, const int32_t *__restrict__ tile_part,
                     const double *__restrict__ beta, int n_root, int n_uses, double *__restrict__ grad_partials) {
   adjoint_walk4<C, NQ, false>(ops, n_ops, L, clv, scl, adj, tips, P, Qd, freqs, seed, tile_part, beta, n_root, n_uses,
-                              grad_partials, nullptr, nullptr);
+                              grad_partials, nullptr);
 }
 
 template <int C, int NQ>
-__global__ void __launch_bounds__(64, 3)
+__global__ void __launch_bounds__(64, C == 8 ? 2 : 3)
     k_model_adjoint(const DevOp *__restrict__ ops, int n_ops, DevLayout L, const double *__restrict__ clv,
                     const int32_t *__restrict__ scl, double *__restrict__ adj, const uint8_t *__restrict__ tips,
                     const double *__restrict__ P, const double *__restrict__ Qd, const double *__restrict__ freqs,
                     const double *__restrict__ seed, const int32_t *__restrict__ tile_part,
-                    const double *__restrict__ beta, int n_root, int n_uses, double *__restrict__ grad_partials,
-                    double *__restrict__ G, double *__restrict__ r_part) {
+                    const double *__restrict__ beta, int n_root, int n_uses, double *__restrict__ r_part) {
   adjoint_walk4<C, NQ, true>(ops, n_ops, L, clv, scl, adj, tips, P, Qd, freqs, seed, tile_part, beta, n_root, n_uses,
-                             grad_partials, G, r_part);
+                             nullptr, r_part);
 }
 
 // ------------------------------------------------ 20 states, FP64 plain form
@@ -1562,14 +1567,17 @@ __global__ void __launch_bounds__(64, 2)
 }
 
 // ---------------------------------------------- model gradient (FP64)
-// dJ/dP of every use from the walks' sums G: per (use, partition, slice of the
+// dJ/dP of every use from the walk's sums: per (use, partition, slice of the
 // partition's waves) the sum over the slice, [use][partition][slice][nl]; the
 // rows after the uses are the roots' sums r_part ([root][wave][4]) likewise.
-// A workgroup holds 256 / nl waves' entries at once and adds them in order.
+// Use u lies at [wave][part] (wave_part doubles) of adjoint row use_row[u] / 2,
+// as its child use_row[u] % 2.  A workgroup holds 256 / nl waves' entries at
+// once and adds them in order.
 __global__ void __launch_bounds__(256)
-    k_model_reduce(const double *__restrict__ G, const double *__restrict__ r_part, int n_uses, int nl, int n_waves,
-                   int waves_per_tile, const int32_t *__restrict__ part_tile_begin, int P, int n_slice,
-                   double *__restrict__ g_sum, double *__restrict__ r_sum) {
+    k_model_reduce(const double *__restrict__ adj, size_t adj_row, int wave_part, const int32_t *__restrict__ use_row,
+                   const double *__restrict__ r_part, int n_uses, int nl, int n_waves, int waves_per_tile,
+                   const int32_t *__restrict__ part_tile_begin, int P, int n_slice, double *__restrict__ g_sum,
+                   double *__restrict__ r_sum) {
   __shared__ double sh[256];
   const bool root = static_cast<int>(blockIdx.x) >= n_uses;
   const int row = root ? blockIdx.x - n_uses : blockIdx.x, width = root ? 4 : nl;
@@ -1578,9 +1586,11 @@ __global__ void __launch_bounds__(256)
   const int w0 = wb + static_cast<int>(static_cast<int64_t>(we - wb) * slice / n_slice);
   const int w1 = wb + static_cast<int>(static_cast<int64_t>(we - wb) * (slice + 1) / n_slice);
   const int i = threadIdx.x % width, lead = threadIdx.x / width, step = 256 / width;
-  const double *in = (root ? r_part : G) + static_cast<size_t>(row) * n_waves * width + i;
+  const int stride = root ? 4 : wave_part;
+  const double *in = i + (root ? r_part + static_cast<size_t>(row) * n_waves * 4
+                               : adj + static_cast<size_t>(use_row[row] >> 1) * adj_row + (use_row[row] & 1) * nl);
   double s = 0.0;
-  for (int w = w0 + lead; w < w1; w += step) s += in[static_cast<size_t>(w) * width];
+  for (int w = w0 + lead; w < w1; w += step) s += in[static_cast<size_t>(w) * stride];
   sh[threadIdx.x] = s;
   __syncthreads();
   if (lead == 0) {
@@ -3675,7 +3685,7 @@ void launch_mixture(Engine &e, int variant, int pw, double *host) {
 
 void launch_adjoint_walk(Engine &e, const DevOp *ops, int n_ops, bool model) {
   if (n_ops == 0) return;
-  const unsigned waves = static_cast<unsigned>(e.L.n_tiles) * e.rpw;
+  const unsigned waves = static_cast<unsigned>(e.L.n_tiles) * (model ? e.model_wpt() : e.rpw);
   if (e.S == AA_STATES) {
     if (model) throw std::logic_error("launch_adjoint_walk: model gradients are built for 4-state data");
     dispatch_c(e.C, [&](auto c) {
@@ -3690,20 +3700,24 @@ void launch_adjoint_walk(Engine &e, const DevOp *ops, int n_ops, bool model) {
     NRX_HIP(hipGetLastError());
     return;
   }
-  dispatch_walk(e.C, e.walk_nq, [&](auto c, auto nq) {
-    constexpr int C = decltype(c)::value, NQ = decltype(nq)::value;
-    auto go = [&](auto kernel, auto... extra) {
-      hipLaunchKernelGGL(kernel, dim3(waves), dim3(64), adjoint_walk_lds(NQ, e.adj_slots), e.stream, ops, n_ops, e.L,
-                         e.d_clv.as<double>(), e.d_scl.as<int32_t>(), e.d_adj.as<double>(), e.d_tips.as<uint8_t>(),
-                         e.d_P.as<double>(), e.d_Qd.as<double>(), e.d_freqs.as<double>(), e.d_site_seed.as<double>(),
-                         e.d_tile_part.as<int32_t>(), e.d_beta.as<double>(), static_cast<int>(e.root_slots.size()),
-                         e.n_uses, e.d_grad_partials.as<double>(), extra...);
-    };
-    if (model)
-      go(k_model_adjoint<C, NQ>, e.d_mg_g.as<double>(), e.d_mg_r.as<double>());
-    else
-      go(k_adjoint_level<C, NQ>);
-  });
+  auto go = [&](auto kernel, int nq, int slots, const DevBuf &partials) {
+    hipLaunchKernelGGL(kernel, dim3(waves), dim3(64), adjoint_walk_lds(nq, slots), e.stream, ops, n_ops, e.L,
+                       e.d_clv.as<double>(), e.d_scl.as<int32_t>(), e.d_adj.as<double>(), e.d_tips.as<uint8_t>(),
+                       e.d_P.as<double>(), e.d_Qd.as<double>(), e.d_freqs.as<double>(), e.d_site_seed.as<double>(),
+                       e.d_tile_part.as<int32_t>(), e.d_beta.as<double>(), static_cast<int>(e.root_slots.size()),
+                       e.n_uses, partials.as<double>());
+  };
+  if (model)
+    dispatch_c(e.C, [&](auto c) {
+      constexpr int C = decltype(c)::value;
+      if (e.model_nq() == 4) return go(k_model_adjoint<C, 4>, 4, e.model_slots, e.d_mg_r);
+      if constexpr (C != 8) go(k_model_adjoint<C, 2>, 2, e.model_slots, e.d_mg_r);
+    });
+  else
+    dispatch_walk(e.C, e.walk_nq, [&](auto c, auto nq) {
+      constexpr int C = decltype(c)::value, NQ = decltype(nq)::value;
+      go(k_adjoint_level<C, NQ>, NQ, e.adj_slots, e.d_grad_partials);
+    });
   NRX_HIP(hipGetLastError());
 }
 
@@ -3871,7 +3885,8 @@ void launch_deriv_fused(Engine &e, const PathStep *steps, const int32_t *path_be
 void launch_model_grad(Engine &e, double *g_sum, double *r_sum, double *edge_out, double *out, int n_slice) {
   const int n_root = static_cast<int>(e.root_slots.size()), nl = e.C == 8 ? 128 : 64;
   hipLaunchKernelGGL(k_model_reduce, dim3(e.n_uses + n_root, e.P * n_slice), dim3(256), 0, e.stream,
-                     e.d_mg_g.as<double>(), e.d_mg_r.as<double>(), e.n_uses, nl, e.L.n_tiles * e.rpw, e.rpw,
+                     e.d_adj.as<double>(), e.clv_elems_per_slot, e.model_nq() * 64, e.d_use_row.as<int32_t>(),
+                     e.d_mg_r.as<double>(), e.n_uses, nl, e.L.n_tiles * e.model_wpt(), e.model_wpt(),
                      e.d_part_tile_begin.as<int32_t>(), e.P, n_slice, g_sum, r_sum);
   NRX_HIP(hipGetLastError());
   dispatch_c(e.C, [&](auto c) {
