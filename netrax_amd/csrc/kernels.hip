@@ -413,7 +413,7 @@ __global__ void __launch_bounds__(256)
 // otherwise the same code runs on the global arrays.  The arithmetic and
 // its order are the same either way.
 constexpr int MIX_LDS_DOUBLES = 6144;  // 48 KiB
-constexpr int MIX_PARTIALS = 2048;  // see launch_mixture
+constexpr int MIX_PARTIALS = 2048, MIX_ROWS = 16;  // see launch_mixture
 __host__ __device__ inline int mixture_lds_doubles(int n_root, int nc, int R, int P) {
   return n_root * P + 2 * nc + nc * P + nc * R;
 }
@@ -468,21 +468,26 @@ __device__ void mixture_body(const DevLayout &L, int n_root, int nc, int R, int 
     const int r = root_of(k);
     put(rl.tree_logl + p * nc + k, r >= 0 ? rs[r * P + p] : 0.0);
   }
-  // a wave per partition, lanes over the classes
+  // a group of lanes per partition, lanes over the classes: as many lanes as
+  // there are classes, at most a wave, so that many partitions with few trees
+  // are done in few rounds (64 partitions, 4 trees: 6.6 us, 34 with a wave each)
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, n_waves = blockDim.x >> 6;
-  for (int p = wave; p < P; p += n_waves) {
+  int width = 64;
+  while (width > 1 && width / 2 >= nc) width /= 2;
+  const int member = threadIdx.x & (width - 1);
+  for (int p0 = 0; p0 < P; p0 += blockDim.x / width) {
+    const int p = p0 + threadIdx.x / width, n = p < P ? nc : 0;  // (every lane takes part in the exchanges)
     // best class (first maximum in class order)
     double best = -INFINITY;
     int arg = -1;
-    for (int k = lane; k < nc; k += 64) {
+    for (int k = member; k < n; k += width) {
       const double v = used(k) ? logprob(k) + rs[root_of(k) * P + p] : -INFINITY;
       if (v > best) {
         best = v;
         arg = k;
       }
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
+    for (int off = width / 2; off > 0; off >>= 1) {
       const double v = __shfl_xor(best, off);
       const int k = __shfl_xor(arg, off);
       if (v > best || (v == best && k >= 0 && (arg < 0 || k < arg))) {
@@ -491,7 +496,7 @@ __device__ void mixture_body(const DevLayout &L, int n_root, int nc, int R, int 
       }
     }
     double sum = 0.0;
-    for (int k = lane; k < nc; k += 64) {
+    for (int k = member; k < n; k += width) {
       double a = 0.0;
       if (variant == 1)
         a = k == arg ? 1.0 : 0.0;
@@ -500,10 +505,10 @@ __device__ void mixture_body(const DevLayout &L, int n_root, int nc, int R, int 
       alpha[p * nc + k] = a;
       sum += a;
     }
-    sum = lane_sum(sum);
+    for (int off = width / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
     if (variant != 1)
-      for (int k = lane; k < nc; k += 64) alpha[p * nc + k] = sum > 0.0 ? alpha[p * nc + k] / sum : 0.0;
-    if (lane == 0) {
+      for (int k = member; k < n; k += width) alpha[p * nc + k] = sum > 0.0 ? alpha[p * nc + k] / sum : 0.0;
+    if (member == 0 && p < P) {
       per_part[p] = variant == 1 ? best : best + log(sum);
       put(rl.per_part + p, per_part[p]);
     }
@@ -3665,10 +3670,12 @@ void launch_forward_walk(Engine &e, const DevOp *ops, int n_ops) {
 
 void launch_mixture(Engine &e, int variant, int pw, double *host) {
   const int nr = static_cast<int>(e.root_slots.size());
-  // root sums of few partials are formed by the mixture's workgroup, which
-  // saves a launch (4.8 us with the gap); it adds about 500 partials per us
+  // few root sums of few partials are formed by the mixture's workgroup, which
+  // saves a launch (4.8 us with the gap): it adds about 500 partials per us, and
+  // a sum takes one of its four waves 1 us (lnL of 12 taxa: 16 sums 47 us either
+  // way, 32 sums 59 us in the workgroup, 54 before it, 256 sums 96 and 42)
   const int64_t n_wt = static_cast<int64_t>(e.L.n_tiles) * pw;
-  const bool fused = nr * n_wt <= MIX_PARTIALS;
+  const bool fused = nr * n_wt <= MIX_PARTIALS && nr * e.P <= MIX_ROWS;
   if (!fused) {
     hipLaunchKernelGGL(k_reduce_segments, dim3(nr * e.P), dim3(256), 0, e.stream, e.d_root_partials.as<double>(),
                        static_cast<size_t>(n_wt), pw, e.d_part_tile_begin.as<int32_t>(), e.P,
