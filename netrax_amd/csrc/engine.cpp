@@ -54,15 +54,22 @@ int guarded(F &&f) {
 }
 
 // Host-to-device copy of a (pageable, possibly short-lived) host vector;
-// waits for completion so the source may be freed right after.
+// waits for completion so the source may be freed right after (`wait` false:
+// the caller waits for the stream while the source lives).
 template <typename T>
-void upload(DevBuf &b, const std::vector<T> &v, hipStream_t s) {
+void upload(DevBuf &b, const std::vector<T> &v, hipStream_t s, bool wait = true) {
   b.alloc(std::max<size_t>(sizeof(T) * v.size(), 16));
-  if (!v.empty()) {
-    NRX_HIP(hipMemcpyAsync(b.p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice, s));
-    NRX_HIP(hipStreamSynchronize(s));
-  }
+  if (v.empty()) return;
+  NRX_HIP(hipMemcpyAsync(b.p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice, s));
+  if (wait) NRX_HIP(hipStreamSynchronize(s));
 }
+
+// Waits for a stream whichever way its scope ends: what was put on it reads
+// host memory of the caller's.
+struct StreamDrain {
+  hipStream_t s;
+  ~StreamDrain() { (void)hipStreamSynchronize(s); }
+};
 
 }  // namespace
 
@@ -1239,7 +1246,7 @@ static void build_batch(Batch &b) {
     assign_reverse_slots(ops.data() + at + n_ops, static_cast<int>(n_ops), b.shape.adj_slots);
     *b.handoffs[i] = lds_handoffs(ops.data() + at + n_ops, n_ops);
   }
-  upload(b.d_ops, ops, b.stream);
+  b.d_ops.alloc(sizeof(DevOp) * std::max<size_t>(ops.size(), 1));
   size_t first_op = 0;
   for (int i = 0; i < n; ++i) {
     const Engine &e = *b.engines[i];
@@ -1270,10 +1277,14 @@ static void build_batch(Batch &b) {
     for (int t = 0; t < b.engines[o.second]->L.n_tiles * gwpt; ++t) work.push_back({o.second, t});
   }
   b.n_work = static_cast<int>(work.size());
-  upload(b.d_nets, nets, b.stream);
-  upload(b.d_small, small, b.stream);
-  upload(b.d_work, work, b.stream);
-  upload(b.d_offsets, b.offsets, b.stream);
+  {
+    const StreamDrain drain{b.stream};  // one wait for all
+    upload(b.d_ops, ops, b.stream, false);
+    upload(b.d_nets, nets, b.stream, false);
+    upload(b.d_small, small, b.stream, false);
+    upload(b.d_work, work, b.stream, false);
+    upload(b.d_offsets, b.offsets, b.stream, false);
+  }
   if (b.h_out) NRX_HIP(hipHostFree(b.h_out));
   NRX_HIP(hipHostMalloc(reinterpret_cast<void **>(&b.h_out), sizeof(double) * b.offsets[n],
                         hipHostMallocDefault));
@@ -1356,10 +1367,7 @@ int nrx_batch_evaluate(nrx_batch *batch, int32_t variant, double *lnl, double *d
     }
     // the batch's kernels read the engines' pinned lengths: they have ended
     // whichever way this call ends
-    struct Drain {
-      hipStream_t s;
-      ~Drain() { (void)hipStreamSynchronize(s); }
-    } drain{b.stream};
+    const StreamDrain drain{b.stream};
     const bool grad = dbrlen != nullptr;
     auto enqueue = [&]() {
       const SmallDesc *sd = b.d_small.as<SmallDesc>();
