@@ -435,7 +435,6 @@ static void build_schedule(Engine &e) {
     dc[k].root_index = e.class_root_index[k];
     dc[k].use = e.class_use[k];
   }
-  upload(e.d_ops, e.ops_all, e.stream);
   if (e.opt.precision == NRX_FP64 || e.S == AA_STATES) {
     choose_walk_shape(e);
     e.gwpt = e.S == AA_STATES ? e.rpw * e.C : e.rpw;
@@ -452,15 +451,14 @@ static void build_schedule(Engine &e) {
   upload(e.d_edge_use_list, e.edge_use_list, e.stream);
   upload(e.d_classes, dc, e.stream);
   upload(e.d_class_dlogprob, e.class_dlogprob, e.stream);
-  std::vector<int32_t> rs(e.root_slots.begin(), e.root_slots.end());
-  upload(e.d_root_slots, rs, e.stream);
+  const size_t n_root = std::max<size_t>(1, e.root_slots.size());
   const size_t n_wt = static_cast<size_t>(e.L.n_tiles) * e.rpw;
   const size_t n_gwt = static_cast<size_t>(e.L.n_tiles) * e.gwpt;
-  e.d_root_partials.alloc(sizeof(double) * std::max<size_t>(1, rs.size()) * n_wt);
-  e.d_beta.alloc(sizeof(double) * std::max<size_t>(1, rs.size()) * e.P);
+  e.d_root_partials.alloc(sizeof(double) * n_root * n_wt);
+  e.d_beta.alloc(sizeof(double) * n_root * e.P);
   e.d_grad_partials.alloc(sizeof(double) * std::max(1, e.n_uses) * n_gwt);
-  e.d_site_seed.alloc(sizeof(double) * std::max<size_t>(1, rs.size()) * e.L.n_sites_pad);
-  e.d_root_sums.alloc(sizeof(double) * std::max<size_t>(1, rs.size()) * e.P);
+  e.d_site_seed.alloc(sizeof(double) * n_root * e.L.n_sites_pad);
+  e.d_root_sums.alloc(sizeof(double) * n_root * e.P);
   e.d_use_sums.alloc(sizeof(double) * std::max(1, e.n_uses) * static_cast<size_t>(e.P) * GRAD_SLICES);
   stream_sync(e);
   upload_netdesc(e);
@@ -1514,7 +1512,6 @@ int nrx_create(const nrx_network_desc *net, const nrx_partition_desc *parts, int
     DevLayout &L = e->L;
     L.n_sites_pad = off;
     L.n_tiles = tile;
-    L.n_tiles_grid = (tile + 7) / 8 * 8;
     L.n_parts = n_parts;
     L.n_edges = e->E;
     L.S = e->S;

@@ -171,7 +171,6 @@ struct DevClass {
 struct DevLayout {
   int64_t n_sites_pad;   // sites over all partitions, tile padded
   int32_t n_tiles;
-  int32_t n_tiles_grid;  // n_tiles rounded up to a multiple of 8 (XCDs)
   int32_t n_parts;
   int32_t n_edges;
   int32_t S;

@@ -154,13 +154,13 @@ struct Engine : nrx_engine {
   DevBuf d_clv, d_scl, d_adj, d_adj_exp, d_Qf;
   DevBuf d_PA;  // 20-state FP64 form: P and P^T in operand order
   DevBuf d_Pa;  // 20-state FP32 form: likewise
-  DevBuf d_ops, d_ops_dirty, d_Qd;
+  DevBuf d_ops_dirty, d_Qd;
   DevBuf d_ops_fwd, d_ops_adj;  // the walks' op lists
   // FP32 form, incremental evaluation: the invalid ops and their descriptor
   DevBuf d_ops_inc, d_netdesc_inc;
   DevBuf d_edge_use_begin, d_edge_use_list;
   DevBuf d_netdesc, d_work;  // FP32 form: this engine's NetDesc and (0, tile) work table
-  DevBuf d_classes, d_class_dlogprob, d_root_slots;
+  DevBuf d_classes, d_class_dlogprob;
   DevBuf d_root_partials, d_beta, d_grad_partials, d_root_sums, d_use_sums;
   DevBuf d_site_seed;  // plain form: adjoint seed factor w / (C Ltilde) [root][site]
   DevBuf d_result;
