@@ -291,10 +291,11 @@ __device__ __forceinline__ void tip_vec(uint32_t mask, double (&x)[S]) {
   for (int i = 0; i < S; ++i) x[i] = ((mask >> i) & 1u) ? 1.0 : 0.0;
 }
 
-// y = M x for one S x S row-major matrix.  (20 states: in pieces of two rows,
-// which keeps M, where it is in scalar registers, from spilling: sumtables of
-// 2,000 patterns, 4 categories 91 us against 108.)
-template <int S>
+// y = M x for one S x S row-major matrix.  PIECES: two rows at a time, which
+// keeps a matrix of 20 states, where it is in scalar registers, from spilling
+// (sumtables of 2,000 patterns, 4 categories 91 us against 108; the kernel that
+// evaluates them as well has more registers in use and is 3 % faster without).
+template <int S, bool PIECES>
 __device__ __forceinline__ void matvec(const double *__restrict__ M, const double (&x)[S],
                                        double (&y)[S]) {
 #pragma unroll
@@ -303,23 +304,31 @@ __device__ __forceinline__ void matvec(const double *__restrict__ M, const doubl
 #pragma unroll
     for (int j = 0; j < S; ++j) s = fma(M[i * S + j], x[j], s);
     y[i] = s;
-    if constexpr (S == AA_STATES)
-      if (i % 2) __builtin_amdgcn_sched_barrier(0);
+    if (PIECES && i % 2) __builtin_amdgcn_sched_barrier(0);
   }
 }
 
-// y = M^T x, row by row of M
-template <int S>
+// y = M^T x (PIECES: row by row of M, which adds each sum's terms in the same order)
+template <int S, bool PIECES>
 __device__ __forceinline__ void matvec_t(const double *__restrict__ M, const double (&x)[S],
                                          double (&y)[S]) {
+  if constexpr (PIECES) {
 #pragma unroll
-  for (int j = 0; j < S; ++j) y[j] = 0.0;
+    for (int j = 0; j < S; ++j) y[j] = 0.0;
 #pragma unroll
-  for (int i = 0; i < S; ++i) {
+    for (int i = 0; i < S; ++i) {
 #pragma unroll
-    for (int j = 0; j < S; ++j) y[j] = fma(M[i * S + j], x[i], y[j]);
-    if constexpr (S == AA_STATES)
+      for (int j = 0; j < S; ++j) y[j] = fma(M[i * S + j], x[i], y[j]);
       if (i % 2) __builtin_amdgcn_sched_barrier(0);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < S; ++j) {
+      double s = 0.0;
+#pragma unroll
+      for (int i = 0; i < S; ++i) s = fma(M[i * S + j], x[i], s);
+      y[j] = s;
+    }
   }
 }
 
@@ -2877,7 +2886,7 @@ __device__ __forceinline__ size_t clv_row(int64_t site, int c) {
   }
 }
 
-template <int S, int C, typename T, typename CatSum>
+template <int S, int C, typename T, bool PIECES, typename CatSum>
 __device__ __forceinline__ void path_sumtable(CatSum over_cats, const PathStep *__restrict__ steps, int b0, int b1,
                                               const double *sPp, int n_staged, const DevLayout &L,
                                               int part, int64_t site, int c, const T *__restrict__ clv,
@@ -2937,7 +2946,7 @@ __device__ __forceinline__ void path_sumtable(CatSum over_cats, const PathStep *
             tip_vec<S>(tm[u], xs[u]);
           else
             ksu = scl_count<S, T>(ks[u]);
-          matvec<S>(prow(j, 1, ps.edge_sib), xs[u], y);
+          matvec<S, PIECES>(prow(j, 1, ps.edge_sib), xs[u], y);
         } else {
 #pragma unroll
           for (int i = 0; i < S; ++i) y[i] = 1.0;
@@ -2948,13 +2957,13 @@ __device__ __forceinline__ void path_sumtable(CatSum over_cats, const PathStep *
 #pragma unroll
         for (int i = 0; i < S; ++i) z[i] = a[i] * F * y[i];
         if (s0 + u + 1 < b1) {
-          matvec_t<S>(prow(j, 0, ps.edge_child), z, a);  // adjoint of the on-path child
+          matvec_t<S, PIECES>(prow(j, 0, ps.edge_child), z, a);  // adjoint of the on-path child
           kq = kcu;
         } else {
           double uu[S], v[S];
           if (low < 0) tip_vec<S>(tmc, xc);
-          matvec_t<S>(V + static_cast<size_t>(part) * S * S, z, uu);  // u_k = sum_i z_i V[i][k]
-          matvec<S>(Vinv + static_cast<size_t>(part) * S * S, xc, v);  // v_k = sum_j Vinv[k][j] x_j
+          matvec_t<S, PIECES>(V + static_cast<size_t>(part) * S * S, z, uu);  // u_k = sum_i z_i V[i][k]
+          matvec<S, PIECES>(Vinv + static_cast<size_t>(part) * S * S, xc, v);  // v_k = sum_j Vinv[k][j] x_j
 #pragma unroll
           for (int kk = 0; kk < S; ++kk) st[kk] = uu[kk] * v[kk];
         }
@@ -2969,13 +2978,14 @@ __device__ __forceinline__ void path_sumtable(CatSum over_cats, const PathStep *
 // through L2 (16 paths, 41,345 patterns: 68 us, 116 with a thread per row and
 // P in LDS, 32 reads of it per row and step).
 constexpr int PATH_BATCH = 4;  // steps whose loads are issued together
-template <int C>
+// put(q, v): a lane's entry of granule q (state lane >> 4).
+template <int C, typename Put>
 __device__ __forceinline__ void path_sumtable4(const PathStep *__restrict__ steps_, int n_steps, const DevLayout &L,
                                                int part, int64_t site0, const double *__restrict__ clv_,
                                                const int32_t *__restrict__ scl_, const uint8_t *__restrict__ tips_,
                                                const double *__restrict__ P_, const double *__restrict__ V,
                                                const double *__restrict__ Vinv, const double *__restrict__ freqs,
-                                               double *__restrict__ st_) {
+                                               Put put) {
   constexpr int NQ = 4;
   using W = Quad<C, NQ>;
   constexpr int NA = W::NA, SPW = W::SPW;
@@ -3060,10 +3070,40 @@ __device__ __forceinline__ void path_sumtable4(const PathStep *__restrict__ step
   // st_k = (z^T V)_k (V^-1 x)_k
   tip_row(low, xc, rawc);
   const double vt = V[part * 16 + state * 4 + (lane & 3)], wi = Vinv[part * 16 + (lane & 3) * 4 + state];
-  GAS double *st = to_global(st_) + site0 * (C * 4);
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) *at(st, off + q * 512) = mfma4(vt, a[q], 0.0) * mfma4(wi, xc[q], 0.0);
+  for (int q = 0; q < NQ; ++q) put(q, mfma4(vt, a[q], 0.0) * mfma4(wi, xc[q], 0.0));
 }
+
+// The (site, category) of a thread that walks a path, and sums over the
+// categories of its site.  4 states: the categories of a site in adjacent lanes.
+// 20 states: a wave per category, so that P is the same for a wave and read
+// through scalar registers (branches of 30 taxa, 8 trees, 2,000 patterns, 4
+// categories: 91 us on average, 242 with every lane reading its category's P).
+template <int S, int C>
+struct PathRow {
+  static constexpr bool WAVES = S == AA_STATES;
+  int c, site;  // site within the tile
+  __device__ __forceinline__ PathRow() {
+    c = C == 1 ? 0 : WAVES ? __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / TILE)) : static_cast<int>(threadIdx.x % C);
+    site = WAVES ? threadIdx.x % TILE : threadIdx.x / C;
+  }
+  // (every thread of the workgroup takes part)
+  __device__ __forceinline__ double over_cats(double v) const {
+    if constexpr (!WAVES || C == 1) return cat_sum<C>(v);
+    __shared__ double cats[C][TILE];
+    __syncthreads();  // the sum before this one has been read
+    cats[c][site] = v;
+    __syncthreads();
+    double s[C];
+#pragma unroll
+    for (int k = 0; k < C; ++k) s[k] = cats[k][site];
+#pragma unroll
+    for (int w = 1; w < C; w *= 2)  // (in cat_sum's order)
+#pragma unroll
+      for (int k = 0; k < C; k += 2 * w) s[k] += s[k + w];
+    return s[0];
+  }
+};
 
 template <int S, int C, typename T>
 __global__ void __launch_bounds__(TILE *C)
@@ -3081,36 +3121,19 @@ __global__ void __launch_bounds__(TILE *C)
     const int tile = group * 8 + r % 8, path = r / 8;
     if (tile >= L.n_tiles) return;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    path_sumtable4<C>(steps + path_begin[path], path_begin[path + 1] - path_begin[path], L, tile_part[tile],
-                      static_cast<int64_t>(tile) * TILE + wave * Quad<C, 4>::SPW, clv, scl, tips, P, V, Vinv, freqs,
-                      st + static_cast<int64_t>(path) * L.n_sites_pad * (C * 4));
+    const int64_t site0 = static_cast<int64_t>(tile) * TILE + wave * Quad<C, 4>::SPW;
+    GAS double *out = to_global(st) + static_cast<int64_t>(path) * L.n_sites_pad * (C * 4) + site0 * (C * 4);
+    const uint32_t off = (threadIdx.x & 63) * 8;
+    path_sumtable4<C>(steps + path_begin[path], path_begin[path + 1] - path_begin[path], L, tile_part[tile], site0, clv,
+                      scl, tips, P, V, Vinv, freqs, [&](int q, double v) { *at(out, off + q * 512) = v; });
     return;
   } else {
   double *sPp = dyn_lds<double>();
   const int tile = blockIdx.x;
   const int part = tile_part[tile];
-  // 4 states: the categories of a site in adjacent lanes.  20 states: a wave per
-  // category, so that P is the same for a wave and read through scalar registers
-  // (branches of 30 taxa, 8 trees, 2,000 patterns, 4 categories: 91 us on average,
-  // 242 with every lane reading its category's P)
-  constexpr bool WAVES = S == AA_STATES;
-  __shared__ double cats[WAVES ? C : 1][TILE];
-  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / TILE)), lane = threadIdx.x % TILE;
-  const int c = WAVES ? wave : static_cast<int>(threadIdx.x % C);
-  const int64_t site = static_cast<int64_t>(tile) * TILE + (WAVES ? lane : static_cast<int>(threadIdx.x / C));
-  auto over_cats = [&](double v) {
-    if constexpr (!WAVES) return cat_sum<C>(v);
-    cats[c][lane] = v;
-    __syncthreads();
-    double s[C];
-#pragma unroll
-    for (int k = 0; k < C; ++k) s[k] = cats[k][lane];
-#pragma unroll
-    for (int w = 1; w < C; w *= 2)  // (in cat_sum's order)
-#pragma unroll
-      for (int k = 0; k < C; k += 2 * w) s[k] += s[k + w];
-    return s[0];
-  };
+  const PathRow<S, C> row;
+  const int c = row.c;
+  const int64_t site = static_cast<int64_t>(tile) * TILE + row.site;
   // one displayed tree's path per workgroup (grid tiles x paths): the path
   // walks are independent, and one per workgroup fills the GPU
   const int j = blockIdx.y;
@@ -3119,8 +3142,8 @@ __global__ void __launch_bounds__(TILE *C)
   const int n_staged = S == 4 ? min(b1 - b0, PATH_STAGED_STEPS) : 0;
   stage_path_p<S, C>(sPp, steps + b0, n_staged, P, part, L);
   double stv[S];
-  path_sumtable<S, C, T>(over_cats, steps, b0, b1, sPp, n_staged, L, part, site, c, clv, scl, scale_unit, tips, P, V,
-                         Vinv, freqs, stv);
+  path_sumtable<S, C, T, S == AA_STATES>([&](double v) { return row.over_cats(v); }, steps, b0, b1, sPp, n_staged, L, part, site, c,
+                         clv, scl, scale_unit, tips, P, V, Vinv, freqs, stv);
   store_st<S>(st + static_cast<size_t>(j) * L.n_sites_pad * (C * S) + st_offset<S, C>(site, c), stv);
   }
 }
@@ -3128,8 +3151,8 @@ __global__ void __launch_bounds__(TILE *C)
 // Per displayed tree j and wave: sums over sites of w log rho(b),
 // w rho'/rho and w (rho''/rho - (rho'/rho)^2) at branch length b, from the
 // sumtable row of (site, category).
-template <int S, int C>
-__device__ __forceinline__ void sumtable_partials(const double (&in)[S], const double (&ex)[S],
+template <int S, int C, typename CatSum>
+__device__ __forceinline__ void sumtable_partials(CatSum over_cats, const double (&in)[S], const double (&ex)[S],
                                                   const double (&lr)[S], double w, int c, double *out3) {
   double t0 = 0.0, t1 = 0.0, t2 = 0.0;
 #pragma unroll
@@ -3139,9 +3162,9 @@ __device__ __forceinline__ void sumtable_partials(const double (&in)[S], const d
     t1 += q * lr[k];
     t2 += q * lr[k] * lr[k];
   }
-  t0 = cat_sum<C>(t0);
-  t1 = cat_sum<C>(t1);
-  t2 = cat_sum<C>(t2);
+  t0 = over_cats(t0);
+  t1 = over_cats(t1);
+  t2 = over_cats(t2);
   double v0 = 0.0, v1 = 0.0, v2 = 0.0;
   if (c == 0 && w != 0.0) {
     const double r1 = t1 / t0;
@@ -3200,7 +3223,7 @@ __global__ void __launch_bounds__(TILE *C)
   for (int j = blockIdx.y; j < min(n_paths, static_cast<int>(blockIdx.y) + 1); ++j) {
     double stv[S], v[3];
     load_st<S>(st + static_cast<size_t>(j) * slot + ro, stv);
-    sumtable_partials<S, C>(stv, ex, lr, w, c, v);
+    sumtable_partials<S, C>([](double x) { return cat_sum<C>(x); }, stv, ex, lr, w, c, v);
     if ((threadIdx.x & 63) == 0)
 #pragma unroll
       for (int q = 0; q < 3; ++q) partials[(static_cast<size_t>(j) * 3 + q) * n_wt + wt] = v[q];
@@ -3241,7 +3264,7 @@ __global__ void __launch_bounds__(TILE *C)
   for (int j = blockIdx.y; j < min(n_paths, static_cast<int>(blockIdx.y) + 1); ++j) {
     double stv[S], v[3];
     load_st<S>(st + static_cast<size_t>(j) * slot + ro, stv);
-    sumtable_partials<S, C>(stv, ex, lr, w, c, v);
+    sumtable_partials<S, C>([](double x) { return cat_sum<C>(x); }, stv, ex, lr, w, c, v);
     if ((threadIdx.x & 63) == 0)
 #pragma unroll
       for (int q = 0; q < 3; ++q) partials[(static_cast<size_t>(j) * 3 + q) * n_wt + wt] = v[q];
@@ -3497,10 +3520,60 @@ __global__ void __launch_bounds__(TILE *C)
   constexpr int PW = TILE * C / 64;
   const int tile = blockIdx.x;
   const int part = tile_part[tile];
-  const int c = threadIdx.x % C;
-  const int64_t site = static_cast<int64_t>(tile) * TILE + threadIdx.x / C;
   const size_t n_wt = static_cast<size_t>(L.n_tiles) * PW;
   const int wt = tile * PW + threadIdx.x / 64;
+  if constexpr (S == 4 && std::is_same<T, double>::value) {
+    // on the matrix cores, as the sumtables; a lane's entries are of one state
+    // and category (of two, with 8 categories), and the sums over the states are
+    // products with ones (30 taxa, 8 trees, 20,000 patterns, 4 categories, the
+    // whole call: 90 us, 107 with a thread per row)
+    using W = Quad<C, 4>;
+    constexpr int NA = W::NA, SPW = W::SPW;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int64_t site0 = static_cast<int64_t>(tile) * TILE + wave * SPW;
+    const double w = lane < SPW ? weights[site0 + lane % SPW] : 0.0;
+    double lr[NA], ex[NA];
+#pragma unroll
+    for (int h = 0; h < NA; ++h) {
+      lr[h] = ev[part * 4 + (lane >> 4)] * rates[part * C + W::cat(lane, h)];
+      ex[h] = exp(lr[h] * brlen);
+    }
+    for (int j = 0; j < n_paths; ++j) {
+      double x[4];
+      path_sumtable4<C>(steps + path_begin[j], path_begin[j + 1] - path_begin[j], L, part, site0, clv, scl, tips, P, V,
+                        Vinv, freqs, [&](int q, double v) { x[q] = v; });
+      double t[3] = {1.0, 0.0, 0.0};  // rho and its derivatives at site lane % SPW
+#pragma unroll
+      for (int q = 0; q < 4; q += NA) {
+        double r[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+        for (int h = 0; h < NA; ++h) {
+          double v = x[q + h] * ex[h];
+#pragma unroll
+          for (int d = 0; d < 3; ++d, v *= lr[h]) r[d] = mfma4(1.0, v, r[d]);
+        }
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          if constexpr (C >= 4) r[d] += dpp<0x124>(r[d]);  // row_ror:4
+          if constexpr (C >= 2) r[d] += dpp<0x128>(r[d]);  // row_ror:8
+          if ((lane % SPW) / (4 * W::SB) == q / NA) t[d] = r[d];
+        }
+      }
+      const double r1 = t[1] / t[0];
+      const double v[3] = {w != 0.0 ? w * log(t[0]) : 0.0, w != 0.0 ? w * r1 : 0.0,
+                           w != 0.0 ? w * (t[2] / t[0] - r1 * r1) : 0.0};
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const double sum = wave_sum(v[d]);
+        if (lane == 0) partials[(static_cast<size_t>(j) * 3 + d) * n_wt + wt] = sum;
+      }
+    }
+    return;
+  } else {
+  const PathRow<S, C> row;
+  const int c = row.c;
+  const int64_t site = static_cast<int64_t>(tile) * TILE + row.site;
+  const auto over_cats = [&](double v) { return row.over_cats(v); };
   const double w = weights[site];
   double ex[S], lr[S];
   stage_exps<S, C>(ev, rates, part, brlen, c, ex, lr);
@@ -3511,12 +3584,13 @@ __global__ void __launch_bounds__(TILE *C)
     const int n_staged = S == 4 ? min(b1 - b0, PATH_STAGED_STEPS) : 0;
     if (S == 4 && j > 0) __syncthreads();  // every lane is done with the previous path's staged P
     stage_path_p<S, C>(sPp, steps + b0, n_staged, P, part, L);
-    path_sumtable<S, C, T>([](double x) { return cat_sum<C>(x); }, steps, b0, b1, sPp, n_staged, L, part, site, c, clv,
-                           scl, scale_unit, tips, P, V, Vinv, freqs, stv);
-    sumtable_partials<S, C>(stv, ex, lr, w, c, v);
+    path_sumtable<S, C, T, false>(over_cats, steps, b0, b1, sPp, n_staged, L, part, site, c, clv, scl, scale_unit, tips, P, V,
+                           Vinv, freqs, stv);
+    sumtable_partials<S, C>(over_cats, stv, ex, lr, w, c, v);
     if ((threadIdx.x & 63) == 0)
 #pragma unroll
       for (int q = 0; q < 3; ++q) partials[(static_cast<size_t>(j) * 3 + q) * n_wt + wt] = v[q];
+  }
   }
 }
 
@@ -3903,7 +3977,7 @@ void launch_deriv_fused(Engine &e, const PathStep *steps, const int32_t *path_be
                          e.d_Vinv.as<double>(), e.d_freqs.as<double>(), e.d_eval.as<double>(),
                          e.d_rates.as<double>(), e.d_weights.as<double>(), brlen, partials);
     else
-      hipLaunchKernelGGL((k_deriv_fused<S, C, double>), dim3(e.L.n_tiles), dim3(TILE * C), lds, e.stream, steps,
+      hipLaunchKernelGGL((k_deriv_fused<S, C, double>), dim3(e.L.n_tiles), dim3(TILE * C), S == 4 ? 0 : lds, e.stream, steps,
                          path_begin, n_paths, e.L, e.d_tile_part.as<int32_t>(),
                          e.d_clv.as<double>(), e.d_scl.as<int32_t>(), 256, e.d_tips.as<TT>(),
                          e.d_P.as<double>(), e.d_V.as<double>(), e.d_Vinv.as<double>(), e.d_freqs.as<double>(),
