@@ -127,6 +127,16 @@ def pmc_traffic(kernel):
         return None
 
 
+def batched_kernel(step, group_width, n_sites_padded, ncat=4):
+    """Name of the FP32 4-state walk (step: "forward" or "adjoint") that a shape
+    runs: the second argument is 2 for two 64-row blocks per wave, 3 for one.
+    Group widths 2 and 3 name them, with any other the engine takes two once
+    that leaves 2,048 waves (walk_blocks_of in engine.cpp)."""
+    blocks = n_sites_padded * ncat // 64
+    two = group_width == 2 or (group_width != 3 and blocks // 2 >= 2048)
+    return f"k_{step}_persistent<{ncat}, {2 if two and ncat > 1 else 3}, 64>"
+
+
 def roofline(res, ncat=4):
     st = res["stats"]
     kern = [("forward pruning", st.fwd_op_bytes, res["fwd_ms_per_eval"], res["fwd_launches_per_eval"]),
@@ -135,11 +145,9 @@ def roofline(res, ncat=4):
     achieved = by / (ms * 1e-3) / 1e9 if ms > 0 else 0.0
     t = res.get("tuning")
     step = "forward" if name.startswith("forward") else "adjoint"
-    if t:  # persistent form: one launch per evaluation
-        split = step == "adjoint" and t.get("row_lanes", 1) == 2
-        kname = (f"k_adjoint_split<{ncat}, {t['group_width']}, {t['tile_sites']}>" if split else
-                 f"k_{step}_persistent<{ncat}, {t['group_width']}, {t['tile_sites']}>")
-    else:  # plain form: one forward and one reverse-sweep launch walking every level
+    if t:
+        kname = batched_kernel(step, t["group_width"], st.n_sites_padded, ncat)
+    else:
         kname = f"k_adjoint_level<4, {ncat}>" if step == "adjoint" else f"k_forward_walk<4, {ncat}, 4>"
     traffic = pmc_traffic(kname)
     return {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBPS, "unit": "GB/s",
@@ -151,15 +159,20 @@ def roofline(res, ncat=4):
 
 
 MFMA_FP32_PEAK_TFLOPS = 157.3
-MFMA_FLOPS_32x32x2 = 32 * 32 * 2 * 2  # one v_mfma_f32_32x32x2f32
+# matrix-instruction flops of one product of the 20-state FP32 walks: a category
+# of 16 sites with a 20 x 20 matrix
+FLOPS_16x16x4, FLOPS_4x4x1 = 16 * 16 * 4 * 2, 16 * 4 * 4 * 1 * 2  # the latter: 16 blocks
+AA_FWD_FLOPS = 10 * FLOPS_16x16x4  # rows 0-15, and rows 16-19 in a 16-row chain
+AA_ADJ_FLOPS = 5 * FLOPS_16x16x4 + 5 * FLOPS_4x4x1  # rows 16-19 in blocks: no padding
+AA_USEFUL_FLOPS = 20 * 20 * 16 * 2
 
 
 def bench_protein(steps, warmup):
     """40 taxa / 2 reticulations / 20,000 amino-acid sites, GTR-like 20-state
     model + G4: plain FP64 form vs the FP32 matrix-core form; matrix-core
-    utilisation of the FP32 kernels from the instruction count the op list
-    implies (10 instructions per (op, child, category, 32-site tile) forward;
-    20 + 10 per inner child in the adjoint)."""
+    utilisation of the FP32 kernels from the products the op list implies (per
+    category of 16 sites one per (op, child) forward; two, and another per
+    inner child, in the adjoint)."""
     from netrax_amd.simulate import workload_protein_20k
 
     w = workload_protein_20k()
@@ -179,16 +192,17 @@ def bench_protein(steps, warmup):
              "adj_hbm_gbps": round(st.adj_bytes / (r["adj_ms_per_eval"] * 1e-3) / 1e9, 1)}
         if prec == 1:
             C = w.partitions[0].model.ncat
-            blocks = st.n_sites_padded // 32 * C
-            fwd_fl = st.n_uses * blocks * 10 * MFMA_FLOPS_32x32x2
-            adj_fl = (2 * st.n_uses + st.n_inner_uses) * blocks * 10 * MFMA_FLOPS_32x32x2
+            waves = st.n_sites_padded // 16 * C
+            fwd_fl = st.n_uses * waves * AA_FWD_FLOPS
+            adj_fl = (2 * st.n_uses + st.n_inner_uses) * waves * AA_ADJ_FLOPS
             fu = fwd_fl / (r["fwd_ms_per_eval"] * 1e-3) / 1e12
             au = adj_fl / (r["adj_ms_per_eval"] * 1e-3) / 1e12
             d["mfma"] = {"peak_tflops": MFMA_FP32_PEAK_TFLOPS,
                          "fwd_tflops": round(fu, 2), "fwd_util": round(fu / MFMA_FP32_PEAK_TFLOPS, 4),
                          "adj_tflops": round(au, 2), "adj_util": round(au / MFMA_FP32_PEAK_TFLOPS, 4),
-                         "useful_fraction": round(400 / 640, 4),
-                         "note": "issued matrix-instruction flops (20 states padded to 32 rows)"}
+                         "fwd_useful_fraction": round(AA_USEFUL_FLOPS / AA_FWD_FLOPS, 4),
+                         "adj_useful_fraction": round(AA_USEFUL_FLOPS / AA_ADJ_FLOPS, 4),
+                         "note": "issued matrix-instruction flops (forward: rows 16-19 in a 16-row chain)"}
             d["tuning"] = r["tuning"]
         out[name] = d
         log(f"protein {name}: {r['evals_per_s']:.1f} evals/s, fwd {r['fwd_ms_per_eval']:.3f} ms, "
@@ -451,13 +465,12 @@ def bench_tile_sweep(tile_counts, steps, warmup, protein=False):
     """Forward and reverse-sweep time of both forms against the number of
     64-site tiles: the headline network (50 taxa, 4 reticulations, seed 3)
     with two uncompressed partitions holding 2/5 and 3/5 of the tiles, the
-    batched form at a fixed shape (3 ops per group, 64-site tiles, or
-    --shape).  A time that stays nearly flat while the tiles per CU grow,
-    then jumps when the tiles outnumber the resident workgroups, marks a
-    walk bound by its per-tile dependency chain, not by HBM.  With
-    `protein`: the 40-taxon, 2-reticulation protein network (seed 4), one
-    uncompressed partition, plain FP64 form and the FP32 matrix-core form
-    (4 ops per group; two 32-site workgroups per tile)."""
+    batched form at a fixed shape (one row block per wave, or --shape).  A
+    time that stays nearly flat while the tiles per CU grow, then jumps when
+    the waves outnumber the resident ones, marks a walk bound by its chain of
+    ops, not by HBM.  With `protein`: the 40-taxon, 2-reticulation protein
+    network (seed 4), one uncompressed partition, plain FP64 form and the
+    FP32 form (both on the matrix cores)."""
     global SHAPE
     from netrax_amd.simulate import make_workload
 
@@ -599,8 +612,8 @@ def main():
     ap.add_argument("--steps", type=int, default=40)
     ap.add_argument("--warmup", type=int, default=5)
     ap.add_argument("--form", choices=["batched", "plain"], default="batched",
-                    help="headline form: batched = FP32 CLVs, persistent site-tile kernels; "
-                         "plain = FP64 CLVs, one launch per pass walking every pruning level")
+                    help="headline form: batched = FP32 CLVs; plain = FP64 CLVs; one launch per "
+                         "pass in either, a wave per 16 (FP32 also 32) sites walking every op")
     ap.add_argument("--only", choices=["batched", "plain", "protein", "candidates", "sweep", "widened"],
                     default=None,
                     help="time only this form or section (profiling runs)")
@@ -615,9 +628,9 @@ def main():
     ap.add_argument("--stream-reference", action="store_true",
                     help="print the plain-stream HBM rates of this GPU (torch kernels) and exit")
     ap.add_argument("--shape", default=None, metavar="GxTSxH",
-                    help="fixed FP32 kernel shape (ops per group x sites per workgroup x lanes "
-                         "per row in the reverse sweep) instead of autotuning, e.g. 3x64x2 "
-                         "(profiling runs)")
+                    help="fixed FP32 kernel shape instead of autotuning, e.g. 3x64x1 (profiling "
+                         "runs): the first number chooses the row blocks of a wave (2: two, "
+                         "3: one, others: by size), the others name the same kernels")
     ap.add_argument("--tile-sweep", default=None, metavar="T1,T2,...",
                     help="only time both forms on the headline network at these numbers of "
                          "64-site tiles (uncompressed synthetic partitions)")
@@ -691,9 +704,9 @@ def main():
     head = forms[head_name]
     st = head["stats"]
     desc = {"plain": "plain FP64 (FP64 CLVs and adjoint; one forward and one reverse-sweep launch, a "
-                     "workgroup per site tile walking every pruning level)",
-            "batched": "batched FP32 (FP32 CLVs + per-site power-of-two exponents, one persistent "
-                       "site-tile launch for all ops and trees, FP32 adjoint with per-site "
+                     "wave per 16 sites walking every op depth first on the matrix cores)",
+            "batched": "batched FP32 (FP32 CLVs + per-site power-of-two exponents, one launch for all "
+                       "ops and trees, a wave per 16 or 32 sites, FP32 adjoint with per-site "
                        "exponents, FP64 site sums / mixture / gradient reduction; each evaluation "
                        "replays one captured HIP graph)"}
     out = {

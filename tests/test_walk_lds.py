@@ -2,39 +2,23 @@
 dynamic LDS of their slots and what the built kernels declare besides
 (group_segment_fixed_size of the code object).  CPU only."""
 import os
-import re
 import shutil
 import subprocess
 
 import pytest
 
+from code_object import kernels
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
-LIB = os.path.join(ROOT, "netrax_amd", "libnetrax_gpu.so")
-LLVM = "/opt/rocm/llvm/bin"
 HIP_INCLUDE = "/opt/rocm/include"
 CUS, LDS_PER_CU, PIECE = 256, 160 * 1024, 1280
 
 
 @pytest.fixture(scope="module")
 def fixed_lds(tmp_path_factory):
-    objcopy = shutil.which("objcopy")
-    bundler, readelf = os.path.join(LLVM, "clang-offload-bundler"), os.path.join(LLVM, "llvm-readelf")
-    if not os.path.exists(LIB) or objcopy is None or not (os.path.exists(bundler) and os.path.exists(readelf)):
-        pytest.skip("the HIP library or the tools are not available")
-    d = tmp_path_factory.mktemp("codeobj")
-    fat, co = str(d / "fatbin.bin"), str(d / "gfx950.co")
-    subprocess.run([objcopy, "--dump-section", f".hip_fatbin={fat}", LIB, str(d / "lib.so")], check=True)
-    subprocess.run([bundler, "--unbundle", "--type=o", f"--input={fat}",
-                    "--targets=hipv4-amdgcn-amd-amdhsa--gfx950", f"--output={co}"], check=True)
-    notes = subprocess.run([readelf, "--notes", co], check=True, capture_output=True, text=True).stdout
-    out = {}
-    for entry in re.split(r"\n  - \.", notes):
-        name = re.search(r"\n\s+\.name:\s+(\S+)", "\n" + entry)
-        size = re.search(r"group_segment_fixed_size:\s+(\d+)", entry)
-        if name and size:
-            out[name.group(1)] = int(size.group(1))
-    return out
+    field = "group_segment_fixed_size"
+    return {n: f[field] for n, f in kernels(tmp_path_factory.mktemp("codeobj"), field).items() if field in f}
 
 
 @pytest.fixture(scope="module")
