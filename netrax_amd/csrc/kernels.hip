@@ -1901,17 +1901,41 @@ __device__ __forceinline__ f32x4 scale4(const f32x4 &x, int e) {
   return y;
 }
 
-// Sums over the 64 lanes of two FP32 values at once, in a fixed order: lane
-// 31 ends with a's total, lane 63 with b's (see pair_wave_sum).
-__device__ __forceinline__ float pair_wave_sum_f32(float a, float b) {
-  const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-  float v = __uint_as_float(s[0]) + __uint_as_float(s[1]);
-  v += dpp<0x111>(v);
-  v += dpp<0x112>(v);
-  v += dpp<0x114>(v);
-  v += dpp<0x118>(v);
-  v += dpp<0x142>(v);
-  return v;
+// Sums over the 64 lanes of pairs of FP32 values at once, in a fixed order: lane
+// 31 of v[r] ends with the total of g[r][0], lane 63 with that of g[r][1] (see
+// pair_wave_sum).  The pairs take each step in turn, so that a step need not
+// wait for the one before it.
+template <int NR>
+__device__ __forceinline__ void pair_wave_sums_f32(const float (&g)[NR][2], float (&v)[NR]) {
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(g[r][0]), __float_as_uint(g[r][1]), false, false);
+    v[r] = __uint_as_float(s[0]) + __uint_as_float(s[1]);
+  }
+  auto step = [&](auto control) {
+#pragma unroll
+    for (int r = 0; r < NR; ++r) v[r] += dpp<decltype(control)::value>(v[r]);
+  };
+  step(std::integral_constant<int, 0x111>{});
+  step(std::integral_constant<int, 0x112>{});
+  step(std::integral_constant<int, 0x114>{});
+  step(std::integral_constant<int, 0x118>{});
+  step(std::integral_constant<int, 0x142>{});
+}
+
+// Sum of v over the lanes of a row block that hold the lane's category (C > 1),
+// in all of them.
+template <int C>
+__device__ __forceinline__ double block_total(double v) {
+  auto add = [](double x, auto &&swap) {
+    const auto lo = swap(__double2loint(x)), hi = swap(__double2hiint(x));
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+  };
+  v += dpp<DPP_XOR1>(v);
+  v += dpp<DPP_XOR2>(v);
+  if constexpr (C == 2) v += dpp<0x141>(v);  // row_half_mirror: the other quad of eight lanes
+  if constexpr (C <= 4) v = add(v, [](int x) { return __builtin_amdgcn_permlane16_swap(x, x, false, false); });
+  return add(v, [](int x) { return __builtin_amdgcn_permlane32_swap(x, x, false, false); });
 }
 
 // x 2^ex + y 2^ey with both aligned to the larger exponent, which is
@@ -2088,19 +2112,27 @@ __device__ __forceinline__ void forward_walk32(const NetDesc &nd, float *lds, in
     }
     if (op.root() >= 0) {
       // (a sum per block, whatever the number of blocks of a wave: an engine
-      // and a batch that it is in leave each other the same sums)
+      // and a batch that it is in leave each other the same sums; category r's
+      // lanes form that of block r)
+      double like = 1.0, w_like = 0.0;
+      int k_like = 0;
 #pragma unroll
       for (int r = 0; r < NR; ++r) {
         double t = 0.0;
 #pragma unroll
         for (int i = 0; i < 4; ++i) t = fma(pi[i], static_cast<double>(v[r][i]), t);
         t = site_total<C>(t) * (1.0 / C);
-        const bool counts = W::cat(lane) == 0 && w[r] != 0.0;
-        const double val = wave_sum(counts ? w[r] * (log(t) - word_k(word[r]) * LN2) : 0.0);
-        if (lane == 0) root_partials[op.root() * n_blocks + r] = val;
+        if (W::cat(lane) == r) {
+          like = t;
+          w_like = w[r];
+          k_like = word_k(word[r]);
+        }
         // the adjoint's seed factor at this root and site, w / (C Ltilde)
         seed[op.root() * static_cast<int64_t>(n) + r * W::SPB] = w[r] != 0.0 ? w[r] / (C * t) : 0.0;
       }
+      const double val = w_like != 0.0 ? w_like * (log(like) - k_like * LN2) : 0.0;
+      const double sum = C == 1 ? wave_sum(val) : block_total<C>(val);
+      if (W::cat(lane) < NR && sl == 0) root_partials[op.root() * n_blocks + W::cat(lane)] = sum;
     }
   };
   walk_ops<FwdIn32<C, NR>>(to_constant(nd.ops_fwd), nd.n_fwd, false, load,
@@ -2345,9 +2377,11 @@ __device__ __forceinline__ void adjoint_walk32(const NetDesc &nd, float *lds, in
       use(0, z);
     }
     // (rows leave as in k_adjoint_level)
-    double total = pair_wave_sum_f32(g[0][0], g[0][1]);
+    float sums[NR];
+    pair_wave_sums_f32<NR>(g, sums);
+    double total = sums[0];
 #pragma unroll
-    for (int r = 1; r < NR; ++r) total += pair_wave_sum_f32(g[r][0], g[r][1]);
+    for (int r = 1; r < NR; ++r) total += sums[r];
     const int k = lane >> 5;
     if ((lane & 31) == 31 && k < op.nk()) ring[(op.gslot() + k) % GRAD_RING] = total;
     const int done = op.gslot() + op.nk();
