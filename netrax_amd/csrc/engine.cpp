@@ -1222,7 +1222,7 @@ static void build_batch(Batch &b) {
   std::vector<std::pair<int, int>> order;  // (cost, engine)
   b.offsets.assign(n + 1, 0);
   b.max_pm = b.max_root_rows = b.max_uses = b.max_parts = b.max_edges = b.max_res = 0;
-  b.versions.resize(n);
+  b.versions.assign(n, -1);  // (of no schedule, until all tables are in place)
   b.G = b.engines[0]->tune_group;
   b.TS = b.engines[0]->tune_tile;
   b.H = b.engines[0]->tune_lanes;
@@ -1255,7 +1255,6 @@ static void build_batch(Batch &b) {
     nets[i].adj_slots = b.shape.adj_slots;
     first_op += 2 * e.ops_all.size();
     small[i] = make_smalldesc(e, gwpt);
-    b.versions[i] = e.schedule_version;
     order.push_back({static_cast<int>(e.ops_all.size()), i});
     b.offsets[i + 1] = b.offsets[i] + e.rl.size;
     b.max_pm = std::max(b.max_pm, e.P * e.E * e.C * e.S * e.S);
@@ -1283,10 +1282,12 @@ static void build_batch(Batch &b) {
     upload(b.d_work, work, b.stream, false);
     upload(b.d_offsets, b.offsets, b.stream, false);
   }
-  if (b.h_out) NRX_HIP(hipHostFree(b.h_out));
+  if (b.h_out) (void)hipHostFree(b.h_out);
+  b.h_out = nullptr;
   NRX_HIP(hipHostMalloc(reinterpret_cast<void **>(&b.h_out), sizeof(double) * b.offsets[n],
                         hipHostMallocDefault));
   NRX_HIP(hipHostGetDevicePointer(reinterpret_cast<void **>(&b.h_out_dev), b.h_out, 0));
+  for (int i = 0; i < n; ++i) b.versions[i] = b.engines[i]->schedule_version;
 }
 
 }  // namespace nrx

@@ -94,6 +94,10 @@ def test_refused_batch_leaves_the_engines_their_changes():
     for a, f in zip(anns, fresh):
         f.set_branch_lengths(a.network.brlen)
         assert a.loglikelihood() == f.loglikelihood(0)
+    # with one shape again it takes them
+    anns[1].set_tuning(4, 64, 1)
+    lnl, _, _, _ = batch.evaluate(0)
+    assert [f.loglikelihood(0) for f in fresh] == list(lnl)
     batch.close()
     for a in anns + fresh:
         a.close()
