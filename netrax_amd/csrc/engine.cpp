@@ -1486,10 +1486,12 @@ int nrx_create(const nrx_network_desc *net, const nrx_partition_desc *parts, int
     if (e->C != 1 && e->C != 2 && e->C != 4 && e->C != 8)
       throw std::invalid_argument("rate categories must be 1, 2, 4 or 8");
     const bool aa32 = e->opt.precision == NRX_FP32 && e->S == AA_STATES;
-    // P (and Q) of one partition are staged in LDS (64 KiB per workgroup)
+    // The range of the 4-state FP32 form: 64 KiB of P per partition (255 edges at
+    // 4 categories), from when its kernels held P in LDS.  They no longer do, but
+    // larger networks have not been tried in this form.
     if (e->opt.precision == NRX_FP32 && !aa32 &&
         sizeof(float) * (static_cast<size_t>(e->E) + 1) * e->C * 16 > 65536)
-      return fail(NRX_ERR_UNSUPPORTED, "network too large for the FP32 form's LDS tables");
+      return fail(NRX_ERR_UNSUPPORTED, "network too large for the FP32 form (64 KiB of P matrices per partition)");
     // site-sum partials per 64-site tile: one per wave
     e->pw = TILE * e->C / 64;
     e->rpw = e->pw;

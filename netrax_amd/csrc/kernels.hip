@@ -2907,16 +2907,15 @@ template <int S, typename T>
 __device__ __forceinline__ int scl_count(int32_t word) {
   return std::is_same<T, double>::value ? word >> 1 : word_k(word);
 }
-// a thread's row in a CLV slot of either form (FP32 rows are kept whole)
+// a thread's row in a CLV slot of either form (FP32, 4 states: rows are kept whole)
 template <int S, int C, typename T>
 __device__ __forceinline__ size_t clv_row(int64_t site, int c) {
   if constexpr (std::is_same<T, double>::value) {
     return row_offset<S, C>(site, c);
-  } else if constexpr (S == 4) {
+  } else {
+    static_assert(S == 4, "branch derivatives of 20 states are of the FP64 form");
     constexpr int SPB = Rows<C, 1>::SPB;
     return static_cast<size_t>(site / SPB * 64 + Rows<C, 1>::lane_of(static_cast<int>(site % SPB), c)) * 4;
-  } else {
-    return static_cast<size_t>(site * C + c) * S;
   }
 }
 
@@ -3939,12 +3938,15 @@ void launch_sumtables(Engine &e, int n_paths, int max_steps) {
     constexpr int S = decltype(s)::value, C = decltype(c)::value;
     using TT = typename TipType<S>::type;
     if (e.opt.precision == NRX_FP32) {
-      hipLaunchKernelGGL((k_sumtables<S, C, float>), dim3(e.L.n_tiles, n_paths), dim3(TILE * C), lds,
-                         e.stream, e.d_steps.as<PathStep>(), e.d_path_begin.as<int32_t>(), n_paths,
-                         e.L, e.d_tile_part.as<int32_t>(),
-                         e.d_clv.as<float>(), e.d_scl.as<int32_t>(), 1, e.d_tips.as<TT>(),
-                         e.d_P.as<double>(), e.d_V.as<double>(), e.d_Vinv.as<double>(),
-                         e.d_freqs.as<double>(), e.d_st.as<double>());
+      if constexpr (S == 4)
+        hipLaunchKernelGGL((k_sumtables<S, C, float>), dim3(e.L.n_tiles, n_paths), dim3(TILE * C), lds,
+                           e.stream, e.d_steps.as<PathStep>(), e.d_path_begin.as<int32_t>(), n_paths,
+                           e.L, e.d_tile_part.as<int32_t>(),
+                           e.d_clv.as<float>(), e.d_scl.as<int32_t>(), 1, e.d_tips.as<TT>(),
+                           e.d_P.as<double>(), e.d_V.as<double>(), e.d_Vinv.as<double>(),
+                           e.d_freqs.as<double>(), e.d_st.as<double>());
+      else
+        throw std::logic_error("sumtables of 20 states are of the FP64 form");
     } else {
       // (4 states: see the kernel)
       const dim3 grid = S == 4 ? dim3((e.L.n_tiles + 7) / 8 * 8 * n_paths) : dim3(e.L.n_tiles, n_paths);
@@ -4004,19 +4006,23 @@ void launch_deriv_fused(Engine &e, const PathStep *steps, const int32_t *path_be
   dispatch_sc(e.S, e.C, [&](auto s, auto c) {
     constexpr int S = decltype(s)::value, C = decltype(c)::value;
     using TT = typename TipType<S>::type;
-    if (e.opt.precision == NRX_FP32)
-      hipLaunchKernelGGL((k_deriv_fused<S, C, float>), dim3(e.L.n_tiles), dim3(TILE * C), lds, e.stream, steps,
-                         path_begin, n_paths, e.L, e.d_tile_part.as<int32_t>(), e.d_clv.as<float>(),
-                         e.d_scl.as<int32_t>(), 1, e.d_tips.as<TT>(), e.d_P.as<double>(), e.d_V.as<double>(),
-                         e.d_Vinv.as<double>(), e.d_freqs.as<double>(), e.d_eval.as<double>(),
-                         e.d_rates.as<double>(), e.d_weights.as<double>(), brlen, partials);
-    else
-      hipLaunchKernelGGL((k_deriv_fused<S, C, double>), dim3(e.L.n_tiles), dim3(TILE * C), S == 4 ? 0 : lds, e.stream, steps,
-                         path_begin, n_paths, e.L, e.d_tile_part.as<int32_t>(),
+    if (e.opt.precision == NRX_FP32) {
+      if constexpr (S == 4)
+        hipLaunchKernelGGL((k_deriv_fused<S, C, float>), dim3(e.L.n_tiles), dim3(TILE * C), lds, e.stream, steps,
+                           path_begin, n_paths, e.L, e.d_tile_part.as<int32_t>(), e.d_clv.as<float>(),
+                           e.d_scl.as<int32_t>(), 1, e.d_tips.as<TT>(), e.d_P.as<double>(), e.d_V.as<double>(),
+                           e.d_Vinv.as<double>(), e.d_freqs.as<double>(), e.d_eval.as<double>(),
+                           e.d_rates.as<double>(), e.d_weights.as<double>(), brlen, partials);
+      else
+        throw std::logic_error("branch derivatives of 20 states are of the FP64 form");
+    } else {
+      hipLaunchKernelGGL((k_deriv_fused<S, C, double>), dim3(e.L.n_tiles), dim3(TILE * C), S == 4 ? 0 : lds, e.stream,
+                         steps, path_begin, n_paths, e.L, e.d_tile_part.as<int32_t>(),
                          e.d_clv.as<double>(), e.d_scl.as<int32_t>(), 256, e.d_tips.as<TT>(),
                          e.d_P.as<double>(), e.d_V.as<double>(), e.d_Vinv.as<double>(), e.d_freqs.as<double>(),
                          e.d_eval.as<double>(), e.d_rates.as<double>(), e.d_weights.as<double>(), brlen,
                          partials);
+    }
   });
   NRX_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_reduce_segments, dim3(n_paths * 3 * e.P), dim3(256), 0, e.stream, partials,
