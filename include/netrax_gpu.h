@@ -57,9 +57,9 @@ extern "C" {
 
 /* arithmetic of the CLV products */
 #define NRX_FP64 0 /* plain form: FP64 CLVs; one forward and one reverse-sweep
-                      launch walking the pruning levels per site tile */
+                      launch walking every op, depth first */
 #define NRX_FP32 1 /* batched form: FP32 CLVs + per-site power-of-two
-                      exponents, persistent site-tile kernels, FP64 sums */
+                      exponents, the same walks, FP64 sums */
 
 /* branch-derivative normalisation for nrx_brlen_derivatives */
 #define NRX_DERIV_REFERENCE 0 /* sums over trees containing the branch only
@@ -270,8 +270,9 @@ int nrx_get_stats(nrx_engine *eng, nrx_stats *out);
  * categories on the same device, must outlive the batch and may appear
  * only once in it (a repeated engine is refused: NRX_ERR_ARG).  With
  * use_graph set on the first engine, the whole batch evaluation (P matrices,
- * persistent forward, reductions, mixture, persistent adjoint, gradient
- * totals, result gather) is one hipGraph launch. */
+ * forward, reductions, mixture, adjoint, gradient totals, result gather) is
+ * one hipGraph launch.  The batch has op lists and a launch shape of its own;
+ * its engines, scored alone, keep theirs. */
 typedef struct nrx_batch nrx_batch;
 
 int nrx_batch_create(nrx_engine *const *engines, int32_t n_engines, nrx_batch **out);
@@ -302,7 +303,7 @@ int nrx_batch_optimize(nrx_batch *batch, int32_t variant, int32_t mode, const in
 
 /* Memory budget of the FP64 form: bytes for the CLV, adjoint and scaler
  * rows (0: every CLV resident, the default).  Under a budget smaller than
- * the resident rows the level schedule is cut into segments; CLVs read by
+ * the resident rows the op list is cut into segments; CLVs read by
  * a later segment keep their rows and each segment's other CLVs share a
  * pool, so the forward pass keeps only those and the reverse sweep
  * recomputes each segment's pooled CLVs before its adjoint (at most one
@@ -326,16 +327,15 @@ int nrx_memory_plan(nrx_engine *eng, nrx_memory_plan_info *out);
 /* Device timing of the last evaluation (zeros unless timing is enabled). */
 int nrx_last_timing(nrx_engine *eng, nrx_timing *out);
 
-/* Shape of the FP32 form's persistent kernels.  No counterpart in the
- * reference (libpll's kernels have no launch shape); the autotuner picks
- * it per engine.  4-state data: group_width (2, 3, 4 or 8) independent ops
- * per group, whose CLV loads are issued together, tile_sites (16, 32
- * or 64, with tile_sites * rate_cats a multiple of 64) sites per
- * workgroup, i.e. tile_sites * rate_cats / 64 wavefronts per site block,
- * and row_lanes (1 or 2) lanes per (site, category) row of 4 states in the
- * reverse sweep (2: each lane holds two states, twice the wavefronts).
- * 20-state data: group_width 1, 2 or 4, 32 sites per workgroup (one
- * matrix-instruction column block) and row_lanes 1. */
+/* Shape of the FP32 form's kernels.  No counterpart in the reference
+ * (libpll's kernels have no launch shape); the autotuner picks it per
+ * engine.  4-state data: group_width 2 puts two blocks of 64 (site,
+ * category) rows on a wavefront, 3 one, 4 and 8 (and the default, 4) as
+ * many as the number of rows in the launch suggests, which for a batch is
+ * that of all its engines.  tile_sites (16, 32 or 64, with tile_sites *
+ * rate_cats a multiple of 64) and row_lanes (1 or 2), and all of a shape
+ * of 20-state data (group_width 1, 2 or 4, tile_sites 32, row_lanes 1), are
+ * accepted and reported as before, and choose nothing any more. */
 typedef struct {
   int32_t group_width;
   int32_t tile_sites;
@@ -344,7 +344,8 @@ typedef struct {
 } nrx_tuning;
 
 /* Times one lnL + gradient evaluation (best of `reps`) for every candidate
- * shape, keeps the fastest for the engine and returns it in *best;
+ * shape (once for those that run the same kernels), keeps the fastest for
+ * the engine (of equal ones the first) and returns it in *best;
  * results[0 .. min(max_results, *n_results)) (may be NULL) receive every
  * candidate's time.  Leaves the engine's CLVs recomputed. */
 int nrx_autotune(nrx_engine *eng, int32_t variant, int32_t reps, nrx_tuning *best,

@@ -176,9 +176,8 @@ static void resize_rows(Engine &e, size_t rows) {
   e.deriv_valid = false;
 }
 
-// Segments of the level schedule whose rows fit the memory budget: the
-// fewest segments (least recomputation) that fit, cut at level boundaries
-// with about equal op counts.  The reverse sweep then recomputes every
+// Segments of the op list whose rows fit the memory budget: the fewest
+// segments (least recomputation) that fit, with about equal op counts.  The reverse sweep then recomputes every
 // segment but the last one, at most one more forward pass.
 static void plan_budget(Engine &e) {
   auto &bp = e.bp;
@@ -277,9 +276,9 @@ static void plan_budget(Engine &e) {
 
 // Granules and LDS slots per wave of the FP64 walks.  4 states: four granules
 // share an op's fixed work best (41,345 patterns x 4 categories, gradient:
-// 0.66 ms, 0.92 with two, 1.00 with one); fewer once they would leave SIMDs
-// without a wave (8,719 patterns: 0.303 / 0.285 / 0.286 ms, 611 patterns, lnL:
-// 53.4 / 50.8 / 50.4 us).  As many slots as let the launch's waves, at most
+// 0.58 ms, 0.75 with two, 1.07 with one); fewer once they would leave SIMDs
+// without a wave (8,719 patterns, which take two: 0.208 / 0.205 / 0.220 ms; 611
+// patterns, which take one, lnL: 40.3 / 38.4 / 38.5 us).  As many slots as let the launch's waves, at most
 // three per SIMD (two in the 20-state reverse walk), be resident together.
 static void choose_walk_shape(Engine &e) {
   if (e.S == AA_STATES) {
@@ -300,9 +299,10 @@ static void choose_walk_shape(Engine &e) {
 
 // 64-row blocks per wave of the FP32 walks, `blocks` of them in a launch: two
 // share an op's fixed work once a launch fills the GPU either way (batch of 32
-// networks, 387,000 patterns, gradients: 2.41 ms against 2.86; 41,345 patterns:
-// 0.44 against 0.41, 1,294 waves leaving most SIMDs one).  Group widths 2 and
-// 3 of a tuned shape name two and one.
+// networks, 387,000 patterns, gradients: 2.16 ms against 2.61; 41,345 patterns:
+// 0.43 against 0.39, 1,294 waves leaving most SIMDs one).  Of a tuned shape's
+// group widths, 2 and 3 ask for two and for one (they are the kernels' template
+// arguments), the others leave the choice to this rule.
 static int walk_blocks_of(int tune_group, int64_t blocks) {
   if (tune_group == 2 || tune_group == 3) return tune_group == 2 ? 2 : 1;
   return blocks / 2 >= 8 * CUS ? 2 : 1;
@@ -339,8 +339,8 @@ static int lds_handoffs(const DevOp *ops, size_t n) {
   return h;
 }
 
-// Builds the level schedule, the batched order, root CLV set and gradient
-// rows for the classes that pass the log-probability cut, and uploads them.
+// Builds the walks' op lists, root CLV set and gradient rows for the classes
+// that pass the log-probability cut, and uploads them.
 static void build_schedule(Engine &e) {
   const int nv = static_cast<int>(e.dag.var.size());
   const int nc = static_cast<int>(e.dag.classes.size());
@@ -467,7 +467,7 @@ static void build_schedule(Engine &e) {
 }
 
 
-// Device descriptor of this engine for the persistent kernels (FP32 form).
+// Device descriptor of this engine for the walks of the FP32 form.
 NetDesc make_netdesc(const Engine &e) {
   NetDesc d{};
   d.L = e.L;
@@ -494,7 +494,7 @@ NetDesc make_netdesc(const Engine &e) {
   d.beta = e.d_beta.as<double>();
   d.root_partials = e.d_root_partials.as<double>();
   d.grad_partials = e.d_grad_partials.as<double>();
-  // every buffer the persistent kernels read must exist before its address
+  // every buffer that the walks read must exist before its address
   // is handed to the device
   const bool aa = e.S == AA_STATES;
   const void *need[] = {d.ops_fwd, d.ops_adj, d.clv, d.scl, d.adj, d.adj_exp, d.tips, aa ? d.Pa : d.Pf,
@@ -877,7 +877,7 @@ static int evaluate(Engine &e, int variant, bool incremental, bool update_pm, bo
   double *host = host_results(e, fetch || graphed);
   bool results_copied = false;
   if (e.opt.precision == NRX_FP32) {
-    // batched form: the op list in one persistent launch, root site sums
+    // batched form: the op list in one launch, root site sums
     // fused into it.  A full evaluation recomputes every CLV (one captured
     // graph with use_graph); an incremental one with some CLVs still valid
     // runs the invalid ops only, through a descriptor of their own, eagerly
@@ -1492,7 +1492,7 @@ int nrx_create(const nrx_network_desc *net, const nrx_partition_desc *parts, int
     if (e->opt.precision == NRX_FP32 && !aa32 &&
         sizeof(float) * (static_cast<size_t>(e->E) + 1) * e->C * 16 > 65536)
       return fail(NRX_ERR_UNSUPPORTED, "network too large for the FP32 form (64 KiB of P matrices per partition)");
-    // site-sum partials per 64-site tile: one per wave
+    // site-sum partials per 64-site tile of the branch derivatives: one per wave
     e->pw = TILE * e->C / 64;
     e->rpw = e->pw;
     e->parts.resize(n_parts);
@@ -2373,9 +2373,11 @@ int nrx_batch_optimize(nrx_batch *batch, int32_t variant, int32_t mode, const in
 
 namespace nrx {
 
-// Shapes of the FP32 form's kernels.  For 4-state data g chooses the row
-// blocks of a wave (walk_blocks_of); ts and h, and all of a shape of 20-state
-// data, are part of its name and choose nothing.
+// Shapes of the FP32 form's kernels, named as when they were groups of ops (g) on
+// tiles of sites (ts) with lanes per row (h), so that shapes that callers keep
+// stay valid.  For 4-state data g chooses the row blocks of a wave
+// (walk_blocks_of); ts and h, and all of a shape of 20-state data, choose
+// nothing.
 struct Shape {
   int g, ts, h;
   bool operator==(const Shape &o) const { return g == o.g && ts == o.ts && h == o.h; }

@@ -11,8 +11,8 @@
 
 namespace nrx {
 
-// Sites of every partition are padded to a multiple of this tile; one tile
-// is the unit of work of every site-parallel kernel.
+// Sites of every partition are padded to a multiple of this tile, so that a
+// wave's sites are of one partition.
 constexpr int TILE = 64;
 constexpr int MAX_CATS = 8;
 
@@ -81,43 +81,42 @@ struct DevOp {
   int32_t root;      // index of the root-CLV site sum this op feeds, or -1
   int32_t flags;     // OP_HAS_CONSUMERS | OP_FIRST_KID0 | OP_FIRST_KID1
   int32_t gslot[2];  // gradient-partial row of (this op, child k)
-  int32_t slots;     // 4-state walks: LDS slots of the uses 0, 1 (children) and 2 (own row), see walk_slot
+  int32_t slots;     // LDS slots of the uses 0, 1 (children) and 2 (own row), see walk_slot
   int32_t pad;
 };
 inline __host__ __device__ int walk_slot(const DevOp &op, int u) { return (op.slots >> (8 * u)) & 255; }
 constexpr int32_t OP_HAS_CONSUMERS = 1;  // adjoint of `out` was accumulated by consumers
 constexpr int32_t OP_FIRST_KID0 = 2;     // first consumer of kid[0] in adjoint order
 constexpr int32_t OP_FIRST_KID1 = 4;
-// FP32 form, first op of a group: no op of the group consumes a CLV of the
-// group before it, so a kernel may load this group's inputs before the
-// previous group's stores (and, walking backwards, load the previous
-// group's inputs before this group delivers)
-constexpr int32_t OP_GROUP_INDEP = 8;
-// FP32 form: child k's adjoint already holds deliveries made in earlier
-// groups of the reverse sweep and none in this group, so the accumulated
-// value may be loaded with the group's other inputs (the kernels issue a
-// group's loads after the previous group's stores)
-constexpr int32_t OP_ACC_EARLY0 = 16;
-constexpr int32_t OP_ACC_EARLY1 = 32;
-// FP32 form, 4 states: a child whose adjoint lives in a per-thread LDS slot
-// instead of HBM.  OP_PASS_KIDk: deliver child k's adjoint to slot
-// pass_slot(flags, k) (written by the first delivery, added to by later
-// ones); OP_A_PASS: this op's own adjoint is in slot pass_slot(flags, 2)
+// A row that a walk hands over in an LDS slot of the wave (DevOp::slots) instead
+// of HBM.  Forward: OP_A_PASS, the op leaves its CLV in slot walk_slot(op, 2);
+// OP_PASS_KIDk, child k is read from slot walk_slot(op, k).  Reverse:
+// OP_PASS_KIDk, child k's adjoint is delivered to slot walk_slot(op, k) (written
+// by the first delivery, added to by later ones); OP_A_PASS, the op's own
+// adjoint is in slot walk_slot(op, 2).
 constexpr int32_t OP_PASS_KID0 = 64;
 constexpr int32_t OP_PASS_KID1 = 128;
 constexpr int32_t OP_A_PASS = 256;
-// 4-state walks (OP_PASS_* and OP_A_PASS name slots of DevOp::slots): the op's own adjoint lies in HBM and the op before it
-// in the sweep delivered to it last, so it is read after that delivery
-// instead of one op ahead
+// reverse: the op's own adjoint lies in HBM and the op before it in the sweep
+// delivered to it last, so it is read after that delivery instead of one op
+// ahead
 constexpr int32_t OP_A_LATE = 512;
-// 4-state walks: child k's adjoint lies in HBM and holds deliveries
+// reverse: child k's adjoint lies in HBM and holds deliveries
 constexpr int32_t OP_ACC0 = 1024;
 constexpr int32_t OP_ACC1 = 2048;
-// 4-state walks, forward: child k's CLV is read from HBM
+// forward: child k's CLV is read from HBM
 constexpr int32_t OP_LOAD0 = 1 << 21;
 constexpr int32_t OP_LOAD1 = 1 << 22;
 constexpr int WALK_SLOTS = 32;  // LDS slots of a wave, at most
-constexpr int PASS_SLOTS = 5;  // at most; fewer where LDS would cost residency
+// Of the order in groups of independent ops that no kernel walks any more
+// (build_batched_order, set_acc_early and set_pass_slots in schedule.hpp):
+// the first op of a group that consumes no CLV of the group before it; child
+// k's adjoint holds deliveries of earlier groups only; slots in the flags,
+// where OP_PASS_* and OP_A_PASS stand for those.
+constexpr int32_t OP_GROUP_INDEP = 8;
+constexpr int32_t OP_ACC_EARLY0 = 16;
+constexpr int32_t OP_ACC_EARLY1 = 32;
+constexpr int PASS_SLOTS = 5;
 constexpr int PASS_SHIFT = 12;  // slot of use u (0, 1: children, 2: own) in bits 12 + 3u
 constexpr int32_t PASS_BITS = 0x1FF << PASS_SHIFT;
 inline __host__ __device__ int pass_slot(int32_t flags, int u) { return (flags >> (PASS_SHIFT + 3 * u)) & 7; }
@@ -177,9 +176,8 @@ struct DevLayout {
   int32_t C;
 };
 
-// Device view of one FP32-form engine, read by the persistent kernels; a
-// launch walks a table of (network, tile) work items, so one launch can
-// score one network or a batch of them.
+// Device view of one FP32-form engine, read by the walks; a 4-state launch has a
+// table of (network, wave) work items, so it scores one network or a batch.
 struct NetDesc {
   DevLayout L;
   int32_t n_root;
@@ -207,7 +205,7 @@ struct NetDesc {
 
 struct WorkItem {
   int32_t net;
-  int32_t tile;
+  int32_t tile;  // the wave's sites, in the launch's blocks per wave
 };
 
 // Per-network parameters of the small kernels when a batch is scored.
@@ -229,7 +227,7 @@ struct SmallDesc {
   int32_t rl_total, rl_per_part, rl_root_logl, rl_tree_logl, rl_alpha, rl_dbrlen,
       rl_part_dbrlen, rl_dprob;
   int32_t pw;           // root partials per 64-site tile
-  int32_t gwpt, pad[2];  // gradient partials per 64-site tile: its waves
+  int32_t gwpt, pad[2];  // gradient partials per 64-site tile: the launch's waves
 };
 
 struct Engine;

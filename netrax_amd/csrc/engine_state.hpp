@@ -78,9 +78,9 @@ struct Engine : nrx_engine {
   std::vector<LevelChunk> chunks;
   std::vector<int32_t> edge_use_begin, edge_use_list;  // gradient rows per edge
   int n_uses = 0;
-  int pw = 1;   // site-sum partials per tile (one per wave)
+  int pw = 1;   // branch derivatives: site-sum partials per tile (one per wave)
   int rpw = 1;  // root site-sum partials per tile
-  // 4-state walks: LDS slots per wave, and granules per wave (FP64)
+  // walks: granules per wave (FP64, 4 states), and LDS slots per wave
   int walk_nq = 4, fwd_slots = 4, adj_slots = 4;
   int walk_blocks = 1;  // 64-row blocks per wave (FP32)
   int gwpt = 1;  // gradient partials [wave][row]: waves per tile

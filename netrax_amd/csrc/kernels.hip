@@ -70,7 +70,7 @@ template <typename T>
 __device__ __forceinline__ GAS T *to_global(T *p) {
   return (GAS T *)p;
 }
-// Op tables and group bounds never change during a launch: read through
+// Op tables never change during a launch: read through
 // the constant address space they are fetched with scalar loads, whatever
 // stores the kernel makes in between.
 template <typename T>
@@ -144,11 +144,6 @@ __device__ __forceinline__ double cat_sum(double m) {
 // path with no pending load, so the compiler needs no conservative waits
 // before the next phase's loads.
 __device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
-// Load phases are bracketed by s_setprio 1 / s_setprio 0.  Measured 1-1.5 %
-// faster in the batched and plain passes; swapping the two priorities
-// measured the same, so the gain comes from the fixed instruction order the
-// pair imposes (the compiler moves nothing across an s_setprio), not from
-// the wave arbitration itself.
 
 __device__ __forceinline__ double readlane(double v, int lane) {
   return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
@@ -171,7 +166,6 @@ __device__ __forceinline__ double wave_sum(double v) {
   return readlane(v, 63);
 }
 
-// Deterministic workgroup sum; result valid in thread 0.
 // Sum over the 64 lanes, in every lane.
 __device__ __forceinline__ double lane_sum(double v) {
 #pragma unroll
@@ -211,6 +205,7 @@ __device__ __forceinline__ double block_sum_exact(Exact x) {
   return sum.value();
 }
 
+// Deterministic workgroup sum; result valid in thread 0.
 template <int NT>
 __device__ __forceinline__ double block_sum(double v, double *sh) {
   v = wave_sum(v);
@@ -738,8 +733,8 @@ struct FwdIn4 {
 
 // Scaler words: 2 x (rescalings below and at this CLV) + (rescaled here).
 //
-// Bound: HBM (a CLV written per op; 50 taxa, 41,345 patterns: 0.92 GB in 0.223
-// ms, 4.1 TB/s; a thread per row with P in LDS and CLVs through HBM took
+// Bound: HBM (a CLV written per op; 50 taxa, 41,345 patterns: 1.01 GB of traffic
+// in 0.222 ms, 4.5 TB/s; a thread per row with P in LDS and CLVs through HBM took
 // 0.311 + 0.023 ms for the root sums), or a wave's chain of ops for few sites.
 template <int S, int C, int NQ>
 __global__ void __launch_bounds__(64, 3)
@@ -925,16 +920,16 @@ struct AdjIn4 {
 };
 
 // Bound: HBM (every inner child's CLV once per use; 50 taxa, 41,345 patterns:
-// 1.6 GB in 0.363 ms, 4.5 TB/s; with P in LDS and every adjoint through HBM
-// 2.99 GB in 0.648 ms).
+// 1.67 GB of traffic in 0.317 ms, 5.3 TB/s, as a large copy; with P in LDS and
+// every adjoint through HBM 2.99 GB in 0.648 ms).
 //
 // MODEL: instead of the gradient's shares, per use, the sums over the wave's
 // sites of z x^T (dJ/dP), one entry per lane of a granule, and per root those of
 // the frequencies' direct share, f x with f = beta w / (C Ltilde) (r_part,
 // [root][wave][4]).  Both are products over sites: z and x are transposed by a
 // product with the identity, which is exact, and multiplied (41,345 patterns,
-// 138 ops: 0.44 ms against 0.32 without, and 0.08 for k_model_reduce; a pass of
-// its own over stored adjoints and CLVs took 0.85 ms, and storing the adjoints
+// 138 ops: 0.39 ms, the gradient's walk 0.32, and 0.08 for k_model_reduce; a pass
+// of its own over stored adjoints and CLVs took 0.85 ms, and storing the adjoints
 // 0.10).  The sums of
 // child k go to [k][NA][64] of the wave's part of the op's own adjoint row: no
 // one reads that any more, it holds both (NQ >= 2 NA), and they take no memory
@@ -1239,11 +1234,10 @@ struct FwdIn20 {
 // Workgroup: 16 sites, a wave per category; scaler words as in
 // k_forward_walk.  Per op the waves trade which of their sites are small
 // (and at a root the categories' likelihoods) through LDS, with one barrier.
-// Bound: each wave's chain of ops, the matrix cores busy two fifths of the
-// time (18,564 patterns x 4 categories, 73 ops: 0.40 ms, 0.45 with both
-// matrices an op ahead at two waves per SIMD; 0.72 in ten launches of a
-// thread per row and category with P in scalar registers, whose FMAs wait for
-// every row of it).
+// Bound: each wave's chain of ops, the matrix cores busy 27 % of the time (18,564
+// patterns x 4 categories, 73 ops: 0.40 ms, 0.45 with both matrices an op ahead
+// at two waves per SIMD; 0.72 in ten launches of a thread per row and category
+// with P in scalar registers, whose FMAs wait for every row of it).
 template <int C>
 __global__ void __launch_bounds__(64 * C, 3)
     k_forward_level_aa(const DevOp *__restrict__ ops_, int n_ops, int n_slots, DevLayout L, double *__restrict__ clv_,
@@ -1409,9 +1403,9 @@ struct AdjIn20 {
 // The reverse sweep of k_adjoint_level at 20 states.  A workgroup is one wave
 // (a category of 16 sites; nothing crosses the categories), categories in the
 // grid's slow direction, so that waves running together read the same tables.
-// Bound: as the forward walk, at two waves per SIMD (18,564 patterns x 4
-// categories: 0.75 ms; 1.79 in 18 launches of a thread per row, with every
-// adjoint through HBM).
+// Bound: as the forward walk, at two waves per SIMD, the matrix cores busy 38 %
+// (18,564 patterns x 4 categories: 0.75 ms; 1.79 in 18 launches of a thread per
+// row, with every adjoint through HBM).
 template <int C>
 __global__ void __launch_bounds__(64, 2)
     k_adjoint_level_aa(const DevOp *__restrict__ ops_, int n_ops, int n_slots, DevLayout L,
@@ -2536,8 +2530,8 @@ struct FwdIn20f {
 };
 
 // Workgroup: 16 sites, a wave per category, as k_forward_level_aa.
-// Bound: each wave's chain of ops (18,564 patterns x 4 categories, 73 ops:
-// 0.24 ms; 0.35 with 32-site waves of v_mfma_f32_32x32x2, whose 12 of 32 rows
+// Bound: each wave's chain of ops, the matrix cores busy 36 % of the time, here and
+// in the reverse walk (18,564 patterns x 4 categories, 73 ops: 0.24 ms; 0.35 with 32-site waves of v_mfma_f32_32x32x2, whose 12 of 32 rows
 // are padding, a group of four ops at a time and every CLV through HBM).
 template <int C, int G>
 __global__ void __launch_bounds__(64 * C, 4)
@@ -3698,7 +3692,7 @@ __global__ void __launch_bounds__(256) k_grad_total_multi(const SmallDesc *__res
                   d.res + d.rl_dbrlen, nullptr, nullptr);
 }
 
-// Copies every network's result block next to each other for one D2H copy.
+// Puts every network's result block next to each other into pinned host memory.
 __global__ void k_gather_results(const SmallDesc *__restrict__ descs,
                                  const int64_t *__restrict__ offsets, double *__restrict__ out) {
   const SmallDesc &d = descs[blockIdx.y];

@@ -316,10 +316,10 @@ class AnnotatedNetwork:
         return t
 
     def autotune(self, variant: Optional[int] = None, reps: int = 3):
-        """FP32 form: times every kernel shape (ops per group, sites per
-        workgroup, lanes per row in the reverse sweep), keeps the fastest;
-        returns (best, [all candidates]) as (group_width, tile_sites,
-        row_lanes, ms) tuples."""
+        """FP32 form: times every kernel shape (nrx_autotune; of 4-state data
+        group_width 2 means two row blocks per wave, 3 one, others as many as
+        the size suggests), keeps the fastest; returns (best, [all
+        candidates]) as (group_width, tile_sites, row_lanes, ms) tuples."""
         v = int(self.options.likelihood_variant if variant is None else variant)
         best = _lib.Tuning()
         res = (_lib.Tuning * 64)()
