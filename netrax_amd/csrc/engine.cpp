@@ -530,21 +530,30 @@ static void upload_classes_only(Engine &e) {
 }
 
 static void set_probs(Engine &e, const double *p) {
-  for (int r = 0; r < e.R; ++r) {
+  for (int r = 0; r < e.R; ++r)
     if (!(p[r] > 0.0 && p[r] < 1.0))
       throw std::invalid_argument("reticulation probabilities must lie in (0, 1)");
-    e.probs[r] = p[r];
-  }
+  const std::vector<double> old_probs = e.probs;
   const std::vector<char> old_use = e.class_use;
+  std::copy(p, p + e.R, e.probs.begin());
   compute_class_probs(e);
+  e.probs_dirty = true;
   if (old_use != e.class_use) {
     e.deriv_valid = false;
-    build_schedule(e);
     std::fill(e.clv_dirty.begin(), e.clv_dirty.end(), 1);
+    try {
+      build_schedule(e);
+    } catch (...) {
+      // (the rows of the trees that count now exceed the memory budget: the
+      // engine keeps the probabilities and the schedule that it had)
+      e.probs = old_probs;
+      compute_class_probs(e);
+      build_schedule(e);
+      throw;
+    }
   } else {
     upload_classes_only(e);
   }
-  e.probs_dirty = true;
 }
 
 static void mark_clv_dirty_for_edges(Engine &e) {
